@@ -1005,6 +1005,12 @@ k_dot_part(int n, const double *__restrict__ x, const double *__restrict__ y,
   block_sum_store(acc, part + blockIdx.x);
 }
 
+// y = x, any length and alignment
+__global__ void k_copy1(size_t n, const double *__restrict__ x, double *__restrict__ y) {
+  const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
+  if (i < n) y[i] = x[i];
+}
+
 // y = x over n2 16-byte pairs (a plain copy: reference kernel for bandwidth
 // and for calibrating hardware byte counters)
 __global__ void k_copy2(size_t n2, const double2 *__restrict__ x, double2 *__restrict__ y) {
@@ -2088,8 +2094,13 @@ void reduce_partials(const double *part, int nblk, int ncol, double *out,
 }
 
 void copy_f64(size_t n, const double *x, double *y, hipStream_t s) {
+  if (n == 0) return;
+  // pairs only where both ends are 16-byte aligned and no element is left
+  // over: columns of an odd length follow each other at 8-byte alignment
   const size_t n2 = n / 2;
-  if (n2)
+  if (n % 2 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15))
+    hipLaunchKernelGGL(k_copy1, dim3(grid_for(n)), dim3(kThreads), 0, s, n, x, y);
+  else
     hipLaunchKernelGGL(k_copy2, dim3(grid_for(n2)), dim3(kThreads), 0, s, n2,
                        reinterpret_cast<const double2 *>(x), reinterpret_cast<double2 *>(y));
 }

@@ -127,6 +127,35 @@ def test_chebav_generalized_matches_oracle(lib, bsol):
         g.close()
 
 
+@pytest.mark.parametrize("grid", [(5, 7, 3), (9, 3, 1), (3, 1, 1)])
+def test_chebav_generalized_odd_order(lib, grid):
+    """Odd orders: the work columns follow each other at odd offsets, and the
+    last element of every vector takes part (two calls on other vectors, so
+    that the work columns hold an earlier call's values)."""
+    banner("generalized ChebAv, odd order %d x %d x %d" % grid)
+    g = Gen(lib, *grid, "lspol")
+    assert g.n % 2 == 1
+    try:
+        for seed in (3, 4):
+            intv = [1.5, 2.5, 0.0, 6.0]
+            pol, rc = driver.find_pol(lib, intv)
+            assert rc == 0
+            v = np.random.default_rng(seed).uniform(-1.0, 1.0, g.n)
+            y = np.zeros(g.n)
+            pv = [capi.Parvec() for _ in range(3)]
+            for q, arr in zip(pv, (v, y, y)):
+                lib.pEVSL_ParvecCreateShell(g.n, g.n, 0, 0, C.byref(q),
+                                            arr.ctypes.data_as(capi.c_double_p))
+            assert lib.pEVSL_ChebAv(g.inst.p, C.byref(pol), *[C.byref(q) for q in pv]) == 0
+            mu = driver.pol_mu(pol)
+            ref = go.cheb_av_gen(g.A, g.solveB, mu, pol.cc, pol.dd, v)
+            lib.pEVSL_FreePol(C.byref(pol))
+            # the same series in FP64 on both sides, as above
+            assert np.linalg.norm(y - ref) < 1e-11 * np.linalg.norm(ref)
+    finally:
+        g.close()
+
+
 def test_kpm_generalized_matches_oracle(lib):
     banner("generalized KPM 8^3, exact B-solve, LSPol L^T solve")
     g = Gen(lib, 8, 8, 8, "host")
