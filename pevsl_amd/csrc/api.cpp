@@ -120,20 +120,10 @@ double KernTimers::seconds_matching(const char *prefix) {
   return t;
 }
 
-// about three nonzeros per lane (measured best for 7-point stencils: 2)
-int auto_lanes(double mean_row) {
-  int L = 1;
-  while (L < 64 && 2 * L <= mean_row / 3.0) L *= 2;
-  return L;
-}
-
 void apply_A(Ctx &c, const double *dx, double *dy) {
   if (c.stats) c.stats->n_mvA++;
   if (c.A) {
-    const int lanes =
-        c.lanes ? c.lanes
-                : auto_lanes(c.A->n ? (double)c.A->nnz / c.A->n : 1.0);
-    spmv_f64(*c.A, dx, dy, lanes, c.stream);
+    spmv_f64(*c.A, dx, dy, c.spmv_lanes(), c.stream);
     return;
   }
   if (!c.host_mv) fatal("matrix A not set", __FILE__, __LINE__);
@@ -296,7 +286,7 @@ int pEVSL_SetAParcsr(pevsl_Data *p, pevsl_Parcsr *A) {
   if (!c.A_src) fatal("SetAParcsr: matrix has no device copy (ParcsrSetup not called)",
                       __FILE__, __LINE__);
   c.A_view = *c.A_src;
-  if (!c.col16) c.A_view.jo16 = nullptr;
+  c.A_view.use_offsets(c.col16);
   c.A = &c.A_view;
   c.host_mv = nullptr;
   return 0;
@@ -396,7 +386,7 @@ int pEVSL_SetColumnOffsets16(pevsl_Data *p, int on) {
   c.col16 = on;
   if (c.A_src) {
     c.A_view = *c.A_src;
-    if (!on) c.A_view.jo16 = nullptr;
+    c.A_view.use_offsets(on);
   }
   return 0;
 }
@@ -533,6 +523,12 @@ int pEVSL_ParcsrSetup(pevsl_Csr *Ai, pevsl_Parcsr *A) {
   M->csr.nrowblk = (int)rb.size() - 1;
   M->csr.rowblk = M->rowblk.ensure(rb.size());
   PV_HIP(hipMemcpy(M->csr.rowblk, rb.data(), sizeof(int) * rb.size(), hipMemcpyHostToDevice));
+  {
+    std::vector<int> bz(rb.size());
+    for (size_t b = 0; b < rb.size(); b++) bz[b] = Ai->ia[rb[b]];
+    M->csr.blknz = M->blknz.ensure(bz.size());
+    PV_HIP(hipMemcpy(M->csr.blknz, bz.data(), sizeof(int) * bz.size(), hipMemcpyHostToDevice));
+  }
   // 16-bit column offsets from each row block's first row, kept when every
   // nonzero's offset fits (banded orderings such as the natural order of a
   // grid Laplacian; not random sparsity)
@@ -648,7 +644,7 @@ void pEVSL_ParcsrMatvec(pevsl_Parcsr *A, pevsl_Parvec *x, pevsl_Parvec *y) {
   double *d = nullptr;
   PV_HIP(hipMalloc(&d, sizeof(double) * ((size_t)n + (size_t)m + 1)));
   PV_HIP(hipMemcpy(d, x->data, sizeof(double) * (size_t)m, hipMemcpyHostToDevice));
-  spmv_f64(*M, d, d + m, auto_lanes(n ? (double)M->nnz / n : 1.0), 0);
+  spmv_f64(*M, d, d + m, 0, 0);
   PV_HIP(hipMemcpy(y->data, d + m, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost));
   PV_HIP(hipFree(d));
 }

@@ -430,7 +430,6 @@ int pEVSL_LanDosG(pevsl_Data *pevsl, const int nvec, int msteps, int npts, doubl
   std::vector<double> wn((size_t)nvec, 0.0);
   std::vector<int> nwn((size_t)nvec, 0);
   std::vector<double> ha((size_t)2 * nvec), betas((size_t)nvec);
-  const int lanes = c.lanes ? c.lanes : auto_lanes((double)c.A->nnz / std::max(1, n));
   const int msk = (1 << shift) - 1;
   (void)msk;
   for (int k = 0; k < maxit; k++) {
@@ -438,7 +437,6 @@ int pEVSL_LanDosG(pevsl_Data *pevsl, const int nvec, int msteps, int npts, doubl
       double *base = vt[(size_t)v];
       apply_A(c, base + (size_t)k * L.ld, base + (size_t)(k + 1) * L.ld);
     }
-    (void)lanes;
     lan_alpha(L, k, s);
     lan_subtract_alpha(L, k, s);
     lan_cgs_pass(L, k, 0, s);

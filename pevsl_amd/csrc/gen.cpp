@@ -54,15 +54,15 @@ void lspol_apply(const LSPolData &L, const double *dx, double *dy, double *wk, h
     scale_vec(n, dy, nullptr, mu[0], s);
     return;
   }
-  const int lanes = auto_lanes(n ? (double)B.nnz / n : 1.0);
   double *b[3] = {wk, wk + n, wk + 2 * (size_t)n};
   const double *vk = dx, *vkm1 = nullptr;
   int nb = 0;
+  YPlan yp;
   for (int k = 1; k <= m; k++) {
     double *vkp1 = b[nb];
     nb = (nb + 1) % 3;
-    cheb_step_vec<double>(B, vk, vkm1, vkp1, dy, L.cc, k == 1 ? 1.0 / L.dd : 2.0 / L.dd, mu[0],
-                          mu[k], k == 1, lanes, s);
+    cheb_step_stream<double>(B, vk, vkm1, vkp1, dy, L.cc, k == 1 ? 1.0 / L.dd : 2.0 / L.dd, mu[0],
+                             k > 2 ? mu[k - 2] : 0.0, mu[k - 1], mu[k], yp.next(k, m), s);
     vkm1 = vk;
     vk = vkp1;
   }
@@ -170,7 +170,7 @@ double ddot(Ctx &c, int n, const double *x, const double *y) {
 
 void apply_B(Ctx &c, pevsl_Data *p, const double *dx, double *dy) {
   if (c.B) {
-    spmv_f64(*c.B, dx, dy, auto_lanes(c.B->n ? (double)c.B->nnz / c.B->n : 1.0), c.stream);
+    spmv_f64(*c.B, dx, dy, 0, c.stream);
     return;
   }
   if (!p->Bmv || !p->Bmv->func) fatal("matrix B not set", __FILE__, __LINE__);

@@ -62,7 +62,7 @@ struct DBuf {
 // Device copy of a CSR matrix (attached to pevsl_Parcsr.dev).
 struct DevMatrix {
   DevCsr csr;
-  DBuf<int> ia, ja, rowblk;
+  DBuf<int> ia, ja, rowblk, blknz;
   DBuf<int> rowblk_q[5];  // partitions of the nnz-balanced kernels, Q >= 2
   DBuf<double> a64;
   DBuf<float> a32;
@@ -105,10 +105,6 @@ struct KernTimers {
   hipEvent_t take();
 };
 
-// Rows longer than this make the batched filter default to the nnz-balanced
-// block kernels.
-constexpr int kUnevenRow = 64;
-
 // Highest filter degree a batched FP32 group runs in Clenshaw form; above it
 // the group runs the three-term form (same vector passes with y updated every
 // other degree, smaller rounding error at high degree).
@@ -134,6 +130,8 @@ struct Ctx {
   unsigned long long rand_offset = 0;
   int lanes = 0;                   // lanes per row of the single-column SpMV
   int use_stream = -1;             // CSR-stream filter kernel: 1 yes, 0 no, -1 auto
+  // lanes argument of the products with A: the tuned vector-CSR kernel, or 0
+  int spmv_lanes() const { return use_stream == 0 ? lanes : 0; }
   int block_width = 0;             // columns per block SpMM (0 = auto)
   int blk_rowkernel = -1;          // block SpMM: 1 row-per-thread, 0 lane per (row, col), -1 auto
   int keep_vectors = 1;
@@ -159,9 +157,6 @@ struct Ctx {
 
 Ctx &ctx_of(pevsl_Data *p);
 const DevCsr *dev_matrix_of(pevsl_Parcsr *A);
-
-// lanes per row for a matrix with mean row length r (power of two, <= 64)
-int auto_lanes(double mean_row);
 
 // Wall-clock + device-event timing helper: measures the device time of the
 // work enqueued between start() and stop() on one stream.

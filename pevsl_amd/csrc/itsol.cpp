@@ -31,7 +31,7 @@ namespace {
 void bmv(const ChebIterData &C, const double *x, double *y, hipStream_t s) {
   const DevCsr *B = dev_matrix_of(C.Bp);
   if (!B) fatal("ChebIter: B has no device copy (pEVSL_ParcsrSetup)", __FILE__, __LINE__);
-  spmv_f64(*B, x, y, auto_lanes(B->n ? (double)B->nnz / B->n : 1.0), s);
+  spmv_f64(*B, x, y, 0, s);
 }
 
 // Templates form; x is left untouched when deg < 1 (chebiter.c:152-155)

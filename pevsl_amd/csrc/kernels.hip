@@ -41,9 +41,8 @@
 // deterministic for a given launch shape.  The filter kernels disable FMA
 // contraction so that, with one lane per row, each element follows the same
 // rounding sequence as the reference's scalar loops.
-#include "kernels.hpp"
+#include "dev.hpp"
 
-#include <hip/hip_runtime.h>
 #include <cfloat>
 #include <cmath>
 #include <algorithm>
@@ -53,7 +52,6 @@ namespace pevsl {
 
 namespace {
 
-constexpr int kThreads = 256;
 // MI355X Infinity Cache (memory-side last-level cache)
 constexpr double kInfinityCacheBytes = 256.0 * 1024 * 1024;
 
@@ -136,18 +134,6 @@ struct Row16<float> {
   }
 };
 
-// Row-block index of this workgroup such that each XCD works on one
-// contiguous range of row blocks.  Workgroups are dispatched to the 8 XCDs
-// round-robin (workgroup i to XCD i mod 8), and each XCD has its own L2: with
-// contiguous ranges the neighbour rows that a stencil-like matrix gathers
-// (+-1, +-nx, +-nx*ny) mostly sit in the same L2.  A bijection of [0, nb).
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_block(int bid, int nb) {
-  const int q = nb / kXcds, r = nb % kXcds;
-  const int x = bid % kXcds, j = bid / kXcds;
-  return x * q + min(x, r) + j;
-}
-
 // Column of nonzero j in a row block that starts at row r0: the 32-bit index,
 // or (J16) r0 plus the nonzero's 16-bit offset from r0 (DevCsr::jo16), which
 // saves 2 of the 4 index bytes per nonzero.
@@ -158,10 +144,6 @@ __device__ __forceinline__ int block_col(const int *__restrict__ ja, const short
     return r0 + (int)jo[j];
   else
     return ja[j];
-}
-
-inline int grid_for(size_t work, int threads = kThreads) {
-  return (int)((work + threads - 1) / threads);
 }
 
 // ---------------------------------------------------------------------------
@@ -227,69 +209,142 @@ k_cheb_vec(int n, const int *__restrict__ ia, const int *__restrict__ ja,
   }
 }
 
-// CSR-stream step: the block's nonzeros are multiplied with the gathered
-// x values in coalesced order and staged in LDS; each thread then sums one
-// row sequentially (the reference's summation order) and applies the
-// recurrence.  A row longer than kStreamNnz forms a block alone and is
-// reduced by the whole block.
+// LDS of a CSR-stream block: staged products (reused by the long row's
+// reduction) and the sums of its rows longer than kUnevenRow.
+template <typename T>
+struct StreamLds {
+  T prod[kStreamNnz];
+  T lsum[kStreamRows];
+};
+
+// Row sums of the CSR-stream row block [r0, r1) with nonzeros [j0, j0 + nz):
+// the block's nonzeros are multiplied with the gathered x values in coalesced
+// order and staged in LDS; thread threadIdx.x then sums row r0 + threadIdx.x,
+// entries [qs, qe), in column order (the reference's order) and returns it.
+//   * A row longer than kUnevenRow entries (uneven: the matrix has some) is
+//     summed by a wave instead, lanes 64 entries apart, the long rows of the
+//     block dealt to its waves in turn.  One thread walking a row of 2,000
+//     entries kept the whole block, and with it the launch, waiting: the
+//     power-law matrix of 1e5 rows took 87 us per FP64 filter step.
+//   * A row longer than kStreamNnz is a block alone, reduced by all threads;
+//     its sum is thread 0's.
+template <typename T, bool J16>
+__device__ __forceinline__ T stream_sum(StreamLds<T> &lds, int r0, int r1, int j0, int nz, int qs,
+                                        int qe, const int *__restrict__ ia,
+                                        const int *__restrict__ ja, const short *__restrict__ jo,
+                                        const T *__restrict__ a, const T *__restrict__ x,
+                                        int uneven) {
+#pragma clang fp contract(off)
+  T acc = 0;
+  if (nz > kStreamNnz) {
+    for (int q = threadIdx.x; q < nz; q += kThreads)
+      acc += a[j0 + q] * x[block_col<J16>(ja, jo, r0, j0 + q)];
+    lds.prod[threadIdx.x] = acc;
+    __syncthreads();
+    for (int w = kThreads / 2; w > 0; w >>= 1) {
+      if (threadIdx.x < w) lds.prod[threadIdx.x] += lds.prod[threadIdx.x + w];
+      __syncthreads();
+    }
+    return lds.prod[0];
+  }
+  for (int q = threadIdx.x; q < nz; q += kThreads)
+    lds.prod[q] = a[j0 + q] * x[block_col<J16>(ja, jo, r0, j0 + q)];
+  __syncthreads();
+  if (uneven) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int turn = 0;
+    for (int c0 = 0; c0 < r1 - r0; c0 += 64) {
+      int s = 0, e = 0;
+      if (c0 + lane < r1 - r0) {
+        s = ia[r0 + c0 + lane] - j0;
+        e = ia[r0 + c0 + lane + 1] - j0;
+      }
+      unsigned long long rows = __ballot(e - s > kUnevenRow);
+      while (rows) {
+        const int b = __ffsll((long long)rows) - 1;
+        rows &= rows - 1;
+        if ((turn++ & (kThreads / 64 - 1)) != wave) continue;
+        const int ss = __shfl(s, b, 64), ee = __shfl(e, b, 64);
+        T p = 0;
+        for (int q = ss + lane; q < ee; q += 64) p += lds.prod[q];
+        p = group_sum<64>(p);
+        if (lane == 0) lds.lsum[c0 + b] = p;
+      }
+    }
+    __syncthreads();
+    if (qe - qs > kUnevenRow) return lds.lsum[threadIdx.x];
+  }
+#pragma unroll 4
+  for (int q = qs; q < qe; q++) acc += lds.prod[q];
+  return acc;
+}
+
+// Block rb's rows and nonzeros: its bounds, and its entry of the offsets of
+// the blocks' first nonzeros, are independent loads.
+struct StreamBlock {
+  int rb, r0, r1, j0, nz;
+  __device__ StreamBlock(const int *__restrict__ rowblk, const int *__restrict__ blknz) {
+    rb = xcd_block(blockIdx.x, gridDim.x);
+    r0 = rowblk[rb];
+    r1 = rowblk[rb + 1];
+    j0 = blknz[rb];
+    nz = blknz[rb + 1] - j0;
+  }
+};
+
+// y = A x, CSR-stream form; column blockIdx.y of X and Y (leading dim ld)
+template <bool J16>
+__global__ void __launch_bounds__(kThreads)
+k_spmv_stream(const int *__restrict__ rowblk, const int *__restrict__ blknz,
+              const int *__restrict__ ia, const int *__restrict__ ja,
+              const short *__restrict__ jo, const double *__restrict__ a,
+              const double *__restrict__ x, double *__restrict__ y, size_t ld, int uneven) {
+  __shared__ StreamLds<double> lds;
+  const StreamBlock b(rowblk, blknz);
+  x += (size_t)blockIdx.y * ld;
+  y += (size_t)blockIdx.y * ld;
+  const int r = b.r0 + threadIdx.x;
+  int qs = 0, qe = 0;
+  if (r < b.r1) {
+    qs = ia[r] - b.j0;
+    qe = ia[r + 1] - b.j0;
+  }
+  const double acc = stream_sum<double, J16>(lds, b.r0, b.r1, b.j0, b.nz, qs, qe, ia, ja, jo, a,
+                                             x, uneven);
+  if (r < b.r1) y[r] = acc;
+}
+
+// CSR-stream step of the filter, one column
 template <typename T, bool J16>
 __global__ void __launch_bounds__(kThreads)
-k_cheb_stream(const int *__restrict__ rowblk, const int *__restrict__ ia,
-              const int *__restrict__ ja, const short *__restrict__ jo, const T *__restrict__ a,
-              const T *__restrict__ vk, const T *__restrict__ vkm1,
-              T *__restrict__ vkp1, T *__restrict__ y, T cc, T t, T mu0, T muk,
-              int first) {
+k_cheb_stream(const int *__restrict__ rowblk, const int *__restrict__ blknz,
+              const int *__restrict__ ia, const int *__restrict__ ja,
+              const short *__restrict__ jo, const T *__restrict__ a, const T *__restrict__ vk,
+              const T *__restrict__ vkm1, T *__restrict__ vkp1, T *__restrict__ y, T cc, T t, T m0,
+              T m3, T m2, T m1, int ymode, int uneven) {
 #pragma clang fp contract(off)
-  __shared__ T prod[kStreamNnz];
-  const int rb = xcd_block(blockIdx.x, gridDim.x);
-  const int r0 = rowblk[rb], r1 = rowblk[rb + 1];
-  const int j0 = ia[r0], nz = ia[r1] - j0;
-  T acc = 0;
-  int r = r0 + threadIdx.x;
+  __shared__ StreamLds<T> lds;
+  const StreamBlock b(rowblk, blknz);
+  const int r = b.r0 + threadIdx.x;
   // the row's own operands and row pointers are loaded before the gathers,
   // so that their latency overlaps the staging (100^3 Laplacian, 16-bit
   // offsets: FP32 15.56 against 16.27 us per step, FP64 19.66 against 19.69)
   T v = 0, vm = 0, yv = 0;
   int qs = 0, qe = 0;
-  if (r < r1) {
+  if (r < b.r1) {
     v = vk[r];
-    if (!first) {
-      vm = vkm1[r];
-      yv = y[r];
-    }
-    qs = ia[r] - j0;
-    qe = ia[r + 1] - j0;
+    if (vkm1) vm = vkm1[r];
+    if (ymode != kYSkip && !(ymode & kYInit)) yv = y[r];
+    qs = ia[r] - b.j0;
+    qe = ia[r + 1] - b.j0;
   }
-  if (nz <= kStreamNnz) {
-    for (int q = threadIdx.x; q < nz; q += kThreads)
-      prod[q] = a[j0 + q] * vk[block_col<J16>(ja, jo, r0, j0 + q)];
-    __syncthreads();
-    if (r >= r1) return;
-    for (int q = qs; q < qe; q++) acc += prod[q];
-  } else {
-    // single long row
-    for (int q = threadIdx.x; q < nz; q += kThreads)
-      acc += a[j0 + q] * vk[block_col<J16>(ja, jo, r0, j0 + q)];
-    __shared__ T red[kThreads];
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = kThreads / 2; w > 0; w >>= 1) {
-      if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x != 0) return;
-    acc = red[0];  // thread 0's operands are those of the block's one row r0
-  }
+  const T acc = stream_sum<T, J16>(lds, b.r0, b.r1, b.j0, b.nz, qs, qe, ia, ja, jo, a, vk, uneven);
+  if (r >= b.r1) return;
   T w = acc + (-cc) * v;
   w = w * t;
-  if (first) {
-    vkp1[r] = w;
-    y[r] = v * mu0 + muk * w;
-  } else {
-    w = w + (T)(-1) * vm;
-    vkp1[r] = w;
-    y[r] = yv + muk * w;
-  }
+  if (vkm1) w = w + (T)(-1) * vm;
+  vkp1[r] = w;
+  if (ymode != kYSkip) y[r] = y_next<T>(ymode, yv, vm, v, w, m0, m3, m2, m1);
 }
 
 // B interleaved columns; lane = (row_in_block, column).
@@ -321,6 +376,17 @@ k_cheb_blk(int n, const int *__restrict__ ia, const int *__restrict__ ja,
     vkp1[idx] = w;
     y[idx] = y[idx] + muk * w;
   }
+}
+
+// y_next of column c of an interleaved block: coefficients mus[d*B + c]
+template <typename T>
+__device__ __forceinline__ T y_col(int ymode, const double *mus, int k, int B, int c, T yv, T vm,
+                                   T v, T w) {
+  const int terms = ymode & 3;
+  const T m0 = (ymode & kYInit) ? (T)mus[c] : (T)0;
+  const T m3 = terms == 3 ? (T)mus[(size_t)(k - 2) * B + c] : (T)0;
+  const T m2 = terms >= 2 ? (T)mus[(size_t)(k - 1) * B + c] : (T)0;
+  return y_next<T>(ymode, yv, vm, v, w, m0, m3, m2, (T)mus[(size_t)k * B + c]);
 }
 
 // Row-per-thread block step for B interleaved columns: the row block's
@@ -420,32 +486,27 @@ k_cheb_blkrow(const int *__restrict__ rowblk, const int *__restrict__ ia,
   }
   T v[B], vm[B], yy[B], w[B];
   load_row<T, B>(vk + (size_t)r * B, v);
+  // with kYInit, columns >= nact still keep y
   if (ymode != kYSkip) load_row<T, B>(y + (size_t)r * B, yy);
-  if (k == 1) {
-#pragma unroll
-    for (int c = 0; c < B; c++) {
-      w[c] = acc[c] + (-cc) * v[c];
-      w[c] = w[c] * t;
-      if (c < nact) yy[c] = v[c] * (T)mus[c] + (T)mus[(size_t)B + c] * w[c];
-    }
-  } else {
+  if (vkm1) {
     load_row<T, B>(vkm1 + (size_t)r * B, vm);
+  } else {
 #pragma unroll
-    for (int c = 0; c < B; c++) {
-      w[c] = acc[c] + (-cc) * v[c];
-      w[c] = w[c] * t;
-      w[c] = w[c] + (T)(-1) * vm[c];
-      if (c < nact) {
-        // kYPair: the term of degree k-1 (v, this step's input) that the
-        // previous step skipped, then degree k: the two updates of two plain
-        // steps, in their order
-        if (ymode == kYPair) yy[c] = yy[c] + (T)mus[(size_t)(k - 1) * B + c] * v[c];
-        if (ymode != kYSkip) yy[c] = yy[c] + (T)mus[(size_t)k * B + c] * w[c];
-      }
-    }
+    for (int c = 0; c < B; c++) vm[c] = 0;
+  }
+#pragma unroll
+  for (int c = 0; c < B; c++) {
+    w[c] = acc[c] + (-cc) * v[c];
+    w[c] = w[c] * t;
+    if (vkm1) w[c] = w[c] + (T)(-1) * vm[c];
+  }
+  if (ymode != kYSkip) {
+#pragma unroll
+    for (int c = 0; c < B; c++)
+      if (c < nact) yy[c] = y_col<T>(ymode, mus, k, B, c, yy[c], vm[c], v[c], w[c]);
+    store_row<T, B>(y + (size_t)r * B, yy);
   }
   store_row<T, B>(vkp1 + (size_t)r * B, w);
-  if (ymode != kYSkip) store_row<T, B>(y + (size_t)r * B, yy);
 }
 
 // One Clenshaw step of the filter on B interleaved columns (row per thread,
@@ -632,39 +693,6 @@ __global__ void k_blk_colscale(size_t n, int B, const T *__restrict__ v, T *__re
 // by the whole workgroup (shuffles, then LDS across waves).  Products are
 // rounded before they are added and staged rows are summed in column order,
 // so those rows round exactly as in the row-per-thread kernels.
-//
-// Budget: NZ = kStreamNnz / Q staged products of B values (32 KiB of LDS when
-// a piece is 16 bytes) and at most kStreamRows / Q rows per block, Q = pieces
-// per row; the host builds one row partition per Q (DevCsr::rowblk_q).
-template <typename T, int B>
-struct Pieces {
-  static constexpr int P = (B * (int)sizeof(T) >= 16) ? 16 / (int)sizeof(T) : B;
-  static constexpr int Q = B / P;
-  static constexpr int NZ = kStreamNnz / Q;
-};
-
-template <typename T, int P>
-__device__ __forceinline__ void ld_piece(const T *p, T (&x)[P]) {
-  if constexpr (P * sizeof(T) == 16) {
-    *reinterpret_cast<float4 *>(x) = *reinterpret_cast<const float4 *>(p);
-  } else if constexpr (P * sizeof(T) == 8) {
-    *reinterpret_cast<float2 *>(x) = *reinterpret_cast<const float2 *>(p);
-  } else {
-#pragma unroll
-    for (int e = 0; e < P; e++) x[e] = p[e];
-  }
-}
-template <typename T, int P>
-__device__ __forceinline__ void st_piece(T *p, const T (&x)[P]) {
-  if constexpr (P * sizeof(T) == 16) {
-    *reinterpret_cast<float4 *>(p) = *reinterpret_cast<const float4 *>(x);
-  } else if constexpr (P * sizeof(T) == 8) {
-    *reinterpret_cast<float2 *>(p) = *reinterpret_cast<const float2 *>(x);
-  } else {
-#pragma unroll
-    for (int e = 0; e < P; e++) p[e] = x[e];
-  }
-}
 
 // Epilogue of the three-term step (same operations as k_cheb_blkrow) on
 // columns [piece*P, piece*P + P) of row r.
@@ -680,34 +708,30 @@ struct EpiCheb {
 #pragma clang fp contract(off)
     constexpr int P = Pieces<T, B>::P;
     const size_t o = (size_t)r * B + piece * P;
-    T v[P], yy[P], w[P];
+    T v[P], vm[P], yy[P], w[P];
     ld_piece<T, P>(vk + o, v);
     if (ymode != kYSkip) ld_piece<T, P>(y + o, yy);
-    if (k == 1) {
-#pragma unroll
-      for (int e = 0; e < P; e++) {
-        const int c = piece * P + e;
-        w[e] = acc[e] + (-cc) * v[e];
-        w[e] = w[e] * t;
-        if (c < nact) yy[e] = v[e] * (T)mus[c] + (T)mus[(size_t)B + c] * w[e];
-      }
-    } else {
-      T vm[P];
+    if (vkm1) {
       ld_piece<T, P>(vkm1 + o, vm);
+    } else {
+#pragma unroll
+      for (int e = 0; e < P; e++) vm[e] = 0;
+    }
+#pragma unroll
+    for (int e = 0; e < P; e++) {
+      w[e] = acc[e] + (-cc) * v[e];
+      w[e] = w[e] * t;
+      if (vkm1) w[e] = w[e] + (T)(-1) * vm[e];
+    }
+    if (ymode != kYSkip) {
 #pragma unroll
       for (int e = 0; e < P; e++) {
         const int c = piece * P + e;
-        w[e] = acc[e] + (-cc) * v[e];
-        w[e] = w[e] * t;
-        w[e] = w[e] + (T)(-1) * vm[e];
-        if (c < nact) {
-          if (ymode == kYPair) yy[e] = yy[e] + (T)mus[(size_t)(k - 1) * B + c] * v[e];
-          if (ymode != kYSkip) yy[e] = yy[e] + (T)mus[(size_t)k * B + c] * w[e];
-        }
+        if (c < nact) yy[e] = y_col<T>(ymode, mus, k, B, c, yy[e], vm[e], v[e], w[e]);
       }
+      st_piece<T, P>(y + o, yy);
     }
     st_piece<T, P>(vkp1 + o, w);
-    if (ymode != kYSkip) st_piece<T, P>(y + o, yy);
   }
 };
 
@@ -1732,9 +1756,39 @@ __global__ void k_rand(size_t n, double *__restrict__ x, uint64_t seed,
 // Launchers
 // ===========================================================================
 
+// lanes per row of the vector-CSR product: about three nonzeros per lane
+// (7-point stencils: 2 measured best)
+static int even_lanes(double mean_row) {
+  int L = 1;
+  while (L < 64 && 2 * L <= mean_row / 3.0) L *= 2;
+  return L;
+}
+
 void spmv_cols_f64(const DevCsr &A, const double *X, double *Y, int ncol,
                    size_t ld, int lanes, hipStream_t s) {
   if (A.n == 0 || ncol == 0) return;
+  if (lanes == 0) {
+    // One column on even rows and fewer than two row blocks per CU: the
+    // vector-CSR kernel, whose loads depend on each other over fewer stages
+    // and which has more blocks.  7-point stencil, whole call of one product,
+    // vector-CSR against CSR-stream: 20^3 13.5 / 14.7 us, 40^3 14.2 / 14.9,
+    // 50^3 (489 blocks) 15.3 / 15.2, 60^3 17.2 / 16.4, 100^3 38.8 / 27.8.
+    // Uneven rows (1e5, up to 2,000 entries): 90 / 33 us.
+    const bool stream = ncol > 1 || A.max_row > kUnevenRow || A.nrowblk >= 512;
+    if (!stream) lanes = even_lanes((double)A.nnz / A.n);
+    auto go = [&](auto kernel) {
+      if (A.nrowblk == 0) return;
+      hipLaunchKernelGGL(kernel, dim3(A.nrowblk, ncol), dim3(kThreads), 0, s, A.rowblk, A.blknz,
+                         A.ia, A.ja, A.jo16, A.a64, X, Y, ld, A.max_row > kUnevenRow ? 1 : 0);
+    };
+    if (stream) {
+      if (A.jo16)
+        go(k_spmv_stream<true>);
+      else
+        go(k_spmv_stream<false>);
+      return;
+    }
+  }
   dim3 grid(grid_for((size_t)A.n * lanes), ncol);
   switch (lanes) {
 #define CASE(L)                                                              \
@@ -1862,28 +1916,28 @@ template void clen_step_bal<float>(const DevCsr &, int, const float *, const flo
 
 template <typename T>
 void cheb_step_stream(const DevCsr &A, const T *vk, const T *vkm1, T *vkp1,
-                      T *y, double cc, double t, double mu0, double muk,
-                      bool first, hipStream_t s) {
+                      T *y, double cc, double t, double mu0, double mu3, double mu2, double mu1,
+                      int ymode, hipStream_t s) {
   if (A.n == 0 || A.nrowblk == 0) return;
   const T *a = std::is_same<T, double>::value ? (const T *)A.a64
                                               : (const T *)A.a32;
+  const int uneven = A.max_row > kUnevenRow;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(A.nrowblk), dim3(kThreads), 0, s, A.rowblk, A.blknz, A.ia,
+                       A.ja, A.jo16, a, vk, vkm1, vkp1, y, (T)cc, (T)t, (T)mu0, (T)mu3, (T)mu2,
+                       (T)mu1, ymode, uneven);
+  };
   if (A.jo16)
-    hipLaunchKernelGGL((k_cheb_stream<T, true>), dim3(A.nrowblk), dim3(kThreads), 0, s,
-                       A.rowblk, A.ia, A.ja, A.jo16, a, vk, vkm1, vkp1, y, (T)cc, (T)t,
-                       (T)mu0, (T)muk, first ? 1 : 0);
+    go(k_cheb_stream<T, true>);
   else
-    hipLaunchKernelGGL((k_cheb_stream<T, false>), dim3(A.nrowblk), dim3(kThreads), 0, s,
-                       A.rowblk, A.ia, A.ja, A.jo16, a, vk, vkm1, vkp1, y, (T)cc, (T)t,
-                       (T)mu0, (T)muk, first ? 1 : 0);
+    go(k_cheb_stream<T, false>);
 }
-template void cheb_step_stream<double>(const DevCsr &, const double *,
-                                       const double *, double *, double *,
-                                       double, double, double, double, bool,
-                                       hipStream_t);
-template void cheb_step_stream<float>(const DevCsr &, const float *,
-                                      const float *, float *, float *, double,
-                                      double, double, double, bool,
-                                      hipStream_t);
+template void cheb_step_stream<double>(const DevCsr &, const double *, const double *, double *,
+                                       double *, double, double, double, double, double, double,
+                                       int, hipStream_t);
+template void cheb_step_stream<float>(const DevCsr &, const float *, const float *, float *,
+                                      float *, double, double, double, double, double, double,
+                                      int, hipStream_t);
 
 template void cheb_step_vec<double>(const DevCsr &, const double *,
                                     const double *, double *, double *, double,

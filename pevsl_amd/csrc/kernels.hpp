@@ -21,6 +21,7 @@ struct DevCsr {
   // row blocks of the CSR-stream kernels: consecutive rows with at most
   // kStreamRows rows and kStreamNnz nonzeros (a longer row is a block alone)
   int *rowblk = nullptr;
+  int *blknz = nullptr;  // first nonzero of each row block, ia[rowblk[b]]
   int nrowblk = 0;
   // row blocks of the nnz-balanced block kernels, one partition per number
   // Q = 2^i of 16-byte pieces in a B-wide row: at most kStreamRows/Q rows and
@@ -31,10 +32,19 @@ struct DevCsr {
   // `rowblk` (null when an offset does not fit in a short): the CSR-stream
   // and row-per-thread block kernels then read 2 index bytes per nonzero
   short *jo16 = nullptr;
+  // on == 0: 32-bit column indices
+  void use_offsets(int on) {
+    if (on) return;
+    jo16 = nullptr;
+  }
 };
 
 // index bytes per nonzero read by the CSR-stream and row-block kernels
 inline int index_bytes(const DevCsr &A) { return A.jo16 ? 2 : 4; }
+
+// Rows longer than this are uneven: the CSR-stream kernels sum them by a wave,
+// and the batched filter defaults to the nnz-balanced block kernels.
+constexpr int kUnevenRow = 64;
 
 constexpr int kStreamRows = 256;
 constexpr int kStreamNnz = 2048;
@@ -46,7 +56,9 @@ void build_row_blocks(int n, const int *ia, std::vector<int> &blk,
                       int max_rows = kStreamRows, int max_nnz = kStreamNnz);
 
 // ---- sparse products -------------------------------------------------------
-// y = A x, one column.  lanes = lanes per row in {1,2,4,8,16,32,64}.
+// y = A x, one column.  lanes = lanes per row in {1,2,4,8,16,32,64}, or 0 for
+// the CSR-stream
+// or vector-CSR form by size.
 void spmv_f64(const DevCsr &A, const double *x, double *y, int lanes,
               hipStream_t s);
 // Y(:,c) = A X(:,c) for ncol column-major columns with leading dim ld.
@@ -61,13 +73,40 @@ void cheb_step_vec(const DevCsr &A, const T *vk, const T *vkm1, T *vkp1, T *y,
                    double cc, double t, double mu0, double muk, bool first,
                    int lanes, hipStream_t s);
 
-// Same step with the CSR-stream kernel (one block per row block: coalesced
-// products staged in LDS, then one sequential sum per row).
+// How a three-term step of degree d updates the accumulator y, whose term of
+// degree d is mu_d v_d (vk = v_{d-1}, vkm1 = v_{d-2}, vkp1 = v_d):
+//   kYSkip       y is neither read nor written: its term waits
+//   1, 2, 3      y += the terms of the last 1, 2 or 3 degrees, in order
+//   kYInit | 1   y = mu_0 v_0 + mu_1 v_1              (d == 1)
+//   kYInit | 2   y = mu_0 v_0 + mu_1 v_1 + mu_2 v_2   (d == 2, v_0 = vkm1)
+// A step holds v_{d-2}, v_{d-1} and v_d anyway, so y need pass through memory
+// only every third degree, with the results of one update per degree bit for
+// bit.  YPlan gives the modes of a run of degrees 1..m.
+constexpr int kYSkip = 0, kYInit = 4;
+struct YPlan {
+  int pend = 0;          // degrees whose terms wait
+  bool started = false;  // y holds the terms of the degrees before them
+  int next(int d, int m) {
+    pend++;
+    const bool flush = d == m || pend == (started ? 3 : 2);
+    if (!flush) return kYSkip;
+    const int mode = (started ? 0 : kYInit) | pend;
+    started = true;
+    pend = 0;
+    return mode;
+  }
+};
+// passes over y of a step: none, a write, or a read and a write
+inline int y_passes(int mode) { return mode == kYSkip ? 0 : (mode & kYInit) ? 1 : 2; }
+
+// Same step, y updated as `ymode` says (mu0, mu3, mu2, mu1: the coefficients
+// of degrees 0, d-2, d-1, d; vkm1 null at d == 1), with the CSR-stream
+// kernel (one block per row block: coalesced products staged in LDS, then one
+// sequential sum per row; rows longer than kUnevenRow by a wave).
 template <typename T>
 void cheb_step_stream(const DevCsr &A, const T *vk, const T *vkm1, T *vkp1,
-                      T *y, double cc, double t, double mu0, double muk,
-                      bool first, hipStream_t s);
-
+                      T *y, double cc, double t, double mu0, double mu3, double mu2, double mu1,
+                      int ymode, hipStream_t s);
 // Same for B interleaved columns (row-major n x B block, column fastest).
 // mus: device array [(deg_max+1) x B] of per-column coefficients; k = degree
 // index of this step (1..); columns c >= nact are left untouched.
@@ -76,23 +115,14 @@ void cheb_step_blk(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1,
                    T *y, double cc, double t, const double *mus, int k,
                    int nact, hipStream_t s);
 
-// y-update modes of the three-term block steps (cheb_step_blkrow,
-// cheb_step_bal; k >= 2 for kYPair):
-//   kYPlain  y += mu_k vkp1 (k == 1: y = mu_0 vk + mu_1 vkp1)
-//   kYSkip   y is neither read nor written (its term waits for the next step)
-//   kYPair   y += mu_{k-1} vk, then y += mu_k vkp1: the updates of a skipped
-//            step and this one, in their order, for columns c < nact (active
-//            at degree k-1; mus is zero past each column's degree)
-// Skip and pair steps alternate, so y costs one read and one write per two
-// degrees, with the results of plain steps bit for bit.
-constexpr int kYPlain = 0, kYSkip = 2, kYPair = 1;
-
 // Same with one thread per row (row blocks of the CSR-stream partition,
-// a/ja staged in LDS, B-wide 16-byte row gathers); B <= 32.
+// a/ja staged in LDS, B-wide 16-byte row gathers); B <= 32.  y is updated as
+// `ymode` says, for columns c < nact (active at the lowest degree whose term
+// is added; mus is zero past each column's degree).
 template <typename T>
 void cheb_step_blkrow(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1,
                       T *y, double cc, double t, const double *mus, int k,
-                      int nact, hipStream_t s, int ymode = kYPlain);
+                      int nact, hipStream_t s, int ymode);
 
 // Clenshaw step on B interleaved columns (row per thread, B <= 32):
 //   out = mu_k v + t (A b1 - cc b1) - b2,  mu_k per column = mus[k*B + c];
@@ -123,7 +153,7 @@ void clen_step_seg(const DevCsr &A, int Bp, const T *b1, const T *b2, const T *v
 template <typename T>
 void cheb_step_bal(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1,
                    T *y, double cc, double t, const double *mus, int k,
-                   int nact, hipStream_t s, int ymode = kYPlain);
+                   int nact, hipStream_t s, int ymode);
 template <typename T>
 void clen_step_bal(const DevCsr &A, int B, const T *b1, const T *b2, const T *v, T *out,
                    double cc, double t, const double *mus, int k, hipStream_t s);
@@ -149,7 +179,8 @@ int kpm_step_bal(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1, co
 // out[c] = sum_b part[b*ncol + c], b < nblk (fixed order); out may be strided.
 void reduce_partials(const double *part, int nblk, int ncol, double *out,
                      hipStream_t s);
-// y = x for n doubles (n even, 16-byte aligned): plain copy kernel
+// y = x for n doubles: plain copy kernel (16-byte pairs where n and the
+// alignment allow)
 void copy_f64(size_t n, const double *x, double *y, hipStream_t s);
 // part[p] (m1 x m2, column-major) = X(rows p*chunk .. , :)^T Y(same rows, :)
 // for p < nparts (the last part ends at row n), FP64 MFMA (hand-written

@@ -90,8 +90,8 @@ double clen_seg_launch_bytes(const DevCsr &A, int elem, int seg, int d, int nseg
   return b;
 }
 
-// three-term step: passes = vector passes per column (5: vk gathered, vkm1,
-// vkp1, y read and written; 3 on the first degree, or with y skipped)
+// three-term step: passes = vector passes per column (3: vk gathered, vkm1,
+// vkp1; 2 on the first degree; and those of y)
 size_t filter_launch_bytes(const DevCsr &A, int elem, int ncol, int passes, int idx) {
   const double vec = (double)A.n * elem;
   return (size_t)((double)A.nnz * (elem + idx) + 4.0 * (A.n + 1) + passes * vec * ncol);
@@ -131,11 +131,12 @@ static void cheb_filter_f32(Ctx &c, const pevsl_Polparams *pol, const float *x32
   const double *mu = pol->mu;
   const double cc = pol->cc, dd = pol->dd;
   const hipStream_t s = c.stream;
-  const int lanes = c.lanes ? c.lanes : auto_lanes((double)A.nnz / std::max(1, n));
+  const int lanes = std::max(c.lanes, 1);
   const bool stream = c.use_stream != 0;
   float *b[3] = {w, w + (size_t)n, w + 2 * (size_t)n};
   const float *vk = x32, *vkm1 = nullptr;
   int nb = 0;
+  YPlan yp;
   const long tok = m > 0 && timed
                        ? c.kt.begin(s, filter_kernel_name(true, 0, 0, stream, lanes).c_str())
                        : -1;
@@ -143,15 +144,17 @@ static void cheb_filter_f32(Ctx &c, const pevsl_Polparams *pol, const float *x32
   for (int k = 1; k <= m; k++) {
     float *vkp1 = b[nb];
     nb = (nb + 1) % 3;
+    const int ymode = stream ? yp.next(k, m) : (k == 1 ? kYInit | 1 : 1);
     if (stream)
       cheb_step_stream<float>(A, vk, vkm1, vkp1, y32, cc, k == 1 ? 1.0 / dd : 2.0 / dd, mu[0],
-                              mu[k], k == 1, s);
+                              k > 2 ? mu[k - 2] : 0.0, mu[k - 1], mu[k], ymode, s);
     else
       cheb_step_vec<float>(A, vk, vkm1, vkp1, y32, cc, k == 1 ? 1.0 / dd : 2.0 / dd, mu[0],
                            mu[k], k == 1, lanes, s);
     vkm1 = vk;
     vk = vkp1;
-    bytes += (double)filter_launch_bytes(A, 4, 1, k == 1 ? 3 : 5, stream ? index_bytes(A) : 4);
+    bytes += (double)filter_launch_bytes(A, 4, 1, (k == 1 ? 2 : 3) + y_passes(ymode),
+                                         stream ? index_bytes(A) : 4);
   }
   if (tok >= 0) c.kt.end(s, tok, m, bytes);
   c.kstats.filter_bytes += bytes;
@@ -191,24 +194,25 @@ void cheb_filter_col(Ctx &c, const pevsl_Polparams *pol, const double *dv,
     return;
   }
   const DevCsr &A = *c.A;
-  const int lanes = c.lanes ? c.lanes : auto_lanes((double)A.nnz / std::max(1, n));
-  // default (-1): the CSR-stream kernel (5.7 vs 4.4 TB/s for the best
-  // vector-CSR lane count on the 7-point stencil)
+  const int lanes = std::max(c.lanes, 1);
+  // default (-1): the CSR-stream kernel
   const bool stream = c.use_stream != 0;
   if (c.filter_prec == PEVSL_PREC_FP64) {
     double *w = work ? work : c.scratch64.ensure((size_t)3 * n);
     double *b[3] = {w, w + n, w + 2 * (size_t)n};
     const double *vk = dv, *vkm1 = nullptr;
     int nb = 0;
+    YPlan yp;
     const long tok =
         work ? -1 : c.kt.begin(s, filter_kernel_name(false, 0, 0, stream, lanes).c_str());
     const double bytes0 = c.kstats.filter_bytes;
     for (int k = 1; k <= m; k++) {
       double *vkp1 = b[nb];
       nb = (nb + 1) % 3;
+      const int ymode = stream ? yp.next(k, m) : (k == 1 ? kYInit | 1 : 1);
       if (stream)
         cheb_step_stream<double>(A, vk, vkm1, vkp1, dy, cc, k == 1 ? 1.0 / dd : 2.0 / dd,
-                                 mu[0], mu[k], k == 1, s);
+                                 mu[0], k > 2 ? mu[k - 2] : 0.0, mu[k - 1], mu[k], ymode, s);
       else
         cheb_step_vec<double>(A, vk, vkm1, vkp1, dy, cc,
                               k == 1 ? 1.0 / dd : 2.0 / dd, mu[0], mu[k], k == 1,
@@ -216,7 +220,8 @@ void cheb_filter_col(Ctx &c, const pevsl_Polparams *pol, const double *dv,
       vkm1 = vk;
       vk = vkp1;
       c.kstats.filter_bytes +=
-          (double)filter_launch_bytes(A, 8, 1, k == 1 ? 3 : 5, stream ? index_bytes(A) : 4);
+          (double)filter_launch_bytes(A, 8, 1, (k == 1 ? 2 : 3) + y_passes(ymode),
+                                      stream ? index_bytes(A) : 4);
     }
     if (tok >= 0) c.kt.end(s, tok, m, c.kstats.filter_bytes - bytes0);
   } else {
@@ -712,7 +717,7 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
     int nb = 0;
     const long tok = degmax > 0 && !capture_ ? c_.kt.begin(c_.stream, kname.c_str()) : -1;
     double kbytes = 0.0;
-    int nprev = g;  // columns whose series reaches degree d - 1
+    YPlan yp;
     for (int d = 1; d <= degmax; d++) {
       int nact = 0;
       while (nact < g && degs[(size_t)nact] >= d) nact++;
@@ -723,18 +728,14 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
         vkp1 = bufs[nb];
       }
       nb = (nb + 1) % 3;
-      // the row kernels update y every other degree (skip, then pair: the
-      // same additions in the same order, one pass over y per two degrees);
-      // the last degree updates it alone when it would be skipped
-      int ymode = kYPlain, ncol = nact, passes = d == 1 ? 3 : 5;
-      if (rowk && d > 1) {
-        if (d % 2 == 1) {
-          ymode = kYPair;
-          ncol = nprev;
-        } else if (d < degmax) {
-          ymode = kYSkip;
-          passes = 3;
-        }
+      // the row kernels update y every third degree (YPlan: the same
+      // additions in the same order, one pass over y per three degrees), for
+      // the columns active at the lowest degree whose term is added
+      const int ymode = rowk ? yp.next(d, degmax) : (d == 1 ? kYInit | 1 : 1);
+      int ncol = nact;
+      if (rowk && ymode != kYSkip) {
+        ncol = 0;
+        while (ncol < g && degs[(size_t)ncol] >= d + 1 - (ymode & 3)) ncol++;
       }
       if (bal)
         cheb_step_bal<T>(A, B, vk, vkm1, vkp1, y, cc, d == 1 ? 1.0 / dd : 2.0 / dd, musp, d,
@@ -745,15 +746,9 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
       else
         cheb_step_blk<T>(A, B, vk, vkm1, vkp1, y, cc, d == 1 ? 1.0 / dd : 2.0 / dd,
                          musp, d, nact, c_.stream);
-      nprev = nact;
-      // pair steps count y over the columns of degree d - 1 (a product of
-      // its own over the columns of degree d); skip steps touch no y
       const int ib = rowk && !bal ? index_bytes(A) : 4;  // only the row kernel reads jo16
-      const double lb =
-          ymode == kYPair
-              ? (double)filter_launch_bytes(A, (int)elem, nact, 3, ib) +
-                    2.0 * (double)n_ * (double)elem * ncol
-              : (double)filter_launch_bytes(A, (int)elem, nact, passes, ib);
+      const double lb = (double)filter_launch_bytes(A, (int)elem, nact, d == 1 ? 2 : 3, ib) +
+                        y_passes(ymode) * (double)n_ * (double)elem * ncol;
       kbytes += lb;
       c_.kstats.filter_bytes += lb;
       c_.kstats.filter_steps += nact;
@@ -1067,9 +1062,7 @@ void BatchSolver::ritz(int s, double tol) {
     col_scale(n_, nb, U.p, ld, red.p, st);
     // W = A U, Rayleigh quotients
     if (c_.A) {
-      spmv_cols_f64(*c_.A, U.p, W.p, nb, ld,
-                    c_.lanes ? c_.lanes : auto_lanes((double)c_.A->nnz / std::max(1, n_)),
-                    st);
+      spmv_cols_f64(*c_.A, U.p, W.p, nb, ld, c_.spmv_lanes(), st);
     } else {
       for (int i = 0; i < nb; i++) apply_A(c_, U.p + (size_t)i * ld, W.p + (size_t)i * ld);
     }
@@ -1155,7 +1148,7 @@ void BatchSolver::ritz_rr(int s, double tol) {
   C.release();
   free_basis(s);  // the basis is no longer needed
   conv_.release();
-  const int lanes = c_.lanes ? c_.lanes : auto_lanes((double)c_.A->nnz / std::max(1, n_));
+  const int lanes = c_.spmv_lanes();
   spmv_cols_f64(*c_.A, U.p, W.p, nsel, ld, lanes, st);
   sl.nmatvec += nsel;
   // Gram matrices (upper triangles are read by SYGVD)

@@ -30,10 +30,12 @@ double time_vec(Ctx &c, int lanes, int reps) {
   b.ensure((size_t)4 * n);
   T *v0 = b.p, *v1 = b.p + n, *v2 = b.p + 2 * (size_t)n, *y = b.p + 3 * (size_t)n;
   PV_HIP(hipMemsetAsync(b.p, 0, sizeof(T) * 4 * (size_t)n, c.stream));
-  // warm-up
+  // the stream kernel updates y every third degree, as a solve runs it
+  int turn = 0;
   auto step = [&](const T *vk, const T *vkm1, T *vkp1) {
     if (lanes == 0)
-      cheb_step_stream<T>(A, vk, vkm1, vkp1, y, 6.0, 1.0 / 6, 0.1, 0.1, false, c.stream);
+      cheb_step_stream<T>(A, vk, vkm1, vkp1, y, 6.0, 1.0 / 6, 0.1, 0.1, 0.1, 0.1,
+                          ++turn % 3 == 0 ? 3 : kYSkip, c.stream);
     else
       cheb_step_vec<T>(A, vk, vkm1, vkp1, y, 6.0, 1.0 / 6, 0.1, 0.1, false, lanes, c.stream);
   };
@@ -66,11 +68,11 @@ double time_blk(Ctx &c, int B, int reps, DBuf<double> &mus, int kind) {
   SegTops tops{};
   for (int p = 0; p < kMaxSegs; p++) tops.top[p] = 100;  // every piece forms the product
   const int nseg = B * (int)sizeof(T) / 16;
-  // the three-term row kernels alternate skip and pair steps, as a batched
-  // solve runs them (on average four vector passes per degree)
-  int parity = 0;
+  // the three-term row kernels update y every third degree, as a batched
+  // solve runs them (on average 11/3 vector passes per degree)
+  int turn = 0;
   auto step = [&](const T *vk, const T *vkm1, T *vkp1) {
-    const int ymode = (parity++ & 1) ? kYPair : kYSkip;
+    const int ymode = ++turn % 3 == 0 ? 3 : kYSkip;
     if (kind == 5)
       clen_step_seg<T>(A, B, vk, vkm1, y, vkp1, 6.0, 1.0 / 3, mus.p, 2, nseg, tops, c.stream);
     else if (kind == 4)
