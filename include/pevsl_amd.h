@@ -41,7 +41,9 @@ typedef struct {
   double t_eig;           /* tridiagonal eigen-solves                   */
   double t_ritz;          /* Ritz vectors, residuals                    */
   double t_kpm;           /* KPM moments                                */
-  double filter_bytes;    /* algorithmic bytes of the filter steps      */
+  double filter_bytes;    /* algorithmic bytes of the filter steps, the
+                             matrix counted in CSR form whichever layout
+                             the kernels read                           */
   double reorth_bytes;    /* algorithmic bytes of the reorthogonalization */
   long long filter_steps; /* column-degree steps                        */
   long long filter_launches;
@@ -188,7 +190,12 @@ int pEVSL_SetGraphFilter(pevsl_Data *pevsl, int on);
  * results are bitwise the same.  on = 1 (default) uses them where the
  * matrix has them, 0 keeps the 32-bit indices for this instance.
  * pEVSL_ColumnOffsets16 returns 1 when the instance's matrix is read
- * through them. */
+ * through them.
+ * A matrix of at most 32 diagonals, each of one value (the main diagonal may
+ * vary: constant-coefficient grid stencils, with or without a potential),
+ * also gets a diagonal layout of one mask byte (four above 8 diagonals) per
+ * row, which the same kernels and the products then read instead; 0
+ * switches it off as well. */
 int pEVSL_SetColumnOffsets16(pevsl_Data *pevsl, int on);
 int pEVSL_ColumnOffsets16(pevsl_Data *pevsl);
 

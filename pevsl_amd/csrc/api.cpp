@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstring>
 #include <ctime>
+#include <memory>
 
 #include "internal.hpp"
 
@@ -214,6 +215,113 @@ static void parcsr_mv_host(double *x, double *y, void *data) {
                           &Y, y);
   pEVSL_ParcsrMatvec(A, &X, &Y);
 }
+
+namespace {
+
+// Diagonal layout of a CSR matrix (DevDia) in host memory.
+struct HostDia {
+  int ndiag = 0, qd = -1;
+  int off[kMaxDiags];
+  double c[kMaxDiags];
+  std::vector<uint8_t> mask8;
+  std::vector<uint32_t> mask32;
+  std::vector<double> dg;
+};
+
+// Fills D and returns true if the matrix has a diagonal layout: columns
+// ascend strictly within rows, at most kMaxDiags diagonals, each of one value
+// (bit for bit), the main diagonal excepted, and at least half of the
+// diagonals' places taken (a kernel loads x for every diagonal of a row).
+// A matrix without the layout is recognised after its first rows: random
+// sparsity has more than kMaxDiags diagonals within two or three rows, and
+// varying coefficients differ at once.  On structured grids most rows repeat
+// the row before, which one comparison per entry establishes.
+bool find_dia(int n, const int *ia, const int *ja, const double *a, HostDia &D) {
+  if (n <= 0 || ia[n] <= 0) return false;
+  int nd = 0, off[kMaxDiags], qrow[kMaxDiags];
+  double c[kMaxDiags];
+  bool varies[kMaxDiags];
+  int prev = -1, plen = -1, nvar = 0;
+  auto same = [](double x, double y) { return memcmp(&x, &y, sizeof x) == 0; };
+  // diagonals in order of first appearance, one value each
+  std::vector<uint32_t> rm((size_t)n);
+  for (int i = 0; i < n; i++) {
+    const int b = ia[i], len = ia[i + 1] - b;
+    bool rep = len == plen;
+    for (int j = 0; rep && j < len; j++) rep = ja[b + j] - i == ja[prev + j] - (i - 1);
+    if (!rep) {
+      if (len > kMaxDiags) return false;
+      for (int j = 0; j < len; j++) {
+        if (j > 0 && ja[b + j] <= ja[b + j - 1]) return false;
+        const int o = ja[b + j] - i;
+        int q = 0;
+        while (q < nd && off[q] != o) q++;
+        if (q == nd) {
+          if (nd == kMaxDiags) return false;
+          off[nd] = o;
+          c[nd] = a[b + j];
+          varies[nd++] = false;
+        }
+        qrow[j] = q;
+      }
+    }
+    uint32_t m = 0;
+    for (int j = 0; j < len; j++) {
+      const int q = qrow[j];
+      m |= 1u << q;
+      if (!varies[q] && !same(a[b + j], c[q])) {
+        varies[q] = true;
+        if (++nvar > 1 || off[q] != 0) return false;
+      }
+    }
+    rm[(size_t)i] = m;
+    prev = b;
+    plen = len;
+  }
+  if (2.0 * ia[n] < (double)nd * n) return false;
+  // ascending diagonals
+  int ord[kMaxDiags], pos[kMaxDiags];
+  for (int q = 0; q < nd; q++) ord[q] = q;
+  std::sort(ord, ord + nd, [&](int x, int y) { return off[x] < off[y]; });
+  bool moved = false;
+  for (int q = 0; q < nd; q++) {
+    pos[ord[q]] = q;
+    moved = moved || ord[q] != q;
+    D.off[q] = off[ord[q]];
+    D.c[q] = c[ord[q]];
+    if (varies[ord[q]]) D.qd = q;
+  }
+  D.ndiag = nd;
+  uint32_t last = ~0u, lastm = 0;
+  if (nd <= 8)
+    D.mask8.resize((size_t)n);
+  else
+    D.mask32.resize((size_t)n);
+  for (int i = 0; i < n; i++) {
+    uint32_t m = rm[(size_t)i];
+    if (moved) {
+      if (m != last) {
+        last = m;
+        lastm = 0;
+        for (int q = 0; q < nd; q++) lastm |= ((m >> q) & 1u) << pos[q];
+      }
+      m = lastm;
+    }
+    if (nd <= 8)
+      D.mask8[(size_t)i] = (uint8_t)m;
+    else
+      D.mask32[(size_t)i] = m;
+  }
+  if (D.qd >= 0) {
+    D.dg.assign((size_t)n, 0.0);
+    for (int i = 0; i < n; i++)
+      for (int j = ia[i]; j < ia[i + 1]; j++)
+        if (ja[j] == i) D.dg[(size_t)i] = a[j];
+  }
+  return true;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -518,21 +626,33 @@ int pEVSL_ParcsrSetup(pevsl_Csr *Ai, pevsl_Parcsr *A) {
   int mr = 0;
   for (int i = 0; i < n; i++) mr = std::max(mr, Ai->ia[i + 1] - Ai->ia[i]);
   M->csr.max_row = mr;
-  std::vector<int> rb;
+  // row partitions, one device array: the CSR-stream blocks, the offsets of
+  // their first nonzeros, the blocks of the balanced kernels
+  std::vector<int> rb, rq, all;
   build_row_blocks(n, Ai->ia, rb);
   M->csr.nrowblk = (int)rb.size() - 1;
-  M->csr.rowblk = M->rowblk.ensure(rb.size());
-  PV_HIP(hipMemcpy(M->csr.rowblk, rb.data(), sizeof(int) * rb.size(), hipMemcpyHostToDevice));
-  {
-    std::vector<int> bz(rb.size());
-    for (size_t b = 0; b < rb.size(); b++) bz[b] = Ai->ia[rb[b]];
-    M->csr.blknz = M->blknz.ensure(bz.size());
-    PV_HIP(hipMemcpy(M->csr.blknz, bz.data(), sizeof(int) * bz.size(), hipMemcpyHostToDevice));
+  size_t at[6];
+  at[0] = 0;
+  all = rb;
+  at[5] = all.size();
+  for (int r0 : rb) all.push_back(Ai->ia[r0]);
+  for (int l = 1; l < 5; l++) {
+    build_row_blocks(n, Ai->ia, rq, kStreamRows >> l, kStreamNnz >> l);
+    M->csr.nrowblk_q[l] = (int)rq.size() - 1;
+    at[l] = all.size();
+    all.insert(all.end(), rq.begin(), rq.end());
   }
+  M->rowblk.ensure(all.size());
+  PV_HIP(hipMemcpy(M->rowblk.p, all.data(), sizeof(int) * all.size(), hipMemcpyHostToDevice));
+  M->csr.rowblk = M->rowblk.p;
+  M->csr.blknz = M->rowblk.p + at[5];
+  M->csr.rowblk_q[0] = M->csr.rowblk;
+  M->csr.nrowblk_q[0] = M->csr.nrowblk;
+  for (int l = 1; l < 5; l++) M->csr.rowblk_q[l] = M->rowblk.p + at[l];
   // 16-bit column offsets from each row block's first row, kept when every
   // nonzero's offset fits (banded orderings such as the natural order of a
   // grid Laplacian; not random sparsity)
-  std::vector<short> jo((size_t)nnz);
+  std::unique_ptr<short[]> jo(new short[(size_t)nnz]);
   bool fits = nnz > 0;
   for (size_t b = 0; fits && b + 1 < rb.size(); b++) {
     const int r0 = rb[b];
@@ -547,19 +667,10 @@ int pEVSL_ParcsrSetup(pevsl_Csr *Ai, pevsl_Parcsr *A) {
   }
   if (fits) {
     M->csr.jo16 = M->jo16.ensure((size_t)nnz);
-    PV_HIP(hipMemcpy(M->csr.jo16, jo.data(), sizeof(short) * (size_t)nnz,
+    PV_HIP(hipMemcpy(M->csr.jo16, jo.get(), sizeof(short) * (size_t)nnz,
                      hipMemcpyHostToDevice));
   }
-  M->csr.rowblk_q[0] = M->csr.rowblk;
-  M->csr.nrowblk_q[0] = M->csr.nrowblk;
-  for (int l = 1; l < 5; l++) {
-    build_row_blocks(n, Ai->ia, rb, kStreamRows >> l, kStreamNnz >> l);
-    M->csr.nrowblk_q[l] = (int)rb.size() - 1;
-    M->csr.rowblk_q[l] = M->rowblk_q[l].ensure(rb.size());
-    PV_HIP(hipMemcpy(M->csr.rowblk_q[l], rb.data(), sizeof(int) * rb.size(),
-                     hipMemcpyHostToDevice));
-  }
-  std::vector<float> a32((size_t)nnz);
+  std::unique_ptr<float[]> a32(new float[(size_t)nnz]);
   for (int j = 0; j < nnz; j++) a32[j] = (float)Ai->a[j];
   PV_HIP(hipMemcpy(M->csr.ia, Ai->ia, sizeof(int) * (size_t)(n + 1),
                    hipMemcpyHostToDevice));
@@ -567,8 +678,34 @@ int pEVSL_ParcsrSetup(pevsl_Csr *Ai, pevsl_Parcsr *A) {
                    hipMemcpyHostToDevice));
   PV_HIP(hipMemcpy(M->csr.a64, Ai->a, sizeof(double) * (size_t)nnz,
                    hipMemcpyHostToDevice));
-  PV_HIP(hipMemcpy(M->csr.a32, a32.data(), sizeof(float) * (size_t)nnz,
+  PV_HIP(hipMemcpy(M->csr.a32, a32.get(), sizeof(float) * (size_t)nnz,
                    hipMemcpyHostToDevice));
+  // diagonal layout, where the matrix has one
+  HostDia hd;
+  if (find_dia(n, Ai->ia, Ai->ja, Ai->a, hd)) {
+    DevDia &dd = M->csr.dia;
+    const size_t mb = hd.ndiag <= 8 ? (size_t)n : sizeof(uint32_t) * (size_t)n;
+    PV_HIP(hipMemcpy(M->dia_mask.ensure(mb),
+                     hd.ndiag <= 8 ? (const void *)hd.mask8.data() : (const void *)hd.mask32.data(),
+                     mb, hipMemcpyHostToDevice));
+    dd.mask = M->dia_mask.p;
+    if (hd.qd >= 0) {
+      std::vector<float> dg32((size_t)n);
+      for (int i = 0; i < n; i++) dg32[(size_t)i] = (float)hd.dg[(size_t)i];
+      PV_HIP(hipMemcpy(M->dia_dg64.ensure((size_t)n), hd.dg.data(), sizeof(double) * (size_t)n,
+                       hipMemcpyHostToDevice));
+      PV_HIP(hipMemcpy(M->dia_dg32.ensure((size_t)n), dg32.data(), sizeof(float) * (size_t)n,
+                       hipMemcpyHostToDevice));
+      dd.dg64 = M->dia_dg64.p;
+      dd.dg32 = M->dia_dg32.p;
+    }
+    for (int q = 0; q < hd.ndiag; q++) {
+      dd.off[q] = hd.off[q];
+      dd.c[q] = hd.c[q];
+    }
+    dd.qd = hd.qd;
+    dd.ndiag = hd.ndiag;
+  }
   A->dev = M;
   return 0;
 }

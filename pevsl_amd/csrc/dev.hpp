@@ -1,4 +1,5 @@
-// dev.hpp -- device-side helpers shared by the kernel files: launch constants, the XCD-aware block order, 16-byte pieces of
+// dev.hpp -- device-side helpers shared by the kernel files (kernels.hip,
+// dia.hip): launch constants, the XCD-aware block order, 16-byte pieces of
 // interleaved rows and the update of the filter's accumulator.
 #pragma once
 #include <hip/hip_runtime.h>

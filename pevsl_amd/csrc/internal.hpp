@@ -62,11 +62,14 @@ struct DBuf {
 // Device copy of a CSR matrix (attached to pevsl_Parcsr.dev).
 struct DevMatrix {
   DevCsr csr;
-  DBuf<int> ia, ja, rowblk, blknz;
-  DBuf<int> rowblk_q[5];  // partitions of the nnz-balanced kernels, Q >= 2
+  DBuf<int> ia, ja;
+  DBuf<int> rowblk;  // the row partitions (DevCsr::rowblk, blknz, rowblk_q)
   DBuf<double> a64;
   DBuf<float> a32;
   DBuf<short> jo16;
+  DBuf<uint8_t> dia_mask;
+  DBuf<double> dia_dg64;
+  DBuf<float> dia_dg32;
 };
 
 // Live per-kernel timing on an instance's stream: HIP events around a run of
@@ -117,8 +120,8 @@ struct Ctx {
   rocblas_handle blas = nullptr;
   const DevCsr *A = nullptr;       // set by SetAParcsr: &A_view
   const DevCsr *A_src = nullptr;   // the matrix's device copy
-  DevCsr A_view;                   // A_src, without jo16 when col16 == 0
-  int col16 = 1;                   // 16-bit column offsets where the matrix has them
+  DevCsr A_view;                   // A_src, as plain CSR when col16 == 0
+  int col16 = 1;                   // 16-bit column offsets / diagonals where the matrix has them
   MVFunc host_mv = nullptr;        // set by SetAMatvec (host callback)
   void *host_mv_data = nullptr;
   int filter_prec = PEVSL_PREC_FP64;

@@ -10,6 +10,7 @@
 //     coalesced order into LDS, then each thread sums one row sequentially
 //     (the reference's order); a longer row is one block, reduced by all of
 //     its threads.  The default single-slice filter.
+//   * (dia.hip) the same steps on matrices with a diagonal layout.
 //   * k_cheb_vec : one column with L lanes per row (tuning alternative).
 //   * k_cheb_blkrow / k_clen_blkrow : B slices as interleaved columns
 //     (row-major n x B), a/ja staged in LDS, one thread per row gathering
@@ -1768,6 +1769,10 @@ void spmv_cols_f64(const DevCsr &A, const double *X, double *Y, int ncol,
                    size_t ld, int lanes, hipStream_t s) {
   if (A.n == 0 || ncol == 0) return;
   if (lanes == 0) {
+    if (use_dia(A, 8, 1)) {
+      dia_spmv_f64(A, X, Y, ncol, ld, s);
+      return;
+    }
     // One column on even rows and fewer than two row blocks per CU: the
     // vector-CSR kernel, whose loads depend on each other over fewer stages
     // and which has more blocks.  7-point stencil, whole call of one product,
@@ -1919,6 +1924,10 @@ void cheb_step_stream(const DevCsr &A, const T *vk, const T *vkm1, T *vkp1,
                       T *y, double cc, double t, double mu0, double mu3, double mu2, double mu1,
                       int ymode, hipStream_t s) {
   if (A.n == 0 || A.nrowblk == 0) return;
+  if (use_dia(A, sizeof(T), 1)) {
+    dia_cheb_step<T>(A, vk, vkm1, vkp1, y, cc, t, mu0, mu3, mu2, mu1, ymode, s);
+    return;
+  }
   const T *a = std::is_same<T, double>::value ? (const T *)A.a64
                                               : (const T *)A.a32;
   const int uneven = A.max_row > kUnevenRow;

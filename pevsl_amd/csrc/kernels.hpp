@@ -9,6 +9,26 @@
 
 namespace pevsl {
 
+// Diagonal layout of a matrix whose nonzeros lie on at most kMaxDiags
+// diagonals, each holding one value wherever it holds an entry -- except the
+// main diagonal, whose values may differ from row to row: the constant-
+// coefficient stencils of structured grids, with or without a potential.
+// Per row it stores a bit mask of the diagonals present (1 byte up to 8
+// diagonals, else 4) and, where they differ, the main diagonal's value,
+// against 8-12 bytes per nonzero in CSR.  Diagonals ascend, as the columns of
+// every row do, so a row's sum has the same terms in the same order.
+constexpr int kMaxDiags = 32;
+struct DevDia {
+  int ndiag = 0;         // 0: the matrix has no such layout
+  int off[kMaxDiags] = {};     // column - row, ascending
+  double c[kMaxDiags] = {};    // the diagonal's value
+  int qd = -1;           // index of the main diagonal if it varies, else -1
+  const void *mask = nullptr;  // per row: bit q set = entry on diagonal q
+  const double *dg64 = nullptr;  // main diagonal per row (qd >= 0)
+  const float *dg32 = nullptr;
+};
+inline int dia_mask_bytes(const DevDia &D) { return D.ndiag <= 8 ? 1 : 4; }
+
 // Device CSR: int32 row pointers / column indices, values in FP64 and FP32.
 struct DevCsr {
   int n = 0;       // rows == cols
@@ -32,10 +52,15 @@ struct DevCsr {
   // `rowblk` (null when an offset does not fit in a short): the CSR-stream
   // and row-per-thread block kernels then read 2 index bytes per nonzero
   short *jo16 = nullptr;
-  // on == 0: 32-bit column indices
+  // diagonal layout, where the matrix has one (dia.ndiag > 0): the one-column
+  // step, the row-per-thread block steps and the products then read it
+  DevDia dia;
+  // on == 0: the plain CSR form (32-bit indices), without the layouts that
+  // replace the column indices
   void use_offsets(int on) {
     if (on) return;
     jo16 = nullptr;
+    dia.ndiag = 0;
   }
 };
 
@@ -57,7 +82,7 @@ void build_row_blocks(int n, const int *ia, std::vector<int> &blk,
 
 // ---- sparse products -------------------------------------------------------
 // y = A x, one column.  lanes = lanes per row in {1,2,4,8,16,32,64}, or 0 for
-// the CSR-stream
+// the kernel that suits the matrix: its diagonal layout, else the CSR-stream
 // or vector-CSR form by size.
 void spmv_f64(const DevCsr &A, const double *x, double *y, int lanes,
               hipStream_t s);
@@ -100,13 +125,26 @@ struct YPlan {
 inline int y_passes(int mode) { return mode == kYSkip ? 0 : (mode & kYInit) ? 1 : 2; }
 
 // Same step, y updated as `ymode` says (mu0, mu3, mu2, mu1: the coefficients
-// of degrees 0, d-2, d-1, d; vkm1 null at d == 1), with the CSR-stream
-// kernel (one block per row block: coalesced products staged in LDS, then one
-// sequential sum per row; rows longer than kUnevenRow by a wave).
+// of degrees 0, d-2, d-1, d; vkm1 null at d == 1), with the kernel that suits
+// the matrix: its diagonal layout, or the CSR-stream kernel (one block per row
+// block: coalesced products staged in LDS, then one sequential sum per row).
 template <typename T>
 void cheb_step_stream(const DevCsr &A, const T *vk, const T *vkm1, T *vkp1,
                       T *y, double cc, double t, double mu0, double mu3, double mu2, double mu1,
                       int ymode, hipStream_t s);
+// whether cheb_step_stream and the row-per-thread block steps of width B read
+// the diagonal layout (32-bit byte offsets into a block of B columns)
+inline bool use_dia(const DevCsr &A, int elem, int B) {
+  return A.dia.ndiag > 0 && (double)A.n * elem * B < 4294967296.0;
+}
+// kernels of the diagonal layout (dia.hip)
+void dia_spmv_f64(const DevCsr &A, const double *X, double *Y, int ncol, size_t ld,
+                  hipStream_t s);
+template <typename T>
+void dia_cheb_step(const DevCsr &A, const T *vk, const T *vkm1, T *vkp1, T *y, double cc,
+                   double t, double mu0, double mu3, double mu2, double mu1, int ymode,
+                   hipStream_t s);
+
 // Same for B interleaved columns (row-major n x B block, column fastest).
 // mus: device array [(deg_max+1) x B] of per-column coefficients; k = degree
 // index of this step (1..); columns c >= nact are left untouched.

@@ -97,7 +97,17 @@ size_t filter_launch_bytes(const DevCsr &A, int elem, int ncol, int passes, int 
   return (size_t)((double)A.nnz * (elem + idx) + 4.0 * (A.n + 1) + passes * vec * ncol);
 }
 
-// name of a filter kernel for the per-kernel timers
+// What a launch on the diagonal layout does not read of the CSR form the byte
+// counts above assume (they feed pevsl_KernelStats, whose figures compare
+// between layouts; the per-kernel timers count what the kernel reads).
+double dia_saved_bytes(const DevCsr &A, int elem, int idx, bool dia) {
+  if (!dia) return 0.0;
+  return (double)A.nnz * (elem + idx) + 4.0 * (A.n + 1) -
+         (double)A.n * (dia_mask_bytes(A.dia) + (A.dia.qd >= 0 ? elem : 0));
+}
+
+// name of a filter step for the per-kernel timers; the stream and row forms
+// keep their names on the diagonal layout
 std::string filter_kernel_name(bool f32, int kind, int B, bool stream, int lanes) {
   const char *t = f32 ? "float" : "double";
   char nm[48];
@@ -137,6 +147,7 @@ static void cheb_filter_f32(Ctx &c, const pevsl_Polparams *pol, const float *x32
   const float *vk = x32, *vkm1 = nullptr;
   int nb = 0;
   YPlan yp;
+  const bool dia = stream && use_dia(A, 4, 1);
   const long tok = m > 0 && timed
                        ? c.kt.begin(s, filter_kernel_name(true, 0, 0, stream, lanes).c_str())
                        : -1;
@@ -156,7 +167,7 @@ static void cheb_filter_f32(Ctx &c, const pevsl_Polparams *pol, const float *x32
     bytes += (double)filter_launch_bytes(A, 4, 1, (k == 1 ? 2 : 3) + y_passes(ymode),
                                          stream ? index_bytes(A) : 4);
   }
-  if (tok >= 0) c.kt.end(s, tok, m, bytes);
+  if (tok >= 0) c.kt.end(s, tok, m, bytes - m * dia_saved_bytes(A, 4, index_bytes(A), dia));
   c.kstats.filter_bytes += bytes;
   c.kstats.filter_steps += m;
   c.kstats.filter_launches += m;
@@ -195,7 +206,7 @@ void cheb_filter_col(Ctx &c, const pevsl_Polparams *pol, const double *dv,
   }
   const DevCsr &A = *c.A;
   const int lanes = std::max(c.lanes, 1);
-  // default (-1): the CSR-stream kernel
+  // default (-1): the diagonal layout's or the CSR-stream kernel
   const bool stream = c.use_stream != 0;
   if (c.filter_prec == PEVSL_PREC_FP64) {
     double *w = work ? work : c.scratch64.ensure((size_t)3 * n);
@@ -203,6 +214,7 @@ void cheb_filter_col(Ctx &c, const pevsl_Polparams *pol, const double *dv,
     const double *vk = dv, *vkm1 = nullptr;
     int nb = 0;
     YPlan yp;
+    const bool dia = stream && use_dia(A, 8, 1);
     const long tok =
         work ? -1 : c.kt.begin(s, filter_kernel_name(false, 0, 0, stream, lanes).c_str());
     const double bytes0 = c.kstats.filter_bytes;
@@ -223,7 +235,9 @@ void cheb_filter_col(Ctx &c, const pevsl_Polparams *pol, const double *dv,
           (double)filter_launch_bytes(A, 8, 1, (k == 1 ? 2 : 3) + y_passes(ymode),
                                       stream ? index_bytes(A) : 4);
     }
-    if (tok >= 0) c.kt.end(s, tok, m, c.kstats.filter_bytes - bytes0);
+    if (tok >= 0)
+      c.kt.end(s, tok, m, c.kstats.filter_bytes - bytes0 -
+                              m * dia_saved_bytes(A, 8, index_bytes(A), dia));
   } else {
     // x32, y32 and three work columns: 5n floats (within 3n doubles)
     float *w = reinterpret_cast<float *>(work ? work

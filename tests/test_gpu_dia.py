@@ -1,0 +1,141 @@
+"""Diagonal layout: matrices of few constant diagonals (the main one may vary)
+are read as a mask per row instead of CSR.  Every call that the layout takes
+is compared with the plain CSR form of the same instance
+(pEVSL_SetColumnOffsets16(0) switches both it and the 16-bit offsets off).
+
+The filter's terms are the same in the same order, each rounded on its own,
+so outputs are equal bit for bit; a product on the CSR side may sum a row in
+several lanes, and is compared to 1e-15 times the row's absolute sum and
+against numpy.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from pevsl_amd import capi, driver
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return capi.load()
+
+
+def banded(n, offs, vary=None, drop=0.0, seed=0):
+    """CSR with constant diagonals `offs` (value by diagonal), `vary` random
+    diagonals among them, and a share `drop` of entries left out."""
+    rng = np.random.default_rng(seed)
+    r, c, v = [], [], []
+    for o in sorted(offs):
+        i = np.arange(max(0, -o), min(n, n - o))
+        i = i[rng.random(len(i)) >= drop] if o != 0 else i
+        r.append(i)
+        c.append(i + o)
+        val = np.full(len(i), 0.3 + 0.1 * (o % 7) - (0.05 if o > 0 else 0.0))
+        if vary and o in vary:
+            val = rng.uniform(1.0, 3.0, len(i))
+        v.append(val)
+    r, c, v = map(np.concatenate, (r, c, v))
+    order = np.lexsort((c, r))
+    ia = np.zeros(n + 1, np.int64)
+    np.add.at(ia, r + 1, 1)
+    return np.cumsum(ia).astype(np.int32), c[order].astype(np.int32), v[order]
+
+
+CASES = {
+    "1x1": lambda: banded(1, [0]),
+    "one_row_block": lambda: banded(255, [-1, 0, 1]),
+    "block_edge": lambda: banded(256, [-1, 0, 1]),
+    "block_edge_1": lambda: banded(257, [-1, 0, 1], vary=[0]),
+    "3_of_4_dropped": lambda: banded(1111, [-5, 0, 5], drop=0.3),
+    "4_no_main": lambda: banded(1000, [-3, -1, 1, 3]),
+    "lap2d": lambda: driver.laplacian3d(31, 17, 1),
+    "lap3d": lambda: driver.laplacian3d(13, 11, 7),
+    "8_diags": lambda: banded(3001, [-700, -31, -1, 0, 1, 31, 700, 2999], drop=0.1, vary=[0]),
+    "9_diags": lambda: banded(3001, [-700, -31, -2, -1, 0, 1, 2, 31, 700], drop=0.1, vary=[0]),
+    "32_diags": lambda: banded(2500, list(range(-16, 16)), vary=[0]),
+    "empty_rows": lambda: banded(700, [-9, 9], drop=0.45),
+    # no such layout: 33 diagonals, a second varying diagonal, mostly absent
+    "33_diags": lambda: banded(900, list(range(-16, 17))),
+    "two_vary": lambda: banded(900, [-1, 0, 1], vary=[0, 1]),
+    "sparse_diags": lambda: banded(900, [-40, -20, 0, 20, 40], drop=0.9),
+}
+
+
+def filt(lib, M, pol, v, prec, on):
+    inst = driver.Instance(lib, M, prec=prec, col16=bool(on))
+    try:
+        y = np.full(M.n, np.nan)
+        pv, py = capi.Parvec(), capi.Parvec()
+        for p, a in ((pv, v), (py, y)):
+            lib.pEVSL_ParvecCreateShell(M.n, M.n, 0, 0, C.byref(p),
+                                        a.ctypes.data_as(capi.c_double_p))
+        assert lib.pEVSL_ChebAv(inst.p, C.byref(pol), C.byref(pv), C.byref(py), None) == 0
+    finally:
+        inst.close()
+    return y
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_filter_equals_csr(lib, name):
+    print("\n[gpu case] diagonal layout, filter, %s" % name, flush=True)
+    ia, ja, a = CASES[name]()
+    n = len(ia) - 1
+    M = driver.Matrix(lib, ia, ja, a)
+    rad = float(np.max(np.bincount(np.repeat(np.arange(n), np.diff(ia)), np.abs(a), n)))
+    rng = np.random.default_rng(n)
+    try:
+        v = rng.uniform(-1, 1, n)
+        # every way a run of degrees can end in the update of y
+        for deg in (1, 2, 3, 4, 5, 6, 17):
+            mu = rng.uniform(-1, 1, deg + 1)
+            pol = capi.Polparams()
+            pol.deg, pol.cc, pol.dd = deg, 0.1 * rad, 1.1 * rad
+            pol.mu = mu.ctypes.data_as(capi.c_double_p)
+            for prec in (capi.PEVSL_PREC_FP64, capi.PEVSL_PREC_FP32):
+                np.testing.assert_array_equal(filt(lib, M, pol, v, prec, 1),
+                                              filt(lib, M, pol, v, prec, 0))
+    finally:
+        M.free()
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_product_equals_csr(lib, name):
+    print("\n[gpu case] diagonal layout, product, %s" % name, flush=True)
+    ia, ja, a = CASES[name]()
+    n = len(ia) - 1
+    M = driver.Matrix(lib, ia, ja, a)
+    try:
+        x = np.random.default_rng(n).uniform(-1, 1, n)
+        y = M.matvec(x)
+        rows = np.repeat(np.arange(n), np.diff(ia))
+        ref = np.bincount(rows, a * x[ja], n)
+        mag = np.bincount(rows, np.abs(a * x[ja]), n)
+        # two summation orders of at most 33 terms
+        assert np.all(np.abs(y - ref) <= 33 * 2.3e-16 * mag)
+    finally:
+        M.free()
+
+
+def test_rectangular_product(lib):
+    print("\n[gpu case] diagonal layout, rectangular products", flush=True)
+    for nr, nc in ((300, 40), (40, 300)):
+        k = min(nr, nc)
+        ia = np.minimum(np.arange(nr + 1), k).astype(np.int32)
+        ja, a = np.arange(k, dtype=np.int32), np.full(k, 2.5)
+        csr = capi.Csr(nr, nc, ia.ctypes.data_as(capi.c_int_p), ja.ctypes.data_as(capi.c_int_p),
+                       a.ctypes.data_as(capi.c_double_p))
+        A = capi.Parcsr()
+        assert lib.pEVSL_ParcsrCreate(nr, nc, None, None, C.byref(A), capi.MPI_COMM_WORLD) == 0
+        assert lib.pEVSL_ParcsrSetup(C.byref(csr), C.byref(A)) == 0
+        x, y = np.random.default_rng(1).uniform(-1, 1, nc), np.full(nr, np.nan)
+        X, Y = capi.Parvec(), capi.Parvec()
+        lib.pEVSL_ParvecCreateShell(nc, nc, 0, 0, C.byref(X), x.ctypes.data_as(capi.c_double_p))
+        lib.pEVSL_ParvecCreateShell(nr, nr, 0, 0, C.byref(Y), y.ctypes.data_as(capi.c_double_p))
+        lib.pEVSL_ParcsrMatvec(C.byref(A), C.byref(X), C.byref(Y))
+        lib.pEVSL_ParcsrFree(C.byref(A))
+        ref = np.zeros(nr)
+        ref[:k] = 2.5 * x[:k]
+        np.testing.assert_array_equal(y, ref)
