@@ -129,14 +129,22 @@ def slice_checks(g, sli, s, o):
             "tol_accept": o["info"]["tol_accept"] if o["info"] else None}
 
 
-# kernels compiled in two forms, 16-bit column offsets (true) or 32-bit
-# indices (false): the profiler names carry the flag, the timers do not
-J16_KERNELS = ("k_clen_blkrow<", "k_cheb_blkrow<", "k_cheb_stream<")
+# steps that read the matrix in its diagonal layout (the Laplacian has one),
+# or as plain CSR with --no-col16: their profiler names differ, the timers'
+# name the step
+STEP_FORMS = ("k_clen_blkrow<", "k_cheb_blkrow<", "k_cheb_stream<")
+DIA_NAMES = {"k_clen_blkrow": "k_dia_blk<%s,%s,8,EpiClen<%s,%s>>",
+             "k_cheb_blkrow": "k_dia_blk<%s,%s,8,EpiCheb<%s,%s>>",
+             "k_cheb_stream": "k_cheb_dia<%s,8>"}
 
 
 def profiler_name(name, col16):
-    if name.startswith(J16_KERNELS):
-        return name[:-1] + (",true>" if col16 else ",false>")
+    if name.startswith(STEP_FORMS):
+        if not col16:
+            return name[:-1] + ",false>"
+        form, args = name[:-1].split("<")
+        a = tuple(args.split(","))
+        return DIA_NAMES[form] % (a + a if len(a) > 1 else a)
     return name
 
 
@@ -520,15 +528,10 @@ def main():
                                    for k_, v in kt.items()}}
         filt = {k_: v for k_, v in kt.items() if k_.startswith("k_")}
         roof = roofline_of(filt, traffic, col16=out["config"]["col16"])
-        if roof and out["config"]["col16"] and roof["kernel"].startswith(
-                ("k_clen_blkrow", "k_cheb_blkrow", "k_cheb_stream")):
-            # the kernel read 2-byte column offsets: `achieved` counts them;
-            # the same launches against the CSR count with 4-byte indices
-            per = roof["us_per_launch"] * 1e-6
-            b32 = roof["bytes_per_launch"] + 2.0 * int(ia[-1])
-            roof["index_bytes"] = 2
-            roof["achieved_csr32"] = round(b32 / per / 1e9, 1)
-            roof["frac_csr32"] = round(b32 / per / 1e9 / HBM_PEAK_GBS, 4)
+        if roof and out["config"]["col16"] and roof["kernel"].startswith(STEP_FORMS):
+            # the Laplacian is read in its diagonal layout: one mask byte per
+            # row in place of values and indices; `achieved` counts that
+            roof["layout"] = "diagonal"
         if roof:
             roof["traffic_source"] = tsrc
             roof["measured"] = ("HIP events around each run of back-to-back launches of the kernel "

@@ -79,4 +79,105 @@ __device__ __forceinline__ T y_next(int mode, T yv, T vm, T v, T w, T m0, T m3, 
   return yv + m1 * w;
 }
 
+// y_next of column c of an interleaved block: coefficients mus[d*B + c]
+template <typename T>
+__device__ __forceinline__ T y_col(int ymode, const double *mus, int k, int B, int c, T yv, T vm,
+                                   T v, T w) {
+  const int terms = ymode & 3;
+  const T m0 = (ymode & kYInit) ? (T)mus[c] : (T)0;
+  const T m3 = terms == 3 ? (T)mus[(size_t)(k - 2) * B + c] : (T)0;
+  const T m2 = terms >= 2 ? (T)mus[(size_t)(k - 1) * B + c] : (T)0;
+  return y_next<T>(ymode, yv, vm, v, w, m0, m3, m2, (T)mus[(size_t)k * B + c]);
+}
+
+// Epilogues of the block steps on piece `piece` (columns piece*P ..) of row r:
+// load() reads the row's own operands (before the row sum where the kernel can,
+// so that their latency overlaps its loads), finish() applies the recurrence
+// to the row sum acc and stores.
+
+// three-term step (same operations as k_cheb_blkrow)
+template <typename T, int B>
+struct EpiCheb {
+  const T *vk, *vkm1;
+  T *vkp1, *y;
+  T cc, t;
+  const double *mus;
+  int k, nact, ymode;
+  static constexpr int P = Pieces<T, B>::P;
+  struct Ops {
+    T v[P], vm[P], yy[P];
+  };
+  __device__ __forceinline__ void load(int r, int piece, Ops &o) const {
+    const size_t at = (size_t)r * B + piece * P;
+    ld_piece<T, P>(vk + at, o.v);
+    // with kYInit, columns >= nact still keep y
+    if (ymode != kYSkip) ld_piece<T, P>(y + at, o.yy);
+    if (vkm1) {
+      ld_piece<T, P>(vkm1 + at, o.vm);
+    } else {
+#pragma unroll
+      for (int e = 0; e < P; e++) o.vm[e] = 0;
+    }
+  }
+  __device__ __forceinline__ void finish(int r, int piece, Ops &o, const T (&acc)[P]) const {
+#pragma clang fp contract(off)
+    const size_t at = (size_t)r * B + piece * P;
+    T w[P];
+#pragma unroll
+    for (int e = 0; e < P; e++) {
+      w[e] = acc[e] + (-cc) * o.v[e];
+      w[e] = w[e] * t;
+      if (vkm1) w[e] = w[e] + (T)(-1) * o.vm[e];
+    }
+    if (ymode != kYSkip) {
+#pragma unroll
+      for (int e = 0; e < P; e++) {
+        const int c = piece * P + e;
+        if (c < nact) o.yy[e] = y_col<T>(ymode, mus, k, B, c, o.yy[e], o.vm[e], o.v[e], w[e]);
+      }
+      st_piece<T, P>(y + at, o.yy);
+    }
+    st_piece<T, P>(vkp1 + at, w);
+  }
+};
+
+// Clenshaw step (same operations as k_clen_blkrow); b1 is the gathered block
+template <typename T, int B>
+struct EpiClen {
+  const T *b1, *b2, *v;
+  T *out;
+  T cc, t;
+  const double *mus;
+  int k;
+  static constexpr int P = Pieces<T, B>::P;
+  struct Ops {
+    T bb[P], vv[P], b2r[P], mu[P];
+  };
+  __device__ __forceinline__ void load(int r, int piece, Ops &o) const {
+    const size_t at = (size_t)r * B + piece * P;
+    ld_piece<T, P>(b1 + at, o.bb);
+    ld_piece<T, P>(v + at, o.vv);
+    if (b2) {
+      ld_piece<T, P>(b2 + at, o.b2r);
+    } else {
+#pragma unroll
+      for (int e = 0; e < P; e++) o.b2r[e] = 0;
+    }
+#pragma unroll
+    for (int e = 0; e < P; e++) o.mu[e] = (T)mus[(size_t)k * B + piece * P + e];
+  }
+  __device__ __forceinline__ void finish(int r, int piece, Ops &o, const T (&acc)[P]) const {
+#pragma clang fp contract(off)
+    T w[P];
+#pragma unroll
+    for (int e = 0; e < P; e++) {
+      T z = acc[e] + (-cc) * o.bb[e];
+      z = z * t;
+      z = z + o.mu[e] * o.vv[e];
+      w[e] = z + (T)(-1) * o.b2r[e];
+    }
+    st_piece<T, P>(out + (size_t)r * B + piece * P, w);
+  }
+};
+
 }  // namespace pevsl

@@ -106,6 +106,65 @@ k_cheb_dia(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask,
   if (ymode != kYSkip) y[r] = y_next<T>(ymode, yv, vm, v, w, m0, m3, m2, m1);
 }
 
+// sum of row r times piece pc (columns pc*P ..) of the interleaved block x
+template <typename T, int B, int UC>
+__device__ __forceinline__ void dia_row_piece(const DiaArg<T, UC> &d, uint32_t m, T dgv, int r,
+                                              int pc, const T *__restrict__ x,
+                                              T (&acc)[Pieces<T, B>::P]) {
+#pragma clang fp contract(off)
+  constexpr int P = Pieces<T, B>::P;
+  constexpr int CH = UC < 8 ? UC : 8;
+#pragma unroll
+  for (int e = 0; e < P; e++) acc[e] = 0;
+#pragma unroll
+  for (int q0 = 0; q0 < UC; q0 += CH) {
+    T xv[CH][P];
+#pragma unroll
+    for (int q = 0; q < CH; q++) {
+      const uint32_t row = (m >> (q0 + q)) & 1 ? (uint32_t)(r + d.off[q0 + q]) : 0u;
+      const uint32_t at = (row * (uint32_t)B + (uint32_t)(pc * P)) * (uint32_t)sizeof(T);
+      ld_piece<T, P>(reinterpret_cast<const T *>(reinterpret_cast<const char *>(x) + at), xv[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < CH; q++) {
+      const T a = q0 + q == d.qd ? dgv : d.c[q0 + q];
+      const bool on = (m >> (q0 + q)) & 1;
+#pragma unroll
+      for (int e = 0; e < P; e++) {
+        const T s = acc[e] + a * xv[q][e];
+        acc[e] = on ? s : acc[e];
+      }
+    }
+  }
+}
+
+// One degree of the filter on B interleaved columns, one thread per (row,
+// 16-byte piece): every load is contiguous over the wave.  Bound by the vector
+// passes (four of n B values) once they exceed the latency of one trip; the
+// row-per-thread CSR kernels gather whole rows with one thread each, wait for
+// their LDS staging, and have Q times fewer threads.  Microseconds per launch,
+// row kernels -> this kernel:
+//   100^3, FP32 Clenshaw    B=4 19.1 -> 11.0  8: 28.9 -> 19.0  16: 77.7 -> 33.8
+//   100^3, FP64 three-term  B=4 38.0 -> 18.4  8: 91.3 -> 32.8
+//   48x40x44, FP32 Clenshaw B=8 5.9 -> 3.7    20^3, FP32 B=8 5.2 -> 2.9
+// (100^3, B=8 FP32: 129 MB, 6.8 TB/s, served by the Infinity Cache.)
+template <typename T, int B, int UC, class Epi>
+__global__ void __launch_bounds__(kThreads)
+k_dia_blk(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask, const T *__restrict__ x,
+          Epi epi) {
+  constexpr uint32_t Q = Pieces<T, B>::Q;
+  const uint32_t g = (uint32_t)xcd_block(blockIdx.x, gridDim.x) * kThreads + threadIdx.x;
+  const int r = (int)(g / Q), pc = (int)(g % Q);
+  if (r >= n) return;
+  const uint32_t m = mask[r];
+  const T dgv = d.qd >= 0 ? d.dg[r] : (T)0;
+  typename Epi::Ops ops;
+  epi.load(r, pc, ops);
+  T acc[Pieces<T, B>::P];
+  dia_row_piece<T, B, UC>(d, m, dgv, r, pc, x, acc);
+  epi.finish(r, pc, ops, acc);
+}
+
 template <typename T, int UC>
 DiaArg<T, UC> dia_arg(const DevDia &D) {
   DiaArg<T, UC> d;
@@ -157,5 +216,63 @@ template void dia_cheb_step<double>(const DevCsr &, const double *, const double
 template void dia_cheb_step<float>(const DevCsr &, const float *, const float *, float *, float *,
                                    double, double, double, double, double, double, int,
                                    hipStream_t);
+
+namespace {
+// k_dia_blk of width B with epilogue `epi`
+template <typename T, int B, class Epi>
+void dia_blk_launch(const DevCsr &A, const T *x, const Epi &epi, hipStream_t s) {
+  dia_dispatch(A.dia, [&](auto uc) {
+    constexpr int UC = decltype(uc)::value;
+    hipLaunchKernelGGL((k_dia_blk<T, B, UC, Epi>),
+                       dim3(grid_for((size_t)A.n * Pieces<T, B>::Q)), dim3(kThreads), 0, s, A.n,
+                       dia_arg<T, UC>(A.dia), (const DiaMask<UC> *)A.dia.mask, x, epi);
+  });
+}
+
+// f(std::integral_constant<int, B>) for the block width
+template <class F>
+void width_dispatch(int B, F &&f) {
+  switch (B) {
+#define CASE(BB)                              \
+  case BB:                                    \
+    f(std::integral_constant<int, BB>{});     \
+    break;
+    CASE(1) CASE(2) CASE(4) CASE(8) CASE(16) CASE(32)
+#undef CASE
+    default:
+      break;
+  }
+}
+}  // namespace
+
+template <typename T>
+void dia_cheb_blk(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1, T *y, double cc,
+                  double t, const double *mus, int k, int nact, hipStream_t s, int ymode) {
+  width_dispatch(B, [&](auto b) {
+    constexpr int BB = decltype(b)::value;
+    dia_blk_launch<T, BB>(
+        A, vk, EpiCheb<T, BB>{vk, vkm1, vkp1, y, (T)cc, (T)t, mus, k, nact, ymode}, s);
+  });
+}
+template <typename T>
+void dia_clen_blk(const DevCsr &A, int B, const T *b1, const T *b2, const T *v, T *out, double cc,
+                  double t, const double *mus, int k, hipStream_t s) {
+  width_dispatch(B, [&](auto b) {
+    constexpr int BB = decltype(b)::value;
+    dia_blk_launch<T, BB>(A, b1, EpiClen<T, BB>{b1, b2, v, out, (T)cc, (T)t, mus, k}, s);
+  });
+}
+template void dia_cheb_blk<double>(const DevCsr &, int, const double *, const double *, double *,
+                                   double *, double, double, const double *, int, int, hipStream_t,
+                                   int);
+template void dia_cheb_blk<float>(const DevCsr &, int, const float *, const float *, float *,
+                                  float *, double, double, const double *, int, int, hipStream_t,
+                                  int);
+template void dia_clen_blk<double>(const DevCsr &, int, const double *, const double *,
+                                   const double *, double *, double, double, const double *, int,
+                                   hipStream_t);
+template void dia_clen_blk<float>(const DevCsr &, int, const float *, const float *,
+                                  const float *, float *, double, double, const double *, int,
+                                  hipStream_t);
 
 }  // namespace pevsl

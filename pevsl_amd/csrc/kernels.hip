@@ -379,17 +379,6 @@ k_cheb_blk(int n, const int *__restrict__ ia, const int *__restrict__ ja,
   }
 }
 
-// y_next of column c of an interleaved block: coefficients mus[d*B + c]
-template <typename T>
-__device__ __forceinline__ T y_col(int ymode, const double *mus, int k, int B, int c, T yv, T vm,
-                                   T v, T w) {
-  const int terms = ymode & 3;
-  const T m0 = (ymode & kYInit) ? (T)mus[c] : (T)0;
-  const T m3 = terms == 3 ? (T)mus[(size_t)(k - 2) * B + c] : (T)0;
-  const T m2 = terms >= 2 ? (T)mus[(size_t)(k - 1) * B + c] : (T)0;
-  return y_next<T>(ymode, yv, vm, v, w, m0, m3, m2, (T)mus[(size_t)k * B + c]);
-}
-
 // Row-per-thread block step for B interleaved columns: the row block's
 // a/ja are staged in LDS (coalesced), then each thread owns one row and
 // gathers whole B-wide rows of vk with 16-byte loads, so one memory
@@ -695,81 +684,6 @@ __global__ void k_blk_colscale(size_t n, int B, const T *__restrict__ v, T *__re
 // rounded before they are added and staged rows are summed in column order,
 // so those rows round exactly as in the row-per-thread kernels.
 
-// Epilogue of the three-term step (same operations as k_cheb_blkrow) on
-// columns [piece*P, piece*P + P) of row r.
-template <typename T, int B>
-struct EpiCheb {
-  const T *vk, *vkm1;
-  T *vkp1, *y;
-  T cc, t;
-  const double *mus;
-  int k, nact, ymode;
-  __device__ __forceinline__ void operator()(int r, int piece,
-                                             const T (&acc)[Pieces<T, B>::P]) const {
-#pragma clang fp contract(off)
-    constexpr int P = Pieces<T, B>::P;
-    const size_t o = (size_t)r * B + piece * P;
-    T v[P], vm[P], yy[P], w[P];
-    ld_piece<T, P>(vk + o, v);
-    if (ymode != kYSkip) ld_piece<T, P>(y + o, yy);
-    if (vkm1) {
-      ld_piece<T, P>(vkm1 + o, vm);
-    } else {
-#pragma unroll
-      for (int e = 0; e < P; e++) vm[e] = 0;
-    }
-#pragma unroll
-    for (int e = 0; e < P; e++) {
-      w[e] = acc[e] + (-cc) * v[e];
-      w[e] = w[e] * t;
-      if (vkm1) w[e] = w[e] + (T)(-1) * vm[e];
-    }
-    if (ymode != kYSkip) {
-#pragma unroll
-      for (int e = 0; e < P; e++) {
-        const int c = piece * P + e;
-        if (c < nact) yy[e] = y_col<T>(ymode, mus, k, B, c, yy[e], vm[e], v[e], w[e]);
-      }
-      st_piece<T, P>(y + o, yy);
-    }
-    st_piece<T, P>(vkp1 + o, w);
-  }
-};
-
-// Epilogue of the Clenshaw step (same operations as k_clen_blkrow); b1 is the
-// gathered block.
-template <typename T, int B>
-struct EpiClen {
-  const T *b1, *b2, *v;
-  T *out;
-  T cc, t;
-  const double *mus;
-  int k;
-  __device__ __forceinline__ void operator()(int r, int piece,
-                                             const T (&acc)[Pieces<T, B>::P]) const {
-#pragma clang fp contract(off)
-    constexpr int P = Pieces<T, B>::P;
-    const size_t o = (size_t)r * B + piece * P;
-    T bb[P], vv[P], b2r[P], w[P];
-    ld_piece<T, P>(b1 + o, bb);
-    ld_piece<T, P>(v + o, vv);
-    if (b2) {
-      ld_piece<T, P>(b2 + o, b2r);
-    } else {
-#pragma unroll
-      for (int e = 0; e < P; e++) b2r[e] = 0;
-    }
-#pragma unroll
-    for (int e = 0; e < P; e++) {
-      T z = acc[e] + (-cc) * bb[e];
-      z = z * t;
-      z = z + (T)mus[(size_t)k * B + piece * P + e] * vv[e];
-      w[e] = z + (T)(-1) * b2r[e];
-    }
-    st_piece<T, P>(out + o, w);
-  }
-};
-
 // U = NZ / S = 8 products per thread and block: each thread first issues
 // its 8 index and value loads (nontemporal: the matrix streams once per step
 // and should not evict the gathered block from the caches), then its 8
@@ -889,7 +803,11 @@ k_blk_bal(const int *__restrict__ rowblk, const int *__restrict__ ia,
           Epi epi) {
   __shared__ T prod[Pieces<T, B>::NZ * B];
   bal_rows<T, B>(xcd_block(blockIdx.x, gridDim.x), rowblk, ia, ja, a, x, prod,
-                 [&](int r, int pc, const T (&acc)[Pieces<T, B>::P]) { epi(r, pc, acc); });
+                 [&](int r, int pc, const T (&acc)[Pieces<T, B>::P]) {
+                   typename Epi::Ops o;
+                   epi.load(r, pc, o);
+                   epi.finish(r, pc, o, acc);
+                 });
 }
 
 // KPM step on B interleaved vectors with the nnz-balanced products (uneven
@@ -1982,6 +1900,10 @@ void cheb_step_blkrow(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp
                       T *y, double cc, double t, const double *mus, int k,
                       int nact, hipStream_t s, int ymode) {
   if (A.n == 0 || nact <= 0 || A.nrowblk == 0) return;
+  if (use_dia(A, sizeof(T), B)) {
+    dia_cheb_blk<T>(A, B, vk, vkm1, vkp1, y, cc, t, mus, k, nact, s, ymode);
+    return;
+  }
   const T *a = std::is_same<T, double>::value ? (const T *)A.a64
                                               : (const T *)A.a32;
   switch (B) {
@@ -2009,6 +1931,10 @@ void clen_step_blkrow(const DevCsr &A, int B, const T *b1, const T *b2, const T 
   if (!b1) {  // top term: no product
     hipLaunchKernelGGL((k_blk_colscale<T>), dim3(grid_for((size_t)A.n * B)), dim3(kThreads), 0,
                        s, (size_t)A.n, B, v, out, mus, k);
+    return;
+  }
+  if (use_dia(A, sizeof(T), B)) {
+    dia_clen_blk<T>(A, B, b1, b2, v, out, cc, t, mus, k, s);
     return;
   }
   const T *a = std::is_same<T, double>::value ? (const T *)A.a64 : (const T *)A.a32;

@@ -145,6 +145,13 @@ void dia_cheb_step(const DevCsr &A, const T *vk, const T *vkm1, T *vkp1, T *y, d
                    double t, double mu0, double mu3, double mu2, double mu1, int ymode,
                    hipStream_t s);
 
+template <typename T>
+void dia_cheb_blk(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1, T *y, double cc,
+                  double t, const double *mus, int k, int nact, hipStream_t s, int ymode);
+template <typename T>
+void dia_clen_blk(const DevCsr &A, int B, const T *b1, const T *b2, const T *v, T *out, double cc,
+                  double t, const double *mus, int k, hipStream_t s);
+
 // Same for B interleaved columns (row-major n x B block, column fastest).
 // mus: device array [(deg_max+1) x B] of per-column coefficients; k = degree
 // index of this step (1..); columns c >= nact are left untouched.
@@ -154,7 +161,8 @@ void cheb_step_blk(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1,
                    int nact, hipStream_t s);
 
 // Same with one thread per row (row blocks of the CSR-stream partition,
-// a/ja staged in LDS, B-wide 16-byte row gathers); B <= 32.  y is updated as
+// a/ja staged in LDS, B-wide 16-byte row gathers), or on the diagonal layout
+// with one thread per (row, 16-byte piece); B <= 32.  y is updated as
 // `ymode` says, for columns c < nact (active at the lowest degree whose term
 // is added; mus is zero past each column's degree).
 template <typename T>
@@ -162,7 +170,7 @@ void cheb_step_blkrow(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp
                       T *y, double cc, double t, const double *mus, int k,
                       int nact, hipStream_t s, int ymode);
 
-// Clenshaw step on B interleaved columns (row per thread, B <= 32):
+// Clenshaw step on B interleaved columns (same kernels, B <= 32):
 //   out = mu_k v + t (A b1 - cc b1) - b2,  mu_k per column = mus[k*B + c];
 // b2 == nullptr reads as zero; b1 == nullptr gives the top term out = mu_k v.
 template <typename T>

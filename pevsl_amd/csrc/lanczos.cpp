@@ -326,6 +326,7 @@ struct GroupGraph {
   hipGraphExec_t exec = nullptr;
   char *blocks = nullptr;  // filter-block allocation the graph was captured on
   double bytes = 0.0;      // algorithmic bytes of one replay
+  double kbytes = 0.0;     // bytes its kernels move
   long long steps = 0, launches = 0;
   std::string kname;
   bool used = false;
@@ -429,6 +430,7 @@ class BatchSolver {
   pevsl_Data *p_;
   int ns_;
   bool capture_ = false;  // filter_block enqueues kernels only (graph capture)
+  double kbytes_ = 0.0;   // bytes the last enqueued group's kernels move
   int n_ = 0;
   bool b32_ = false;  // FP32 basis storage
   size_t vb_ = 8;     // basis element bytes
@@ -632,6 +634,8 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
   const bool segk = kind == 5;
   const bool clen = kind == 2 || kind == 4;
   const bool bal = kind == 3 || kind == 4;
+  const bool dia = (kind == 1 || kind == 2) && use_dia(A, (int)elem, B);
+  kbytes_ = 0.0;
   auto run = [&](auto *tag) {
     using T = std::remove_pointer_t<decltype(tag)>;
     T *x = (T *)xb[0], *y = (T *)xb[1];
@@ -683,6 +687,7 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
         b1 = out;
         yout = out;
       }
+      kbytes_ += kbytes;
       if (tok >= 0) c_.kt.end(c_.stream, tok, degmax + 1, kbytes);
     } else if (clen && degmax >= 1) {
       // Clenshaw sums from the top degree down: b_d = mu_d x + (2/dd)(A - cc)
@@ -723,6 +728,8 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
         b1 = out;
         yout = out;
       }
+      kbytes -= degmax * dia_saved_bytes(A, (int)elem, index_bytes(A), dia);
+      kbytes_ += kbytes;
       if (tok >= 0) c_.kt.end(c_.stream, tok, degmax, kbytes);
     } else {
     // third work buffer: reuse x once it is no longer read (after step 2)
@@ -770,6 +777,8 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
       vkm1 = vk;
       vk = vkp1;
     }
+    kbytes -= degmax * dia_saved_bytes(A, (int)elem, index_bytes(A), dia);
+    kbytes_ += kbytes;
     if (tok >= 0) c_.kt.end(c_.stream, tok, degmax, kbytes);
     }
     if constexpr (std::is_same<T, float>::value) {
@@ -899,13 +908,14 @@ void BatchSolver::filter_group_graph(const std::vector<int> &grp, int k) {
     gg->blocks = base;
     // the capture counted one application that has not run
     gg->bytes = c_.kstats.filter_bytes - ks.filter_bytes;
+    gg->kbytes = kbytes_;
     gg->steps = c_.kstats.filter_steps - ks.filter_steps;
     gg->launches = c_.kstats.filter_launches - ks.filter_launches;
     c_.kstats = ks;
   }
   const long tok = c_.kt.begin(c_.stream, gg->kname.c_str());
   PV_HIP(hipGraphLaunch(gg->exec, c_.stream));
-  c_.kt.end(c_.stream, tok, gg->launches, gg->bytes);
+  c_.kt.end(c_.stream, tok, gg->launches, gg->kbytes);
   c_.kstats.filter_bytes += gg->bytes;
   c_.kstats.filter_steps += gg->steps;
   c_.kstats.filter_launches += gg->launches;

@@ -119,6 +119,54 @@ def test_product_equals_csr(lib, name):
         M.free()
 
 
+@pytest.mark.parametrize("mat", ["lap3d", "pot", "9_diags"])
+@pytest.mark.parametrize("prec,kind,width", [(0, 1, 2), (0, 1, 4), (0, 1, 8), (0, 1, 16),
+                                             (1, 1, 2), (1, 1, 4), (1, 2, 8), (1, 1, 16),
+                                             (1, 2, 32)])
+def test_block_steps_equal_csr(lib, mat, prec, kind, width):
+    """Batched solves of 7 slices (groups of the width and a remainder), with
+    slices whose degrees differ: same steps, eigenvalues and residuals."""
+    print("\n[gpu case] diagonal layout, block %s prec %d kind %d width %d" % (
+        mat, prec, kind, width), flush=True)
+    if mat == "9_diags":
+        ia, ja, a = banded(1201, [-90, -11, -2, -1, 0, 1, 2, 11, 90], vary=[0], seed=2)
+        top = 20.0
+        i = np.repeat(np.arange(1201), np.diff(ia))
+        a = np.where(ja == i, 10.0 + a, 0.3 + 0.1 * (np.abs(ja - i) % 7))  # symmetric
+    else:
+        ia, ja, a = driver.laplacian3d(9, 8, 11)
+        top = 12.0
+        if mat == "pot":
+            i = np.repeat(np.arange(len(ia) - 1), np.diff(ia))
+            a = np.where(ja == i, a + np.random.default_rng(3).random(len(a)), a)
+            top = 13.0
+    M = driver.Matrix(lib, ia, ja, a)
+    edges = np.array([0.02, 0.1, 0.15, 0.3, 0.33, 0.5, 0.55, 0.65]) * top
+    intvs = [[edges[i], edges[i + 1], 0.0, top] for i in range(7)]
+    pols = [driver.find_pol(lib, iv)[0] for iv in intvs]
+    vinit = np.random.default_rng(5).uniform(-1, 1, M.n)
+    runs = []
+    try:
+        for on in (True, False):
+            inst = driver.Instance(lib, M, prec=prec, block_rowkernel=kind, block_width=width,
+                                   col16=on)
+            try:
+                rc, outs = driver.cheblan_batch(inst, intvs, [60] * 7, 1e-8, vinit, pols)
+                assert rc == 0
+                runs.append(outs)
+            finally:
+                inst.close()
+    finally:
+        for p_ in pols:
+            lib.pEVSL_FreePol(C.byref(p_))
+        M.free()
+    for x, y in zip(*runs):
+        assert x["info"]["its"] == y["info"]["its"]
+        assert x["info"]["tr"] == y["info"]["tr"]
+        np.testing.assert_array_equal(x["lam"], y["lam"])
+        np.testing.assert_array_equal(x["res"], y["res"])
+
+
 def test_rectangular_product(lib):
     print("\n[gpu case] diagonal layout, rectangular products", flush=True)
     for nr, nc in ((300, 40), (40, 300)):
