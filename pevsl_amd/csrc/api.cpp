@@ -193,6 +193,12 @@ void rand_vectors(Ctx &c, int n, int nvec, double *d_out, size_t ld) {
     }
     return;
   }
+  if (ld == (size_t)n) {  // consecutive counters: one launch for all vectors
+    rand_fill((size_t)n * nvec, d_out, c.rand_seed, c.rand_offset,
+              c.rand_mode == PEVSL_RAND_RADEMACHER, c.stream);
+    c.rand_offset += (unsigned long long)n * nvec;
+    return;
+  }
   for (int v = 0; v < nvec; v++) {
     rand_fill((size_t)n, d_out + (size_t)v * ld, c.rand_seed, c.rand_offset,
               c.rand_mode == PEVSL_RAND_RADEMACHER, c.stream);

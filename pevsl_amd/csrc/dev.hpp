@@ -180,4 +180,105 @@ struct EpiClen {
   }
 };
 
+// ---- KPM step --------------------------------------------------------------
+// Sums of one thread over its rows' piece of P columns, in FP64: s[0] = w.w,
+// s[1] = w.v and (first step) s[2] = v.v for the step v -> w; or, with the
+// start vectors v0 given, s[0] = w.v0 alone.
+template <int P>
+struct KpmSums {
+  double s[3][P];
+  __device__ __forceinline__ KpmSums() {
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int e = 0; e < P; e++) s[i][e] = 0.0;
+  }
+};
+
+// The step on piece pc of row r: w = scal (acc - ctr v) - vm, written over vm
+// (vw; vm is zero, and not read, on the first step), and its sums.  acc, ctr
+// and scal are of type AT: with AT = double on FP32 vectors the step rounds to
+// FP32 once, where it stores w.
+template <typename T, int B, typename AT>
+struct EpiKpm {
+  const T *v;
+  T *vw;
+  const T *v0;
+  AT ctr, scal;
+  int first;
+  static constexpr int P = Pieces<T, B>::P;
+  struct Ops {
+    T v[P], vm[P], z[P];
+  };
+  __device__ __forceinline__ void load(int r, int pc, Ops &o) const {
+    const size_t at = (size_t)r * B + pc * P;
+    ld_piece<T, P>(v + at, o.v);
+    if (v0) ld_piece<T, P>(v0 + at, o.z);
+    if (!first) {
+      ld_piece<T, P>(vw + at, o.vm);
+    } else {
+#pragma unroll
+      for (int e = 0; e < P; e++) o.vm[e] = 0;
+    }
+  }
+  __device__ __forceinline__ void finish(int r, int pc, const Ops &o, const AT (&acc)[P],
+                                         KpmSums<P> &s) const {
+#pragma clang fp contract(off)
+    T w[P];
+#pragma unroll
+    for (int e = 0; e < P; e++) {
+      AT x = acc[e] + (-ctr) * (AT)o.v[e];
+      x = x * scal;
+      w[e] = (T)(x + (AT)(-1) * (AT)o.vm[e]);
+      const double we = w[e], ve = o.v[e];
+      if (v0) {
+        s.s[0][e] += we * (double)o.z[e];
+      } else {
+        s.s[0][e] += we * we;
+        s.s[1][e] += we * ve;
+        if (first) s.s[2][e] += ve * ve;
+      }
+    }
+    st_piece<T, P>(vw + (size_t)r * B + pc * P, w);
+  }
+  // sums a launch writes per column
+  __device__ __forceinline__ int nsum() const { return v0 ? 1 : first ? 3 : 2; }
+  // group `g` of vectors, gstride elements apart
+  __device__ __forceinline__ void group(int g, size_t gstride) {
+    v += g * gstride;
+    vw += g * gstride;
+    if (v0) v0 += g * gstride;
+  }
+};
+
+// Block sums of the threads' KpmSums (thread t holds piece t % Q) in a fixed
+// order: lanes of a wave that hold the same piece, then the waves.  Sum i <
+// nsum of column c goes to part[(i*ncol + c) * nblk + blk].
+template <typename T, int B>
+__device__ __forceinline__ void kpm_block_sums(const KpmSums<Pieces<T, B>::P> &s, int nsum,
+                                               int ncol, int nblk, int blk, double *part) {
+  constexpr int P = Pieces<T, B>::P, Q = Pieces<T, B>::Q, W = kThreads / 64;
+  __shared__ double red[3][W][B];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, pc = threadIdx.x % Q;
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    if (i >= nsum) break;
+#pragma unroll
+    for (int e = 0; e < P; e++) {
+      double x = s.s[i][e];
+#pragma unroll
+      for (int off = 32; off >= Q; off >>= 1) x += __shfl_xor(x, off, 64);
+      if (lane < Q) red[i][wave][pc * P + e] = x;
+    }
+  }
+  __syncthreads();
+  for (int u = threadIdx.x; u < nsum * B; u += kThreads) {
+    const int i = u / B, c = u % B;
+    double x = 0.0;
+#pragma unroll
+    for (int w = 0; w < W; w++) x += red[i][w][c];
+    part[((size_t)i * ncol + c) * nblk + blk] = x;
+  }
+}
+
 }  // namespace pevsl

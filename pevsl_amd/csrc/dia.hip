@@ -16,6 +16,7 @@
 // results equal the CSR kernels' bit for bit.
 #include "dev.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace pevsl {
@@ -24,10 +25,10 @@ namespace {
 
 // Diagonals as kernel arguments (scalar registers); entries past ndiag have
 // no mask bit.
-template <typename T, int UC>
+template <typename T, int UC, typename C = T>
 struct DiaArg {
   int off[UC];
-  T c[UC];
+  C c[UC];
   int qd;
   const T *dg;
 };
@@ -106,11 +107,12 @@ k_cheb_dia(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask,
   if (ymode != kYSkip) y[r] = y_next<T>(ymode, yv, vm, v, w, m0, m3, m2, m1);
 }
 
-// sum of row r times piece pc (columns pc*P ..) of the interleaved block x
-template <typename T, int B, int UC>
-__device__ __forceinline__ void dia_row_piece(const DiaArg<T, UC> &d, uint32_t m, T dgv, int r,
+// sum of row r times piece pc (columns pc*P ..) of the interleaved block x,
+// in type C
+template <typename T, int B, int UC, typename C = T>
+__device__ __forceinline__ void dia_row_piece(const DiaArg<T, UC, C> &d, uint32_t m, T dgv, int r,
                                               int pc, const T *__restrict__ x,
-                                              T (&acc)[Pieces<T, B>::P]) {
+                                              C (&acc)[Pieces<T, B>::P]) {
 #pragma clang fp contract(off)
   constexpr int P = Pieces<T, B>::P;
   constexpr int CH = UC < 8 ? UC : 8;
@@ -127,11 +129,11 @@ __device__ __forceinline__ void dia_row_piece(const DiaArg<T, UC> &d, uint32_t m
     }
 #pragma unroll
     for (int q = 0; q < CH; q++) {
-      const T a = q0 + q == d.qd ? dgv : d.c[q0 + q];
+      const C a = q0 + q == d.qd ? (C)dgv : d.c[q0 + q];
       const bool on = (m >> (q0 + q)) & 1;
 #pragma unroll
       for (int e = 0; e < P; e++) {
-        const T s = acc[e] + a * xv[q][e];
+        const C s = acc[e] + a * (C)xv[q][e];
         acc[e] = on ? s : acc[e];
       }
     }
@@ -165,12 +167,45 @@ k_dia_blk(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask, const T 
   epi.finish(r, pc, ops, acc);
 }
 
-template <typename T, int UC>
-DiaArg<T, UC> dia_arg(const DevDia &D) {
-  DiaArg<T, UC> d;
+// One KPM step on B interleaved columns, group blockIdx.y: each workgroup
+// takes `iters` runs of kThreads (row, piece) items, so that its sums end in
+// one reduction and one set of partials.  Bound by the three vector passes
+// (u_j, u_j-1 read, u_j+1 over it).  Whole pEVSL_Kpmdos, against one thread per
+// (row, column) and one product per moment: 100^3, Mdeg 300, 64 FP32 vectors
+// 263 -> 33.6 ms (600 launches of 192 MB: 3.4 TB/s); 20^3, 60 FP64 vectors 8.8
+// -> 3.5 ms, of which 2.5 ms are the rand() stream on the host.
+template <typename T, int B, int UC>
+__global__ void __launch_bounds__(kThreads)
+k_dia_kpm(int n, DiaArg<T, UC, double> d, const DiaMask<UC> *__restrict__ mask,
+          EpiKpm<T, B, double> epi, size_t gstride, int iters, int ncol,
+          double *__restrict__ part) {
+  constexpr uint32_t Q = Pieces<T, B>::Q;
+  constexpr int P = Pieces<T, B>::P;
+  const int blk = xcd_block(blockIdx.x, gridDim.x);
+  epi.group(blockIdx.y, gstride);
+  KpmSums<P> sums;
+  for (int it = 0; it < iters; it++) {
+    const uint32_t g = ((uint32_t)blk * iters + it) * kThreads + threadIdx.x;
+    const int r = (int)(g / Q), pc = (int)(g % Q);
+    if (r >= n) break;
+    const uint32_t m = mask[r];
+    const T dgv = d.qd >= 0 ? d.dg[r] : (T)0;
+    typename EpiKpm<T, B, double>::Ops ops;
+    epi.load(r, pc, ops);
+    double acc[P];
+    dia_row_piece<T, B, UC, double>(d, m, dgv, r, pc, epi.v, acc);
+    epi.finish(r, pc, ops, acc, sums);
+  }
+  kpm_block_sums<T, B>(sums, epi.nsum(), ncol, gridDim.x, blk,
+                       part + (size_t)blockIdx.y * B * gridDim.x);
+}
+
+template <typename T, int UC, typename C = T>
+DiaArg<T, UC, C> dia_arg(const DevDia &D) {
+  DiaArg<T, UC, C> d;
   for (int q = 0; q < UC; q++) {
     d.off[q] = q < D.ndiag ? D.off[q] : 0;
-    d.c[q] = q < D.ndiag ? (T)D.c[q] : (T)0;
+    d.c[q] = q < D.ndiag ? (C)D.c[q] : (C)0;
   }
   d.qd = D.qd;
   d.dg = std::is_same<T, double>::value ? (const T *)D.dg64 : (const T *)D.dg32;
@@ -274,5 +309,38 @@ template void dia_clen_blk<double>(const DevCsr &, int, const double *, const do
 template void dia_clen_blk<float>(const DevCsr &, int, const float *, const float *,
                                   const float *, float *, double, double, const double *, int,
                                   hipStream_t);
+
+// runs of kThreads (row, piece) items per workgroup: as many as leave about
+// kKpmBlocks workgroups (eight per CU)
+constexpr int kKpmBlocks = 2048;
+static int dia_kpm_iters(int n, int elem, int B) {
+  const long long items = (long long)n * std::max(1, B * elem / 16);
+  return (int)((items + (long long)kThreads * kKpmBlocks - 1) / ((long long)kThreads * kKpmBlocks));
+}
+int dia_kpm_blocks(int n, int elem, int B) {
+  const long long items = (long long)n * std::max(1, B * elem / 16);
+  const long long per = (long long)kThreads * dia_kpm_iters(n, elem, B);
+  return (int)((items + per - 1) / per);
+}
+
+template <typename T>
+void dia_kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, double ctr,
+                  double scal, bool first, double *part, hipStream_t s) {
+  width_dispatch(B, [&](auto b) {
+    constexpr int BB = decltype(b)::value;
+    dia_dispatch(A.dia, [&](auto uc) {
+      constexpr int UC = decltype(uc)::value;
+      hipLaunchKernelGGL((k_dia_kpm<T, BB, UC>),
+                         dim3(dia_kpm_blocks(A.n, sizeof(T), BB), ng), dim3(kThreads), 0, s, A.n,
+                         dia_arg<T, UC, double>(A.dia), (const DiaMask<UC> *)A.dia.mask,
+                         EpiKpm<T, BB, double>{v, vw, v0, ctr, scal, first ? 1 : 0},
+                         (size_t)A.n * BB, dia_kpm_iters(A.n, sizeof(T), BB), ng * BB, part);
+    });
+  });
+}
+template void dia_kpm_step<double>(const DevCsr &, int, int, const double *, double *,
+                                   const double *, double, double, bool, double *, hipStream_t);
+template void dia_kpm_step<float>(const DevCsr &, int, int, const float *, float *, const float *,
+                                  double, double, bool, double *, hipStream_t);
 
 }  // namespace pevsl

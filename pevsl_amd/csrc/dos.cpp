@@ -1,10 +1,9 @@
 // dos.cpp -- density of states and spectrum slicing on the GPU.
 //
 // pEVSL_Kpmdos (SRC/kpmdos.c:36-197): all nvec random vectors advance
-// together as the columns of one interleaved block; each degree is one fused
-// launch (kernels.hip k_kpm_blk: SpMM + three-term recurrence + per-column
-// dot with v0; k_kpm_bal, in blocks of at most 32 vectors, when a row has
-// more than 64 entries).  For the generalized problem the moments come from
+// together as the columns of interleaved blocks; a step is one fused launch
+// (dia.hip k_dia_kpm or kernels.hip k_kpm_bal: SpMM + three-term recurrence +
+// dot products), and half as many steps as moments suffice (kpm_moments).  For the generalized problem the moments come from
 // the B-solve form (gen.cpp).  The per-(vector, degree) dots come back to the host, where
 // mu and the eigenvalue count are accumulated in the reference's order
 // (vector-major), so the host arithmetic matches the reference exactly.
@@ -76,70 +75,103 @@ Aux &aux() {
   return *a;
 }
 
+// dots[m*Mdeg + k-1] = <v_m, T_k v_m> of unit random vectors v_m, T_k the
+// Chebyshev polynomials of the scaled matrix.  With u_j = T_j v they follow
+// from the products of neighbours (T_2j = 2 T_j^2 - 1, T_2j+1 = 2 T_j+1 T_j -
+// T_1, A symmetric):
+//   <v, T_2j v> = 2 <u_j, u_j> - <v, v>,  <v, T_2j+1 v> = 2 <u_j+1, u_j> - <v, T_1 v>
+// so that half of the products with A give all Mdeg moments, and a step reads
+// u_j and u_j-1 and writes u_j+1, without v.  All is divided by <v, v>, whose
+// distance from 1 is the rounding of v.
+//
+// These differences carry the rounding errors of u_j in full, where <v, T_k v>
+// carries them scaled by the moment.  In FP64, and on the diagonal layout,
+// whose steps compute in FP64 and round FP32 vectors once, the moments are as
+// accurate or more so (relative error of mu, FP32 vectors: 100^3 3.6e-8 ->
+// 2.1e-8, 20^3 1.2e-7 -> 3.4e-9); with FP32 arithmetic throughout they would
+// be ten times worse (100^3: 4e-7).  FP32 on the other matrices therefore
+// takes one product per moment and the dot product with v.
 template <typename T>
 void kpm_moments(Ctx &c, int n, int Mdeg, int nvec, double ctr, double wid,
                  std::vector<double> &dots /* [nvec][Mdeg] */) {
   const DevCsr &A = *c.A;
   const hipStream_t s = c.stream;
-  // uneven rows: nnz-balanced step, blocks of at most 32 vectors
-  const bool bal = A.max_row > kUnevenRow;
-  const int bmax = bal ? 32 : 64;
+  const int elem = (int)sizeof(T);
+  if (Mdeg < 1 || nvec < 1) return;
+  // Width of a group of interleaved vectors: 32, or on the diagonal layout
+  // what leaves its two blocks in the Infinity Cache from step to step (the
+  // balanced kernels gather whole rows and gain from width in any case); as
+  // many groups in one launch as fit there together.
+  constexpr double kResident = 160e6;
+  const bool dia = use_dia(A, elem, 32);
+  const bool direct = !dia && elem == 4;
   int B = 1;
-  while (B < nvec && B < bmax) B *= 2;
-  const size_t blk = (size_t)n * B;
-  DBuf<double> raw, part, dd;
-  DBuf<T> v0, b0, b1, b2;
-  raw.ensure((size_t)n * B);
-  v0.ensure(blk);
-  b0.ensure(blk);
-  b1.ensure(blk);
-  b2.ensure(blk);
-  int nrb = kpm_part_blocks(n, B);
-  if (bal) nrb = std::max(nrb, A.nrowblk_q[bal_level((int)sizeof(T), B)]);
-  part.ensure((size_t)nrb * B);
-  dd.ensure((size_t)Mdeg * B + (size_t)dot_part_blocks(n) + 8);
-  DBuf<double *> cp;
-  cp.ensure((size_t)B);
-  std::vector<double> hd((size_t)Mdeg * B);
-  std::vector<double> nrm((size_t)B);
-  for (int v0i = 0; v0i < nvec; v0i += B) {
-    const int nb = std::min(B, nvec - v0i);
-    // random vectors, unit 2-norm (SRC/kpmdos.c:117-121)
+  while (B < nvec && B < 32 && (!dia || B < 4 || 4.0 * n * B * elem <= kResident)) B *= 2;
+  const double gbytes = 2.0 * n * B * elem;
+  const int ng = std::max(1, std::min((nvec + B - 1) / B, (int)std::min(64.0, kResident / gbytes)));
+  const int W = ng * B;                            // vectors per run
+  const int nst = direct ? Mdeg : (Mdeg + 1) / 2;  // products
+  const int ns = direct ? 1 : 2;                   // sums per step and column
+  const int nblk = kpm_blocks(A, elem, B);
+  // partials of `keep` steps before they are summed
+  const int keep = (int)std::max(1.0, std::min((double)std::min(nst, 64),
+                                               64e6 / (16.0 * W * nblk)));
+  const size_t blk = (size_t)n * W;
+  DBuf<double> raw, part, sums, nrm;
+  DBuf<T> buf;
+  raw.ensure(blk);
+  part.ensure((size_t)(ns * keep + 1) * W * nblk);
+  sums.ensure((size_t)(ns * nst + 1) * W);
+  nrm.ensure((size_t)W * (col_part_blocks(n) + 1));
+  T *b0 = buf.ensure((direct ? 3 : 2) * blk);
+  std::vector<double> hs((size_t)(ns * nst + 1) * W);
+  for (int m0 = 0; m0 < nvec; m0 += W) {
+    const int nb = std::min(W, nvec - m0);
     rand_vectors(c, n, nb, raw.p, (size_t)n);
-    for (int j = 0; j < nb; j++) {
-      double *col = raw.p + (size_t)j * n;
-      double *pt = dd.p + (size_t)Mdeg * B;
-      const int np = dot_partials(n, col, col, pt, s);
-      reduce_partials(pt, np, 1, dd.p + j, s);
+    col_dots(n, nb, raw.p, (size_t)n, raw.p, (size_t)n, nrm.p + W, nrm.p, s);
+    kpm_pack<T>(n, B, ng, nb, raw.p, nrm.p, b0, s);
+    const T *v = b0, *v0 = nullptr;
+    T *vw = b0 + blk;
+    if (direct) {
+      v0 = b0 + 2 * blk;
+      PV_HIP(hipMemcpyAsync(b0 + 2 * blk, b0, sizeof(T) * blk, hipMemcpyDeviceToDevice, s));
     }
-    PV_HIP(hipMemcpyAsync(nrm.data(), dd.p, sizeof(double) * nb, hipMemcpyDeviceToHost, s));
-    PV_HIP(hipStreamSynchronize(s));
-    for (int j = 0; j < nb; j++)
-      scale_vec(n, raw.p + (size_t)j * n, nullptr, 1.0 / sqrt(nrm[(size_t)j]), s);
-    std::vector<double *> ptrs((size_t)B, nullptr);
-    for (int j = 0; j < nb; j++) ptrs[(size_t)j] = raw.p + (size_t)j * n;
-    PV_HIP(hipMemcpyAsync(cp.p, ptrs.data(), sizeof(double *) * B, hipMemcpyHostToDevice, s));
-    pack_cols<T>(n, B, nb, cp.p, v0.p, s);
-    // vk = v0, vkm1 = 0
-    PV_HIP(hipMemcpyAsync(b0.p, v0.p, sizeof(T) * blk, hipMemcpyDeviceToDevice, s));
-    PV_HIP(hipMemsetAsync(b1.p, 0, sizeof(T) * blk, s));
-    T *vk = b0.p, *vkm1 = b1.p, *vkp1 = b2.p;
-    for (int k = 0; k < Mdeg; k++) {
-      const double scal = (k == 0 ? 1.0 : 2.0) / wid;
-      const int nbk = bal ? kpm_step_bal<T>(A, B, vk, vkm1, vkp1, v0.p, ctr, scal, part.p, s)
-                          : kpm_step_blk<T>(A, B, vk, vkm1, vkp1, v0.p, ctr, scal, part.p, s);
-      reduce_partials(part.p, nbk, B, dd.p + (size_t)k * B, s);
-      T *t = vkm1;
-      vkm1 = vk;
-      vk = vkp1;
-      vkp1 = t;
+    // step j's sums: rows ns j W .. (w.w, w.v; or w.v0) of `sums`; v.v (step
+    // 0's third) goes to the end
+    int pend = 0, done = 0;
+    for (int j = 0; j < nst; j++) {
+      double *pt = part.p + (size_t)ns * pend * W * nblk;
+      kpm_step<T>(A, B, ng, v, vw, v0, ctr, (j == 0 ? 1.0 : 2.0) / wid, j == 0, pt, s);
+      if (j == 0 && !direct)
+        row_sums(pt + (size_t)2 * W * nblk, W, nblk, sums.p + (size_t)2 * nst * W, s);
+      pend++;
+      if (pend == keep || j == nst - 1) {
+        row_sums(part.p, ns * pend * W, nblk, sums.p + (size_t)ns * done * W, s);
+        done += pend;
+        pend = 0;
+      }
+      T *t = const_cast<T *>(v);
+      v = vw;
+      vw = t;
       c.kstats.filter_steps += nb;
     }
-    PV_HIP(hipMemcpyAsync(hd.data(), dd.p, sizeof(double) * Mdeg * B, hipMemcpyDeviceToHost, s));
+    PV_HIP(hipMemcpyAsync(hs.data(), sums.p, sizeof(double) * hs.size(), hipMemcpyDeviceToHost,
+                          s));
     PV_HIP(hipStreamSynchronize(s));
-    for (int j = 0; j < nb; j++)
-      for (int k = 0; k < Mdeg; k++)
-        dots[(size_t)(v0i + j) * Mdeg + k] = hd[(size_t)k * B + j];
+    for (int m = 0; m < nb; m++) {
+      double *d = dots.data() + (size_t)(m0 + m) * Mdeg;
+      if (direct) {
+        for (int k = 0; k < Mdeg; k++) d[k] = hs[(size_t)k * W + m];
+        continue;
+      }
+      const double vv = hs[(size_t)2 * nst * W + m], d1 = hs[(size_t)W + m];
+      for (int j = 0; j < nst; j++) {
+        // step j gives <u_j+1, u_j> and <u_j+1, u_j+1>
+        if (2 * j < Mdeg)
+          d[2 * j] = (j == 0 ? d1 : 2.0 * hs[(size_t)(2 * j + 1) * W + m] - d1) / vv;
+        if (2 * j + 1 < Mdeg) d[2 * j + 1] = (2.0 * hs[(size_t)2 * j * W + m] - vv) / vv;
+      }
+    }
   }
 }
 
@@ -213,6 +245,7 @@ int pEVSL_Kpmdos(pevsl_Data *pevsl, int Mdeg, int damping, int nvec, double *int
   jackson_like(Mdeg, damping, jac);
   jac[0] = 1.0;
   std::vector<double> dots((size_t)nvec * Mdeg);
+  const long long steps0 = c.kstats.filter_steps;
   EvTimer ev;
   ev.start(c.stream);
   if (pevsl->ifGenEv) {
@@ -230,7 +263,7 @@ int pEVSL_Kpmdos(pevsl_Data *pevsl, int Mdeg, int damping, int nvec, double *int
     kpm_moments<double>(c, n, Mdeg, nvec, ctr, wid, dots);
   ev.stop(c.stream);
   c.kstats.t_kpm += ev.seconds();
-  if (c.A && !pevsl->ifGenEv) pevsl->stats->n_mvA += (size_t)nvec * Mdeg;
+  if (c.A && !pevsl->ifGenEv) pevsl->stats->n_mvA += (size_t)(c.kstats.filter_steps - steps0);
   // accumulation in the reference order (SRC/kpmdos.c:104-157)
   memset(mu, 0, sizeof(double) * (size_t)(Mdeg + 1));
   double tcnt = 0.0;

@@ -20,13 +20,13 @@
 //     of columns), up to 64 FP32 columns in one pass over the matrix, each
 //     piece active from its own top degree (uneven degrees cost their own
 //     steps only, at 4-column granularity).
-//   * k_blk_bal (epilogues EpiCheb / EpiClen) and k_kpm_bal : the same steps
+//   * k_blk_bal (epilogues EpiCheb / EpiClen) : the same steps
 //     for matrices with uneven rows, parallel over (nonzero, 16-byte piece)
 //     with the products staged in LDS and summed per row in column order.
 //   * k_cheb_blk : B columns with one lane per (row, column).
-//   * k_kpm_blk : one degree of the KPM recurrence (SRC/kpmdos.c:129-156) for
-//     all random vectors at once, fused with the per-column dot product
-//     against v0 (block partial sums, deterministic second stage).
+//   * k_kpm_bal : one degree of the KPM recurrence (SRC/kpmdos.c:129-156) for
+//     up to 32 random vectors a group, fused with the per-column dot products
+//     (block partial sums, deterministic second stage).
 //   * k_lan_* : Lanczos vector updates and classical Gram-Schmidt with the
 //     DGKS test (SRC/cheblanNr.c:219-246, SRC/miscla.c:211-240) as batched
 //     tall-skinny GEMV-T / GEMV-N over chunked Lanczos bases (FP64 or FP32
@@ -810,93 +810,66 @@ k_blk_bal(const int *__restrict__ rowblk, const int *__restrict__ ia,
                  });
 }
 
-// KPM step on B interleaved vectors with the nnz-balanced products (uneven
-// rows): vkp1 = scal (A vk - ctr vk) - vkm1 and, per column, the partial dot
-// of vkp1 with v0 over the row block, part[rb * B + c] (rb = row block, so
-// the second-stage sum runs in row order whatever the dispatch order).
+// KPM step on B interleaved vectors with the nnz-balanced products; group
+// blockIdx.y of vectors (stride gstride elements, B columns of ncol each).
 template <typename T, int B>
 __global__ void __launch_bounds__(kThreads)
 k_kpm_bal(const int *__restrict__ rowblk, const int *__restrict__ ia,
-          const int *__restrict__ ja, const T *__restrict__ a, const T *__restrict__ vk,
-          const T *__restrict__ vkm1, T *__restrict__ vkp1, const T *__restrict__ v0, T ctr,
-          T scal, double *__restrict__ part) {
-#pragma clang fp contract(off)
-  using PC = Pieces<T, B>;
-  constexpr int P = PC::P, Q = PC::Q;
-  __shared__ T prod[PC::NZ * B];
+          const int *__restrict__ ja, const T *__restrict__ a, EpiKpm<T, B, T> epi, size_t gstride,
+          int ncol, double *__restrict__ part) {
+  constexpr int P = Pieces<T, B>::P;
+  __shared__ T prod[Pieces<T, B>::NZ * B];
   const int rb = xcd_block(blockIdx.x, gridDim.x);
-  double dsum[P];
-#pragma unroll
-  for (int e = 0; e < P; e++) dsum[e] = 0.0;
-  bal_rows<T, B>(rb, rowblk, ia, ja, a, vk, prod, [&](int r, int pc, const T (&acc)[P]) {
-    const size_t o = (size_t)r * B + pc * P;
-    T v[P], vm[P], z[P], w[P];
-    ld_piece<T, P>(vk + o, v);
-    ld_piece<T, P>(vkm1 + o, vm);
-    ld_piece<T, P>(v0 + o, z);
-#pragma unroll
-    for (int e = 0; e < P; e++) {
-      w[e] = acc[e] + (-ctr) * v[e];
-      w[e] = w[e] * scal;
-      w[e] = w[e] + (T)(-1) * vm[e];
-      dsum[e] += (double)w[e] * (double)z[e];
-    }
-    st_piece<T, P>(vkp1 + o, w);
+  epi.group(blockIdx.y, gstride);
+  KpmSums<P> sums;
+  bal_rows<T, B>(rb, rowblk, ia, ja, a, epi.v, prod, [&](int r, int pc, const T (&acc)[P]) {
+    typename EpiKpm<T, B, T>::Ops o;
+    epi.load(r, pc, o);
+    epi.finish(r, pc, o, acc, sums);
   });
-  // per column: sum over the threads holding its piece, in thread order
+  kpm_block_sums<T, B>(sums, epi.nsum(), ncol, gridDim.x, rb,
+                       part + (size_t)blockIdx.y * B * gridDim.x);
+}
+
+// Packs column-major FP64 vectors (leading dim n) as unit vectors into groups
+// of B interleaved columns of type T: column c of the batch, divided by
+// sqrt(nrm2[c]) (SRC/kpmdos.c:117-121), is column c % B of group c / B; columns
+// past ncol are zero.  Blocks of 64 rows turn through LDS, so that both sides
+// are read and written in runs.
+template <typename T>
+__global__ void __launch_bounds__(kThreads)
+k_kpm_pack(int n, int B, int ncol, const double *__restrict__ raw,
+           const double *__restrict__ nrm2, T *__restrict__ blk) {
+  __shared__ T tile[64][33];
+  const int r0 = blockIdx.x * 64, g = blockIdx.y;
+  blk += (size_t)g * n * B;
+  for (int u = threadIdx.x; u < 64 * B; u += kThreads) {
+    const int r = u & 63, c = u >> 6, gc = g * B + c;
+    double x = 0.0;
+    if (r0 + r < n && gc < ncol) x = raw[(size_t)gc * n + r0 + r] * (1.0 / sqrt(nrm2[gc]));
+    tile[r][c] = (T)x;
+  }
   __syncthreads();
-  double *red = reinterpret_cast<double *>(prod);
-  static_assert(kThreads * P * sizeof(double) <= PC::NZ * B * sizeof(T), "LDS reuse");
-#pragma unroll
-  for (int e = 0; e < P; e++) red[threadIdx.x * P + e] = dsum[e];
-  __syncthreads();
-  if (threadIdx.x < B) {
-    const int c = threadIdx.x, pc = c / P, e = c % P;
-    double sum = 0.0;
-    for (int t = pc; t < kThreads; t += Q) sum += red[t * P + e];
-    part[(size_t)rb * B + c] = sum;
+  for (int u = threadIdx.x; u < 64 * B; u += kThreads) {
+    const int r = u / B, c = u % B;
+    if (r0 + r < n) blk[(size_t)(r0 + r) * B + c] = tile[r][c];
   }
 }
 
-// KPM step + per-column partial dot with v0 over the block's rows.
-template <typename T, int B>
+// out[i] = sum of part[i*nblk ..], one block per sum, fixed order
 __global__ void __launch_bounds__(kThreads)
-k_kpm_blk(int n, const int *__restrict__ ia, const int *__restrict__ ja,
-          const T *__restrict__ a, const T *__restrict__ vk,
-          const T *__restrict__ vkm1, T *__restrict__ vkp1,
-          const T *__restrict__ v0, T ctr, T scal, double *__restrict__ part,
-          int rows_per_block) {
-#pragma clang fp contract(off)
-  constexpr int RPW = 64 / B;  // rows per wave per sweep
-  __shared__ double red[kThreads / 64][B];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int c = lane % B;
-  const int rsub = lane / B;
-  const int row0 = blockIdx.x * rows_per_block;
-  const int row_end = min(n, row0 + rows_per_block);
-  double dsum = 0.0;
-  for (int row = row0 + wave * RPW + rsub; row < row_end;
-       row += (kThreads / 64) * RPW) {
-    T acc = 0;
-    const int e = ia[row + 1];
-    for (int j = ia[row]; j < e; j++) acc += a[j] * vk[(size_t)ja[j] * B + c];
-    const size_t idx = (size_t)row * B + c;
-    T w = acc + (-ctr) * vk[idx];
-    w = w * scal;
-    w = w + (T)(-1) * vkm1[idx];
-    vkp1[idx] = w;
-    dsum += (double)w * (double)v0[idx];
-  }
-  // reduce over the rows held by this wave (lanes with equal c)
-#pragma unroll
-  for (int off = 32; off >= B; off >>= 1) dsum += __shfl_xor(dsum, off, 64);
-  if (rsub == 0) red[wave][c] = dsum;
+k_row_sums(const double *__restrict__ part, int nblk, double *__restrict__ out) {
+  __shared__ double red[kThreads / 64];
+  const double *p = part + (size_t)blockIdx.x * nblk;
+  double s = 0.0;
+  for (int b = threadIdx.x; b < nblk; b += kThreads) s += p[b];
+  s = wave_sum(s);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x < B) {
-    double s = 0.0;
-#pragma unroll
-    for (int w = 0; w < kThreads / 64; w++) s += red[w][threadIdx.x];
-    part[(size_t)blockIdx.x * B + threadIdx.x] = s;
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int w = 0; w < kThreads / 64; w++) t += red[w];
+    out[blockIdx.x] = t;
   }
 }
 
@@ -2006,74 +1979,57 @@ template void cheb_step_blk<float>(const DevCsr &, int, const float *,
                                    double, const double *, int, int,
                                    hipStream_t);
 
-// rows per block of the KPM kernel: enough rows that every block does a few
-// sweeps, and at most ~4096 blocks.
-static int kpm_rows_per_block(int n, int B) {
-  const int rpw = 64 / B;
-  const int sweep = (kThreads / 64) * rpw;
-  int rpb = sweep * 4;
-  while ((n + rpb - 1) / rpb > 4096) rpb *= 2;
-  return rpb;
-}
-
-int kpm_part_blocks(int n, int B) {
-  const int rpb = kpm_rows_per_block(n, B);
-  return (n + rpb - 1) / rpb;
+int kpm_blocks(const DevCsr &A, int elem, int B) {
+  if (use_dia(A, elem, B)) return dia_kpm_blocks(A.n, elem, B);
+  return A.nrowblk_q[bal_level(elem, B)];
 }
 
 template <typename T>
-int kpm_step_blk(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1,
-                 const T *v0, double ctr, double scal, double *part,
-                 hipStream_t s) {
-  const int rpb = kpm_rows_per_block(A.n, B);
-  const int nb = (A.n + rpb - 1) / rpb;
-  const T *a = std::is_same<T, double>::value ? (const T *)A.a64
-                                              : (const T *)A.a32;
-  switch (B) {
-#define CASE(BB)                                                             \
-  case BB:                                                                   \
-    hipLaunchKernelGGL((k_kpm_blk<T, BB>), dim3(nb), dim3(kThreads), 0, s,   \
-                       A.n, A.ia, A.ja, a, vk, vkm1, vkp1, v0, (T)ctr,       \
-                       (T)scal, part, rpb);                                  \
-    break;
-    CASE(1) CASE(2) CASE(4) CASE(8) CASE(16) CASE(32) CASE(64)
-#undef CASE
-    default:
-      return 0;
+void kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, double ctr,
+              double scal, bool first, double *part, hipStream_t s) {
+  if (A.n == 0) return;
+  if (use_dia(A, sizeof(T), B)) {
+    dia_kpm_step<T>(A, B, ng, v, vw, v0, ctr, scal, first, part, s);
+    return;
   }
-  return nb;
-}
-template <typename T>
-int kpm_step_bal(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1, const T *v0,
-                 double ctr, double scal, double *part, hipStream_t s) {
   const int lv = bal_level((int)sizeof(T), B);
-  if (lv > 4 || !A.rowblk_q[lv] || A.nrowblk_q[lv] == 0) return 0;
+  if (lv > 4 || A.nrowblk_q[lv] == 0) return;
   const T *a = std::is_same<T, double>::value ? (const T *)A.a64 : (const T *)A.a32;
   switch (B) {
-#define CASE(BB)                                                                          \
-  case BB:                                                                                \
-    hipLaunchKernelGGL((k_kpm_bal<T, BB>), dim3(A.nrowblk_q[lv]), dim3(kThreads), 0, s,   \
-                       A.rowblk_q[lv], A.ia, A.ja, a, vk, vkm1, vkp1, v0, (T)ctr, (T)scal, \
-                       part);                                                             \
+#define CASE(BB)                                                                           \
+  case BB:                                                                                 \
+    hipLaunchKernelGGL((k_kpm_bal<T, BB>), dim3(A.nrowblk_q[lv], ng), dim3(kThreads), 0, s, \
+                       A.rowblk_q[lv], A.ia, A.ja, a,                                       \
+                       EpiKpm<T, BB, T>{v, vw, v0, (T)ctr, (T)scal, first ? 1 : 0},         \
+                       (size_t)A.n * BB, ng * BB, part);                                    \
     break;
     CASE(1) CASE(2) CASE(4) CASE(8) CASE(16) CASE(32)
 #undef CASE
     default:
-      return 0;
+      break;
   }
-  return A.nrowblk_q[lv];
 }
-template int kpm_step_bal<double>(const DevCsr &, int, const double *, const double *, double *,
-                                  const double *, double, double, double *, hipStream_t);
-template int kpm_step_bal<float>(const DevCsr &, int, const float *, const float *, float *,
-                                 const float *, double, double, double *, hipStream_t);
+template void kpm_step<double>(const DevCsr &, int, int, const double *, double *, const double *,
+                               double, double, bool, double *, hipStream_t);
+template void kpm_step<float>(const DevCsr &, int, int, const float *, float *, const float *,
+                              double, double, bool, double *, hipStream_t);
 
-template int kpm_step_blk<double>(const DevCsr &, int, const double *,
-                                  const double *, double *, const double *,
-                                  double, double, double *, hipStream_t);
-template int kpm_step_blk<float>(const DevCsr &, int, const float *,
-                                 const float *, float *, const float *, double,
-                                 double, double *, hipStream_t);
+template <typename T>
+void kpm_pack(int n, int B, int ng, int ncol, const double *raw, const double *nrm2, T *blk,
+              hipStream_t s) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL((k_kpm_pack<T>), dim3((n + 63) / 64, ng), dim3(kThreads), 0, s, n, B, ncol,
+                     raw, nrm2, blk);
+}
+template void kpm_pack<double>(int, int, int, int, const double *, const double *, double *,
+                               hipStream_t);
+template void kpm_pack<float>(int, int, int, int, const double *, const double *, float *,
+                              hipStream_t);
+
+void row_sums(const double *part, int nrows, int nblk, double *out, hipStream_t s) {
+  if (nrows <= 0) return;
+  hipLaunchKernelGGL(k_row_sums, dim3(nrows), dim3(kThreads), 0, s, part, nblk, out);
+}
 
 void reduce_partials(const double *part, int nblk, int ncol, double *out,
                      hipStream_t s) {

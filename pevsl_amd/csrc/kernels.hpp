@@ -206,20 +206,28 @@ void clen_step_bal(const DevCsr &A, int B, const T *b1, const T *b2, const T *v,
 // partition index of the balanced kernels for element size elem, width B
 int bal_level(int elem, int B);
 
-// KPM step on B interleaved columns:
-//   vkp1 = scal (A vk - ctr vk) - vkm1,   part[blk][c] = sum_rows vkp1*v0
-// returns the number of row blocks (partials per column) written.
+// One KPM step v -> w = scal (A v - ctr v) - vm of ng groups of B interleaved
+// columns (group g at v + g n B; B a power of two <= 32), w written over vm
+// (vw); vm is zero, and not read, if `first`.  Per column c = g B + b the block
+// partials of w.w, w.v and (first) v.v, or of w.v0 alone where v0 is given:
+// part[(i ng B + c) nblk + blk] for sum i and blk < nblk = kpm_blocks(A,
+// sizeof(T), B).  On the diagonal layout (row sums and recurrence in FP64
+// whatever T is) or with the nnz-balanced products (in T).
 template <typename T>
-int kpm_step_blk(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1,
-                 const T *v0, double ctr, double scal, double *part,
-                 hipStream_t s);
-int kpm_part_blocks(int n, int B);
-// The same step with the nnz-balanced products (uneven rows, B <= 32):
-// partials per row block of the balanced partition, returns their number
-// (0 if B has no partition).
+void kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, double ctr,
+              double scal, bool first, double *part, hipStream_t s);
+int kpm_blocks(const DevCsr &A, int elem, int B);
+int dia_kpm_blocks(int n, int elem, int B);
 template <typename T>
-int kpm_step_bal(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1, const T *v0,
-                 double ctr, double scal, double *part, hipStream_t s);
+void dia_kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, double ctr,
+                  double scal, bool first, double *part, hipStream_t s);
+// raw: ncol column-major n-vectors; group g of blk gets columns g B .. as
+// x / sqrt(nrm2[c]), zero past ncol
+template <typename T>
+void kpm_pack(int n, int B, int ng, int ncol, const double *raw, const double *nrm2, T *blk,
+              hipStream_t s);
+// out[i] = sum of part[i*nblk .. (i+1)*nblk), i < nrows
+void row_sums(const double *part, int nrows, int nblk, double *out, hipStream_t s);
 
 // ---- dense / vector kernels (FP64 unless stated) --------------------------
 // out[c] = sum_b part[b*ncol + c], b < nblk (fixed order); out may be strided.

@@ -187,3 +187,42 @@ def test_rectangular_product(lib):
         ref = np.zeros(nr)
         ref[:k] = 2.5 * x[:k]
         np.testing.assert_array_equal(y, ref)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("Mdeg,nvec", [(1, 1), (2, 3), (5, 33), (30, 70)])
+def test_kpm_on_both_layouts(lib, prec, Mdeg, nvec):
+    """Moments of odd and even counts, single vectors, padded groups and more
+    vectors than one group holds, on the diagonal layout and as CSR, against
+    the recurrence in FP64 numpy on the same rand() stream."""
+    print("\n[gpu case] KPM Mdeg %d nvec %d prec %d" % (Mdeg, nvec, prec), flush=True)
+    ia, ja, a = driver.laplacian3d(7, 9, 5)
+    n = len(ia) - 1
+    dense = np.zeros((n, n))
+    dense[np.repeat(np.arange(n), np.diff(ia)), ja] = a
+    libc = C.CDLL(None)
+    libc.srand(7)
+    t = 2147483647.0 / 2
+    v = (np.array([libc.rand() for _ in range(n * nvec)], float).reshape(nvec, n).T - t) / t
+    v /= np.linalg.norm(v, axis=0)
+    u, um, dots = v, None, []
+    for k in range(Mdeg):
+        w = (dense @ u - 6.0 * u) * ((2.0 if k else 1.0) / 6.0) - (um if k else 0.0)
+        um, u = u, w
+        dots.append(float((w * v).sum()))
+    # damping 0: mu_k = 2 / (nvec pi) sum of the dots
+    ref = np.array([1.0 / np.pi] + [2.0 / (nvec * np.pi) * d for d in dots])
+    M = driver.Matrix(lib, ia, ja, a)
+    try:
+        for on in (True, False):
+            inst = driver.Instance(lib, M, prec=prec, col16=on)
+            try:
+                lib.pEVSL_RandSeed(7)
+                rc, mu, _ = inst.kpmdos(Mdeg, 0, nvec, [3.0, 5.0, 0.0, 12.0])
+            finally:
+                inst.close()
+            assert rc == 0
+            # FP64: a few roundings of unit quantities; FP32: the path's 2e-5
+            assert np.max(np.abs(mu - ref)) <= (1e-13 if prec == 0 else 2e-5)
+    finally:
+        M.free()
