@@ -10,7 +10,6 @@
 #include <cmath>
 #include <cstring>
 #include <ctime>
-#include <memory>
 
 #include "internal.hpp"
 
@@ -655,37 +654,32 @@ int pEVSL_ParcsrSetup(pevsl_Csr *Ai, pevsl_Parcsr *A) {
   M->csr.rowblk_q[0] = M->csr.rowblk;
   M->csr.nrowblk_q[0] = M->csr.nrowblk;
   for (int l = 1; l < 5; l++) M->csr.rowblk_q[l] = M->rowblk.p + at[l];
-  // 16-bit column offsets from each row block's first row, kept when every
-  // nonzero's offset fits (banded orderings such as the natural order of a
-  // grid Laplacian; not random sparsity)
-  std::unique_ptr<short[]> jo(new short[(size_t)nnz]);
-  bool fits = nnz > 0;
-  for (size_t b = 0; fits && b + 1 < rb.size(); b++) {
-    const int r0 = rb[b];
-    for (int j = Ai->ia[r0]; j < Ai->ia[rb[b + 1]]; j++) {
-      const int d = Ai->ja[j] - r0;
-      if (d < -32768 || d > 32767) {
-        fits = false;
-        break;
-      }
-      jo[(size_t)j] = (short)d;
-    }
-  }
-  if (fits) {
-    M->csr.jo16 = M->jo16.ensure((size_t)nnz);
-    PV_HIP(hipMemcpy(M->csr.jo16, jo.get(), sizeof(short) * (size_t)nnz,
-                     hipMemcpyHostToDevice));
-  }
-  std::unique_ptr<float[]> a32(new float[(size_t)nnz]);
-  for (int j = 0; j < nnz; j++) a32[j] = (float)Ai->a[j];
   PV_HIP(hipMemcpy(M->csr.ia, Ai->ia, sizeof(int) * (size_t)(n + 1),
                    hipMemcpyHostToDevice));
   PV_HIP(hipMemcpy(M->csr.ja, Ai->ja, sizeof(int) * (size_t)nnz,
                    hipMemcpyHostToDevice));
   PV_HIP(hipMemcpy(M->csr.a64, Ai->a, sizeof(double) * (size_t)nnz,
                    hipMemcpyHostToDevice));
-  PV_HIP(hipMemcpy(M->csr.a32, a32.get(), sizeof(float) * (size_t)nnz,
-                   hipMemcpyHostToDevice));
+  // FP32 values and 16-bit column offsets are formed on the device from what
+  // is there already.  Offsets are from each row block's first row, kept when
+  // every nonzero's offset fits (banded orderings such as the natural order of
+  // a grid Laplacian; not random sparsity: a few rows tell)
+  copy_f64_to_f32((size_t)nnz, M->csr.a64, M->csr.a32, nullptr);
+  bool fits = nnz > 0;
+  for (int i = 0; fits && i < n; i += std::max(1, n / 64))
+    for (int j = Ai->ia[i]; fits && j < Ai->ia[i + 1]; j++)
+      fits = std::abs((long)Ai->ja[j] - i) < 32768 + kStreamRows;
+  if (fits) {
+    DBuf<int> over;
+    int bad = 0;
+    PV_HIP(hipMemcpy(over.ensure(1), &bad, sizeof(int), hipMemcpyHostToDevice));
+    offsets16(M->csr, M->jo16.ensure((size_t)nnz), over.p, nullptr);
+    PV_HIP(hipMemcpy(&bad, over.p, sizeof(int), hipMemcpyDeviceToHost));
+    if (bad)
+      M->jo16.release();
+    else
+      M->csr.jo16 = M->jo16.p;
+  }
   // diagonal layout, where the matrix has one
   HostDia hd;
   if (find_dia(n, Ai->ia, Ai->ja, Ai->a, hd)) {
@@ -712,6 +706,8 @@ int pEVSL_ParcsrSetup(pevsl_Csr *Ai, pevsl_Parcsr *A) {
     dd.qd = hd.qd;
     dd.ndiag = hd.ndiag;
   }
+  // instances read the copy from streams of their own
+  PV_HIP(hipStreamSynchronize(nullptr));
   A->dev = M;
   return 0;
 }

@@ -151,6 +151,20 @@ __device__ __forceinline__ int block_col(const int *__restrict__ ja, const short
 // Sparse products
 // ---------------------------------------------------------------------------
 
+// jo[j] = ja[j] - first row of j's row block; *over = 1 if one does not fit
+__global__ void __launch_bounds__(kThreads)
+k_offsets16(const int *__restrict__ rowblk, const int *__restrict__ blknz,
+            const int *__restrict__ ja, short *__restrict__ jo, int *__restrict__ over) {
+  const int r0 = rowblk[blockIdx.x], e = blknz[blockIdx.x + 1];
+  bool bad = false;
+  for (int j = blknz[blockIdx.x] + threadIdx.x; j < e; j += kThreads) {
+    const int d = ja[j] - r0;
+    bad = bad || d < -32768 || d > 32767;
+    jo[j] = (short)d;
+  }
+  if (bad) *over = 1;
+}
+
 // y = A x, L lanes per row (rows of a wave: 64/L).
 template <int L>
 __global__ void __launch_bounds__(kThreads)
@@ -1703,6 +1717,12 @@ void spmv_cols_f64(const DevCsr &A, const double *X, double *Y, int ncol,
 void spmv_f64(const DevCsr &A, const double *x, double *y, int lanes,
               hipStream_t s) {
   spmv_cols_f64(A, x, y, 1, (size_t)A.n, lanes, s);
+}
+
+void offsets16(const DevCsr &A, short *jo, int *over, hipStream_t s) {
+  if (A.nrowblk == 0) return;
+  hipLaunchKernelGGL(k_offsets16, dim3(A.nrowblk), dim3(kThreads), 0, s, A.rowblk, A.blknz, A.ja,
+                     jo, over);
 }
 
 template <typename T>

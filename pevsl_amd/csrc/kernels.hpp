@@ -80,6 +80,10 @@ constexpr int kStreamNnz = 2048;
 void build_row_blocks(int n, const int *ia, std::vector<int> &blk,
                       int max_rows = kStreamRows, int max_nnz = kStreamNnz);
 
+// jo[j] = ja[j] - (first row of nonzero j's row block); *over set to 1 if one
+// does not fit in 16 bits
+void offsets16(const DevCsr &A, short *jo, int *over, hipStream_t s);
+
 // ---- sparse products -------------------------------------------------------
 // y = A x, one column.  lanes = lanes per row in {1,2,4,8,16,32,64}, or 0 for
 // the kernel that suits the matrix: its diagonal layout, else the CSR-stream
