@@ -107,6 +107,96 @@ k_cheb_dia(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask,
   if (ymode != kYSkip) y[r] = y_next<T>(ymode, yv, vm, v, w, m0, m3, m2, m1);
 }
 
+// Coefficients of the degrees of one k_cheb_multi launch.
+template <typename T>
+struct MuArg {
+  T m0, mu[kMultiMax];
+};
+
+// Degrees d0 .. d0+s-1 of the filter for one column in one launch: a workgroup
+// owns R rows and keeps them, with the s*bw rows on either side that they
+// depend on (bw: the widest diagonal), in LDS; it steps the window, which
+// shrinks by bw at both ends per degree, with one barrier per degree, and
+// writes its own rows' last two vectors and y.  Each row goes through the
+// operations of k_cheb_dia in their order, hence the same bits; rows in the
+// overlap of two windows are computed by both.
+//
+// For grids and chains whose degree takes less than the launch around it:
+// k_cheb_dia needs 2.7-4 us a degree at any size below 1e5 rows (launch, one
+// trip to memory).  Bound by LDS reads and barriers inside, by the overlap of
+// the windows where the band is wide.  FP64, microseconds per degree, a launch
+// per degree -> best s:
+//   chain 64,000 rows 4.0 -> 0.50 (s = 32)   1e6 rows 6.6 -> 1.5 (s = 32)
+//   12^3 3.0 -> 1.34 (s = 6)    20^3 3.0 -> 2.35 (s = 5), FP32 3.0 -> 1.91
+//   60^2 4.0 -> 0.97 (s = 8)    250^2 3.8 -> 2.3 (s = 6)  400^2 4.0 -> 3.5
+// K rows of the window per thread, blockDim.x apart.
+template <typename T, int UC, int K>
+__global__ void __launch_bounds__(1024)
+k_cheb_multi(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask, int bw, int R, int d0,
+             int s, int last, const T *__restrict__ vin, const T *__restrict__ vmin,
+             T *__restrict__ vout, T *__restrict__ vmout, T *__restrict__ y, T cc, T t1, T t2,
+             MuArg<T> mus) {
+#pragma clang fp contract(off)
+  extern __shared__ char multi_lds[];
+  const int r0 = blockIdx.x * R, r1 = min(n, r0 + R);
+  const int w0 = max(0, r0 - s * bw), w1 = min(n, r1 + s * bw), L = w1 - w0;
+  T *a = reinterpret_cast<T *>(multi_lds), *b = a + L;
+  uint32_t mk[K];
+  T dg[K], yv[K];
+#pragma unroll
+  for (int i = 0; i < K; i++) {
+    const int x = threadIdx.x + i * (int)blockDim.x, r = w0 + x;
+    mk[i] = 0;
+    dg[i] = yv[i] = 0;
+    if (x < L) {
+      mk[i] = mask[r];
+      if (d.qd >= 0) dg[i] = d.dg[r];
+      const T v = vin[r];
+      a[x] = v;
+      b[x] = d0 > 1 ? vmin[r] : (T)0;
+      if (r >= r0 && r < r1) yv[i] = d0 > 1 ? y[r] : v * mus.m0;
+    }
+  }
+  __syncthreads();
+  for (int j = 0; j < s; j++) {
+    const int h = (s - 1 - j) * bw;
+    const int lo = max(0, r0 - h), hi = min(n, r1 + h);
+    const T t = d0 + j == 1 ? t1 : t2;
+#pragma unroll
+    for (int i = 0; i < K; i++) {
+      const int x = threadIdx.x + i * (int)blockDim.x, r = w0 + x;
+      if (r < lo || r >= hi) continue;
+      T acc = 0;
+#pragma unroll
+      for (int q = 0; q < UC; q++) {
+        const bool on = (mk[i] >> q) & 1;
+        const T av = q == d.qd ? dg[i] : d.c[q];
+        const T z = acc + av * a[on ? x + d.off[q] : 0];
+        acc = on ? z : acc;
+      }
+      T w = acc + (-cc) * a[x];
+      w = w * t;
+      if (d0 + j > 1) w = w + (T)(-1) * b[x];
+      b[x] = w;
+      if (r >= r0 && r < r1) yv[i] = yv[i] + mus.mu[j] * w;
+    }
+    __syncthreads();
+    T *sw = a;
+    a = b;
+    b = sw;
+  }
+#pragma unroll
+  for (int i = 0; i < K; i++) {
+    const int x = threadIdx.x + i * (int)blockDim.x, r = w0 + x;
+    if (r < r0 || r >= r1) continue;
+    y[r] = yv[i];
+    if (!last) {
+      vout[r] = a[x];
+      vmout[r] = b[x];
+    }
+  }
+}
+
 // sum of row r times piece pc (columns pc*P ..) of the interleaved block x,
 // in type C
 template <typename T, int B, int UC, typename C = T>
@@ -309,6 +399,120 @@ template void dia_clen_blk<double>(const DevCsr &, int, const double *, const do
 template void dia_clen_blk<float>(const DevCsr &, int, const float *, const float *,
                                   const float *, float *, double, double, const double *, int,
                                   hipStream_t);
+
+// Degrees per launch s and rows per workgroup R of k_cheb_multi for a filter of
+// degree m; s = 1 where one launch per degree is at least as good.  Model in
+// microseconds, fitted to the times of s = 2 .. 32 on the grids at
+// k_cheb_multi: a launch costs 4.5 and 0.8e-3 per row of the window it loads; a
+// degree inside it 0.2, and 0.5e-3 (U + 3)/10 per row it steps for U diagonals,
+// for each round of workgroups over the CUs; one launch per degree costs 3.0 +
+// 5.6e-6 n.  The window must fit 64 KiB of LDS, which ends the gain where the
+// band is wide (30^3: 900 rows either side per degree) or the grid large.
+MultiPlan dia_multi_plan(const DevCsr &A, int elem, int m) {
+  MultiPlan best;
+  if (!use_dia(A, elem, 1) || m < 2 || A.n > (1 << 20) || A.dia.ndiag > 8) return best;
+  int bw = 0;
+  for (int q = 0; q < A.dia.ndiag; q++) bw = std::max(bw, std::abs(A.dia.off[q]));
+  const double row = 0.5e-3 * (A.dia.ndiag + 3) / 10.0;
+  double tbest = 3.0 + 5.6e-6 * A.n;
+  for (int per = 1; per <= 8; per *= 2) {
+    const int R = std::max(64, (A.n + 256 * per - 1) / (256 * per));
+    const int wgs = (A.n + R - 1) / R;
+    for (int s = 2; s <= std::min(m, kMultiMax); s++) {
+      const long long L = (long long)R + 2LL * s * bw;
+      if (L > kMultiRows || 2 * L * elem > kMultiLds) break;
+      const double t = (4.5 + 0.8e-3 * (double)L) / s +
+                       ((wgs + 255) / 256) * (0.2 + row * (R + (double)bw * (s - 1)));
+      if (t < tbest) {
+        tbest = t;
+        best.s = s;
+        best.R = R;
+        best.bw = bw;
+      }
+    }
+  }
+  // equal launches
+  if (best.s > 1) best.s = (m + (m + best.s - 1) / best.s - 1) / ((m + best.s - 1) / best.s);
+  return best;
+}
+
+template <typename T>
+void dia_cheb_multi(const DevCsr &A, const MultiPlan &p, const T *v, const T *vm, T *vout,
+                    T *vmout, T *y, double cc, double dd, const double *mu, int d0, int s,
+                    bool last, hipStream_t st) {
+  MuArg<T> ma;
+  ma.m0 = (T)mu[0];
+  for (int j = 0; j < kMultiMax; j++) ma.mu[j] = j < s ? (T)mu[d0 + j] : (T)0;
+  const int L = p.R + 2 * s * p.bw;
+  const int nt = std::min(1024, (L + 63) / 64 * 64);
+  const int K = (L + nt - 1) / nt;
+  auto go = [&](auto uc, auto k) {
+    constexpr int UC = decltype(uc)::value, KK = decltype(k)::value;
+    hipLaunchKernelGGL((k_cheb_multi<T, UC, KK>), dim3((A.n + p.R - 1) / p.R), dim3(nt),
+                       2 * (size_t)L * sizeof(T), st, A.n, dia_arg<T, UC>(A.dia),
+                       (const DiaMask<UC> *)A.dia.mask, p.bw, p.R, d0, s, last ? 1 : 0, v, vm,
+                       vout, vmout, y, (T)cc, (T)(1.0 / dd), (T)(2.0 / dd), ma);
+  };
+  auto width = [&](auto uc) {
+    if (K <= 1)
+      go(uc, std::integral_constant<int, 1>{});
+    else if (K <= 2)
+      go(uc, std::integral_constant<int, 2>{});
+    else
+      go(uc, std::integral_constant<int, 4>{});
+  };
+  if (A.dia.ndiag <= 4)
+    width(std::integral_constant<int, 4>{});
+  else
+    width(std::integral_constant<int, 8>{});
+}
+template void dia_cheb_multi<double>(const DevCsr &, const MultiPlan &, const double *,
+                                     const double *, double *, double *, double *, double, double,
+                                     const double *, int, int, bool, hipStream_t);
+template void dia_cheb_multi<float>(const DevCsr &, const MultiPlan &, const float *,
+                                    const float *, float *, float *, float *, double, double,
+                                    const double *, int, int, bool, hipStream_t);
+
+template <typename T>
+double cheb_run(const DevCsr &A, const double *mu, int m, double cc, double dd, const T *x, T *y,
+                T *w, hipStream_t st) {
+  const int n = A.n;
+  const double vec = (double)n * sizeof(T);
+  const bool dia = use_dia(A, sizeof(T), 1);
+  const double mat = dia ? (double)n * (dia_mask_bytes(A.dia) + (A.dia.qd >= 0 ? sizeof(T) : 0))
+                         : (double)A.nnz * (sizeof(T) + index_bytes(A)) + 4.0 * (n + 1);
+  const T *vk = x, *vkm1 = nullptr;
+  double bytes = 0.0;
+  const MultiPlan p = dia_multi_plan(A, sizeof(T), m);
+  if (p.s > 1) {
+    int set = 0;
+    for (int d = 1; d <= m; d += p.s, set ^= 1) {
+      const int s = std::min(p.s, m + 1 - d);
+      T *vo = w + (size_t)2 * set * n, *vmo = vo + n;
+      dia_cheb_multi<T>(A, p, vk, vkm1, vo, vmo, y, cc, dd, mu, d, s, d + s > m, st);
+      vk = vo;
+      vkm1 = vmo;
+      bytes += mat + (d == 1 ? 2.0 : 4.0) * vec + (d + s > m ? 0.0 : 2.0) * vec;
+    }
+    return bytes;
+  }
+  T *b[3] = {w, w + n, w + 2 * (size_t)n};
+  YPlan yp;
+  for (int k = 1; k <= m; k++) {
+    T *vkp1 = b[(k - 1) % 3];
+    const int ymode = yp.next(k, m);
+    cheb_step_stream<T>(A, vk, vkm1, vkp1, y, cc, k == 1 ? 1.0 / dd : 2.0 / dd, mu[0],
+                        k > 2 ? mu[k - 2] : 0.0, mu[k - 1], mu[k], ymode, st);
+    vkm1 = vk;
+    vk = vkp1;
+    bytes += mat + ((k == 1 ? 2 : 3) + y_passes(ymode)) * vec;
+  }
+  return bytes;
+}
+template double cheb_run<double>(const DevCsr &, const double *, int, double, double,
+                                 const double *, double *, double *, hipStream_t);
+template double cheb_run<float>(const DevCsr &, const double *, int, double, double, const float *,
+                                float *, float *, hipStream_t);
 
 // runs of kThreads (row, piece) items per workgroup: as many as leave about
 // kKpmBlocks workgroups (eight per CU)

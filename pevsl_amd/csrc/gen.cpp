@@ -35,7 +35,7 @@ struct LSPolData {
   double cc = 0.0, dd = 1.0, tol = 0.0;
   std::vector<double> mu;
   pevsl_Parcsr *Bp = nullptr;  // its HBM copy is looked up at the first solve
-  DBuf<double> wk;          // 3 n recurrence vectors + 2 n staging for host calls
+  DBuf<double> wk;          // 4 n recurrence vectors + 2 n staging for host calls
   hipStream_t s = nullptr;  // stream of host-array calls (pEVSL_LSPolSol)
 };
 
@@ -54,18 +54,7 @@ void lspol_apply(const LSPolData &L, const double *dx, double *dy, double *wk, h
     scale_vec(n, dy, nullptr, mu[0], s);
     return;
   }
-  double *b[3] = {wk, wk + n, wk + 2 * (size_t)n};
-  const double *vk = dx, *vkm1 = nullptr;
-  int nb = 0;
-  YPlan yp;
-  for (int k = 1; k <= m; k++) {
-    double *vkp1 = b[nb];
-    nb = (nb + 1) % 3;
-    cheb_step_stream<double>(B, vk, vkm1, vkp1, dy, L.cc, k == 1 ? 1.0 / L.dd : 2.0 / L.dd, mu[0],
-                             k > 2 ? mu[k - 2] : 0.0, mu[k - 1], mu[k], yp.next(k, m), s);
-    vkm1 = vk;
-    vk = vkp1;
-  }
+  cheb_run<double>(B, mu, m, L.cc, L.dd, dx, dy, wk, s);
 }
 
 // sum_{j <= m} mu_j T_j(x) by the three-term recurrence (chebxPltd,
@@ -144,7 +133,7 @@ void solve_with(Ctx &c, pevsl_Data *p, SVFunc f, void *data, const double *dx, d
   if (f == pEVSL_LSPolSol) {
     const LSPolData &L = *static_cast<const LSPolData *>(data);
     if (L.n != p->n) fatal("LSPol data of another size", __FILE__, __LINE__);
-    lspol_apply(L, dx, dy, c.gen_lsw.ensure((size_t)3 * p->n), c.stream);
+    lspol_apply(L, dx, dy, c.gen_lsw.ensure((size_t)4 * p->n), c.stream);
     return;
   }
   if (f == pEVSL_ChebIterSolv1 || f == pEVSL_ChebIterSolv2) {
@@ -580,10 +569,10 @@ void pEVSL_LSPolSol(double *db, double *dx, void *data) {
   LSPolData &L = *static_cast<LSPolData *>(data);
   const int n = L.n;
   if (!L.s) PV_HIP(hipStreamCreateWithFlags(&L.s, hipStreamNonBlocking));
-  double *w = L.wk.ensure((size_t)5 * n);
-  PV_HIP(hipMemcpyAsync(w + 3 * (size_t)n, db, sizeof(double) * n, hipMemcpyHostToDevice, L.s));
-  lspol_apply(L, w + 3 * (size_t)n, w + 4 * (size_t)n, w, L.s);
-  PV_HIP(hipMemcpyAsync(dx, w + 4 * (size_t)n, sizeof(double) * n, hipMemcpyDeviceToHost, L.s));
+  double *w = L.wk.ensure((size_t)6 * n), *b = w + 4 * (size_t)n, *x = b + n;
+  PV_HIP(hipMemcpyAsync(b, db, sizeof(double) * n, hipMemcpyHostToDevice, L.s));
+  lspol_apply(L, b, x, w, L.s);
+  PV_HIP(hipMemcpyAsync(dx, x, sizeof(double) * n, hipMemcpyDeviceToHost, L.s));
   PV_HIP(hipStreamSynchronize(L.s));
 }
 

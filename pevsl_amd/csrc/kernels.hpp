@@ -156,6 +156,28 @@ template <typename T>
 void dia_clen_blk(const DevCsr &A, int B, const T *b1, const T *b2, const T *v, T *out, double cc,
                   double t, const double *mus, int k, hipStream_t s);
 
+// The degrees 1..m >= 1 of the filter y = sum mu_k T_k((A - cc)/dd) x for one
+// column in the stream form: a launch per degree, or on the diagonal layout of
+// a small or narrow matrix several degrees per launch (k_cheb_multi), with the
+// same bits.  w: 4 n elements (3 n if n > 2^20).  Returns the bytes of the
+// passes over memory.
+template <typename T>
+double cheb_run(const DevCsr &A, const double *mu, int m, double cc, double dd, const T *x, T *y,
+                T *w, hipStream_t s);
+// launches of several degrees: degrees per launch (1: none), rows per
+// workgroup, widest diagonal
+struct MultiPlan {
+  int s = 1, R = 0, bw = 0;
+};
+constexpr int kMultiMax = 32;      // degrees per launch at most
+constexpr int kMultiRows = 4096;   // rows of a workgroup's window at most
+constexpr int kMultiLds = 65536;   // bytes of LDS for its two vectors
+MultiPlan dia_multi_plan(const DevCsr &A, int elem, int m);
+template <typename T>
+void dia_cheb_multi(const DevCsr &A, const MultiPlan &p, const T *v, const T *vm, T *vout,
+                    T *vmout, T *y, double cc, double dd, const double *mu, int d0, int s,
+                    bool last, hipStream_t st);
+
 // Same for B interleaved columns (row-major n x B block, column fastest).
 // mus: device array [(deg_max+1) x B] of per-column coefficients; k = degree
 // index of this step (1..); columns c >= nact are left untouched.

@@ -132,43 +132,46 @@ std::string filter_kernel_name(bool f32, int kind, int B, bool stream, int lanes
 
 }  // namespace
 
-// FP32 filter y = p((A - cc)/dd) v on FP32 columns; w holds 3n floats.
-// `timed`: record the run in the instance's per-kernel HIP-event timers.
-static void cheb_filter_f32(Ctx &c, const pevsl_Polparams *pol, const float *x32, float *y32,
-                            float *w, bool timed = true) {
+// Filter y = p((A - cc)/dd) x, degree >= 1, on columns of type T; w holds 4n
+// elements.  `timed`: record the run in the instance's per-kernel HIP-event
+// timers.
+template <typename T>
+static void cheb_filter_run(Ctx &c, const pevsl_Polparams *pol, const T *x, T *y, T *w,
+                            bool timed) {
   const DevCsr &A = *c.A;
-  const int n = A.n, m = pol->deg;
+  const int n = A.n, m = pol->deg, elem = (int)sizeof(T);
   const double *mu = pol->mu;
   const double cc = pol->cc, dd = pol->dd;
   const hipStream_t s = c.stream;
   const int lanes = std::max(c.lanes, 1);
+  // default (-1): the stream form
   const bool stream = c.use_stream != 0;
-  float *b[3] = {w, w + (size_t)n, w + 2 * (size_t)n};
-  const float *vk = x32, *vkm1 = nullptr;
-  int nb = 0;
+  const long tok =
+      timed ? c.kt.begin(s, filter_kernel_name(elem == 4, 0, 0, stream, lanes).c_str()) : -1;
+  // statistics count the CSR form, a launch per degree
+  double csr = 0.0;
   YPlan yp;
-  const bool dia = stream && use_dia(A, 4, 1);
-  const long tok = m > 0 && timed
-                       ? c.kt.begin(s, filter_kernel_name(true, 0, 0, stream, lanes).c_str())
-                       : -1;
-  double bytes = 0.0;
   for (int k = 1; k <= m; k++) {
-    float *vkp1 = b[nb];
-    nb = (nb + 1) % 3;
     const int ymode = stream ? yp.next(k, m) : (k == 1 ? kYInit | 1 : 1);
-    if (stream)
-      cheb_step_stream<float>(A, vk, vkm1, vkp1, y32, cc, k == 1 ? 1.0 / dd : 2.0 / dd, mu[0],
-                              k > 2 ? mu[k - 2] : 0.0, mu[k - 1], mu[k], ymode, s);
-    else
-      cheb_step_vec<float>(A, vk, vkm1, vkp1, y32, cc, k == 1 ? 1.0 / dd : 2.0 / dd, mu[0],
-                           mu[k], k == 1, lanes, s);
-    vkm1 = vk;
-    vk = vkp1;
-    bytes += (double)filter_launch_bytes(A, 4, 1, (k == 1 ? 2 : 3) + y_passes(ymode),
-                                         stream ? index_bytes(A) : 4);
+    csr += (double)filter_launch_bytes(A, elem, 1, (k == 1 ? 2 : 3) + y_passes(ymode),
+                                       stream ? index_bytes(A) : 4);
   }
-  if (tok >= 0) c.kt.end(s, tok, m, bytes - m * dia_saved_bytes(A, 4, index_bytes(A), dia));
-  c.kstats.filter_bytes += bytes;
+  double bytes = csr;
+  if (stream) {
+    bytes = cheb_run<T>(A, mu, m, cc, dd, x, y, w, s);
+  } else {
+    T *b[3] = {w, w + (size_t)n, w + 2 * (size_t)n};
+    const T *vk = x, *vkm1 = nullptr;
+    for (int k = 1; k <= m; k++) {
+      T *vkp1 = b[(k - 1) % 3];
+      cheb_step_vec<T>(A, vk, vkm1, vkp1, y, cc, k == 1 ? 1.0 / dd : 2.0 / dd, mu[0], mu[k],
+                       k == 1, lanes, s);
+      vkm1 = vk;
+      vk = vkp1;
+    }
+  }
+  if (tok >= 0) c.kt.end(s, tok, m, bytes);
+  c.kstats.filter_bytes += csr;
   c.kstats.filter_steps += m;
   c.kstats.filter_launches += m;
 }
@@ -204,58 +207,23 @@ void cheb_filter_col(Ctx &c, const pevsl_Polparams *pol, const double *dv,
     c.kstats.filter_steps += m;
     return;
   }
-  const DevCsr &A = *c.A;
-  const int lanes = std::max(c.lanes, 1);
-  // default (-1): the diagonal layout's or the CSR-stream kernel
-  const bool stream = c.use_stream != 0;
   if (c.filter_prec == PEVSL_PREC_FP64) {
-    double *w = work ? work : c.scratch64.ensure((size_t)3 * n);
-    double *b[3] = {w, w + n, w + 2 * (size_t)n};
-    const double *vk = dv, *vkm1 = nullptr;
-    int nb = 0;
-    YPlan yp;
-    const bool dia = stream && use_dia(A, 8, 1);
-    const long tok =
-        work ? -1 : c.kt.begin(s, filter_kernel_name(false, 0, 0, stream, lanes).c_str());
-    const double bytes0 = c.kstats.filter_bytes;
-    for (int k = 1; k <= m; k++) {
-      double *vkp1 = b[nb];
-      nb = (nb + 1) % 3;
-      const int ymode = stream ? yp.next(k, m) : (k == 1 ? kYInit | 1 : 1);
-      if (stream)
-        cheb_step_stream<double>(A, vk, vkm1, vkp1, dy, cc, k == 1 ? 1.0 / dd : 2.0 / dd,
-                                 mu[0], k > 2 ? mu[k - 2] : 0.0, mu[k - 1], mu[k], ymode, s);
-      else
-        cheb_step_vec<double>(A, vk, vkm1, vkp1, dy, cc,
-                              k == 1 ? 1.0 / dd : 2.0 / dd, mu[0], mu[k], k == 1,
-                              lanes, s);
-      vkm1 = vk;
-      vk = vkp1;
-      c.kstats.filter_bytes +=
-          (double)filter_launch_bytes(A, 8, 1, (k == 1 ? 2 : 3) + y_passes(ymode),
-                                      stream ? index_bytes(A) : 4);
-    }
-    if (tok >= 0)
-      c.kt.end(s, tok, m, c.kstats.filter_bytes - bytes0 -
-                              m * dia_saved_bytes(A, 8, index_bytes(A), dia));
-  } else {
-    // x32, y32 and three work columns: 5n floats (within 3n doubles)
-    float *w = reinterpret_cast<float *>(work ? work
-                                              : c.scratch64.ensure((size_t)5 * n / 2 + 8));
-    float *x32 = w, *y32 = w + n;
-    copy_f64_to_f32((size_t)n, dv, x32, s);
-    cheb_filter_f32(c, pol, x32, y32, w + 2 * (size_t)n, work == nullptr);
-    copy_f32_to_f64((size_t)n, y32, dy, s);
+    double *w = work ? work : c.scratch64.ensure((size_t)4 * n);
+    cheb_filter_run<double>(c, pol, dv, dy, w, work == nullptr);
     return;
   }
-  c.kstats.filter_steps += m;
-  c.kstats.filter_launches += m;
+  // x32, y32 and four work columns: 6n floats (3n doubles)
+  float *w = reinterpret_cast<float *>(work ? work : c.scratch64.ensure((size_t)3 * n + 8));
+  float *x32 = w, *y32 = w + n;
+  copy_f64_to_f32((size_t)n, dv, x32, s);
+  cheb_filter_run<float>(c, pol, x32, y32, w + 2 * (size_t)n, work == nullptr);
+  copy_f32_to_f64((size_t)n, y32, dy, s);
 }
 
 void cheb_filter_col32(Ctx &c, const pevsl_Polparams *pol, const float *dv, float *dy) {
   const int n = c.A->n;
-  float *w = reinterpret_cast<float *>(c.scratch64.ensure((size_t)3 * n / 2 + 8));
-  cheb_filter_f32(c, pol, dv, dy, w);
+  float *w = reinterpret_cast<float *>(c.scratch64.ensure((size_t)2 * n + 8));
+  cheb_filter_run<float>(c, pol, dv, dy, w, true);
 }
 
 namespace {

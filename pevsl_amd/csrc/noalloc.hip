@@ -3,8 +3,8 @@
 // must not allocate device memory (code under HIP graph capture, serving
 // loops, harnesses that forbid hipMalloc).
 //
-// The filter's work vectors (three n-vectors in FP64; x, y and three columns
-// in FP32 on the mixed path, which fit in the same space) live in `scratch`,
+// The filter's work vectors (three n-vectors in FP64, four up to 2^20 rows; x, y and
+// four columns in FP32 on the mixed path, which fit in the same space) live in `scratch`,
 // a file-scope device array of kScratchDoubles doubles that every GPU the
 // library runs on holds until the process ends.  Host code never passes the
 // array's name to a kernel: the first call on a device resolves its device
@@ -22,7 +22,8 @@ namespace {
 
 // Rows of the largest matrix the entry point accepts (2^21 = 2,097,152).
 constexpr size_t kMaxRows = size_t(1) << 21;
-// three n-vectors of doubles; 5n floats on the FP32 filter path fit as well
+// three n-vectors of doubles, four up to 2^20 rows (kernels.hpp cheb_run); 6n
+// floats on the FP32 filter path fit as well
 constexpr size_t kScratchDoubles = 3 * kMaxRows + 64;  // 48 MiB + 512 B
 
 static __device__ __align__(256) double scratch[kScratchDoubles];

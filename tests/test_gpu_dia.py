@@ -51,6 +51,11 @@ CASES = {
     "block_edge_1": lambda: banded(257, [-1, 0, 1], vary=[0]),
     "3_of_4_dropped": lambda: banded(1111, [-5, 0, 5], drop=0.3),
     "4_no_main": lambda: banded(1000, [-3, -1, 1, 3]),
+    # several degrees per launch: one window, many windows, the widest band
+    "chain_wide": lambda: banded(70001, [-1, 0, 1], vary=[0]),
+    "band_31": lambda: banded(20011, [-31, -30, 0, 30, 31], drop=0.1),
+    "band_400": lambda: banded(8000, [-400, -20, -1, 0, 1, 20, 400]),
+    "lower_only": lambda: banded(5000, [-3, -2, 0]),
     "lap2d": lambda: driver.laplacian3d(31, 17, 1),
     "lap3d": lambda: driver.laplacian3d(13, 11, 7),
     "8_diags": lambda: banded(3001, [-700, -31, -1, 0, 1, 31, 700, 2999], drop=0.1, vary=[0]),
@@ -89,7 +94,7 @@ def test_filter_equals_csr(lib, name):
     try:
         v = rng.uniform(-1, 1, n)
         # every way a run of degrees can end in the update of y
-        for deg in (1, 2, 3, 4, 5, 6, 17):
+        for deg in (1, 2, 3, 4, 5, 6, 17, 70):
             mu = rng.uniform(-1, 1, deg + 1)
             pol = capi.Polparams()
             pol.deg, pol.cc, pol.dd = deg, 0.1 * rad, 1.1 * rad
