@@ -462,7 +462,8 @@ int pEVSL_LanDosG(pevsl_Data *pevsl, const int nvec, int msteps, int npts, doubl
   }
   std::vector<double> wn((size_t)nvec, 0.0);
   std::vector<int> nwn((size_t)nvec, 0);
-  std::vector<double> ha((size_t)2 * nvec), betas((size_t)nvec);
+  PinnedBuf<double> ha((size_t)3 * nvec);
+  std::vector<double> betas((size_t)nvec);
   const int msk = (1 << shift) - 1;
   (void)msk;
   for (int k = 0; k < maxit; k++) {
@@ -470,25 +471,26 @@ int pEVSL_LanDosG(pevsl_Data *pevsl, const int nvec, int msteps, int npts, doubl
       double *base = vt[(size_t)v];
       apply_A(c, base + (size_t)k * L.ld, base + (size_t)(k + 1) * L.ld);
     }
-    lan_alpha(L, k, s);
-    lan_subtract_alpha(L, k, s);
+    lan_update(L, k, false, s);
     lan_cgs_pass(L, k, 0, s);
-    lan_cgs_pass(L, k, 1, s);
-    PV_HIP(hipMemcpyAsync(ha.data(), L.alpha, sizeof(double) * nvec, hipMemcpyDeviceToHost, s));
-    PV_HIP(hipMemcpyAsync(ha.data() + nvec, L.nrm2b, sizeof(double) * nvec,
-                          hipMemcpyDeviceToHost, s));
+    lan_finish(L, k, 0, ha.p, s);
     PV_HIP(hipStreamSynchronize(s));
+    if (std::any_of(ha.p, ha.p + 3 * nvec, [&](const double &x) {
+          return (&x - ha.p) % 3 == 2 && x != 0.0;
+        })) {
+      lan_cgs_pass(L, k, 1, s);
+      lan_finish(L, k, 1, ha.p, s);
+      PV_HIP(hipStreamSynchronize(s));
+    }
     std::vector<int> brk;
     for (int v = 0; v < nvec; v++) {
-      const double alpha = ha[(size_t)v], beta = sqrt(ha[(size_t)nvec + v]);
+      const double alpha = ha.p[3 * v], beta = sqrt(ha.p[3 * v + 1]);
       dT[(size_t)v * maxit + k] = alpha;
       wn[(size_t)v] += fabs(alpha) + 2.0 * beta;
       nwn[(size_t)v] += 3;
       betas[(size_t)v] = beta;
       if (beta * nwn[(size_t)v] < orthTol * wn[(size_t)v]) brk.push_back(v);
     }
-    PV_HIP(hipMemcpyAsync(L.beta, betas.data(), sizeof(double) * nvec, hipMemcpyHostToDevice, s));
-    lan_scale_new(L, k, s);  // breakdown columns are overwritten below
     for (int v : brk) {
       // fresh random vector orthogonalized against the basis (SRC/landos.c:209-232)
       double *col = vt[(size_t)v] + (size_t)(k + 1) * L.ld;
@@ -496,16 +498,13 @@ int pEVSL_LanDosG(pevsl_Data *pevsl, const int nvec, int msteps, int npts, doubl
       std::vector<int> one((size_t)nvec, 0);
       one[(size_t)v] = 1;
       PV_HIP(hipMemcpyAsync(L.active, one.data(), sizeof(int) * nvec, hipMemcpyHostToDevice, s));
-      PV_HIP(hipMemsetAsync(L.alpha + v, 0, sizeof(double), s));
-      lan_subtract_alpha(L, k, s);
-      lan_cgs_pass(L, k, 0, s);
-      lan_cgs_pass(L, k, 1, s);
-      double nb2 = 0;
-      PV_HIP(hipMemcpyAsync(&nb2, L.nrm2b + v, sizeof(double), hipMemcpyDeviceToHost, s));
-      PV_HIP(hipStreamSynchronize(s));
-      const double b = sqrt(nb2);
-      PV_HIP(hipMemcpyAsync(L.beta + v, &b, sizeof(double), hipMemcpyHostToDevice, s));
-      lan_scale_new(L, k, s);
+      lan_update(L, k, true, s);
+      for (int pass = 0; pass < 2; pass++) {
+        lan_cgs_pass(L, k, pass, s);
+        lan_finish(L, k, pass, ha.p, s);
+        PV_HIP(hipStreamSynchronize(s));
+        if (pass == 0 && ha.p[3 * v + 2] == 0.0) break;
+      }
       const double zero = 0.0;
       PV_HIP(hipMemcpyAsync(L.beta + v, &zero, sizeof(double), hipMemcpyHostToDevice, s));
       PV_HIP(hipMemcpyAsync(L.active, ones.data(), sizeof(int) * nvec, hipMemcpyHostToDevice, s));

@@ -59,6 +59,20 @@ struct DBuf {
   }
 };
 
+// Owned pinned host memory that kernels write.
+template <typename T>
+struct PinnedBuf {
+  T *p = nullptr;
+  explicit PinnedBuf(size_t cnt) {
+    void *q = nullptr;
+    PV_HIP(hipHostMalloc(&q, sizeof(T) * cnt));
+    p = static_cast<T *>(q);
+  }
+  PinnedBuf(const PinnedBuf &) = delete;
+  PinnedBuf &operator=(const PinnedBuf &) = delete;
+  ~PinnedBuf() { (void)hipHostFree(p); }
+};
+
 // Device copy of a CSR matrix (attached to pevsl_Parcsr.dev).
 struct DevMatrix {
   DevCsr csr;

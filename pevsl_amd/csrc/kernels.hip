@@ -106,9 +106,8 @@ template <>
 struct Row16<double> {
   using vec = double2;
   static constexpr int R = 2;
-  static constexpr int kTiters = 16;   // GEMV-T row groups per thread
-  static constexpr int kGnPairs = 2;   // GEMV-N row groups per thread
-  static constexpr int kGnUnroll = 8;  // GEMV-N columns per load batch
+  static constexpr int kTrips = 16;   // GEMV-T row groups per thread at most
+  static constexpr int kGnPairs = 2;  // GEMV-N row groups per thread
   template <bool NT>
   __device__ static __forceinline__ vec ld(const vec *p) { return ld_basis<NT>(p); }
   __device__ static __forceinline__ double get(const vec &v, int r) { return r ? v.y : v.x; }
@@ -121,9 +120,8 @@ template <>
 struct Row16<float> {
   using vec = float4;
   static constexpr int R = 4;
-  static constexpr int kTiters = 8;
+  static constexpr int kTrips = 8;
   static constexpr int kGnPairs = 1;
-  static constexpr int kGnUnroll = 16;
   template <bool NT>
   __device__ static __forceinline__ vec ld(const vec *p) { return NT ? ld_basis_nt(p) : *p; }
   __device__ static __forceinline__ double get(const vec &v, int r) {
@@ -1139,6 +1137,24 @@ k_gram_mfma(int n, int m1, int m2, const double *__restrict__ X, size_t ldx,
 // Lanczos (batched over slices; blockIdx.y = slice)
 // ---------------------------------------------------------------------------
 
+// rows of a GEMV-N block and of one GEMV-T trip, the smaller of the two storage
+// types' (FP64): 16-byte row groups of kThreads threads
+constexpr int kLanRows = kThreads * 2;
+
+// per-slice sizes of the partials (see LanArgs)
+struct LanParts {
+  size_t nbmax, tcap;
+};
+LanParts lan_parts(size_t ld, int hcap) {
+  const size_t trips = (ld + kLanRows - 1) / kLanRows;
+  LanParts p;
+  p.nbmax = trips;
+  // GEMV-T: full-size row blocks for every column, or one trip per block for
+  // the first columns
+  p.tcap = std::max((size_t)hcap * ((trips + 15) / 16), trips * (size_t)std::min(hcap, 256));
+  return p;
+}
+
 template <typename TV>
 struct LanArgs {
   int n;
@@ -1150,7 +1166,11 @@ struct LanArgs {
   int *pass2, *active;
   double *h;
   int hcap;
-  double *part;
+  // block partials: <z, znew>, |znew|^2 before and after Gram-Schmidt (kDotBlocksMax,
+  // kDotBlocksMax and nbmax per slice), GEMV-T partials (tcap per slice)
+  double *pa, *pn, *pb, *pt;
+  int nbmax;
+  size_t tcap;
 };
 
 template <typename TV>
@@ -1169,7 +1189,14 @@ LanArgs<TV> make_args(const LanBatch &L) {
   a.active = L.active;
   a.h = L.h;
   a.hcap = L.hcap;
-  a.part = L.part;
+  const LanParts p = lan_parts(L.ld, L.hcap);
+  const size_t ns = (size_t)L.nslice;
+  a.pa = L.part;
+  a.pn = a.pa + ns * kDotBlocksMax;
+  a.pb = a.pn + ns * kDotBlocksMax;
+  a.pt = a.pb + ns * p.nbmax;
+  a.nbmax = (int)p.nbmax;
+  a.tcap = p.tcap;
   return a;
 }
 
@@ -1184,6 +1211,22 @@ __device__ __forceinline__ TV *lan_col(const LanArgs<TV> &L, int s, int j) {
 inline int lan_vec_blocks(int n) {
   int b = (n + kThreads * 4 - 1) / (kThreads * 4);
   return b < 1 ? 1 : (b > kDotBlocksMax ? kDotBlocksMax : b);
+}
+
+// sum of cnt partials by the whole workgroup, the same in every thread and in
+// every workgroup (fixed order)
+__device__ __forceinline__ double block_sum_all(const double *p, int cnt) {
+  __shared__ double red[kThreads / 64];
+  double v = 0.0;
+  for (int b = threadIdx.x; b < cnt; b += kThreads) v += p[b];
+  v = wave_sum(v);
+  __syncthreads();  // `red` may still be read from an earlier sum
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double t = 0.0;
+#pragma unroll
+  for (int w = 0; w < kThreads / 64; w++) t += red[w];
+  return t;
 }
 
 // znew -= beta zold (k > 0); partial <z, znew>
@@ -1207,69 +1250,114 @@ k_lan_alpha(LanArgs<TV> L, int k) {
     }
     acc += (double)z[i] * w;
   }
-  block_sum_store(acc, L.part + (size_t)s * gridDim.x + blockIdx.x);
+  block_sum_store(acc, L.pa + (size_t)s * kDotBlocksMax + blockIdx.x);
 }
 
-// znew -= alpha z; partial |znew|^2
+// alpha = sum of k_lan_alpha's partials (each workgroup sums them: a read of at
+// most 8 KB in place of a launch); znew -= alpha z; partial |znew|^2.  zero:
+// alpha = 0, only the norm.
 template <typename TV>
 __global__ void __launch_bounds__(kThreads)
-k_lan_sub_alpha(LanArgs<TV> L, int k) {
+k_lan_sub_alpha(LanArgs<TV> L, int k, int zero) {
 #pragma clang fp contract(off)
   const int s = blockIdx.y;
   if (!L.active[s]) return;
   TV *znew = lan_col(L, s, k + 1);
-  const TV *z = lan_col(L, s, k);
-  const double ma = -L.alpha[s];
   double acc = 0.0;
-  for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < (size_t)L.n;
-       i += (size_t)gridDim.x * kThreads) {
-    const TV w = (TV)((double)znew[i] + ma * (double)z[i]);
-    znew[i] = w;
-    acc += (double)w * (double)w;
-  }
-  block_sum_store(acc, L.part + (size_t)s * gridDim.x + blockIdx.x);
-}
-
-// per-slice sums of the vector partials into one of the scalar arrays
-// which: 0 alpha, 1 nrm2a, 2 nrm2b (pass 0, sets pass2), 3 nrm2b (pass 1)
-template <typename TV>
-__global__ void k_lan_reduce(LanArgs<TV> L, int nblk, int which) {
-  const int s = blockIdx.x;
-  if (!L.active[s]) return;
-  if (which == 3 && !L.pass2[s]) return;
-  double v = 0.0;
-  for (int b = threadIdx.x; b < nblk; b += 64)
-    v += L.part[(size_t)s * nblk + b];
-  v = wave_sum(v);
-  if (threadIdx.x != 0) return;
-  if (which == 0) {
-    L.alpha[s] = v;
-  } else if (which == 1) {
-    L.nrm2a[s] = v;
+  if (zero) {
+    for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < (size_t)L.n;
+         i += (size_t)gridDim.x * kThreads)
+      acc += (double)znew[i] * (double)znew[i];
   } else {
-    L.nrm2b[s] = v;
-    if (which == 2) {
-      const double eta = 1.0 / sqrt(2.0);
-      L.pass2[s] = (sqrt(v) > eta * sqrt(L.nrm2a[s])) ? 0 : 1;
+    const double alpha = block_sum_all(L.pa + (size_t)s * kDotBlocksMax, gridDim.x);
+    if (blockIdx.x == 0 && threadIdx.x == 0) L.alpha[s] = alpha;
+    const TV *z = lan_col(L, s, k);
+    const double ma = -alpha;
+    for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < (size_t)L.n;
+         i += (size_t)gridDim.x * kThreads) {
+      const TV w = (TV)((double)znew[i] + ma * (double)z[i]);
+      znew[i] = w;
+      acc += (double)w * (double)w;
     }
   }
+  block_sum_store(acc, L.pn + (size_t)s * kDotBlocksMax + blockIdx.x);
 }
 
-// GEMV-T partials: part[(s*hcap + j)*nrb + rb] = sum over row block rb of
+// DGKS test: a second pass when the norm fell to 1/sqrt(2) of what it was
+__device__ __forceinline__ int dgks_again(double after, double before) {
+  const double eta = 1.0 / sqrt(2.0);
+  return sqrt(after) > eta * sqrt(before) ? 0 : 1;
+}
+
+// |znew|^2 after a pass, from the GEMV-N partials; the DGKS test against the
+// norm in nrm2a
+template <typename TV>
+__global__ void __launch_bounds__(kThreads)
+k_lan_norm(LanArgs<TV> L, int nbn) {
+  const int s = blockIdx.x;
+  if (!L.active[s]) return;
+  const double v = block_sum_all(L.pb + (size_t)s * L.nbmax, nbn);
+  if (threadIdx.x != 0) return;
+  L.nrm2b[s] = v;
+  L.pass2[s] = dgks_again(v, L.nrm2a[s]);
+}
+
+// End of a Lanczos step: |znew|^2 after Gram-Schmidt from its partials (nbn),
+// for pass 0 also before it (nba) and the DGKS test; beta = |znew| and znew /=
+// beta where no second pass is due.  Every workgroup sums the partials itself.
+// host (pinned memory): alpha, |znew|^2, second pass due, per slice.
+template <typename TV>
+__global__ void __launch_bounds__(kThreads)
+k_lan_finish(LanArgs<TV> L, int k, int pass, int nba, int nbn, double *host) {
+  const int s = blockIdx.y;
+  if (!L.active[s]) return;
+  if (pass && !L.pass2[s]) return;
+  const double v = block_sum_all(L.pb + (size_t)s * L.nbmax, nbn);
+  int again = 0;
+  double before = 0.0;
+  if (!pass) {
+    before = block_sum_all(L.pn + (size_t)s * kDotBlocksMax, nba);
+    again = dgks_again(v, before);
+  }
+  const double beta = sqrt(v);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    // pass 1 leaves pass2 set for the workgroups still to come
+    if (!pass) {
+      L.nrm2a[s] = before;
+      L.pass2[s] = again;
+    }
+    L.nrm2b[s] = v;
+    L.beta[s] = beta;
+    host[3 * s] = L.alpha[s];
+    host[3 * s + 1] = v;
+    host[3 * s + 2] = again;
+  }
+  if (again) return;
+  TV *z = lan_col(L, s, k + 1);
+  const double t = 1.0 / beta;
+  for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < (size_t)L.n;
+       i += (size_t)gridDim.x * kThreads)
+    z[i] = (TV)((double)z[i] * t);
+}
+
+// GEMV-T partials: pt[s*tcap + j*nrb + rb] = sum over row block rb of
 // V_s(:,j) * znew_s, for the kTcols columns of this block.  Each lane keeps
 // one accumulator per column and streams 16-byte row groups (2 FP64 or 4
 // FP32 rows, one independent load per column per iteration); the cross-lane
 // reduction runs once per column at the end.  Rows in [n, ld) are zero in
 // every basis column, so whole row groups up to ld are read without masks.
 constexpr int kTcols = 32;               // columns per block
+// A block takes `trips` trips of one 16-byte row group per thread; 8192 rows
+// where that gives blocks enough, fewer for short vectors and few columns (see
+// lan_cgs_pass_t).
 template <typename TV>
-constexpr int gt_rows() {  // rows per block: 8192 for both storage types
-  return kThreads * Row16<TV>::R * Row16<TV>::kTiters;
+constexpr int gt_trip() {  // rows of one trip
+  return kThreads * Row16<TV>::R;
 }
 
 template <bool NT, typename TV>
 __global__ void __launch_bounds__(kThreads)
-k_lan_gemvt(LanArgs<TV> L, int k, int pass, int nrb) {
+k_lan_gemvt(LanArgs<TV> L, int k, int pass, int nrb, int trips) {
   using RV = Row16<TV>;
   using vec = typename RV::vec;
   constexpr int R = RV::R;
@@ -1291,11 +1379,11 @@ k_lan_gemvt(LanArgs<TV> L, int k, int pass, int nrb) {
 #pragma unroll
   for (int c = 0; c < kTcols; c++) acc[c] = 0.0;
   const size_t ngrp = L.ld / R;
-  const size_t p0 = (size_t)rb * (gt_rows<TV>() / R) + threadIdx.x;
+  const size_t p0 = (size_t)rb * ((size_t)trips * kThreads) + threadIdx.x;
   // full column groups load without guards; the last group of a basis
   // guards its columns
   auto sweep = [&](auto full) {
-    for (int i = 0; i < RV::kTiters; i++) {
+    for (int i = 0; i < trips; i++) {
       const size_t p = p0 + (size_t)i * kThreads;
       if (p >= ngrp) break;
       const vec zv = z[p];
@@ -1332,44 +1420,41 @@ k_lan_gemvt(LanArgs<TV> L, int k, int pass, int nrb) {
     double t = 0.0;
 #pragma unroll
     for (int w = 0; w < kThreads / 64; w++) t += red[w][threadIdx.x];
-    L.part[((size_t)s * L.hcap + j0 + threadIdx.x) * nrb + rb] = t;
+    L.pt[(size_t)s * L.tcap + (size_t)(j0 + threadIdx.x) * nrb + rb] = t;
   }
 }
 
-// h_s[j] = sum_rb part[(s*hcap + j)*nrb + rb]
+// h_s[j] = sum_rb pt[s*tcap + j*nrb + rb], one wave per column
 template <typename TV>
 __global__ void __launch_bounds__(kThreads)
 k_lan_reduce_h(LanArgs<TV> L, int k, int pass, int nrb) {
   const int s = blockIdx.y;
   if (!L.active[s]) return;
   if (pass && !L.pass2[s]) return;
-  const int j = blockIdx.x * kThreads + threadIdx.x;
+  const int j = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
   if (j > k) return;
-  const double *p = L.part + ((size_t)s * L.hcap + j) * nrb;
+  const double *p = L.pt + (size_t)s * L.tcap + (size_t)j * nrb;
   double v = 0.0;
-  for (int b = 0; b < nrb; b++) v += p[b];
-  L.h[(size_t)s * L.hcap + j] = v;
+  for (int b = threadIdx.x & 63; b < nrb; b += 64) v += p[b];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) L.h[(size_t)s * L.hcap + j] = v;
 }
 
 // znew -= V(:,0:k) h, column by column in the order of DGEMV 'N'
 // (y_i += (-h_j) V_ij for j = 0..k), with the block partial of |znew|^2.
-// Each thread owns kGnPairs 16-byte row groups and walks the columns
-// kGnUnroll at a time so that 16 loads are in flight per thread.  The
-// running sums are FP64; an FP32 basis is rounded once, when znew is stored.
-template <typename TV>
-constexpr int gn_rows() {  // rows per block: 1024 for both storage types
-  return kThreads * Row16<TV>::R * Row16<TV>::kGnPairs;
-}
-
-template <bool NT, typename TV>
+// Each thread owns P 16-byte row groups and walks the columns U at a time, P U
+// = 16, so that 16 loads are in flight per thread: P = kGnPairs, or 1 for short
+// vectors, which gives twice the blocks and half the trips over the columns.
+// The running sums are FP64; an FP32 basis is rounded once, when znew is
+// stored.
+template <bool NT, typename TV, int P>
 __global__ void __launch_bounds__(kThreads)
-k_lan_gemvn(LanArgs<TV> L, int k, int pass, int nblk) {
+k_lan_gemvn(LanArgs<TV> L, int k, int pass) {
 #pragma clang fp contract(off)
   using RV = Row16<TV>;
   using vec = typename RV::vec;
   constexpr int R = RV::R;
-  constexpr int P = RV::kGnPairs;
-  constexpr int U = RV::kGnUnroll;
+  constexpr int U = 16 / P;
   const int s = blockIdx.y;
   if (!L.active[s]) return;
   if (pass && !L.pass2[s]) return;
@@ -1381,7 +1466,7 @@ k_lan_gemvn(LanArgs<TV> L, int k, int pass, int nblk) {
   bool ok[P];
 #pragma unroll
   for (int i = 0; i < P; i++) {
-    pr[i] = (size_t)blockIdx.x * (gn_rows<TV>() / R) + (size_t)i * kThreads + threadIdx.x;
+    pr[i] = ((size_t)blockIdx.x * P + i) * kThreads + threadIdx.x;
     ok[i] = pr[i] < ngrp;
     const vec zv = ok[i] ? z[pr[i]] : RV::zero();
 #pragma unroll
@@ -1436,18 +1521,7 @@ k_lan_gemvn(LanArgs<TV> L, int k, int pass, int nblk) {
       sq += t;
     }
   }
-  block_sum_store(sq, L.part + (size_t)s * nblk + blockIdx.x);
-}
-
-template <typename TV>
-__global__ void k_lan_scale(LanArgs<TV> L, int k) {
-  const int s = blockIdx.y;
-  if (!L.active[s]) return;
-  TV *z = lan_col(L, s, k + 1);
-  const double t = 1.0 / L.beta[s];
-  for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < (size_t)L.n;
-       i += (size_t)gridDim.x * kThreads)
-    z[i] = (TV)((double)z[i] * t);
+  block_sum_store(sq, L.pb + (size_t)s * L.nbmax + blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -2191,68 +2265,84 @@ void scale_vec_f32(int n, float *x, double hostscale, hipStream_t s) {
 }
 
 size_t lan_part_doubles(int n, int nslice, int hcap) {
-  // sized for FP64 storage, the larger of the two row-block counts
-  const size_t ld = ((size_t)n + 63) / 64 * 64;
-  const size_t nrb = (ld + gt_rows<double>() - 1) / gt_rows<double>();
-  const size_t nbn = (ld + gn_rows<double>() - 1) / gn_rows<double>();
-  const size_t per = std::max(std::max((size_t)hcap * nrb, nbn),
-                              (size_t)lan_vec_blocks(n));
-  return (size_t)nslice * per + 64;
+  const LanParts p = lan_parts(((size_t)n + 63) / 64 * 64, hcap);
+  return (size_t)nslice * (2 * kDotBlocksMax + p.nbmax + p.tcap) + 64;
 }
 
 namespace {
+// GEMV-N blocks of a slice and row groups per thread: kGnPairs, or 1 where
+// that leaves CUs without a block (20^3: 8 blocks of 1024 rows)
 template <typename TV>
-void lan_alpha_t(const LanBatch &L, int k, hipStream_t s) {
-  const int nb = lan_vec_blocks(L.n);
-  LanArgs<TV> a = make_args<TV>(L);
-  hipLaunchKernelGGL(k_lan_alpha<TV>, dim3(nb, L.nslice), dim3(kThreads), 0, s, a, k);
-  hipLaunchKernelGGL(k_lan_reduce<TV>, dim3(L.nslice), dim3(64), 0, s, a, nb, 0);
+int gn_pairs(const LanBatch &L) {
+  constexpr int P = Row16<TV>::kGnPairs;
+  const size_t rows = (size_t)gt_trip<TV>() * P;
+  return L.nslice * ((L.ld + rows - 1) / rows) < 512 ? 1 : P;
+}
+template <typename TV>
+int gn_blocks(const LanBatch &L) {
+  const size_t rows = (size_t)gt_trip<TV>() * gn_pairs<TV>(L);
+  return (int)((L.ld + rows - 1) / rows);
 }
 
 template <typename TV>
-void lan_subtract_alpha_t(const LanBatch &L, int k, hipStream_t s) {
+void lan_update_t(const LanBatch &L, int k, bool norm_only, hipStream_t s) {
   const int nb = lan_vec_blocks(L.n);
   LanArgs<TV> a = make_args<TV>(L);
-  hipLaunchKernelGGL(k_lan_sub_alpha<TV>, dim3(nb, L.nslice), dim3(kThreads), 0, s, a, k);
-  hipLaunchKernelGGL(k_lan_reduce<TV>, dim3(L.nslice), dim3(64), 0, s, a, nb, 1);
+  if (!norm_only)
+    hipLaunchKernelGGL(k_lan_alpha<TV>, dim3(nb, L.nslice), dim3(kThreads), 0, s, a, k);
+  hipLaunchKernelGGL(k_lan_sub_alpha<TV>, dim3(nb, L.nslice), dim3(kThreads), 0, s, a, k,
+                     norm_only ? 1 : 0);
 }
 
 template <typename TV>
 void lan_cgs_pass_t(const LanBatch &L, int k, int pass, hipStream_t s) {
   LanArgs<TV> a = make_args<TV>(L);
-  const int nrb = (int)((L.ld + gt_rows<TV>() - 1) / gt_rows<TV>());
   const int ncb = (k + 1 + kTcols - 1) / kTcols;
+  // GEMV-T row blocks: full-size ones unless they are fewer than four per CU;
+  // then fewer trips each, as far as the partials have room.  One row block
+  // per column group left the chip idle on short vectors (n = 8,000: 15.5 us a
+  // pass, n = 1e5, k = 50: 44 us).
+  const size_t trips_all = (L.ld + gt_trip<TV>() - 1) / gt_trip<TV>();
+  int trips = Row16<TV>::kTrips;
+  while (trips > 1 && ((trips_all + trips - 1) / trips) * ncb * L.nslice < 1024 &&
+         ((trips_all + trips / 2 - 1) / (trips / 2)) * (k + 1) <= a.tcap)
+    trips /= 2;
+  const int nrb = (int)((trips_all + trips - 1) / trips);
   // nontemporal basis loads: measured 6.5 vs 5.9 TB/s at k = 4096 (C2)
   hipLaunchKernelGGL((k_lan_gemvt<true, TV>), dim3(nrb, ncb, L.nslice), dim3(kThreads), 0,
-                     s, a, k, pass, nrb);
-  hipLaunchKernelGGL(k_lan_reduce_h<TV>, dim3(grid_for(k + 1), L.nslice), dim3(kThreads), 0,
-                     s, a, k, pass, nrb);
-  const int nbn = (int)((L.ld + gn_rows<TV>() - 1) / gn_rows<TV>());
-  hipLaunchKernelGGL((k_lan_gemvn<true, TV>), dim3(nbn, L.nslice), dim3(kThreads), 0, s, a,
-                     k, pass, nbn);
-  hipLaunchKernelGGL(k_lan_reduce<TV>, dim3(L.nslice), dim3(64), 0, s, a, nbn, pass ? 3 : 2);
+                     s, a, k, pass, nrb, trips);
+  hipLaunchKernelGGL(k_lan_reduce_h<TV>, dim3(grid_for(k + 1, kThreads / 64), L.nslice),
+                     dim3(kThreads), 0, s, a, k, pass, nrb);
+  constexpr int P = Row16<TV>::kGnPairs;
+  const int nbn = gn_blocks<TV>(L);
+  if (gn_pairs<TV>(L) == P)
+    hipLaunchKernelGGL((k_lan_gemvn<true, TV, P>), dim3(nbn, L.nslice), dim3(kThreads), 0, s, a,
+                       k, pass);
+  else
+    hipLaunchKernelGGL((k_lan_gemvn<true, TV, 1>), dim3(nbn, L.nslice), dim3(kThreads), 0, s, a,
+                       k, pass);
 }
 
 template <typename TV>
-void lan_scale_new_t(const LanBatch &L, int k, hipStream_t s) {
+void lan_finish_t(const LanBatch &L, int k, int pass, double *host, hipStream_t s) {
   LanArgs<TV> a = make_args<TV>(L);
   const int nb = lan_vec_blocks(L.n);
-  hipLaunchKernelGGL(k_lan_scale<TV>, dim3(nb, L.nslice), dim3(kThreads), 0, s, a, k);
+  hipLaunchKernelGGL(k_lan_finish<TV>, dim3(nb, L.nslice), dim3(kThreads), 0, s, a, k, pass, nb,
+                     gn_blocks<TV>(L), host);
+}
+
+template <typename TV>
+void lan_cgs_norm_t(const LanBatch &L, hipStream_t s) {
+  hipLaunchKernelGGL(k_lan_norm<TV>, dim3(L.nslice), dim3(kThreads), 0, s, make_args<TV>(L),
+                     gn_blocks<TV>(L));
 }
 }  // namespace
 
-void lan_alpha(const LanBatch &L, int k, hipStream_t s) {
+void lan_update(const LanBatch &L, int k, bool norm_only, hipStream_t s) {
   if (L.vbytes == 4)
-    lan_alpha_t<float>(L, k, s);
+    lan_update_t<float>(L, k, norm_only, s);
   else
-    lan_alpha_t<double>(L, k, s);
-}
-
-void lan_subtract_alpha(const LanBatch &L, int k, hipStream_t s) {
-  if (L.vbytes == 4)
-    lan_subtract_alpha_t<float>(L, k, s);
-  else
-    lan_subtract_alpha_t<double>(L, k, s);
+    lan_update_t<double>(L, k, norm_only, s);
 }
 
 void lan_cgs_pass(const LanBatch &L, int k, int pass, hipStream_t s) {
@@ -2262,11 +2352,18 @@ void lan_cgs_pass(const LanBatch &L, int k, int pass, hipStream_t s) {
     lan_cgs_pass_t<double>(L, k, pass, s);
 }
 
-void lan_scale_new(const LanBatch &L, int k, hipStream_t s) {
+void lan_cgs_norm(const LanBatch &L, hipStream_t s) {
   if (L.vbytes == 4)
-    lan_scale_new_t<float>(L, k, s);
+    lan_cgs_norm_t<float>(L, s);
   else
-    lan_scale_new_t<double>(L, k, s);
+    lan_cgs_norm_t<double>(L, s);
+}
+
+void lan_finish(const LanBatch &L, int k, int pass, double *host, hipStream_t s) {
+  if (L.vbytes == 4)
+    lan_finish_t<float>(L, k, pass, host, s);
+  else
+    lan_finish_t<double>(L, k, pass, host, s);
 }
 
 void tridiag_trace_above(int m, const double *d, const double *e, double thr,

@@ -334,16 +334,22 @@ struct LanBatch {
 // reorthogonalization coefficients per slice
 size_t lan_part_doubles(int n, int nslice, int hcap);
 
-// znew_s -= beta_s zold_s (k > 0);  alpha_s = <z_s, znew_s>
-void lan_alpha(const LanBatch &L, int k, hipStream_t s);
-// znew_s -= alpha_s z_s;  nrm2a_s = |znew_s|^2
-void lan_subtract_alpha(const LanBatch &L, int k, hipStream_t s);
+// Three-term update: znew_s -= beta_s zold_s (k > 0), alpha_s = <z_s, znew_s>,
+// znew_s -= alpha_s z_s, and partials of |znew_s|^2.  norm_only: only these.
+void lan_update(const LanBatch &L, int k, bool norm_only, hipStream_t s);
 // One classical Gram-Schmidt pass against V_s(:,0:k): h = V^T znew,
-// znew -= V h, nrm2b = |znew|^2.  pass = 0 always runs; pass = 1 runs only
-// for slices whose pass2 flag is set (decided on the device after pass 0).
+// znew -= V h, and partials of |znew|^2.  pass = 0 runs for active slices;
+// pass = 1 only for those among them whose pass2 flag is set.
 void lan_cgs_pass(const LanBatch &L, int k, int pass, hipStream_t s);
-// znew_s /= beta_s for active slices (beta read from the device array).
-void lan_scale_new(const LanBatch &L, int k, hipStream_t s);
+// nrm2b = |znew|^2 from the partials of a pass, pass2 = the DGKS test against
+// nrm2a (a Gram-Schmidt pass outside a Lanczos step)
+void lan_cgs_norm(const LanBatch &L, hipStream_t s);
+// End of a Lanczos step after lan_update and lan_cgs_pass(pass): nrm2b and beta
+// = |znew|; with pass 0 also nrm2a and pass2 (DGKS test); znew /= beta unless a
+// second pass is due.  host[3s ..] = alpha, nrm2b, pass2 of slice s, in memory
+// that the device writes and the host reads once the stream has drained.  With
+// a second pass due: lan_cgs_pass(1), lan_finish(1).
+void lan_finish(const LanBatch &L, int k, int pass, double *host, hipStream_t s);
 
 // ---- tridiagonal (FP64) ---------------------------------------------------
 // Restricted trace of T (diag d[0..m-1], sub-diag e[0..m-2]): eigenvalues

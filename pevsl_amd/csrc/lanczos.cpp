@@ -371,7 +371,7 @@ class BatchSolver {
                      void *const *colp);
   void filter_group_graph(const std::vector<int> &grp, int k);
   void lanczos_update(const std::vector<int> &act, int k);
-  void cgs(const std::vector<int> &act, int k);
+  void cgs(const std::vector<int> &act, int k, int pass);
   void breakdown(int s, int k);
   void convergence_tests(const std::vector<int> &ts, int k);
   void ritz(int s, double tol);
@@ -419,6 +419,7 @@ class BatchSolver {
   double *pinned_ = nullptr;
   int *pinned_i_ = nullptr;
   std::vector<int> mus_key_;
+  std::vector<int> active_h_;  // slices whose device `active` flag is set
   std::vector<double> mus_h_, betas_h_;
   std::vector<void *> cp_h_;
   std::vector<std::unique_ptr<GroupGraph>> graphs_;  // captured filter groups
@@ -477,12 +478,14 @@ void BatchSolver::sync_vtab() {
 }
 
 void BatchSolver::set_active(const std::vector<int> &act) {
+  if (act == active_h_) return;
   // the staging buffer may still feed an earlier copy
   PV_HIP(hipStreamSynchronize(c_.stream));
   for (int s = 0; s < ns_; s++) pinned_i_[s] = 0;
   for (int s : act) pinned_i_[s] = 1;
   PV_HIP(hipMemcpyAsync(L_.active, pinned_i_, sizeof(int) * ns_,
                         hipMemcpyHostToDevice, c_.stream));
+  active_h_ = act;
 }
 
 void BatchSolver::free_basis(int s) {
@@ -892,23 +895,22 @@ void BatchSolver::filter_group_graph(const std::vector<int> &grp, int k) {
 // three-term update: alpha and |z_{k+1}|^2 before reorthogonalization
 void BatchSolver::lanczos_update(const std::vector<int> &act, int k) {
   set_active(act);
-  lan_alpha(L_, k, c_.stream);
-  lan_subtract_alpha(L_, k, c_.stream);
+  lan_update(L_, k, false, c_.stream);
   const double vecb = (double)vb_ * n_;
   c_.kstats.reorth_bytes += act.size() * (4 * vecb + 3 * vecb);
 }
 
-// classical Gram-Schmidt with the DGKS test: pass 0 always, pass 1 only
-// for slices whose norm dropped below 1/sqrt(2) (decided on the device)
-void BatchSolver::cgs(const std::vector<int> &act, int k) {
+// classical Gram-Schmidt pass and the end of the step; pass 1 for the slices
+// whose norm dropped below 1/sqrt(2) in pass 0 (decided on the device)
+void BatchSolver::cgs(const std::vector<int> &act, int k, int pass) {
   const double vecb = (double)vb_ * n_;
-  const double pass = 2.0 * (k + 1) * vecb + 3 * vecb;
-  const long tok = c_.kt.begin(c_.stream, b32_ ? "cgs_pass<float>" : "cgs_pass<double>");
-  lan_cgs_pass(L_, k, 0, c_.stream);
-  c_.kt.end(c_.stream, tok, 1, act.size() * pass);
-  lan_cgs_pass(L_, k, 1, c_.stream);
-  c_.kstats.reorth_bytes += act.size() * pass;
-  c_.kstats.cgs_bytes += act.size() * pass;
+  const double bytes = act.size() * (2.0 * (k + 1) * vecb + 3 * vecb);
+  const long tok =
+      pass ? -1 : c_.kt.begin(c_.stream, b32_ ? "cgs_pass<float>" : "cgs_pass<double>");
+  lan_cgs_pass(L_, k, pass, c_.stream);
+  if (tok >= 0) c_.kt.end(c_.stream, tok, 1, bytes);
+  c_.kstats.reorth_bytes += bytes;
+  c_.kstats.cgs_bytes += bytes;
   c_.kstats.cgs_passes += (long long)act.size();
 }
 
@@ -923,18 +925,14 @@ void BatchSolver::breakdown(int s, int k) {
   sl.nmatvec += sl.pol->deg;
   std::vector<int> one{s};
   set_active(one);
-  // nrm2a of the fresh vector, then the DGKS passes
-  PV_HIP(hipMemsetAsync(L_.alpha + s, 0, sizeof(double), c_.stream));
-  lan_subtract_alpha(L_, k, c_.stream);  // alpha = 0: only |v|^2
-  lan_cgs_pass(L_, k, 0, c_.stream);
-  lan_cgs_pass(L_, k, 1, c_.stream);
-  PV_HIP(hipMemcpyAsync(pinned_, L_.nrm2b + s, sizeof(double), hipMemcpyDeviceToHost,
-                        c_.stream));
-  PV_HIP(hipStreamSynchronize(c_.stream));
-  const double beta = sqrt(pinned_[0]);
-  PV_HIP(hipMemcpyAsync(L_.beta + s, &beta, sizeof(double), hipMemcpyHostToDevice,
-                        c_.stream));
-  lan_scale_new(L_, k, c_.stream);
+  // the norm of the fresh vector, then the DGKS passes
+  lan_update(L_, k, true, c_.stream);
+  for (int pass = 0; pass < 2; pass++) {
+    lan_cgs_pass(L_, k, pass, c_.stream);
+    lan_finish(L_, k, pass, pinned_, c_.stream);
+    PV_HIP(hipStreamSynchronize(c_.stream));
+    if (pass == 0 && pinned_[3 * s + 2] == 0.0) break;
+  }
   const double zero = 0.0;
   PV_HIP(hipMemcpyAsync(L_.beta + s, &zero, sizeof(double), hipMemcpyHostToDevice,
                         c_.stream));
@@ -1276,7 +1274,7 @@ int BatchSolver::prepare(double *intvs, int *maxits, pevsl_Polparams *pols, doub
   L_.h = h_.ensure((size_t)ns_ * L_.hcap);
   L_.part_cap = lan_part_doubles(n_, ns_, L_.hcap);
   L_.part = part_.ensure(L_.part_cap);
-  PV_HIP(hipHostMalloc(&pinned_, sizeof(double) * (2 * ns_ + 8)));
+  PV_HIP(hipHostMalloc(&pinned_, sizeof(double) * (3 * ns_ + 8)));
   PV_HIP(hipHostMalloc(&pinned_i_, sizeof(int) * (ns_ + 8)));
   return 0;
 }
@@ -1304,8 +1302,8 @@ int BatchSolver::run(double *intvs, int *maxits, double tol, pevsl_Parvec *vinit
   }
   if (!act.empty()) {
     // |v|: reuse the Lanczos kernels with the basis column 0 as "znew"
-    // (z = zold = nothing): nrm2a via lan_subtract_alpha with alpha = 0 is
-    // not applicable at k = -1, so use the dot kernels directly.
+    // (z = zold = nothing): the norm of lan_update is not available at
+    // k = -1, so use the dot kernels directly.
     DBuf<double> pt;
     pt.ensure((size_t)dot_part_blocks(n_) + 8);
     for (int s : act) {
@@ -1325,56 +1323,44 @@ int BatchSolver::run(double *intvs, int *maxits, double tol, pevsl_Parvec *vinit
     ev_f.start(st);
     filter_step(act, k);
     ev_f.stop(st);
-    // ---- three-term update and full reorthogonalization
+    // ---- three-term update, full reorthogonalization, normalization; the
+    // host reads alpha and the norms for T and the breakdown test
     ev_r.start(st);
     lanczos_update(act, k);
     ev_c.start(st);
-    cgs(act, k);
+    cgs(act, k, 0);
     ev_c.stop(st);
+    lan_finish(L_, k, 0, pinned_, st);
     ev_r.stop(st);
-    for (int s = 0; s < ns_; s++) {
-      pinned_[s] = 0;
-      pinned_[ns_ + s] = 0;
-    }
-    PV_HIP(hipMemcpyAsync(pinned_, L_.alpha, sizeof(double) * ns_, hipMemcpyDeviceToHost, st));
-    PV_HIP(hipMemcpyAsync(pinned_ + ns_, L_.nrm2b, sizeof(double) * ns_,
-                          hipMemcpyDeviceToHost, st));
-    PV_HIP(hipMemcpyAsync(pinned_i_, L_.pass2, sizeof(int) * ns_, hipMemcpyDeviceToHost, st));
     PV_HIP(hipStreamSynchronize(st));
     t_filter += ev_f.seconds();
     t_reorth += ev_r.seconds();
     t_cgs += ev_c.seconds();
-    for (int s : act) {
-      if (pinned_i_[s]) {  // second DGKS pass ran
-        const double pass = 2.0 * (k + 1) * (double)vb_ * n_ + 3.0 * (double)vb_ * n_;
-        c_.kstats.reorth_bytes += pass;
-        c_.kstats.cgs_bytes += pass;
-        c_.kstats.cgs_passes++;
-      }
+    std::vector<int> again;
+    for (int s : act)
+      if (pinned_[3 * s + 2] != 0.0) again.push_back(s);
+    if (!again.empty()) {
+      ev_r.start(st);
+      cgs(again, k, 1);
+      ev_r.stop(st);
+      lan_finish(L_, k, 1, pinned_, st);
+      PV_HIP(hipStreamSynchronize(st));
+      t_reorth += ev_r.seconds();
+      t_cgs += ev_r.seconds();
     }
     std::vector<int> brk;
     std::vector<double> &betas = betas_h_;
     betas.assign((size_t)ns_, 0.0);
     for (int s : act) {
       Slice &sl = S_[(size_t)s];
-      const double alpha = pinned_[s];
-      const double beta = sqrt(pinned_[ns_ + s]);
+      const double alpha = pinned_[3 * s];
+      const double beta = sqrt(pinned_[3 * s + 1]);
       sl.dT[(size_t)k] = alpha;
       sl.wn += fabs(alpha);
       sl.wn += 2.0 * beta;
       sl.nwn += 3;
       betas[(size_t)s] = beta;
       if (beta * sl.nwn < orthTol * sl.wn) brk.push_back(s);
-    }
-    // regular normalization for the slices without breakdown
-    PV_HIP(hipMemcpyAsync(L_.beta, betas.data(), sizeof(double) * ns_, hipMemcpyHostToDevice,
-                          st));
-    std::vector<int> reg;
-    for (int s : act)
-      if (std::find(brk.begin(), brk.end(), s) == brk.end()) reg.push_back(s);
-    if (!reg.empty()) {
-      set_active(reg);
-      lan_scale_new(L_, k, st);
     }
     for (int s : brk) {
       if (fstats) fprintf(fstats, "it %4d: Lucky breakdown, beta = %.15e\n", k, betas[(size_t)s]);
@@ -1511,8 +1497,9 @@ int BatchSolver::bench(double *intvs, pevsl_Polparams *pols, int k, int warmup, 
     ev_r.start(st);
     lanczos_update(act, k);
     ev_c.start(st);
-    cgs(act, k);
+    cgs(act, k, 0);
     ev_c.stop(st);
+    lan_finish(L_, k, 0, pinned_, st);
     ev_r.stop(st);
     ev_all.stop(st);
     PV_HIP(hipStreamSynchronize(st));

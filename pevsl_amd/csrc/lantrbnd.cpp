@@ -309,26 +309,32 @@ int pEVSL_LanTrbounds(pevsl_Data *pevsl, int lanm, int maxit, double tol, pevsl_
     PV_HIP(hipStreamSynchronize(st));
     return r;
   };
-  auto set_dev = [&](double *dst, double v) {
-    PV_HIP(hipMemcpyAsync(dst, &v, sizeof(double), hipMemcpyHostToDevice, st));
+  // L.beta on the device, which lan_finish sets as well
+  double dev_beta = 0.0;
+  auto set_beta = [&](double v) {
+    if (v == dev_beta) return;
+    PV_HIP(hipMemcpyAsync(L.beta, &v, sizeof(double), hipMemcpyHostToDevice, st));
     PV_HIP(hipStreamSynchronize(st));
+    dev_beta = v;
   };
-  auto get_dev = [&](const double *src) {
-    double v = 0.0;
-    PV_HIP(hipMemcpyAsync(&v, src, sizeof(double), hipMemcpyDeviceToHost, st));
-    PV_HIP(hipStreamSynchronize(st));
-    return v;
+  // Gram-Schmidt of column kk + 1 with the DGKS test, and its normalization;
+  // host.p: alpha, |.|^2
+  PinnedBuf<double> host(3);
+  auto cgs_finish = [&](int kk) {
+    for (int pass = 0; pass < 2; pass++) {
+      lan_cgs_pass(L, kk, pass, st);
+      lan_finish(L, kk, pass, host.p, st);
+      PV_HIP(hipStreamSynchronize(st));
+      if (pass == 0 && host.p[2] == 0.0) break;
+    }
+    dev_beta = std::sqrt(host.p[1]);
   };
   // vnew = random vector orthogonalized against V(:,0:k-1), unit norm,
   // beta = 0 (lucky breakdown, SRC/lantrbnd.c:192-211, 278-301)
   auto restart_random = [&](int k) {
     rand_vectors(c, n, 1, col(k), ld);
-    set_dev(L.alpha, 0.0);
-    lan_subtract_alpha(L, k - 1, st);  // alpha = 0: only |v|^2
-    lan_cgs_pass(L, k - 1, 0, st);
-    lan_cgs_pass(L, k - 1, 1, st);
-    const double b = std::sqrt(get_dev(L.nrm2b));
-    scale_vec(n, col(k), nullptr, 1.0 / b, st);
+    lan_update(L, k - 1, true, st);
+    cgs_finish(k - 1);
   };
   // V(:,0) = vinit / |vinit|
   PV_HIP(hipMemcpyAsync(col(0), vinit->data, sizeof(double) * n, hipMemcpyHostToDevice, st));
@@ -381,27 +387,19 @@ int pEVSL_LanTrbounds(pevsl_Data *pevsl, int lanm, int maxit, double tol, pevsl_
       k++;
       apply_A(c, col(k - 1), col(k));
       it++;
-      set_dev(L.beta, beta);  // znew -= beta zold (k > 1), alpha = <v, znew>
-      lan_alpha(L, k - 1, st);
-      lan_subtract_alpha(L, k - 1, st);
-      lan_cgs_pass(L, k - 1, 0, st);
-      lan_cgs_pass(L, k - 1, 1, st);
-      double sc2[4];
-      PV_HIP(hipMemcpyAsync(sc2, s4, sizeof(double) * 4, hipMemcpyDeviceToHost, st));
-      PV_HIP(hipStreamSynchronize(st));
-      const double alpha = sc2[0];
+      set_beta(beta);
+      lan_update(L, k - 1, false, st);  // znew -= beta zold (k > 1), alpha = <v, znew>
+      cgs_finish(k - 1);
+      const double alpha = host.p[0];
       Tat(k - 1, k - 1) = alpha;
       wn += std::fabs(alpha);
-      beta = std::sqrt(sc2[3]);
+      beta = std::sqrt(host.p[1]);
       wn += 2.0 * beta;
       nwn += 3;
       if (beta * nwn < orthTol * wn) {
         if (fstats) fprintf(fstats, "it %4d: Lucky breakdown, beta = %.15e\n", it, beta);
         restart_random(k);
         beta = 0.0;
-      } else {
-        set_dev(L.beta, beta);
-        lan_scale_new(L, k - 1, st);
       }
       Tat(k, k - 1) = beta;
       Tat(k - 1, k) = beta;

@@ -372,6 +372,7 @@ int pEVSL_CGS_DGKS(pevsl_Data *p, int k, int i_max, pevsl_Parvecs *Q, pevsl_Parv
   }
   for (int it = 0; k > 0 && it < i_max; it++) {
     lan_cgs_pass(L, k - 1, 0, c.stream);  // basis columns 0..k-1, vector in column k
+    lan_cgs_norm(L, c.stream);
     int again = 0;
     PV_HIP(hipMemcpyAsync(&nrm2, L.nrm2b, sizeof(double), hipMemcpyDeviceToHost, c.stream));
     PV_HIP(hipMemcpyAsync(&again, L.pass2, sizeof(int), hipMemcpyDeviceToHost, c.stream));
