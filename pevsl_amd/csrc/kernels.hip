@@ -691,8 +691,9 @@ __global__ void k_blk_colscale(size_t n, int B, const T *__restrict__ v, T *__re
 //            independent gathers, and staged in LDS;
 //   phase 2: one thread per (row, piece) sums the row's staged products in
 //            column order and runs the fused epilogue on its piece.
-// A row with more nonzeros than a block stages is a block alone and is reduced
-// by the whole workgroup (shuffles, then LDS across waves).  Products are
+// Rows beyond kUnevenRow entries are summed by a wave; a row with more nonzeros
+// than a block stages is a block alone and is reduced by the whole workgroup
+// (shuffles, then LDS across waves).  Products are
 // rounded before they are added and staged rows are summed in column order,
 // so those rows round exactly as in the row-per-thread kernels.
 
@@ -711,7 +712,7 @@ template <typename T, int B, class F>
 __device__ __forceinline__ void bal_rows(int rb, const int *__restrict__ rowblk,
                                          const int *__restrict__ ia, const int *__restrict__ ja,
                                          const T *__restrict__ a, const T *__restrict__ x,
-                                         T *prod, F &&f) {
+                                         T *prod, int uneven, F &&f) {
 #pragma clang fp contract(off)
   using PC = Pieces<T, B>;
   constexpr int P = PC::P, Q = PC::Q, S = kThreads / Q, U = kBalUnroll;
@@ -791,13 +792,52 @@ __device__ __forceinline__ void bal_rows(int rb, const int *__restrict__ rowblk,
     }
   }
   __syncthreads();
+  if (uneven) {
+    // Rows of more than kUnevenRow entries: a wave each, dealt to the block's
+    // waves in turn; lane l sums piece l % Q of the entries 64/Q apart.  With
+    // one thread per (row, piece) a row of 2,000 entries set the time of the
+    // launch, 77-100 us at any width (1e5 rows, power law).
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int turn = 0;
+    for (int c0 = 0; c0 < r1 - r0; c0 += 64) {
+      int s = 0, e = 0;
+      if (c0 + lane < r1 - r0) {
+        s = ia[r0 + c0 + lane] - j0;
+        e = ia[r0 + c0 + lane + 1] - j0;
+      }
+      unsigned long long rows = __ballot(e - s > kUnevenRow);
+      while (rows) {
+        const int b = __ffsll((long long)rows) - 1;
+        rows &= rows - 1;
+        if ((turn++ & (kThreads / 64 - 1)) != wave) continue;
+        const int ss = __shfl(s, b, 64), ee = __shfl(e, b, 64);
+        T acc[P];
+#pragma unroll
+        for (int i = 0; i < P; i++) acc[i] = 0;
+        for (int q = ss + lane / Q; q < ee; q += 64 / Q) {
+          T pv[P];
+          ld_piece<T, P>(prod + (size_t)q * B + piece * P, pv);
+#pragma unroll
+          for (int i = 0; i < P; i++) acc[i] += pv[i];
+        }
+#pragma unroll
+        for (int off = 32; off >= Q; off >>= 1) {
+#pragma unroll
+          for (int i = 0; i < P; i++) acc[i] += __shfl_xor(acc[i], off, 64);
+        }
+        if (lane < Q) f(r0 + c0 + b, piece, acc);
+      }
+    }
+  }
   const int nrq = (r1 - r0) * Q;
   for (int u = threadIdx.x; u < nrq; u += kThreads) {
     const int r = r0 + u / Q, pc = u % Q;
     const int qs = ia[r] - j0, qe = ia[r + 1] - j0;
+    if (uneven && qe - qs > kUnevenRow) continue;
     T acc[P];
 #pragma unroll
     for (int e = 0; e < P; e++) acc[e] = 0;
+#pragma unroll 4
     for (int q = qs; q < qe; q++) {
       T pv[P];
       ld_piece<T, P>(prod + (size_t)q * B + pc * P, pv);
@@ -812,9 +852,9 @@ template <typename T, int B, class Epi>
 __global__ void __launch_bounds__(kThreads)
 k_blk_bal(const int *__restrict__ rowblk, const int *__restrict__ ia,
           const int *__restrict__ ja, const T *__restrict__ a, const T *__restrict__ x,
-          Epi epi) {
+          int uneven, Epi epi) {
   __shared__ T prod[Pieces<T, B>::NZ * B];
-  bal_rows<T, B>(xcd_block(blockIdx.x, gridDim.x), rowblk, ia, ja, a, x, prod,
+  bal_rows<T, B>(xcd_block(blockIdx.x, gridDim.x), rowblk, ia, ja, a, x, prod, uneven,
                  [&](int r, int pc, const T (&acc)[Pieces<T, B>::P]) {
                    typename Epi::Ops o;
                    epi.load(r, pc, o);
@@ -828,13 +868,13 @@ template <typename T, int B>
 __global__ void __launch_bounds__(kThreads)
 k_kpm_bal(const int *__restrict__ rowblk, const int *__restrict__ ia,
           const int *__restrict__ ja, const T *__restrict__ a, EpiKpm<T, B, T> epi, size_t gstride,
-          int ncol, double *__restrict__ part) {
+          int ncol, int uneven, double *__restrict__ part) {
   constexpr int P = Pieces<T, B>::P;
   __shared__ T prod[Pieces<T, B>::NZ * B];
   const int rb = xcd_block(blockIdx.x, gridDim.x);
   epi.group(blockIdx.y, gstride);
   KpmSums<P> sums;
-  bal_rows<T, B>(rb, rowblk, ia, ja, a, epi.v, prod, [&](int r, int pc, const T (&acc)[P]) {
+  bal_rows<T, B>(rb, rowblk, ia, ja, a, epi.v, prod, uneven, [&](int r, int pc, const T (&acc)[P]) {
     typename EpiKpm<T, B, T>::Ops o;
     epi.load(r, pc, o);
     epi.finish(r, pc, o, acc, sums);
@@ -1856,7 +1896,8 @@ void cheb_step_bal(const DevCsr &A, int B, const T *vk, const T *vkm1, T *vkp1,
   case BB: {                                                                             \
     const EpiCheb<T, BB> epi{vk, vkm1, vkp1, y, (T)cc, (T)t, mus, k, nact, ymode};       \
     hipLaunchKernelGGL((k_blk_bal<T, BB, EpiCheb<T, BB>>), dim3(A.nrowblk_q[lv]),        \
-                       dim3(kThreads), 0, s, A.rowblk_q[lv], A.ia, A.ja, a, vk, epi);    \
+                       dim3(kThreads), 0, s, A.rowblk_q[lv], A.ia, A.ja, a, vk,          \
+                       A.max_row > kUnevenRow ? 1 : 0, epi);    \
     break;                                                                               \
   }
     CASE(1) CASE(2) CASE(4) CASE(8) CASE(16) CASE(32)
@@ -1882,7 +1923,8 @@ void clen_step_bal(const DevCsr &A, int B, const T *b1, const T *b2, const T *v,
   case BB: {                                                                             \
     const EpiClen<T, BB> epi{b1, b2, v, out, (T)cc, (T)t, mus, k};                       \
     hipLaunchKernelGGL((k_blk_bal<T, BB, EpiClen<T, BB>>), dim3(A.nrowblk_q[lv]),        \
-                       dim3(kThreads), 0, s, A.rowblk_q[lv], A.ia, A.ja, a, b1, epi);    \
+                       dim3(kThreads), 0, s, A.rowblk_q[lv], A.ia, A.ja, a, b1,          \
+                       A.max_row > kUnevenRow ? 1 : 0, epi);    \
     break;                                                                               \
   }
     CASE(1) CASE(2) CASE(4) CASE(8) CASE(16) CASE(32)
@@ -2095,7 +2137,7 @@ void kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, do
     hipLaunchKernelGGL((k_kpm_bal<T, BB>), dim3(A.nrowblk_q[lv], ng), dim3(kThreads), 0, s, \
                        A.rowblk_q[lv], A.ia, A.ja, a,                                       \
                        EpiKpm<T, BB, T>{v, vw, v0, (T)ctr, (T)scal, first ? 1 : 0},         \
-                       (size_t)A.n * BB, ng * BB, part);                                    \
+                       (size_t)A.n * BB, ng * BB, A.max_row > kUnevenRow ? 1 : 0, part);                                    \
     break;
     CASE(1) CASE(2) CASE(4) CASE(8) CASE(16) CASE(32)
 #undef CASE
