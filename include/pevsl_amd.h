@@ -122,9 +122,8 @@ void pEVSL_RandSeed(unsigned seed);
 /* Kernel of the one-column filter step: lanes per row of the vector-CSR
  * kernel (1..64, power of two), PEVSL_SPMV_STREAM for the CSR-stream kernel
  * (row blocks staged in LDS), or 0 = automatic; and the block width of
- * batched solves (1..64, power of two; 0 = 8 columns per block for an
- * FP32 filter and 4 for FP64, the widths pEVSL_Autotune picks on the
- * 7-point stencil). */
+ * batched solves (1..64, power of two; 0 = by the block kernel and the
+ * matrix: 4 to 32 columns per block). */
 #define PEVSL_SPMV_STREAM 128
 int pEVSL_SetSpmvTuning(pevsl_Data *pevsl, int lanes_per_row, int block_width);
 

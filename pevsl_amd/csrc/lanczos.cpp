@@ -381,6 +381,7 @@ class BatchSolver {
 
   // the filter groups of one step: at most the tuned width, one interval map
   std::vector<std::vector<int>> filter_groups(const std::vector<int> &act) const;
+  int group_max() const;
   // block SpMM kernel of the batched filter: 0 lane per (row, column), 1
   // row per thread, 2 its Clenshaw form, 3 / 4 the nnz-balanced forms of 1 /
   // 2, 5 the segmented Clenshaw form (FP32).  Default: 2 on the FP32 path,
@@ -770,6 +771,27 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
     run((double *)nullptr);
 }
 
+// Most slices a filter group holds: the tuned width, else by kernel, from the
+// times per column and launch (microseconds; 7-point stencil and power-law
+// matrices):
+//   segmented kernel: its widest block, one pass over the matrix for all;
+//   nnz-balanced kernels: 16 (2e6 rows, FP64: width 4 292, 8 153, 16 126; FP32:
+//     8 141, 16 74: a gathered row of x is a line of memory at any width);
+//   diagonal layout: 32 or 16 while the four blocks of a launch stay small, as
+//     a launch then costs much the same at every width (20^3, FP32: 8 0.37, 32
+//     0.09; 48x40x44: 8 0.47, 16 0.34; wider groups run more columns past their
+//     own degree), else 8 (100^3, FP64: 4 4.6, 8 4.1);
+//   row kernels: 8 (FP32) / 4 (FP64), as wider row gathers cost more per column.
+int BatchSolver::group_max() const {
+  const int elem = c_.filter_prec == PEVSL_PREC_FP32 ? 4 : 8, kind = block_kind();
+  if (c_.block_width) return c_.block_width;
+  if (kind == 5) return kMaxSegs * 16 / elem;
+  if (kind == 3 || kind == 4) return 16;
+  if ((kind == 1 || kind == 2) && use_dia(*c_.A, elem, 32))
+    return 4.0 * n_ * 32 * elem <= 16e6 ? 32 : 4.0 * n_ * 16 * elem <= 32e6 ? 16 : 8;
+  return elem == 4 ? 8 : 4;
+}
+
 std::vector<std::vector<int>> BatchSolver::filter_groups(const std::vector<int> &act) const {
   // groups of at most gmax slices that share the filter's interval map
   // (cc, dd: FindPol sets them from each slice's own [lmin, lmax],
@@ -782,14 +804,7 @@ std::vector<std::vector<int>> BatchSolver::filter_groups(const std::vector<int> 
     if (pa->dd != pb->dd) return pa->dd < pb->dd;
     return pa->deg > pb->deg;
   });
-  // group width: the tuned one, else the widest block of the segmented
-  // kernel (one pass over the matrix for all columns), else 8 (FP32) / 4
-  // (FP64), which pEVSL_Autotune picks for the row kernels on the 7-point
-  // stencil (wider row gathers cost more per column)
-  const int kind = block_kind();
-  const int gmax = c_.block_width ? c_.block_width
-                   : kind == 5    ? kMaxSegs * 16 / (c_.filter_prec == PEVSL_PREC_FP32 ? 4 : 8)
-                   : (c_.filter_prec == PEVSL_PREC_FP32 ? 8 : 4);
+  const int gmax = group_max();
   std::vector<std::vector<int>> out;
   for (size_t i = 0; i < order.size();) {
     const pevsl_Polparams *p0 = S_[(size_t)order[i]].pol;
