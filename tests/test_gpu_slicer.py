@@ -355,3 +355,56 @@ def test_irregular_slicer_beats_cheap_kpm_on_unseen_powerlaw(lib):
     assert len(net_i) >= 3
     assert np.mean(net_i) < np.mean(cheap_i), (net_i, cheap_i)
     assert np.mean(net_e) < np.mean(cheap_e), (net_e, cheap_e)
+
+
+@pytest.mark.parametrize("batch,nin,nh,nl,nout", [(1, 1, 1, 1, 1), (31, 7, 33, 2, 5),
+                                                   (32, 32, 32, 1, 32), (33, 65, 31, 3, 34),
+                                                   (70, 138, 64, 0, 513), (129, 9, 100, 1, 66)])
+def test_mlp_gradient_at_tile_edges(lib, batch, nin, nh, nl, nout):
+    """Loss and gradient where the 32 x 32 tiles and the turns of 32 over k have
+    remainders, against float64 numpy."""
+    print("\n[gpu case] MLP gradient batch %d %d-%dx%d-%d" % (batch, nin, nh, nl, nout), flush=True)
+    import math
+    rng = np.random.default_rng(batch)
+    nsoft = nout - nout // 3
+    net = slicer.Mlp(lib, nin, nh, nl, nout, nsoft)
+    dims = [nin] + [nh] * nl + [nout]
+    w = rng.normal(0, 0.3, net.nweights).astype(np.float32)
+    net.set_weights(w)
+    X = rng.normal(size=(batch, nin)).astype(np.float32)
+    Q = rng.normal(size=(batch, nout)).astype(np.float32)
+    T = rng.normal(size=(batch, nout)).astype(np.float32)
+    T[:, :nsoft] = np.abs(T[:, :nsoft]) + 0.1
+    T[:, :nsoft] /= T[:, :nsoft].sum(1, keepdims=True)
+    try:
+        loss, grad = net.loss_grad(X, Q, T)
+    finally:
+        net.free()
+    erf = np.vectorize(math.erf)
+    Ws, bs, off = [], [], 0
+    for i, o in zip(dims, dims[1:]):
+        Ws.append(w[off:off + i * o].reshape(o, i).astype(float))
+        bs.append(w[off + i * o:off + i * o + o].astype(float))
+        off += i * o + o
+    hs, zs = [X.astype(float)], []
+    for l, (W, b) in enumerate(zip(Ws, bs)):
+        zs.append(hs[-1] @ W.T + b)
+        hs.append(0.5 * zs[-1] * (1 + erf(zs[-1] / math.sqrt(2))) if l < nl else zs[-1])
+    y = hs[-1] + Q
+    s = y[:, :nsoft] - y[:, :nsoft].max(1, keepdims=True)
+    lse = np.log(np.exp(s).sum(1, keepdims=True))
+    Td = T.astype(float)
+    t = Td[:, :nsoft]
+    ref = float((-(t * (s - lse)).sum(1) + ((y[:, nsoft:] - Td[:, nsoft:]) ** 2).sum(1)).mean())
+    d = np.concatenate([np.exp(s - lse) - t, 2 * (y[:, nsoft:] - Td[:, nsoft:])], 1) / batch
+    parts = []
+    for l in range(nl, -1, -1):
+        parts = [(d.T @ hs[l]).ravel(), d.sum(0)] + parts
+        if l:
+            z = zs[l - 1]
+            d = (d @ Ws[l]) * (0.5 * (1 + erf(z / math.sqrt(2)))
+                               + z * np.exp(-0.5 * z * z) / math.sqrt(2 * math.pi))
+    g = np.concatenate(parts)
+    # FP32 products of at most 513 terms through at most 4 layers
+    assert abs(loss - ref) <= 2e-5 * max(1.0, abs(ref))
+    assert np.linalg.norm(grad - g) <= 2e-5 * np.linalg.norm(g)
