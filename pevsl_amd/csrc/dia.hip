@@ -126,39 +126,57 @@ struct MuArg {
 // trip to memory).  Bound by LDS reads and barriers inside, by the overlap of
 // the windows where the band is wide.  FP64, microseconds per degree, a launch
 // per degree -> best s:
-//   chain 64,000 rows 4.0 -> 0.50 (s = 32)   1e6 rows 6.6 -> 1.5 (s = 32)
-//   12^3 3.0 -> 1.34 (s = 6)    20^3 3.0 -> 2.35 (s = 5), FP32 3.0 -> 1.91
-//   60^2 4.0 -> 0.97 (s = 8)    250^2 3.8 -> 2.3 (s = 6)  400^2 4.0 -> 3.5
+//   chain 64,000 rows 3.8 -> 0.46 (s = 32)   1e6 rows 6.6 -> 1.3 (s = 32)
+//   12^3 3.8 -> 1.1 (s = 12)    20^3 3.0-4.1 -> 1.95 (s = 5), FP32 1.92
+//   60^2 3.8 -> 0.82 (s = 16)   250^2 3.8 -> 1.8 (s = 7)  400^2 3.9 -> 2.95
+// (with a select per absent diagonal instead of the zeros below: 20^3 2.35,
+// 250^2 2.3)
 // K rows of the window per thread, blockDim.x apart.
-template <typename T, int UC, int K>
+template <typename T, int UC, int K, bool DV>
 __global__ void __launch_bounds__(1024)
 k_cheb_multi(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask, int bw, int R, int d0,
              int s, int last, const T *__restrict__ vin, const T *__restrict__ vmin,
              T *__restrict__ vout, T *__restrict__ vmout, T *__restrict__ y, T cc, T t1, T t2,
              MuArg<T> mus) {
 #pragma clang fp contract(off)
+  // the window's two vectors, each with a zero at its end that absent
+  // diagonals read: adding c times zero leaves the sum as it is, bit for bit (a
+  // sum that starts at +0 never becomes -0), and an entry costs no selects
+  constexpr int kSlot = kMultiRows + 8;
   extern __shared__ char multi_lds[];
   const int r0 = blockIdx.x * R, r1 = min(n, r0 + R);
   const int w0 = max(0, r0 - s * bw), w1 = min(n, r1 + s * bw), L = w1 - w0;
-  T *a = reinterpret_cast<T *>(multi_lds), *b = a + L;
-  uint32_t mk[K];
+  T *const va = reinterpret_cast<T *>(multi_lds), *const vb = va + kSlot;
+  // byte offsets of each row's neighbours in a vector, two to a register
+  uint32_t at[K][UC / 2];
   T dg[K], yv[K];
 #pragma unroll
   for (int i = 0; i < K; i++) {
     const int x = threadIdx.x + i * (int)blockDim.x, r = w0 + x;
-    mk[i] = 0;
     dg[i] = yv[i] = 0;
+    uint32_t m = 0;
     if (x < L) {
-      mk[i] = mask[r];
-      if (d.qd >= 0) dg[i] = d.dg[r];
+      m = mask[r];
+      if (DV) dg[i] = d.dg[r];
       const T v = vin[r];
-      a[x] = v;
-      b[x] = d0 > 1 ? vmin[r] : (T)0;
+      va[x] = v;
+      vb[x] = d0 > 1 ? vmin[r] : (T)0;
       if (r >= r0 && r < r1) yv[i] = d0 > 1 ? y[r] : v * mus.m0;
     }
+#pragma unroll
+    for (int q = 0; q < UC; q++) {
+      const int c = x + d.off[q];
+      // rows near the window's ends have neighbours outside it, in steps that
+      // do not compute them
+      const bool on = ((m >> q) & 1) && c >= 0 && c < L;
+      const uint32_t o = (uint32_t)(on ? c : L) * (uint32_t)sizeof(T);
+      at[i][q / 2] = q % 2 ? at[i][q / 2] | (o << 16) : o;
+    }
   }
+  if (threadIdx.x == 0) va[L] = vb[L] = 0;
   __syncthreads();
-  for (int j = 0; j < s; j++) {
+  // degree d0 + j from `from` (v_{d-1}) over `to` (v_{d-2} -> v_d)
+  auto step = [&](int j, const T *from, T *to) {
     const int h = (s - 1 - j) * bw;
     const int lo = max(0, r0 - h), hi = min(n, r1 + h);
     const T t = d0 + j == 1 ? t1 : t2;
@@ -166,24 +184,33 @@ k_cheb_multi(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask, int b
     for (int i = 0; i < K; i++) {
       const int x = threadIdx.x + i * (int)blockDim.x, r = w0 + x;
       if (r < lo || r >= hi) continue;
-      T acc = 0;
+      T xv[UC];
 #pragma unroll
       for (int q = 0; q < UC; q++) {
-        const bool on = (mk[i] >> q) & 1;
-        const T av = q == d.qd ? dg[i] : d.c[q];
-        const T z = acc + av * a[on ? x + d.off[q] : 0];
-        acc = on ? z : acc;
+        const uint32_t o = q % 2 ? at[i][q / 2] >> 16 : at[i][q / 2] & 0xffffu;
+        xv[q] = *reinterpret_cast<const T *>(reinterpret_cast<const char *>(from) + o);
       }
-      T w = acc + (-cc) * a[x];
+      T acc = 0;
+#pragma unroll
+      for (int q = 0; q < UC; q++) acc = acc + (DV && q == d.qd ? dg[i] : d.c[q]) * xv[q];
+      T w = acc + (-cc) * from[x];
       w = w * t;
-      if (d0 + j > 1) w = w + (T)(-1) * b[x];
-      b[x] = w;
+      if (d0 + j > 1) w = w + (T)(-1) * to[x];
+      to[x] = w;
       if (r >= r0 && r < r1) yv[i] = yv[i] + mus.mu[j] * w;
     }
     __syncthreads();
-    T *sw = a;
-    a = b;
-    b = sw;
+  };
+  int j = 0;
+  for (; j + 1 < s; j += 2) {
+    step(j, va, vb);
+    step(j + 1, vb, va);
+  }
+  const T *fin = va, *prev = vb;
+  if (j < s) {
+    step(j, va, vb);
+    fin = vb;
+    prev = va;
   }
 #pragma unroll
   for (int i = 0; i < K; i++) {
@@ -191,8 +218,8 @@ k_cheb_multi(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask, int b
     if (r < r0 || r >= r1) continue;
     y[r] = yv[i];
     if (!last) {
-      vout[r] = a[x];
-      vmout[r] = b[x];
+      vout[r] = fin[x];
+      vmout[r] = prev[x];
     }
   }
 }
@@ -404,7 +431,7 @@ template void dia_clen_blk<float>(const DevCsr &, int, const float *, const floa
 // degree m; s = 1 where one launch per degree is at least as good.  Model in
 // microseconds, fitted to the times of s = 2 .. 32 on the grids at
 // k_cheb_multi: a launch costs 4.5 and 0.8e-3 per row of the window it loads; a
-// degree inside it 0.2, and 0.5e-3 (U + 3)/10 per row it steps for U diagonals,
+// degree inside it 0.2, and 0.35e-3 (U + 3)/10 per row it steps for U diagonals,
 // for each round of workgroups over the CUs; one launch per degree costs 3.0 +
 // 5.6e-6 n.  The window must fit 64 KiB of LDS, which ends the gain where the
 // band is wide (30^3: 900 rows either side per degree) or the grid large.
@@ -413,14 +440,14 @@ MultiPlan dia_multi_plan(const DevCsr &A, int elem, int m) {
   if (!use_dia(A, elem, 1) || m < 2 || A.n > (1 << 20) || A.dia.ndiag > 8) return best;
   int bw = 0;
   for (int q = 0; q < A.dia.ndiag; q++) bw = std::max(bw, std::abs(A.dia.off[q]));
-  const double row = 0.5e-3 * (A.dia.ndiag + 3) / 10.0;
+  const double row = 0.35e-3 * (A.dia.ndiag + 3) / 10.0;
   double tbest = 3.0 + 5.6e-6 * A.n;
   for (int per = 1; per <= 8; per *= 2) {
     const int R = std::max(64, (A.n + 256 * per - 1) / (256 * per));
     const int wgs = (A.n + R - 1) / R;
     for (int s = 2; s <= std::min(m, kMultiMax); s++) {
       const long long L = (long long)R + 2LL * s * bw;
-      if (L > kMultiRows || 2 * L * elem > kMultiLds) break;
+      if (L > kMultiRows) break;
       const double t = (4.5 + 0.8e-3 * (double)L) / s +
                        ((wgs + 255) / 256) * (0.2 + row * (R + (double)bw * (s - 1)));
       if (t < tbest) {
@@ -448,10 +475,17 @@ void dia_cheb_multi(const DevCsr &A, const MultiPlan &p, const T *v, const T *vm
   const int K = (L + nt - 1) / nt;
   auto go = [&](auto uc, auto k) {
     constexpr int UC = decltype(uc)::value, KK = decltype(k)::value;
-    hipLaunchKernelGGL((k_cheb_multi<T, UC, KK>), dim3((A.n + p.R - 1) / p.R), dim3(nt),
-                       2 * (size_t)L * sizeof(T), st, A.n, dia_arg<T, UC>(A.dia),
-                       (const DiaMask<UC> *)A.dia.mask, p.bw, p.R, d0, s, last ? 1 : 0, v, vm,
-                       vout, vmout, y, (T)cc, (T)(1.0 / dd), (T)(2.0 / dd), ma);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((A.n + p.R - 1) / p.R), dim3(nt),
+                         (size_t)(kMultiRows + 8 + L + 1) * sizeof(T), st, A.n,
+                         dia_arg<T, UC>(A.dia), (const DiaMask<UC> *)A.dia.mask, p.bw, p.R, d0, s,
+                         last ? 1 : 0, v, vm, vout, vmout, y, (T)cc, (T)(1.0 / dd), (T)(2.0 / dd),
+                         ma);
+    };
+    if (A.dia.qd >= 0)
+      launch(k_cheb_multi<T, UC, KK, true>);
+    else
+      launch(k_cheb_multi<T, UC, KK, false>);
   };
   auto width = [&](auto uc) {
     if (K <= 1)

@@ -170,8 +170,8 @@ struct MultiPlan {
   int s = 1, R = 0, bw = 0;
 };
 constexpr int kMultiMax = 32;      // degrees per launch at most
-constexpr int kMultiRows = 4096;   // rows of a workgroup's window at most
-constexpr int kMultiLds = 65536;   // bytes of LDS for its two vectors
+// rows of a workgroup's window at most: its two FP64 vectors fill 64 KiB of LDS
+constexpr int kMultiRows = 4080;
 MultiPlan dia_multi_plan(const DevCsr &A, int elem, int m);
 template <typename T>
 void dia_cheb_multi(const DevCsr &A, const MultiPlan &p, const T *v, const T *vm, T *vout,
