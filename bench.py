@@ -133,9 +133,9 @@ def slice_checks(g, sli, s, o):
 # or as plain CSR with --no-col16: their profiler names differ, the timers'
 # name the step
 STEP_FORMS = ("k_clen_blkrow<", "k_cheb_blkrow<", "k_cheb_stream<")
-DIA_NAMES = {"k_clen_blkrow": "k_dia_blk<%s,%s,8,EpiClen<%s,%s>>",
-             "k_cheb_blkrow": "k_dia_blk<%s,%s,8,EpiCheb<%s,%s>>",
-             "k_cheb_stream": "k_cheb_dia<%s,8>"}
+DIA_NAMES = {"k_clen_blkrow": "k_dia_blk<%s,%s,7,EpiClen<%s,%s>>",
+             "k_cheb_blkrow": "k_dia_blk<%s,%s,7,EpiCheb<%s,%s>>",
+             "k_cheb_stream": "k_cheb_dia<%s,7>"}
 
 
 def profiler_name(name, col16):

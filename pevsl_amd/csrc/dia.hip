@@ -127,10 +127,10 @@ struct MuArg {
 // the windows where the band is wide.  FP64, microseconds per degree, a launch
 // per degree -> best s:
 //   chain 64,000 rows 3.8 -> 0.46 (s = 32)   1e6 rows 6.6 -> 1.3 (s = 32)
-//   12^3 3.8 -> 1.1 (s = 12)    20^3 3.0-4.1 -> 1.95 (s = 5), FP32 1.92
-//   60^2 3.8 -> 0.82 (s = 16)   250^2 3.8 -> 1.8 (s = 7)  400^2 3.9 -> 2.95
-// (with a select per absent diagonal instead of the zeros below: 20^3 2.35,
-// 250^2 2.3)
+//   12^3 3.7 -> 1.06 (s = 12)   20^3 3.0-4.1 -> 1.89 (s = 5), FP32 1.86
+//   60^2 3.8 -> 0.75 (s = 8)    250^2 3.7 -> 1.65 (s = 7)  400^2 3.8 -> 2.7
+// (with a select per absent diagonal instead of the zeros below: 20^3 2.4,
+// 250^2 2.1)
 // K rows of the window per thread, blockDim.x apart.
 template <typename T, int UC, int K, bool DV>
 __global__ void __launch_bounds__(1024)
@@ -148,7 +148,7 @@ k_cheb_multi(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask, int b
   const int w0 = max(0, r0 - s * bw), w1 = min(n, r1 + s * bw), L = w1 - w0;
   T *const va = reinterpret_cast<T *>(multi_lds), *const vb = va + kSlot;
   // byte offsets of each row's neighbours in a vector, two to a register
-  uint32_t at[K][UC / 2];
+  uint32_t at[K][(UC + 1) / 2];
   T dg[K], yv[K];
 #pragma unroll
   for (int i = 0; i < K; i++) {
@@ -329,12 +329,20 @@ DiaArg<T, UC, C> dia_arg(const DevDia &D) {
   return d;
 }
 
-// f(std::integral_constant<int, UC>) for the diagonal count's kernel
+// f(std::integral_constant<int, UC>) for the diagonal count's kernel.  Chains
+// and grids of two and three dimensions have 3, 5 and 7 diagonals; a slot more
+// than that costs its load and its arithmetic as a real one does (with 4 and 8
+// slots instead of these: 100^3 block steps 2-5% longer, 250^2 filter 1.8
+// instead of 1.65 us a degree, 20^3 1.95 instead of 1.89).
 template <class F>
 void dia_dispatch(const DevDia &D, F &&f) {
-  if (D.ndiag <= 4)
-    f(std::integral_constant<int, 4>{});
-  else if (D.ndiag <= 8)
+  if (D.ndiag <= 3)
+    f(std::integral_constant<int, 3>{});
+  else if (D.ndiag <= 5)
+    f(std::integral_constant<int, 5>{});
+  else if (D.ndiag <= 7)
+    f(std::integral_constant<int, 7>{});
+  else if (D.ndiag == 8)
     f(std::integral_constant<int, 8>{});
   else
     f(std::integral_constant<int, kMaxDiags>{});
@@ -495,10 +503,9 @@ void dia_cheb_multi(const DevCsr &A, const MultiPlan &p, const T *v, const T *vm
     else
       go(uc, std::integral_constant<int, 4>{});
   };
-  if (A.dia.ndiag <= 4)
-    width(std::integral_constant<int, 4>{});
-  else
-    width(std::integral_constant<int, 8>{});
+  dia_dispatch(A.dia, [&](auto uc) {
+    if constexpr (decltype(uc)::value <= 8) width(uc);
+  });
 }
 template void dia_cheb_multi<double>(const DevCsr &, const MultiPlan &, const double *,
                                      const double *, double *, double *, double *, double, double,

@@ -58,6 +58,7 @@ CASES = {
     "lower_only": lambda: banded(5000, [-3, -2, 0]),
     "lap2d": lambda: driver.laplacian3d(31, 17, 1),
     "lap3d": lambda: driver.laplacian3d(13, 11, 7),
+    "6_diags": lambda: banded(2000, [-90, -7, 0, 7, 90, 91], drop=0.1, vary=[0]),
     "8_diags": lambda: banded(3001, [-700, -31, -1, 0, 1, 31, 700, 2999], drop=0.1, vary=[0]),
     "9_diags": lambda: banded(3001, [-700, -31, -2, -1, 0, 1, 2, 31, 700], drop=0.1, vary=[0]),
     "32_diags": lambda: banded(2500, list(range(-16, 16)), vary=[0]),
