@@ -28,6 +28,11 @@ __device__ __forceinline__ int xcd_block(int bid, int nb) {
   return x * q + min(x, r) + j;
 }
 
+// number of row blocks of XCD x; its first is xcd_block(x, nb)
+__device__ __forceinline__ int xcd_count(int x, int nb) {
+  return nb / kXcds + (x < nb % kXcds ? 1 : 0);
+}
+
 // B-wide rows of an interleaved block cut into Q pieces of P columns (16
 // bytes where the row has that much).
 //
@@ -223,20 +228,18 @@ struct EpiKpm {
   }
   __device__ __forceinline__ void finish(int r, int pc, const Ops &o, const AT (&acc)[P],
                                          KpmSums<P> &s) const {
-#pragma clang fp contract(off)
     T w[P];
 #pragma unroll
     for (int e = 0; e < P; e++) {
-      AT x = acc[e] + (-ctr) * (AT)o.v[e];
-      x = x * scal;
-      w[e] = (T)(x + (AT)(-1) * (AT)o.vm[e]);
+      const AT x = __builtin_elementwise_fma(-ctr, (AT)o.v[e], acc[e]);
+      w[e] = (T)__builtin_elementwise_fma(scal, x, -(AT)o.vm[e]);
       const double we = w[e], ve = o.v[e];
       if (v0) {
-        s.s[0][e] += we * (double)o.z[e];
+        s.s[0][e] = __builtin_fma(we, (double)o.z[e], s.s[0][e]);
       } else {
-        s.s[0][e] += we * we;
-        s.s[1][e] += we * ve;
-        if (first) s.s[2][e] += ve * ve;
+        s.s[0][e] = __builtin_fma(we, we, s.s[0][e]);
+        s.s[1][e] = __builtin_fma(we, ve, s.s[1][e]);
+        if (first) s.s[2][e] = __builtin_fma(ve, ve, s.s[2][e]);
       }
     }
     st_piece<T, P>(vw + (size_t)r * B + pc * P, w);

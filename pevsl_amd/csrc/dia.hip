@@ -224,11 +224,14 @@ k_cheb_multi(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask, int b
   }
 }
 
-// sum of row r times piece pc (columns pc*P ..) of the interleaved block x,
-// in type C
-template <typename T, int B, int UC, typename C = T>
+// sum of row r times piece pc (columns pc*P ..) of the interleaved block x of
+// n rows, in type C.  Absent diagonals read a row inside the block, so that the
+// loads need not wait for the mask (100^3 FP32: B=4 11.4 -> 10.4 us, B=8 20.7
+// -> 20.1).  FMA: with fused multiply-adds and their operand selected before
+// the conversion, for sums in FP64 that need not repeat the scalar loop's bits.
+template <typename T, int B, int UC, bool FMA = false, typename C = T>
 __device__ __forceinline__ void dia_row_piece(const DiaArg<T, UC, C> &d, uint32_t m, T dgv, int r,
-                                              int pc, const T *__restrict__ x,
+                                              int pc, int n, const T *__restrict__ x,
                                               C (&acc)[Pieces<T, B>::P]) {
 #pragma clang fp contract(off)
   constexpr int P = Pieces<T, B>::P;
@@ -240,7 +243,7 @@ __device__ __forceinline__ void dia_row_piece(const DiaArg<T, UC, C> &d, uint32_
     T xv[CH][P];
 #pragma unroll
     for (int q = 0; q < CH; q++) {
-      const uint32_t row = (m >> (q0 + q)) & 1 ? (uint32_t)(r + d.off[q0 + q]) : 0u;
+      const uint32_t row = (uint32_t)min(max(r + d.off[q0 + q], 0), n - 1);
       const uint32_t at = (row * (uint32_t)B + (uint32_t)(pc * P)) * (uint32_t)sizeof(T);
       ld_piece<T, P>(reinterpret_cast<const T *>(reinterpret_cast<const char *>(x) + at), xv[q]);
     }
@@ -250,8 +253,12 @@ __device__ __forceinline__ void dia_row_piece(const DiaArg<T, UC, C> &d, uint32_
       const bool on = (m >> (q0 + q)) & 1;
 #pragma unroll
       for (int e = 0; e < P; e++) {
-        const C s = acc[e] + a * (C)xv[q][e];
-        acc[e] = on ? s : acc[e];
+        if constexpr (FMA) {
+          acc[e] = __builtin_elementwise_fma(a, (C)(on ? xv[q][e] : (T)0), acc[e]);
+        } else {
+          const C s = acc[e] + a * (C)xv[q][e];
+          acc[e] = on ? s : acc[e];
+        }
       }
     }
   }
@@ -263,10 +270,10 @@ __device__ __forceinline__ void dia_row_piece(const DiaArg<T, UC, C> &d, uint32_
 // row-per-thread CSR kernels gather whole rows with one thread each, wait for
 // their LDS staging, and have Q times fewer threads.  Microseconds per launch,
 // row kernels -> this kernel:
-//   100^3, FP32 Clenshaw    B=4 19.1 -> 11.0  8: 28.9 -> 19.0  16: 77.7 -> 33.8
-//   100^3, FP64 three-term  B=4 38.0 -> 18.4  8: 91.3 -> 32.8
-//   48x40x44, FP32 Clenshaw B=8 5.9 -> 3.7    20^3, FP32 B=8 5.2 -> 2.9
-// (100^3, B=8 FP32: 129 MB, 6.8 TB/s, served by the Infinity Cache.)
+//   100^3, FP32 Clenshaw    B=4 19.1 -> 10.0  8: 28.9 -> 17.4  16: 77.7 -> 33-40
+//   100^3, FP64 three-term  B=4 38.0 -> 17.6  8: 91.3 -> 32.6
+//   48x40x44, FP32 Clenshaw B=8 5.9 -> 3.6    20^3, FP32 B=8 5.2 -> 2.9
+// (100^3, B=8 FP32: 129 MB, 7.4 TB/s, served by the Infinity Cache.)
 template <typename T, int B, int UC, class Epi>
 __global__ void __launch_bounds__(kThreads)
 k_dia_blk(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask, const T *__restrict__ x,
@@ -280,29 +287,38 @@ k_dia_blk(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask, const T 
   typename Epi::Ops ops;
   epi.load(r, pc, ops);
   T acc[Pieces<T, B>::P];
-  dia_row_piece<T, B, UC>(d, m, dgv, r, pc, x, acc);
+  dia_row_piece<T, B, UC>(d, m, dgv, r, pc, n, x, acc);
   epi.finish(r, pc, ops, acc);
 }
 
-// One KPM step on B interleaved columns, group blockIdx.y: each workgroup
-// takes `iters` runs of kThreads (row, piece) items, so that its sums end in
-// one reduction and one set of partials.  Bound by the three vector passes
-// (u_j, u_j-1 read, u_j+1 over it).  Whole pEVSL_Kpmdos, against one thread per
-// (row, column) and one product per moment: 100^3, Mdeg 300, 64 FP32 vectors
-// 263 -> 33.6 ms (600 launches of 192 MB: 3.4 TB/s); 20^3, 60 FP64 vectors 8.8
-// -> 3.5 ms, of which 2.5 ms are the rand() stream on the host.
-template <typename T, int B, int UC>
+// One KPM step on B interleaved columns, group blockIdx.y: the workgroups of
+// an XCD sweep its contiguous range of (row, piece) items together, kThreads
+// each at a time, `iters` times, so that the rows in use at one moment are few
+// and stay in its L2, and a workgroup's sums end in one reduction and one set of
+// partials.  Bound by the three vector passes (u_j, u_j-1 read, u_j+1 over it)
+// in FP64, by the FP64 arithmetic on FP32 vectors.  Whole
+// pEVSL_Kpmdos, one thread per (row, column) and one product per moment -> this:
+// 100^3, Mdeg 300, 64 FP32 vectors 263 -> 24.0 ms (600 launches of 192 MB: 4.8
+// TB/s); 20^3, 60 FP64 vectors 8.8 -> 3.4 ms, of which 2.0 ms are the rand()
+// stream on the host.  Each workgroup a contiguous range of its own, and
+// products, sums and selections of absent entries in separate FP64
+// instructions: 33.3 ms at 100^3.
+template <typename T, int B, int UC, bool FIRST>
 __global__ void __launch_bounds__(kThreads)
 k_dia_kpm(int n, DiaArg<T, UC, double> d, const DiaMask<UC> *__restrict__ mask,
           EpiKpm<T, B, double> epi, size_t gstride, int iters, int ncol,
           double *__restrict__ part) {
   constexpr uint32_t Q = Pieces<T, B>::Q;
   constexpr int P = Pieces<T, B>::P;
-  const int blk = xcd_block(blockIdx.x, gridDim.x);
+  // this XCD's workgroups lo .. lo + cnt - 1, this one number j of them
+  const int x = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
+  const int lo = xcd_block(x, gridDim.x), cnt = xcd_count(x, gridDim.x);
   epi.group(blockIdx.y, gstride);
+  epi.v0 = nullptr;
+  epi.first = FIRST;
   KpmSums<P> sums;
   for (int it = 0; it < iters; it++) {
-    const uint32_t g = ((uint32_t)blk * iters + it) * kThreads + threadIdx.x;
+    const uint32_t g = ((uint32_t)lo * iters + (uint32_t)it * cnt + j) * kThreads + threadIdx.x;
     const int r = (int)(g / Q), pc = (int)(g % Q);
     if (r >= n) break;
     const uint32_t m = mask[r];
@@ -310,10 +326,10 @@ k_dia_kpm(int n, DiaArg<T, UC, double> d, const DiaMask<UC> *__restrict__ mask,
     typename EpiKpm<T, B, double>::Ops ops;
     epi.load(r, pc, ops);
     double acc[P];
-    dia_row_piece<T, B, UC, double>(d, m, dgv, r, pc, epi.v, acc);
+    dia_row_piece<T, B, UC, true>(d, m, dgv, r, pc, n, epi.v, acc);
     epi.finish(r, pc, ops, acc, sums);
   }
-  kpm_block_sums<T, B>(sums, epi.nsum(), ncol, gridDim.x, blk,
+  kpm_block_sums<T, B>(sums, epi.nsum(), ncol, gridDim.x, lo + j,
                        part + (size_t)blockIdx.y * B * gridDim.x);
 }
 
@@ -556,8 +572,10 @@ template double cheb_run<float>(const DevCsr &, const double *, int, double, dou
                                 float *, float *, hipStream_t);
 
 // runs of kThreads (row, piece) items per workgroup: as many as leave about
-// kKpmBlocks workgroups (eight per CU)
-constexpr int kKpmBlocks = 2048;
+// kKpmBlocks workgroups (four per CU).  100^3 FP32, 64 vectors: 512 29.5 ms,
+// 768 26.0, 1024 25.3, 2048 28.3, 4096 29.2; FP64, 32 vectors: 21.0, 20.5, 23.6,
+// 27.4, 27.7; 48x40x44 and 300^2: 1024 the best or within 3%
+constexpr int kKpmBlocks = 1024;
 static int dia_kpm_iters(int n, int elem, int B) {
   const long long items = (long long)n * std::max(1, B * elem / 16);
   return (int)((items + (long long)kThreads * kKpmBlocks - 1) / ((long long)kThreads * kKpmBlocks));
@@ -569,23 +587,29 @@ int dia_kpm_blocks(int n, int elem, int B) {
 }
 
 template <typename T>
-void dia_kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, double ctr,
-                  double scal, bool first, double *part, hipStream_t s) {
+void dia_kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, double ctr, double scal,
+                  bool first, double *part, hipStream_t s) {
   width_dispatch(B, [&](auto b) {
     constexpr int BB = decltype(b)::value;
     dia_dispatch(A.dia, [&](auto uc) {
       constexpr int UC = decltype(uc)::value;
-      hipLaunchKernelGGL((k_dia_kpm<T, BB, UC>),
-                         dim3(dia_kpm_blocks(A.n, sizeof(T), BB), ng), dim3(kThreads), 0, s, A.n,
-                         dia_arg<T, UC, double>(A.dia), (const DiaMask<UC> *)A.dia.mask,
-                         EpiKpm<T, BB, double>{v, vw, v0, ctr, scal, first ? 1 : 0},
-                         (size_t)A.n * BB, dia_kpm_iters(A.n, sizeof(T), BB), ng * BB, part);
+      auto go = [&](auto fi) {
+        hipLaunchKernelGGL((k_dia_kpm<T, BB, UC, decltype(fi)::value>),
+                           dim3(dia_kpm_blocks(A.n, sizeof(T), BB), ng), dim3(kThreads), 0, s, A.n,
+                           dia_arg<T, UC, double>(A.dia), (const DiaMask<UC> *)A.dia.mask,
+                           EpiKpm<T, BB, double>{v, vw, nullptr, ctr, scal, 0},
+                           (size_t)A.n * BB, dia_kpm_iters(A.n, sizeof(T), BB), ng * BB, part);
+      };
+      if (first)
+        go(std::true_type{});
+      else
+        go(std::false_type{});
     });
   });
 }
-template void dia_kpm_step<double>(const DevCsr &, int, int, const double *, double *,
-                                   const double *, double, double, bool, double *, hipStream_t);
-template void dia_kpm_step<float>(const DevCsr &, int, int, const float *, float *, const float *,
-                                  double, double, bool, double *, hipStream_t);
+template void dia_kpm_step<double>(const DevCsr &, int, int, const double *, double *, double,
+                                   double, bool, double *, hipStream_t);
+template void dia_kpm_step<float>(const DevCsr &, int, int, const float *, float *, double, double,
+                                  bool, double *, hipStream_t);
 
 }  // namespace pevsl

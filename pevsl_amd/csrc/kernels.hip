@@ -2125,7 +2125,7 @@ void kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, do
               double scal, bool first, double *part, hipStream_t s) {
   if (A.n == 0) return;
   if (use_dia(A, sizeof(T), B)) {
-    dia_kpm_step<T>(A, B, ng, v, vw, v0, ctr, scal, first, part, s);
+    dia_kpm_step<T>(A, B, ng, v, vw, ctr, scal, first, part, s);
     return;
   }
   const int lv = bal_level((int)sizeof(T), B);

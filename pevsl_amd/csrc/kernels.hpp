@@ -245,8 +245,8 @@ void kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, do
 int kpm_blocks(const DevCsr &A, int elem, int B);
 int dia_kpm_blocks(int n, int elem, int B);
 template <typename T>
-void dia_kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, double ctr,
-                  double scal, bool first, double *part, hipStream_t s);
+void dia_kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, double ctr, double scal,
+                  bool first, double *part, hipStream_t s);
 // raw: ncol column-major n-vectors; group g of blk gets columns g B .. as
 // x / sqrt(nrm2[c]), zero past ncol
 template <typename T>

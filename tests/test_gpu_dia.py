@@ -232,3 +232,37 @@ def test_kpm_on_both_layouts(lib, prec, Mdeg, nvec):
             assert np.max(np.abs(mu - ref)) <= (1e-13 if prec == 0 else 2e-5)
     finally:
         M.free()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_kpm_several_runs_of_rows(lib, prec):
+    """Enough rows that each workgroup takes several runs of them, the last
+    ones partly or wholly past the end, against the recurrence in FP64."""
+    print("\n[gpu case] KPM several runs, prec %d" % prec, flush=True)
+    sp = pytest.importorskip("scipy.sparse")
+    ia, ja, a = driver.laplacian3d(33, 33, 31)
+    n, nvec, Mdeg = len(ia) - 1, 33, 5
+    A = sp.csr_matrix((a, ja, ia), shape=(n, n))
+    M = driver.Matrix(lib, ia, ja, a)
+    try:
+        inst = driver.Instance(lib, M, prec=prec)
+        try:
+            lib.pEVSL_RandSeed(11)
+            rc, mu, _ = inst.kpmdos(Mdeg, 0, nvec, [3.0, 5.0, 0.0, 12.0])
+        finally:
+            inst.close()
+    finally:
+        M.free()
+    assert rc == 0
+    libc = C.CDLL(None)
+    libc.srand(11)
+    t = 2147483647.0 / 2
+    v = (np.array([libc.rand() for _ in range(n * nvec)], float).reshape(nvec, n).T - t) / t
+    v /= np.linalg.norm(v, axis=0)
+    u, um, ref = v, None, [1.0 / np.pi]
+    for k in range(Mdeg):
+        w = (A @ u - 6.0 * u) * ((2.0 if k else 1.0) / 6.0) - (um if k else 0.0)
+        um, u = u, w
+        ref.append(2.0 / (nvec * np.pi) * float((w * v).sum()))
+    # as in test_kpm_on_both_layouts
+    assert np.max(np.abs(mu - np.array(ref))) <= (1e-13 if prec == 0 else 2e-5)
