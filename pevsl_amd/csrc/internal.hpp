@@ -145,6 +145,7 @@ struct Ctx {
   int rand_mode = PEVSL_RAND_LIBC;
   unsigned long long rand_seed = 0;
   unsigned long long rand_offset = 0;
+  DBuf<uint32_t> d_rand;           // workspace of rand_vectors, at most 4 MiB
   int lanes = 0;                   // lanes per row of the single-column SpMV
   int use_stream = -1;             // CSR-stream filter kernel: 1 yes, 0 no, -1 auto
   // lanes argument of the products with A: the tuned vector-CSR kernel, or 0

@@ -1759,6 +1759,18 @@ __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
   return x ^ (x >> 31);
 }
 
+// Outputs of the rand() stream to [-1, 1], the host's operations (an exact
+// difference, a correctly rounded quotient) and so its bits.
+__global__ void __launch_bounds__(kThreads)
+k_rand_convert(int n, size_t i0, size_t cnt, const uint32_t *__restrict__ r,
+               double *__restrict__ X, size_t ld) {
+  const size_t k = (size_t)blockIdx.x * kThreads + threadIdx.x;
+  if (k >= cnt) return;
+  const size_t e = i0 + k, col = e / (size_t)n;
+  const double t = 2147483647.0 / 2.0;
+  X[col * ld + (e - col * (size_t)n)] = ((double)(r[k] >> 1) - t) / t;
+}
+
 __global__ void k_rand(size_t n, double *__restrict__ x, uint64_t seed,
                        uint64_t offset, int rademacher) {
   const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
@@ -2471,6 +2483,13 @@ void col_axpy(int n, int ncol, const double *a, const double *X, size_t ldx,
   if (ncol <= 0 || n == 0) return;
   hipLaunchKernelGGL(k_col_axpy, dim3(grid_for(n), ncol), dim3(kThreads), 0,
                      s, n, a, X, ldx, Y, ldy);
+}
+
+void rand_convert(int n, size_t i0, size_t cnt, const uint32_t *r, double *X, size_t ld,
+                  hipStream_t s) {
+  if (cnt == 0) return;
+  hipLaunchKernelGGL(k_rand_convert, dim3(grid_for(cnt)), dim3(kThreads), 0, s, n, i0, cnt, r, X,
+                     ld);
 }
 
 void rand_fill(size_t n, double *x, uint64_t seed, uint64_t offset,

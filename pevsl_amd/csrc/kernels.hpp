@@ -385,6 +385,10 @@ void col_axpy(int n, int ncol, const double *a, const double *X, size_t ldx,
 // sum over degrees as the reference does).
 void kpm_intchx(int Mdeg, const double *mu, int npts, const double *th,
                 double th0, double *yi, hipStream_t s);
+// Elements i0 .. i0 + cnt - 1 of the columns X (n rows, column stride ld) from
+// outputs r of the rand() stream: ((r >> 1) - t) / t, t = RAND_MAX / 2.
+void rand_convert(int n, size_t i0, size_t cnt, const uint32_t *r, double *X, size_t ld,
+                  hipStream_t s);
 // Rademacher (+-1) or uniform [-1,1] counter-based random numbers.
 void rand_fill(size_t n, double *x, uint64_t seed, uint64_t offset,
                int rademacher, hipStream_t s);
