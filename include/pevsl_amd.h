@@ -129,7 +129,7 @@ int pEVSL_SetSpmvTuning(pevsl_Data *pevsl, int lanes_per_row, int block_width);
 
 /* Block SpMM kernel of batched solves: 1 = one thread per row with B-wide
  * row gathers (B <= 32) and the reference's three-term recurrence with an
- * accumulator updated every other degree (4 vector passes per degree on
+ * accumulator updated every third degree (3 2/3 vector passes per degree on
  * average, the sums of one update per degree bit for bit), 2 = the same
  * kernel in Clenshaw form (4 passes), 3 / 4 = the nnz-balanced forms of
  * 1 / 2 (products formed in parallel over nonzeros and staged in LDS, long

@@ -222,7 +222,7 @@ int pEVSL_BenchBlock(pevsl_Data *p, int B, int reps, double *sec, double *bytes)
   *sec = f32 ? time_blk<float>(c, B, reps, mus, kind) : time_blk<double>(c, B, reps, mus, kind);
   const int idx = (kind == 1 || kind == 2) ? index_bytes(*c.A) : 4;
   // four vector passes per degree for all but the lane-per-(row, column)
-  // kernel (Clenshaw; three-term row kernels with y every other degree)
+  // kernel (Clenshaw; three-term kernels with y every third degree move 3 2/3)
   *bytes = kind != 0 ? step_bytes(*c.A, elem, B, idx) - (double)c.A->n * B * elem
                      : step_bytes(*c.A, elem, B, idx);
   return 0;
