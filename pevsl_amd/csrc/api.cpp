@@ -262,42 +262,56 @@ struct HostDia {
 // the row before, which one comparison per entry establishes.
 bool find_dia(int n, const int *ia, const int *ja, const double *a, HostDia &D) {
   if (n <= 0 || ia[n] <= 0) return false;
-  int nd = 0, off[kMaxDiags], qrow[kMaxDiags];
+  int nd = 0, off[kMaxDiags];
   double c[kMaxDiags];
   bool varies[kMaxDiags];
   int prev = -1, plen = -1, nvar = 0;
-  auto same = [](double x, double y) { return memcmp(&x, &y, sizeof x) == 0; };
+  auto bits = [](double x) {
+    uint64_t u;
+    memcpy(&u, &x, sizeof u);
+    return u;
+  };
+  // the row's entries: their diagonals' bits and which of them must be equal
+  uint64_t want[kMaxDiags], fixed[kMaxDiags];
+  uint32_t m = 0;
   // diagonals in order of first appearance, one value each
   std::vector<uint32_t> rm((size_t)n);
   for (int i = 0; i < n; i++) {
     const int b = ia[i], len = ia[i + 1] - b;
-    bool rep = len == plen;
-    for (int j = 0; rep && j < len; j++) rep = ja[b + j] - i == ja[prev + j] - (i - 1);
-    if (!rep) {
-      if (len > kMaxDiags) return false;
+    if (len == plen) {
+      int dj = 0;
+      uint64_t da = 0;
       for (int j = 0; j < len; j++) {
-        if (j > 0 && ja[b + j] <= ja[b + j - 1]) return false;
-        const int o = ja[b + j] - i;
-        int q = 0;
-        while (q < nd && off[q] != o) q++;
-        if (q == nd) {
-          if (nd == kMaxDiags) return false;
-          if (!std::isfinite(a[b + j])) return false;
-          off[nd] = o;
-          c[nd] = a[b + j];
-          varies[nd++] = false;
-        }
-        qrow[j] = q;
+        dj |= (ja[b + j] - i) ^ (ja[prev + j] - (i - 1));
+        da |= (bits(a[b + j]) ^ want[j]) & fixed[j];
+      }
+      if (dj == 0 && da == 0) {
+        rm[(size_t)i] = m;
+        prev = b;
+        continue;
       }
     }
-    uint32_t m = 0;
+    if (len > kMaxDiags) return false;
+    m = 0;
     for (int j = 0; j < len; j++) {
-      const int q = qrow[j];
+      if (j > 0 && ja[b + j] <= ja[b + j - 1]) return false;
+      const int o = ja[b + j] - i;
+      int q = 0;
+      while (q < nd && off[q] != o) q++;
+      if (q == nd) {
+        if (nd == kMaxDiags) return false;
+        if (!std::isfinite(a[b + j])) return false;
+        off[nd] = o;
+        c[nd] = a[b + j];
+        varies[nd++] = false;
+      }
       m |= 1u << q;
-      if (!varies[q] && !same(a[b + j], c[q])) {
+      if (!varies[q] && bits(a[b + j]) != bits(c[q])) {
         varies[q] = true;
         if (++nvar > 1 || off[q] != 0) return false;
       }
+      want[j] = bits(c[q]);
+      fixed[j] = varies[q] ? 0 : ~(uint64_t)0;
     }
     rm[(size_t)i] = m;
     prev = b;
@@ -339,9 +353,12 @@ bool find_dia(int n, const int *ia, const int *ja, const double *a, HostDia &D) 
   }
   if (D.qd >= 0) {
     D.dg.assign((size_t)n, 0.0);
-    for (int i = 0; i < n; i++)
-      for (int j = ia[i]; j < ia[i + 1]; j++)
-        if (ja[j] == i) D.dg[(size_t)i] = a[j];
+    for (int i = 0, at = 0; i < n; i++) {
+      const int b = ia[i], e = ia[i + 1];
+      if (b + at >= e || ja[b + at] != i)  // not where the row before has it
+        for (at = 0; b + at < e && ja[b + at] < i;) at++;
+      if (b + at < e && ja[b + at] == i) D.dg[(size_t)i] = a[b + at];
+    }
   }
   return true;
 }
