@@ -27,6 +27,31 @@
 #include "internal.hpp"
 
 namespace pevsl {
+
+// The layout is decided once, for the widest group, and B follows from it: the
+// host's form (sums per step, v0) and the kernel that runs must agree, and at
+// 2^25 rows in FP32 a group of 16 still fits the layout's 32-bit offsets where
+// one of 32 does not.
+//
+// Width of a group of interleaved vectors: 32, or on the diagonal layout what
+// leaves its two blocks in the Infinity Cache from step to step (the balanced
+// kernels gather whole rows and gain from width in any case); as many groups
+// in one launch as fit there together.
+KpmPlan kpm_plan(const DevCsr &A, int elem, int nvec) {
+  constexpr double kResident = 160e6;
+  constexpr int kWidest = 32;
+  KpmPlan p;
+  p.dia = use_dia(A, elem, kWidest);
+  p.direct = !p.dia && elem == 4;
+  p.B = 1;
+  while (p.B < nvec && p.B < kWidest &&
+         (!p.dia || p.B < 4 || 4.0 * A.n * p.B * elem <= kResident))
+    p.B *= 2;
+  const double gbytes = 2.0 * A.n * p.B * elem;
+  p.ng = std::max(1, std::min((nvec + p.B - 1) / p.B, (int)std::min(64.0, kResident / gbytes)));
+  return p;
+}
+
 namespace {
 
 int check_intv(const double *intv, FILE *f) {
@@ -98,21 +123,13 @@ void kpm_moments(Ctx &c, int n, int Mdeg, int nvec, double ctr, double wid,
   const hipStream_t s = c.stream;
   const int elem = (int)sizeof(T);
   if (Mdeg < 1 || nvec < 1) return;
-  // Width of a group of interleaved vectors: 32, or on the diagonal layout
-  // what leaves its two blocks in the Infinity Cache from step to step (the
-  // balanced kernels gather whole rows and gain from width in any case); as
-  // many groups in one launch as fit there together.
-  constexpr double kResident = 160e6;
-  const bool dia = use_dia(A, elem, 32);
-  const bool direct = !dia && elem == 4;
-  int B = 1;
-  while (B < nvec && B < 32 && (!dia || B < 4 || 4.0 * n * B * elem <= kResident)) B *= 2;
-  const double gbytes = 2.0 * n * B * elem;
-  const int ng = std::max(1, std::min((nvec + B - 1) / B, (int)std::min(64.0, kResident / gbytes)));
+  const KpmPlan p = kpm_plan(A, elem, nvec);
+  const bool direct = p.direct;
+  const int B = p.B, ng = p.ng;
   const int W = ng * B;                            // vectors per run
   const int nst = direct ? Mdeg : (Mdeg + 1) / 2;  // products
   const int ns = direct ? 1 : 2;                   // sums per step and column
-  const int nblk = kpm_blocks(A, elem, B);
+  const int nblk = kpm_blocks(A, p.dia, elem, B);
   // partials of `keep` steps before they are summed
   const int keep = (int)std::max(1.0, std::min((double)std::min(nst, 64),
                                                64e6 / (16.0 * W * nblk)));
@@ -141,7 +158,7 @@ void kpm_moments(Ctx &c, int n, int Mdeg, int nvec, double ctr, double wid,
     int pend = 0, done = 0;
     for (int j = 0; j < nst; j++) {
       double *pt = part.p + (size_t)ns * pend * W * nblk;
-      kpm_step<T>(A, B, ng, v, vw, v0, ctr, (j == 0 ? 1.0 : 2.0) / wid, j == 0, pt, s);
+      kpm_step<T>(A, p.dia, B, ng, v, vw, v0, ctr, (j == 0 ? 1.0 : 2.0) / wid, j == 0, pt, s);
       if (j == 0 && !direct)
         row_sums(pt + (size_t)2 * W * nblk, W, nblk, sums.p + (size_t)2 * nst * W, s);
       pend++;
@@ -221,6 +238,19 @@ void kpm_moments_op(Ctx &c, int n, int Mdeg, int nvec, double ctr, double wid,
 using namespace pevsl;
 
 extern "C" {
+
+int pEVSL_KpmForm(int n, int ndiag, int prec, int nvec, int *width, int *groups) {
+  if (n < 1 || ndiag < 0 || ndiag > kMaxDiags || nvec < 1 ||
+      (prec != PEVSL_PREC_FP64 && prec != PEVSL_PREC_FP32))
+    return -1;
+  DevCsr A;
+  A.n = n;
+  A.dia.ndiag = ndiag;
+  const KpmPlan p = kpm_plan(A, prec == PEVSL_PREC_FP32 ? 4 : 8, nvec);
+  if (width) *width = p.B;
+  if (groups) *groups = p.ng;
+  return p.dia ? 2 : p.direct ? 0 : 1;
+}
 
 int pEVSL_Kpmdos(pevsl_Data *pevsl, int Mdeg, int damping, int nvec, double *intv,
                  int ngroups, int groupid, MPI_Comm gl_comm, double *mu, double *ecnt) {

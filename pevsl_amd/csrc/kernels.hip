@@ -2127,16 +2127,16 @@ template void cheb_step_blk<float>(const DevCsr &, int, const float *,
                                    double, const double *, int, int,
                                    hipStream_t);
 
-int kpm_blocks(const DevCsr &A, int elem, int B) {
-  if (use_dia(A, elem, B)) return dia_kpm_blocks(A.n, elem, B);
+int kpm_blocks(const DevCsr &A, bool dia, int elem, int B) {
+  if (dia) return dia_kpm_blocks(A.n, elem, B);
   return A.nrowblk_q[bal_level(elem, B)];
 }
 
 template <typename T>
-void kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, double ctr,
+void kpm_step(const DevCsr &A, bool dia, int B, int ng, const T *v, T *vw, const T *v0, double ctr,
               double scal, bool first, double *part, hipStream_t s) {
   if (A.n == 0) return;
-  if (use_dia(A, sizeof(T), B)) {
+  if (dia) {
     dia_kpm_step<T>(A, B, ng, v, vw, ctr, scal, first, part, s);
     return;
   }
@@ -2157,9 +2157,9 @@ void kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, do
       break;
   }
 }
-template void kpm_step<double>(const DevCsr &, int, int, const double *, double *, const double *,
-                               double, double, bool, double *, hipStream_t);
-template void kpm_step<float>(const DevCsr &, int, int, const float *, float *, const float *,
+template void kpm_step<double>(const DevCsr &, bool, int, int, const double *, double *,
+                               const double *, double, double, bool, double *, hipStream_t);
+template void kpm_step<float>(const DevCsr &, bool, int, int, const float *, float *, const float *,
                               double, double, bool, double *, hipStream_t);
 
 template <typename T>

@@ -236,13 +236,21 @@ int bal_level(int elem, int B);
 // columns (group g at v + g n B; B a power of two <= 32), w written over vm
 // (vw); vm is zero, and not read, if `first`.  Per column c = g B + b the block
 // partials of w.w, w.v and (first) v.v, or of w.v0 alone where v0 is given:
-// part[(i ng B + c) nblk + blk] for sum i and blk < nblk = kpm_blocks(A,
-// sizeof(T), B).  On the diagonal layout (row sums and recurrence in FP64
-// whatever T is) or with the nnz-balanced products (in T).
+// part[(i ng B + c) nblk + blk] for sum i and blk < nblk = kpm_blocks(A, dia,
+// sizeof(T), B).  On the diagonal layout (dia: row sums and recurrence in FP64
+// whatever T is, without v0) or with the nnz-balanced products (in T); `dia`
+// is the caller's KpmPlan::dia, since the two forms differ in their sums.
 template <typename T>
-void kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, const T *v0, double ctr,
+void kpm_step(const DevCsr &A, bool dia, int B, int ng, const T *v, T *vw, const T *v0, double ctr,
               double scal, bool first, double *part, hipStream_t s);
-int kpm_blocks(const DevCsr &A, int elem, int B);
+int kpm_blocks(const DevCsr &A, bool dia, int elem, int B);
+// How pEVSL_Kpmdos forms the moments of nvec vectors of `elem` bytes an element.
+struct KpmPlan {
+  bool dia;     // steps on the diagonal layout
+  bool direct;  // one product per moment and <w, v0>; else two moments a product
+  int B, ng;    // vectors in a group, groups in a run
+};
+KpmPlan kpm_plan(const DevCsr &A, int elem, int nvec);
 int dia_kpm_blocks(int n, int elem, int B);
 template <typename T>
 void dia_kpm_step(const DevCsr &A, int B, int ng, const T *v, T *vw, double ctr, double scal,

@@ -308,3 +308,31 @@ def test_missing_library_fails_loudly(tmp_path):
     with pytest.raises(RuntimeError) as e:
         capi.load(str(tmp_path / "libpevsl_amd.so"))
     assert "not found" in str(e.value) and "build" in str(e.value)
+
+
+@pytest.mark.parametrize("prec,elem", [(capi.PEVSL_PREC_FP64, 8), (capi.PEVSL_PREC_FP32, 4)])
+@pytest.mark.parametrize("nvec", [1, 3, 4, 8, 16, 17, 32, 64])
+def test_kpm_form_at_the_diagonal_layouts_limit(lib, prec, elem, nvec):
+    """The diagonal layout's steps address a block of 32 columns with 32-bit
+    byte offsets: 2^25 rows in FP32, 2^24 in FP64.  From there on every number
+    of vectors takes the CSR form, in FP32 with one product per moment: whether
+    a narrower group would still fit plays no part."""
+    width, groups = C.c_int(), C.c_int()
+
+    def form(n, ndiag):
+        f = lib.pEVSL_KpmForm(n, ndiag, prec, nvec, C.byref(width), C.byref(groups))
+        assert 1 <= width.value <= 32 and width.value & (width.value - 1) == 0
+        assert groups.value >= 1
+        return f
+
+    limit = 2 ** 32 // (32 * elem)
+    csr = 0 if prec == capi.PEVSL_PREC_FP32 else 1
+    for n in (315, 10 ** 6, limit - 1):
+        assert form(n, 7) == 2
+        assert n * width.value * elem < 2 ** 32
+        assert form(n, 0) == csr
+    for n in (limit, limit + 1, 324 ** 3, 2 ** 31 - 1):
+        assert form(n, 7) == csr
+    assert lib.pEVSL_KpmForm(0, 7, prec, nvec, None, None) == -1
+    assert lib.pEVSL_KpmForm(10, 33, prec, nvec, None, None) == -1
+    assert lib.pEVSL_KpmForm(10, 7, 2, nvec, None, None) == -1
