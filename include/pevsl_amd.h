@@ -275,10 +275,13 @@ size_t pEVSL_ChebAvNoAllocMaxRows(void);
  * on a matrix of n rows with ndiag diagonals in its diagonal layout (0: the
  * matrix has none): 0 one product with A per moment on the CSR form, 1 two
  * moments per product on the CSR form, 2 two moments per product on the
- * diagonal layout; -1 on invalid arguments.  *width: vectors interleaved in a
+ * diagonal layout; -1 on invalid arguments.  Two moments per product need a
+ * symmetric matrix (columns ascending within rows); pevsl_Stat.n_mvA counts
+ * the products.  *width: vectors interleaved in a
  * group, *groups: groups advanced together (either may be NULL).  Host
  * arithmetic, no device needed. */
-int pEVSL_KpmForm(int n, int ndiag, int prec, int nvec, int *width, int *groups);
+int pEVSL_KpmForm(int n, int ndiag, int symmetric, int prec, int nvec, int *width,
+                  int *groups);
 
 /* Device name and HBM size of the current device; 0 on success. */
 int pEVSL_DeviceInfo(char *name, int len, size_t *hbm_bytes);

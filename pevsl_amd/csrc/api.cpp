@@ -706,16 +706,18 @@ int pEVSL_ParcsrSetup(pevsl_Csr *Ai, pevsl_Parcsr *A) {
   for (int i = 0; fits && i < n; i += std::max(1, n / 64))
     for (int j = Ai->ia[i]; fits && j < Ai->ia[i + 1]; j++)
       fits = std::abs((long)Ai->ja[j] - i) < 32768 + kStreamRows;
-  if (fits) {
-    DBuf<int> over;
-    int bad = 0;
-    PV_HIP(hipMemcpy(over.ensure(1), &bad, sizeof(int), hipMemcpyHostToDevice));
-    offsets16(M->csr, M->jo16.ensure((size_t)nnz), over.p, nullptr);
-    PV_HIP(hipMemcpy(&bad, over.p, sizeof(int), hipMemcpyDeviceToHost));
-    if (bad)
+  {
+    DBuf<int> flags;
+    int bad[2] = {0, n == A->ncol_local ? 0 : 1};  // an offset too far, not symmetric
+    PV_HIP(hipMemcpy(flags.ensure(2), bad, sizeof bad, hipMemcpyHostToDevice));
+    if (fits) offsets16(M->csr, M->jo16.ensure((size_t)nnz), flags.p, nullptr);
+    if (!bad[1]) check_symmetric(M->csr, flags.p + 1, nullptr);
+    PV_HIP(hipMemcpy(bad, flags.p, sizeof bad, hipMemcpyDeviceToHost));
+    if (fits && bad[0])
       M->jo16.release();
-    else
+    else if (fits)
       M->csr.jo16 = M->jo16.p;
+    M->csr.sym = !bad[1];
   }
   // diagonal layout, where the matrix has one
   HostDia hd;

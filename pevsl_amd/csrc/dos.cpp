@@ -41,8 +41,8 @@ KpmPlan kpm_plan(const DevCsr &A, int elem, int nvec) {
   constexpr double kResident = 160e6;
   constexpr int kWidest = 32;
   KpmPlan p;
-  p.dia = use_dia(A, elem, kWidest);
-  p.direct = !p.dia && elem == 4;
+  p.dia = A.sym && use_dia(A, elem, kWidest);
+  p.direct = !A.sym || (!p.dia && elem == 4);
   p.B = 1;
   while (p.B < nvec && p.B < kWidest &&
          (!p.dia || p.B < 4 || 4.0 * A.n * p.B * elem <= kResident))
@@ -115,7 +115,8 @@ Aux &aux() {
 // accurate or more so (relative error of mu, FP32 vectors: 100^3 3.6e-8 ->
 // 2.1e-8, 20^3 1.2e-7 -> 3.4e-9); with FP32 arithmetic throughout they would
 // be ten times worse (100^3: 4e-7).  FP32 on the other matrices therefore
-// takes one product per moment and the dot product with v.
+// takes one product per moment and the dot product with v, and so does a matrix
+// that is not symmetric, for which the products of neighbours say nothing.
 template <typename T>
 void kpm_moments(Ctx &c, int n, int Mdeg, int nvec, double ctr, double wid,
                  std::vector<double> &dots /* [nvec][Mdeg] */) {
@@ -239,13 +240,14 @@ using namespace pevsl;
 
 extern "C" {
 
-int pEVSL_KpmForm(int n, int ndiag, int prec, int nvec, int *width, int *groups) {
+int pEVSL_KpmForm(int n, int ndiag, int symmetric, int prec, int nvec, int *width, int *groups) {
   if (n < 1 || ndiag < 0 || ndiag > kMaxDiags || nvec < 1 ||
       (prec != PEVSL_PREC_FP64 && prec != PEVSL_PREC_FP32))
     return -1;
   DevCsr A;
   A.n = n;
   A.dia.ndiag = ndiag;
+  A.sym = symmetric != 0;
   const KpmPlan p = kpm_plan(A, prec == PEVSL_PREC_FP32 ? 4 : 8, nvec);
   if (width) *width = p.B;
   if (groups) *groups = p.ng;

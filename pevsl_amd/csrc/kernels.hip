@@ -163,6 +163,33 @@ k_offsets16(const int *__restrict__ rowblk, const int *__restrict__ blknz,
   if (bad) *over = 1;
 }
 
+// *bad = 1 unless the matrix is symmetric with ascending columns, a wave per
+// row: each entry's mirror by bisection in its column's row.  Values may differ
+// by the rounding of an assembly that adds them in another order.
+__global__ void __launch_bounds__(kThreads)
+k_symmetric(int n, const int *__restrict__ ia, const int *__restrict__ ja,
+            const double *__restrict__ a, int *__restrict__ bad) {
+  const int i = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+  if (i >= n) return;
+  const int b = ia[i], e = ia[i + 1];
+  for (int j = b + (threadIdx.x & 63); j < e; j += 64) {
+    const int c = ja[j];
+    const double v = a[j];
+    int lo = ia[c], hi = ia[c + 1];
+    const int end = hi;
+    while (lo < hi) {
+      const int m = (lo + hi) / 2;
+      if (ja[m] < i)
+        lo = m + 1;
+      else
+        hi = m;
+    }
+    bool ok = lo < end && ja[lo] == i && (j == b || ja[j - 1] < c);
+    if (ok) ok = fabs(v - a[lo]) <= 4 * DBL_EPSILON * fabs(v);
+    if (!ok) *bad = 1;
+  }
+}
+
 // y = A x, L lanes per row (rows of a wave: 64/L).
 template <int L>
 __global__ void __launch_bounds__(kThreads)
@@ -1849,6 +1876,12 @@ void offsets16(const DevCsr &A, short *jo, int *over, hipStream_t s) {
   if (A.nrowblk == 0) return;
   hipLaunchKernelGGL(k_offsets16, dim3(A.nrowblk), dim3(kThreads), 0, s, A.rowblk, A.blknz, A.ja,
                      jo, over);
+}
+
+void check_symmetric(const DevCsr &A, int *bad, hipStream_t s) {
+  if (A.n == 0) return;
+  hipLaunchKernelGGL(k_symmetric, dim3(grid_for((size_t)A.n, kThreads / 64)), dim3(kThreads), 0, s,
+                     A.n, A.ia, A.ja, A.a64, bad);
 }
 
 template <typename T>

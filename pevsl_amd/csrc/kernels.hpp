@@ -52,6 +52,9 @@ struct DevCsr {
   // `rowblk` (null when an offset does not fit in a short): the CSR-stream
   // and row-per-thread block kernels then read 2 index bytes per nonzero
   short *jo16 = nullptr;
+  // every entry has its mirror, equal to a few roundings (square, columns
+  // ascending within rows): pEVSL_Kpmdos then forms two moments per product
+  bool sym = false;
   // diagonal layout, where the matrix has one (dia.ndiag > 0): the one-column
   // step, the row-per-thread block steps and the products then read it
   DevDia dia;
@@ -83,6 +86,9 @@ void build_row_blocks(int n, const int *ia, std::vector<int> &blk,
 // jo[j] = ja[j] - (first row of nonzero j's row block); *over set to 1 if one
 // does not fit in 16 bits
 void offsets16(const DevCsr &A, short *jo, int *over, hipStream_t s);
+// *bad set to 1 unless every entry (i, j) has a mirror (j, i) of its value and
+// columns ascend strictly within rows (A square)
+void check_symmetric(const DevCsr &A, int *bad, hipStream_t s);
 
 // ---- sparse products -------------------------------------------------------
 // y = A x, one column.  lanes = lanes per row in {1,2,4,8,16,32,64}, or 0 for

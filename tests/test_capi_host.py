@@ -319,8 +319,8 @@ def test_kpm_form_at_the_diagonal_layouts_limit(lib, prec, elem, nvec):
     a narrower group would still fit plays no part."""
     width, groups = C.c_int(), C.c_int()
 
-    def form(n, ndiag):
-        f = lib.pEVSL_KpmForm(n, ndiag, prec, nvec, C.byref(width), C.byref(groups))
+    def form(n, ndiag, sym=1):
+        f = lib.pEVSL_KpmForm(n, ndiag, sym, prec, nvec, C.byref(width), C.byref(groups))
         assert 1 <= width.value <= 32 and width.value & (width.value - 1) == 0
         assert groups.value >= 1
         return f
@@ -331,8 +331,9 @@ def test_kpm_form_at_the_diagonal_layouts_limit(lib, prec, elem, nvec):
         assert form(n, 7) == 2
         assert n * width.value * elem < 2 ** 32
         assert form(n, 0) == csr
+        assert form(n, 7, 0) == form(n, 0, 0) == 0
     for n in (limit, limit + 1, 324 ** 3, 2 ** 31 - 1):
         assert form(n, 7) == csr
-    assert lib.pEVSL_KpmForm(0, 7, prec, nvec, None, None) == -1
-    assert lib.pEVSL_KpmForm(10, 33, prec, nvec, None, None) == -1
-    assert lib.pEVSL_KpmForm(10, 7, 2, nvec, None, None) == -1
+    assert lib.pEVSL_KpmForm(0, 7, 1, prec, nvec, None, None) == -1
+    assert lib.pEVSL_KpmForm(10, 33, 1, prec, nvec, None, None) == -1
+    assert lib.pEVSL_KpmForm(10, 7, 1, 2, nvec, None, None) == -1

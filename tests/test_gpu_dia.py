@@ -266,3 +266,71 @@ def test_kpm_several_runs_of_rows(lib, prec):
         ref.append(2.0 / (nvec * np.pi) * float((w * v).sum()))
     # as in test_kpm_on_both_layouts
     assert np.max(np.abs(mu - np.array(ref))) <= (1e-13 if prec == 0 else 2e-5)
+
+
+def not_symmetric(which):
+    """Matrices for which the products of neighbouring vectors give no
+    moments, and one (unsorted columns) whose symmetry is not looked for."""
+    rng = np.random.default_rng(21)
+    if which == "diagonals":
+        return banded(700, [-3, -2, 0, 1])
+    if which == "values":  # symmetric pattern with a diagonal layout
+        return banded(700, [-1, 0, 1])
+    if which == "one_entry":  # a symmetric layout with one entry missing
+        ia, ja, a = driver.laplacian3d(9, 8, 7)
+        k = int(np.flatnonzero(ja != np.repeat(np.arange(len(ia) - 1), np.diff(ia)))[100])
+        row = int(np.searchsorted(ia, k, side="right")) - 1
+        ia = ia.copy()
+        ia[row + 1:] -= 1
+        return ia, np.delete(ja, k), np.delete(a, k)
+    if which == "csr":
+        n, m = 600, 5
+        ja = np.concatenate([np.sort(rng.choice(n, m, replace=False)) for _ in range(n)])
+        return (np.arange(n + 1, dtype=np.int32) * m, ja.astype(np.int32),
+                rng.uniform(-1, 1, n * m))
+    ia, ja, a = driver.laplacian3d(9, 8, 7)  # "unsorted"
+    for i in range(len(ia) - 1):
+        ja[ia[i]:ia[i + 1]] = ja[ia[i]:ia[i + 1]][::-1].copy()
+        a[ia[i]:ia[i + 1]] = a[ia[i]:ia[i + 1]][::-1].copy()
+    return ia, ja, a
+
+
+@pytest.mark.parametrize("which", ["diagonals", "values", "one_entry", "csr", "unsorted"])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_kpm_without_symmetry(lib, which, prec):
+    """<v, T_k v> of a matrix that is not symmetric, against the recurrence in
+    FP64 numpy: one product per moment, whatever the layout."""
+    print("\n[gpu case] KPM without symmetry, %s prec %d" % (which, prec), flush=True)
+    ia, ja, a = not_symmetric(which)
+    n, nvec, Mdeg = len(ia) - 1, 5, 8
+    dense = np.zeros((n, n))
+    np.add.at(dense, (np.repeat(np.arange(n), np.diff(ia)), ja), a)
+    # |A| <= sqrt(|A|_1 |A|_inf); T_k of a non-normal matrix may still grow
+    c0 = 6.0 if which in ("one_entry", "unsorted") else 0.0
+    off = np.abs(dense - c0 * np.eye(n))
+    wid = 2.0 * float(np.sqrt(off.sum(0).max() * off.sum(1).max()))
+    libc = C.CDLL(None)
+    libc.srand(7)
+    t = 2147483647.0 / 2
+    v = (np.array([libc.rand() for _ in range(n * nvec)], float).reshape(nvec, n).T - t) / t
+    v /= np.linalg.norm(v, axis=0)
+    u, um, ref, top = v, None, [1.0 / np.pi], 1.0
+    for k in range(Mdeg):
+        w = (dense @ u - c0 * u) * ((2.0 if k else 1.0) / wid) - (um if k else 0.0)
+        um, u = u, w
+        top = max(top, float(np.linalg.norm(w, axis=0).max()))
+        ref.append(2.0 / (nvec * np.pi) * float((w * v).sum()))
+    M = driver.Matrix(lib, ia, ja, a)
+    try:
+        inst = driver.Instance(lib, M, prec=prec)
+        try:
+            lib.pEVSL_RandSeed(7)
+            rc, mu, _ = inst.kpmdos(Mdeg, 0, nvec, [c0 - 0.1, c0 + 0.1, c0 - wid, c0 + wid])
+            assert inst.stats()["n_mvA"] == nvec * Mdeg
+        finally:
+            inst.close()
+    finally:
+        M.free()
+    assert rc == 0
+    # as in test_kpm_on_both_layouts, times the vectors' largest norm
+    assert np.max(np.abs(mu - np.array(ref))) <= top * (1e-13 if prec == 0 else 2e-5)
