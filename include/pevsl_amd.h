@@ -197,6 +197,10 @@ int pEVSL_SetGraphFilter(pevsl_Data *pevsl, int on);
  * switches it off as well. */
 int pEVSL_SetColumnOffsets16(pevsl_Data *pevsl, int on);
 int pEVSL_ColumnOffsets16(pevsl_Data *pevsl);
+/* Number of diagonals of the layout the instance's matrix is read through, 0
+ * without one; *slots (may be NULL): diagonals of the kernels that run it, the
+ * next of 3, 5, 7, 8, 9, 13, 19, 27, 32. */
+int pEVSL_DiagonalLayout(pevsl_Data *pevsl, int *slots);
 
 /* Return code of pEVSL_ChebLanNrBatch / pEVSL_ChebLanNr when a Lanczos
  * basis does not fit in device memory; the call releases what it held and

@@ -546,6 +546,13 @@ int pEVSL_ColumnOffsets16(pevsl_Data *p) {
   return c.A && c.A->jo16 ? 1 : 0;
 }
 
+int pEVSL_DiagonalLayout(pevsl_Data *p, int *slots) {
+  const Ctx &c = ctx_of(p);
+  const int nd = c.A ? c.A->dia.ndiag : 0;
+  if (slots) *slots = nd ? dia_slots(nd) : 0;
+  return nd;
+}
+
 int pEVSL_SetBatchWave(pevsl_Data *p, int wave) {
   if (wave < 0) return -1;
   ctx_of(p).batch_wave = wave;

@@ -36,6 +36,9 @@ struct DiaArg {
 template <int UC>
 using DiaMask = std::conditional_t<UC <= 8, uint8_t, uint32_t>;
 
+// loads of a row in flight together
+constexpr int dia_chunk(int uc) { return uc <= 9 ? uc : 8; }
+
 // x[i] with a 32-bit byte offset from a uniform base (use_dia bounds it)
 template <typename T>
 __device__ __forceinline__ T ld32(const T *x, uint32_t i) {
@@ -49,15 +52,15 @@ __device__ __forceinline__ T dia_row(const DiaArg<T, UC> &d, uint32_t m, T dgv, 
                                      const T *__restrict__ x) {
 #pragma clang fp contract(off)
   T acc = 0;
-  constexpr int CH = UC < 8 ? UC : 8;
+  constexpr int CH = dia_chunk(UC);
 #pragma unroll
   for (int q0 = 0; q0 < UC; q0 += CH) {
     T xv[CH];
 #pragma unroll
-    for (int q = 0; q < CH; q++)
+    for (int q = 0; q < CH && q0 + q < UC; q++)
       xv[q] = ld32(x, (m >> (q0 + q)) & 1 ? (uint32_t)(r + d.off[q0 + q]) : 0u);
 #pragma unroll
-    for (int q = 0; q < CH; q++) {
+    for (int q = 0; q < CH && q0 + q < UC; q++) {
       const T a = q0 + q == d.qd ? dgv : d.c[q0 + q];
       const T s = acc + a * xv[q];
       acc = (m >> (q0 + q)) & 1 ? s : acc;
@@ -235,20 +238,20 @@ __device__ __forceinline__ void dia_row_piece(const DiaArg<T, UC, C> &d, uint32_
                                               C (&acc)[Pieces<T, B>::P]) {
 #pragma clang fp contract(off)
   constexpr int P = Pieces<T, B>::P;
-  constexpr int CH = UC < 8 ? UC : 8;
+  constexpr int CH = dia_chunk(UC);
 #pragma unroll
   for (int e = 0; e < P; e++) acc[e] = 0;
 #pragma unroll
   for (int q0 = 0; q0 < UC; q0 += CH) {
     T xv[CH][P];
 #pragma unroll
-    for (int q = 0; q < CH; q++) {
+    for (int q = 0; q < CH && q0 + q < UC; q++) {
       const uint32_t row = (uint32_t)min(max(r + d.off[q0 + q], 0), n - 1);
       const uint32_t at = (row * (uint32_t)B + (uint32_t)(pc * P)) * (uint32_t)sizeof(T);
       ld_piece<T, P>(reinterpret_cast<const T *>(reinterpret_cast<const char *>(x) + at), xv[q]);
     }
 #pragma unroll
-    for (int q = 0; q < CH; q++) {
+    for (int q = 0; q < CH && q0 + q < UC; q++) {
       const C a = q0 + q == d.qd ? (C)dgv : d.c[q0 + q];
       const bool on = (m >> (q0 + q)) & 1;
 #pragma unroll
@@ -344,23 +347,18 @@ DiaArg<T, UC, C> dia_arg(const DevDia &D) {
   return d;
 }
 
-// f(std::integral_constant<int, UC>) for the diagonal count's kernel.  Chains
-// and grids of two and three dimensions have 3, 5 and 7 diagonals; a slot more
-// than that costs its load and its arithmetic as a real one does (with 4 and 8
-// slots instead of these: 100^3 block steps 2-5% longer, 250^2 filter 1.8
-// instead of 1.65 us a degree, 20^3 1.95 instead of 1.89).
+// f(std::integral_constant<int, UC>) for the diagonal count's kernel
+// (dia_slots).
 template <class F>
 void dia_dispatch(const DevDia &D, F &&f) {
-  if (D.ndiag <= 3)
-    f(std::integral_constant<int, 3>{});
-  else if (D.ndiag <= 5)
-    f(std::integral_constant<int, 5>{});
-  else if (D.ndiag <= 7)
-    f(std::integral_constant<int, 7>{});
-  else if (D.ndiag == 8)
-    f(std::integral_constant<int, 8>{});
-  else
-    f(std::integral_constant<int, kMaxDiags>{});
+  switch (dia_slots(D.ndiag)) {
+#define CASE(UC)                           \
+  case UC:                                 \
+    f(std::integral_constant<int, UC>{});  \
+    break;
+    CASE(3) CASE(5) CASE(7) CASE(8) CASE(9) CASE(13) CASE(19) CASE(27) CASE(kMaxDiags)
+#undef CASE
+  }
 }
 
 }  // namespace

@@ -27,6 +27,20 @@ struct DevDia {
   const double *dg64 = nullptr;  // main diagonal per row (qd >= 0)
   const float *dg32 = nullptr;
 };
+// Diagonals of the kernel that runs a layout of ndiag: the counts of the usual
+// stencils (chains, 5- and 9-point, 7-, 13-, 19- and 27-point), so that from two
+// diagonals on at most a third of the slots are spare: one costs its load and its
+// arithmetic as a real one does.  Microseconds with more slots -> with these:
+//   8 -> 5, 250^2 filter 1.8 -> 1.65 a degree     8 -> 7, 20^3 1.95 -> 1.89
+//   32 -> 9, 9-point 1000^2: filter FP64 19.6 -> 9.4, FP32 9.9 -> 5.5; width 8
+//     FP64 77 -> 34, FP32 36.8 -> 17.9 (CSR 34.4: 32 slots lost to it)
+//   32 -> 13, 19, 27, 100^3: width 8 FP32 38 -> 23, 27, 33; FP64 73 -> 47, 51, 70
+inline int dia_slots(int ndiag) {
+  constexpr int kSlots[] = {3, 5, 7, 8, 9, 13, 19, 27, kMaxDiags};
+  for (int s : kSlots)
+    if (ndiag <= s) return s;
+  return 0;
+}
 inline int dia_mask_bytes(const DevDia &D) { return D.ndiag <= 8 ? 1 : 4; }
 
 // Device CSR: int32 row pointers / column indices, values in FP64 and FP32.

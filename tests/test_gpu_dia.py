@@ -44,6 +44,15 @@ def banded(n, offs, vary=None, drop=0.0, seed=0):
     return np.cumsum(ia).astype(np.int32), c[order].astype(np.int32), v[order]
 
 
+def count_band(n, count):
+    """Symmetric band of `count` diagonals, a varying main one among them if
+    the count is odd."""
+    up = [1 + k * k // 2 + k for k in range(count // 2)]
+    ia, ja, a = banded(n, [-o for o in up] + up + [0] * (count % 2), vary=[0], seed=count)
+    o = np.abs(ja - np.repeat(np.arange(n), np.diff(ia)))
+    return ia, ja, np.where(o > 0, 0.3 + 0.1 * (o % 7), a)
+
+
 CASES = {
     "1x1": lambda: banded(1, [0]),
     "one_row_block": lambda: banded(255, [-1, 0, 1]),
@@ -62,6 +71,9 @@ CASES = {
     "8_diags": lambda: banded(3001, [-700, -31, -1, 0, 1, 31, 700, 2999], drop=0.1, vary=[0]),
     "9_diags": lambda: banded(3001, [-700, -31, -2, -1, 0, 1, 2, 31, 700], drop=0.1, vary=[0]),
     "32_diags": lambda: banded(2500, list(range(-16, 16)), vary=[0]),
+    # the last count of each kernel above 8 diagonals, and the first of the next
+    **{"count_%d" % k: (lambda k=k: count_band(1500 + k, k)) for k in
+       (10, 13, 14, 19, 20, 27, 28)},
     "empty_rows": lambda: banded(700, [-9, 9], drop=0.45),
     # no such layout: 33 diagonals, a second varying diagonal, mostly absent
     "33_diags": lambda: banded(900, list(range(-16, 17))),
@@ -334,3 +346,102 @@ def test_kpm_without_symmetry(lib, which, prec):
     assert rc == 0
     # as in test_kpm_on_both_layouts, times the vectors' largest norm
     assert np.max(np.abs(mu - np.array(ref))) <= top * (1e-13 if prec == 0 else 2e-5)
+
+
+# diagonals and slots of each case's layout (0: none)
+LAYOUT = {"1x1": 1, "one_row_block": 3, "block_edge": 3, "block_edge_1": 3, "3_of_4_dropped": 3,
+          "4_no_main": 4, "chain_wide": 3, "band_31": 5, "band_400": 7, "lower_only": 3, "lap2d": 5,
+          "lap3d": 7, "6_diags": 6, "8_diags": 8, "9_diags": 9, "32_diags": 32, "empty_rows": 2,
+          "33_diags": 0, "two_vary": 0, "sparse_diags": 0,
+          **{"count_%d" % k: k for k in (10, 13, 14, 19, 20, 27, 28)}}
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_layout_is_taken(lib, name):
+    """The cases above run, or do not run, on the layout they are meant for,
+    with spare slots of at most a third from two diagonals on."""
+    print("\n[gpu case] diagonal layout taken, %s" % name, flush=True)
+    M = driver.Matrix(lib, *CASES[name]())
+    slots = C.c_int(-1)
+    try:
+        for on in (True, False):
+            inst = driver.Instance(lib, M, col16=on)
+            try:
+                nd = lib.pEVSL_DiagonalLayout(inst.p, C.byref(slots))
+            finally:
+                inst.close()
+            assert nd == (LAYOUT[name] if on else 0)
+            assert slots.value >= nd and (nd < 2 or 3 * (slots.value - nd) <= slots.value)
+            assert nd > 0 or slots.value == 0
+    finally:
+        M.free()
+
+
+COUNTS = [9, 10, 13, 14, 19, 20, 27, 28, 32]
+
+
+@pytest.mark.parametrize("prec,kind,width", [(0, 1, 4), (1, 2, 8), (1, 1, 2)])
+@pytest.mark.parametrize("count", COUNTS)
+def test_block_steps_by_diagonal_count(lib, count, prec, kind, width):
+    print("\n[gpu case] diagonal layout, block, %d diagonals prec %d kind %d width %d" % (
+        count, prec, kind, width), flush=True)
+    M = driver.Matrix(lib, *count_band(901, count))
+    rad = 20.0
+    intvs = [[0.05 * rad * i, 0.05 * rad * (i + 0.9), -rad, rad] for i in range(5)]
+    pols = [driver.find_pol(lib, iv)[0] for iv in intvs]
+    vinit = np.random.default_rng(5).uniform(-1, 1, M.n)
+    runs = []
+    try:
+        for on in (True, False):
+            inst = driver.Instance(lib, M, prec=prec, block_rowkernel=kind, block_width=width,
+                                   col16=on)
+            try:
+                assert lib.pEVSL_DiagonalLayout(inst.p, None) == (count if on else 0)
+                rc, outs = driver.cheblan_batch(inst, intvs, [40] * 5, 1e-8, vinit, pols)
+                assert rc == 0
+                runs.append(outs)
+            finally:
+                inst.close()
+    finally:
+        for p_ in pols:
+            lib.pEVSL_FreePol(C.byref(p_))
+        M.free()
+    for x, y in zip(*runs):
+        assert x["info"]["its"] == y["info"]["its"]
+        assert x["info"]["tr"] == y["info"]["tr"]
+        np.testing.assert_array_equal(x["lam"], y["lam"])
+        np.testing.assert_array_equal(x["res"], y["res"])
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("count", COUNTS)
+def test_kpm_by_diagonal_count(lib, count, prec):
+    print("\n[gpu case] KPM, %d diagonals prec %d" % (count, prec), flush=True)
+    ia, ja, a = count_band(901, count)
+    n, nvec, Mdeg, rad = 901, 9, 11, 24.0
+    dense = np.zeros((n, n))
+    dense[np.repeat(np.arange(n), np.diff(ia)), ja] = a
+    libc = C.CDLL(None)
+    libc.srand(3)
+    t = 2147483647.0 / 2
+    v = (np.array([libc.rand() for _ in range(n * nvec)], float).reshape(nvec, n).T - t) / t
+    v /= np.linalg.norm(v, axis=0)
+    u, um, ref = v, None, [1.0 / np.pi]
+    for k in range(Mdeg):
+        w = (dense @ u) * ((2.0 if k else 1.0) / rad) - (um if k else 0.0)
+        um, u = u, w
+        ref.append(2.0 / (nvec * np.pi) * float((w * v).sum()))
+    M = driver.Matrix(lib, ia, ja, a)
+    try:
+        inst = driver.Instance(lib, M, prec=prec)
+        try:
+            lib.pEVSL_RandSeed(3)
+            rc, mu, _ = inst.kpmdos(Mdeg, 0, nvec, [1.0, 2.0, -rad, rad])
+            assert inst.stats()["n_mvA"] == nvec * ((Mdeg + 1) // 2)  # on the layout
+        finally:
+            inst.close()
+    finally:
+        M.free()
+    assert rc == 0
+    # as in test_kpm_on_both_layouts
+    assert np.max(np.abs(mu - np.array(ref))) <= (1e-13 if prec == 0 else 2e-5)
