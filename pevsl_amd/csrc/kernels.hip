@@ -1208,6 +1208,8 @@ k_gram_mfma(int n, int m1, int m2, const double *__restrict__ X, size_t ldx,
 // types' (FP64): 16-byte row groups of kThreads threads
 constexpr int kLanRows = kThreads * 2;
 
+constexpr int kGtCols = 256;  // see gt_trips
+
 // per-slice sizes of the partials (see LanArgs)
 struct LanParts {
   size_t nbmax, tcap;
@@ -1217,8 +1219,8 @@ LanParts lan_parts(size_t ld, int hcap) {
   LanParts p;
   p.nbmax = trips;
   // GEMV-T: full-size row blocks for every column, or one trip per block for
-  // the first columns
-  p.tcap = std::max((size_t)hcap * ((trips + 15) / 16), trips * (size_t)std::min(hcap, 256));
+  // the first kGtCols columns (gt_trips)
+  p.tcap = std::max((size_t)hcap * ((trips + 15) / 16), trips * (size_t)std::min(hcap, kGtCols));
   return p;
 }
 
@@ -2357,18 +2359,45 @@ size_t lan_part_doubles(int n, int nslice, int hcap) {
 }
 
 namespace {
+// The splits below decide the order of the sums, so they follow from the vector
+// length and the step alone: a slice rounds alike by itself, in a batch of any
+// size and in any wave.
+
 // GEMV-N blocks of a slice and row groups per thread: kGnPairs, or 1 where
 // that leaves CUs without a block (20^3: 8 blocks of 1024 rows)
+constexpr size_t kGnBlocks = 256;
 template <typename TV>
 int gn_pairs(const LanBatch &L) {
   constexpr int P = Row16<TV>::kGnPairs;
   const size_t rows = (size_t)gt_trip<TV>() * P;
-  return L.nslice * ((L.ld + rows - 1) / rows) < 512 ? 1 : P;
+  return (L.ld + rows - 1) / rows < kGnBlocks ? 1 : P;
 }
 template <typename TV>
 int gn_blocks(const LanBatch &L) {
   const size_t rows = (size_t)gt_trip<TV>() * gn_pairs<TV>(L);
   return (int)((L.ld + rows - 1) / rows);
+}
+
+// GEMV-T trips of a block for k + 1 columns: full-size blocks unless they are
+// fewer than half the CUs, then fewer trips each, as far as every LanParts has
+// room (a block per kLanRows rows for the first kGtCols columns).  One row
+// block per column group left the chip idle on short vectors (n = 8,000: 15.5
+// us a pass).  Microseconds of update and pass with at least 64 / 128 / 1024
+// blocks a slice, FP64: one slice n = 84,480, k = 50 63 / 58 / 58, k = 150
+// 89 / 80 / 87; n = 1e6, k = 16 115 / 106 / 132; 16 slices n = 84,480, k = 16
+// 134 / 153 / 153, k = 150 579 / 571 / 650, n = 1e6, k = 16 991 / 990 / 1325.
+constexpr size_t kGtBlocks = 128;
+template <typename TV>
+int gt_trips(const LanBatch &L, int k) {
+  const size_t all = (L.ld + gt_trip<TV>() - 1) / gt_trip<TV>();
+  const size_t room = (L.ld + kLanRows - 1) / kLanRows * kGtCols;
+  const size_t ncb = (k + 1 + kTcols - 1) / kTcols;
+  auto blocks = [&](size_t trips) { return (all + trips - 1) / trips; };
+  size_t trips = Row16<TV>::kTrips;
+  while (trips > 1 && blocks(trips) * ncb < kGtBlocks &&
+         blocks(trips / 2) * (size_t)(k + 1) <= room)
+    trips /= 2;
+  return (int)trips;
 }
 
 template <typename TV>
@@ -2385,16 +2414,8 @@ template <typename TV>
 void lan_cgs_pass_t(const LanBatch &L, int k, int pass, hipStream_t s) {
   LanArgs<TV> a = make_args<TV>(L);
   const int ncb = (k + 1 + kTcols - 1) / kTcols;
-  // GEMV-T row blocks: full-size ones unless they are fewer than four per CU;
-  // then fewer trips each, as far as the partials have room.  One row block
-  // per column group left the chip idle on short vectors (n = 8,000: 15.5 us a
-  // pass, n = 1e5, k = 50: 44 us).
-  const size_t trips_all = (L.ld + gt_trip<TV>() - 1) / gt_trip<TV>();
-  int trips = Row16<TV>::kTrips;
-  while (trips > 1 && ((trips_all + trips - 1) / trips) * ncb * L.nslice < 1024 &&
-         ((trips_all + trips / 2 - 1) / (trips / 2)) * (k + 1) <= a.tcap)
-    trips /= 2;
-  const int nrb = (int)((trips_all + trips - 1) / trips);
+  const int trips = gt_trips<TV>(L, k);
+  const int nrb = (int)((L.ld + (size_t)trips * gt_trip<TV>() - 1) / ((size_t)trips * gt_trip<TV>()));
   // nontemporal basis loads: measured 6.5 vs 5.9 TB/s at k = 4096 (C2)
   hipLaunchKernelGGL((k_lan_gemvt<true, TV>), dim3(nrb, ncb, L.nslice), dim3(kThreads), 0,
                      s, a, k, pass, nrb, trips);

@@ -183,3 +183,46 @@ def test_graph_filter_equals_eager(lib, prec, kind):
     assert blk and all(k_ in kt1 for k_ in blk)
     for k_ in blk:
         assert kt1[k_]["launches"] == kt0[k_]["launches"]
+
+
+@pytest.mark.parametrize("grid", [(11, 12, 10), (20, 20, 20), (60, 40, 30)])
+def test_a_slice_rounds_alike_alone_and_in_any_batch(lib, grid):
+    """FP64 on a grid, whose filter gives every column the same bits in any
+    block: the Gram-Schmidt sums follow from the vector length and the step
+    alone, so a slice solved by itself, in batches of other sizes, beside
+    slices with more room for steps, and in waves gives the same steps, trace,
+    eigenvalues and residuals bit for bit."""
+    banner("one slice alone and in batches, %dx%dx%d" % grid)
+    M = driver.Matrix(lib, *driver.laplacian3d(*grid))
+    ex = np.unique(np.round(driver.exact_eig_lap3(*grid, 0.0, 12.0), 12))
+    edges = [0.5 * (ex[j] + ex[j + 1]) for j in range(0, 46, 5)]  # 5 distinct each
+    intvs = [[edges[i], edges[i + 1], 0.0, 12.0] for i in range(9)]
+    pols = [driver.find_pol(lib, iv)[0] for iv in intvs]
+    vinit = driver.rand_vinit(lib, M.n)
+    pick, maxits, out = 4, 200, {}
+    try:
+        for name, sl, its, wave in (("alone", [4], [maxits], 0),
+                                    ("two", [4, 7], [maxits] * 2, 0),
+                                    ("nine", list(range(9)), [maxits] * 9, 0),
+                                    ("more room", [2, 4, 6], [400, maxits, 300], 0),
+                                    ("waves", list(range(9)), [maxits] * 9, 4)):
+            inst = driver.Instance(lib, M)
+            try:
+                lib.pEVSL_SetBatchWave(inst.p, wave)
+                rc, o = driver.cheblan_batch(inst, [intvs[s] for s in sl], its, 1e-8, vinit,
+                                             [pols[s] for s in sl])
+                assert rc == 0
+                out[name] = o[sl.index(pick)]
+            finally:
+                inst.close()
+    finally:
+        for p_ in pols:
+            lib.pEVSL_FreePol(C.byref(p_))
+        M.free()
+    ref = out.pop("alone")
+    assert len(ref["lam"]) >= 5 and ref["info"]["its"] < maxits
+    for name, o in out.items():
+        assert o["info"]["its"] == ref["info"]["its"], name
+        assert o["info"]["tr"] == ref["info"]["tr"], name
+        np.testing.assert_array_equal(o["lam"], ref["lam"], err_msg=name)
+        np.testing.assert_array_equal(o["res"], ref["res"], err_msg=name)
