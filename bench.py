@@ -129,23 +129,23 @@ def slice_checks(g, sli, s, o):
             "tol_accept": o["info"]["tol_accept"] if o["info"] else None}
 
 
-# steps that read the matrix in its diagonal layout (the Laplacian has one),
-# or as plain CSR with --no-col16: their profiler names differ, the timers'
-# name the step
-STEP_FORMS = ("k_clen_blkrow<", "k_cheb_blkrow<", "k_cheb_stream<")
-DIA_NAMES = {"k_clen_blkrow": "k_dia_blk<%s,%s,7,EpiClen<%s,%s>>",
-             "k_cheb_blkrow": "k_dia_blk<%s,%s,7,EpiCheb<%s,%s>>",
-             "k_cheb_stream": "k_cheb_dia<%s,7>"}
+# CSR forms compiled for 16-bit column offsets (true) and 32-bit indices
+# (false): the profiler's names carry the flag, the timers' do not
+J16_KERNELS = ("k_clen_blkrow<", "k_cheb_blkrow<", "k_cheb_stream<")
 
 
 def profiler_name(name, col16):
-    if name.startswith(STEP_FORMS):
-        if not col16:
-            return name[:-1] + ",false>"
-        form, args = name[:-1].split("<")
-        a = tuple(args.split(","))
-        return DIA_NAMES[form] % (a + a if len(a) > 1 else a)
+    if name.startswith(J16_KERNELS):
+        return name[:-1] + (",true>" if col16 else ",false>")
     return name
+
+
+def filter_rate(ktimes):
+    """GB/s of the filter kernels (names k_*): bytes they read and wrote over
+    their own time."""
+    f = [v for k, v in ktimes.items() if k.startswith("k_")]
+    t = sum(v["seconds"] for v in f)
+    return round(sum(v["bytes"] for v in f) / max(t, 1e-12) / 1e9, 1)
 
 
 def roofline_of(ktimes, traffic, prefer=None, col16=False):
@@ -318,15 +318,16 @@ def probe(kind):
                 log("probe   %2d | %s | %s | %s | %s" % (
                     B, fmt(tr.t_blockclen[i], B), fmt(tr.t_blockseg[i], B),
                     fmt(tr.t_blockrow[i], B), fmt(tr.t_blockbalclen[i], B)))
-            # the Clenshaw row kernel with 16-bit column offsets and with the
-            # 32-bit indices
+            # the Clenshaw row step on the diagonal layout and on plain CSR
             lib.pEVSL_SetBlockKernel(inst.p, 2)
             for col16 in (1, 0):
                 lib.pEVSL_SetColumnOffsets16(inst.p, col16)
                 for B in (4, 8):
                     assert lib.pEVSL_BenchBlock(inst.p, B, 50, C.byref(sec), C.byref(byt)) == 0
                     log("probe clen row kernel width %d, %s: %.2f us, %.1f MB, %.2f TB/s" % (
-                        B, "16-bit offsets" if col16 else "32-bit indices", sec.value * 1e6,
+                        B, "diagonal layout" if lib.pEVSL_DiagonalLayout(inst.p, None)
+                        else "16-bit offsets" if lib.pEVSL_ColumnOffsets16(inst.p)
+                        else "32-bit indices", sec.value * 1e6,
                         byt.value / 1e6, byt.value / sec.value / 1e12))
         finally:
             inst.close()
@@ -364,8 +365,8 @@ def main():
                     help="replays of the captured filter group in the hipGraph-vs-eager "
                          "comparison (0: no comparison)")
     ap.add_argument("--no-col16", action="store_true",
-                    help="32-bit column indices in the filter kernels (default: 16-bit offsets "
-                         "where the matrix has them, pEVSL_SetColumnOffsets16)")
+                    help="plain CSR with 32-bit column indices in the filter kernels (default: "
+                         "the matrix's diagonal layout, pEVSL_SetColumnOffsets16)")
     ap.add_argument("--progress", action="store_true",
                     help="the solver's convergence-test lines (ChebLanNr fstats) on stderr")
     args = ap.parse_args()
@@ -424,6 +425,7 @@ def main():
     inst = driver.Instance(lib, M, prec=capi.PEVSL_PREC_FP32, basis_prec=basis,
                            col16=not args.no_col16)
     out["config"]["col16"] = bool(lib.pEVSL_ColumnOffsets16(inst.p))
+    out["config"]["diagonals"] = lib.pEVSL_DiagonalLayout(inst.p, None)
     lib.pEVSL_SetBatchWave(inst.p, wave)
     lib.pEVSL_SetGraphFilter(inst.p, 1 if args.graph_filter else 0)
     tune = capi.TuneResult()
@@ -485,7 +487,7 @@ def main():
                                                                     "t_eig", "t_ritz")},
                           "stats": {k: st[k] for k in ("n_mvA", "n_polAv", "t_mvA", "t_polAv",
                                                        "t_reorth", "t_eig", "t_ritz")},
-                          "filter_GBs": round(ks["filter_bytes"] / max(ks["t_filter"], 1e-9) / 1e9, 1),
+                          "filter_GBs": filter_rate(inst.kernel_times()),
                           "cgs_GBs": round(ks["cgs_bytes"] / max(ks["t_cgs"], 1e-9) / 1e9, 1),
                           "per_slice": [{"slice": r["slice"], "deg": d, "its": r["its"],
                                          "found": r["found"], "exact": r["exact"]}
@@ -516,7 +518,7 @@ def main():
                        if sb.wall_step > 0 else None,
                        "ms_filter": round(sb.sec_filter * 1e3, 3),
                        "ms_cgs": round(sb.sec_cgs * 1e3, 3),
-                       "filter_GBs": round(sb.filter_bytes / max(sb.sec_filter, 1e-12) / 1e9, 1),
+                       "filter_GBs": filter_rate(kt),
                        "cgs_GBs": round(sb.cgs_bytes / max(sb.sec_cgs, 1e-12) / 1e9, 1),
                        "graph_vs_eager": {"group_width": sb.graph_group_width,
                                           "nodes": sb.graph_nodes,
@@ -528,7 +530,7 @@ def main():
                                    for k_, v in kt.items()}}
         filt = {k_: v for k_, v in kt.items() if k_.startswith("k_")}
         roof = roofline_of(filt, traffic, col16=out["config"]["col16"])
-        if roof and out["config"]["col16"] and roof["kernel"].startswith(STEP_FORMS):
+        if roof and roof["kernel"].startswith(("k_dia_blk<", "k_cheb_dia<", "k_cheb_multi<")):
             # the Laplacian is read in its diagonal layout: one mask byte per
             # row in place of values and indices; `achieved` counts that
             roof["layout"] = "diagonal"

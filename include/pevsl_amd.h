@@ -42,11 +42,11 @@ typedef struct {
   double t_ritz;          /* Ritz vectors, residuals                    */
   double t_kpm;           /* KPM moments                                */
   double filter_bytes;    /* algorithmic bytes of the filter steps, the
-                             matrix counted in CSR form whichever layout
-                             the kernels read                           */
+                             matrix in the layout that they read        */
   double reorth_bytes;    /* algorithmic bytes of the reorthogonalization */
   long long filter_steps; /* column-degree steps                        */
-  long long filter_launches;
+  long long filter_launches; /* their kernel launches; one covers several
+                             degrees on small or narrow diagonal layouts */
   double t_cgs;           /* Gram-Schmidt passes only (GEMV-T + GEMV-N)  */
   double cgs_bytes;       /* algorithmic bytes of those passes           */
   long long cgs_passes;   /* passes run (first + DGKS second passes)     */
@@ -190,11 +190,13 @@ int pEVSL_SetGraphFilter(pevsl_Data *pevsl, int on);
  * matrix has them, 0 keeps the 32-bit indices for this instance.
  * pEVSL_ColumnOffsets16 returns 1 when the instance's matrix is read
  * through them.
+ *
  * A matrix of at most 32 diagonals, each of one value (the main diagonal may
  * vary: constant-coefficient grid stencils, with or without a potential),
  * also gets a diagonal layout of one mask byte (four above 8 diagonals) per
- * row, which the same kernels and the products then read instead; 0
- * switches it off as well. */
+ * row, which the products and the one-column and row-per-thread block steps
+ * then read instead (pEVSL_ColumnOffsets16 is then 0); 0 switches it off as
+ * well. */
 int pEVSL_SetColumnOffsets16(pevsl_Data *pevsl, int on);
 int pEVSL_ColumnOffsets16(pevsl_Data *pevsl);
 /* Number of diagonals of the layout the instance's matrix is read through, 0
@@ -249,7 +251,11 @@ int pEVSL_GetKernelStats(pevsl_Data *pevsl, pevsl_KernelStats *st);
  * last pEVSL_StatsReset: launches, seconds, algorithmic bytes.  Copies up
  * to maxn entries to out and sets *count to the number recorded. */
 typedef struct {
-  char name[48];      /* e.g. "k_clen_blkrow<float,8>"                     */
+  char name[48];      /* e.g. "k_clen_blkrow<float,8>"; on the diagonal
+                         layout "k_dia_blk<float,8,7,EpiClen<float,8>>",
+                         "k_cheb_dia<double,7>" or, several degrees per
+                         launch, "k_cheb_multi<double,7>" (7: the slots of
+                         pEVSL_DiagonalLayout)                             */
   long long launches;
   double seconds;
   double bytes;

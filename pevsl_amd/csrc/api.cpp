@@ -543,7 +543,7 @@ int pEVSL_SetColumnOffsets16(pevsl_Data *p, int on) {
 
 int pEVSL_ColumnOffsets16(pevsl_Data *p) {
   const Ctx &c = ctx_of(p);
-  return c.A && c.A->jo16 ? 1 : 0;
+  return c.A && c.A->jo16 && c.A->dia.ndiag == 0 ? 1 : 0;
 }
 
 int pEVSL_DiagonalLayout(pevsl_Data *p, int *slots) {

@@ -528,16 +528,13 @@ template void dia_cheb_multi<float>(const DevCsr &, const MultiPlan &, const flo
                                     const double *, int, int, bool, hipStream_t);
 
 template <typename T>
-double cheb_run(const DevCsr &A, const double *mu, int m, double cc, double dd, const T *x, T *y,
-                T *w, hipStream_t st) {
+ChebRun cheb_run(const DevCsr &A, const MultiPlan &p, const double *mu, int m, double cc, double dd,
+                 const T *x, T *y, T *w, hipStream_t st) {
   const int n = A.n;
   const double vec = (double)n * sizeof(T);
-  const bool dia = use_dia(A, sizeof(T), 1);
-  const double mat = dia ? (double)n * (dia_mask_bytes(A.dia) + (A.dia.qd >= 0 ? sizeof(T) : 0))
-                         : (double)A.nnz * (sizeof(T) + index_bytes(A)) + 4.0 * (n + 1);
+  const double mat = matrix_bytes(A, sizeof(T), index_bytes(A), use_dia(A, sizeof(T), 1));
   const T *vk = x, *vkm1 = nullptr;
-  double bytes = 0.0;
-  const MultiPlan p = dia_multi_plan(A, sizeof(T), m);
+  ChebRun run;
   if (p.s > 1) {
     int set = 0;
     for (int d = 1; d <= m; d += p.s, set ^= 1) {
@@ -546,9 +543,10 @@ double cheb_run(const DevCsr &A, const double *mu, int m, double cc, double dd, 
       dia_cheb_multi<T>(A, p, vk, vkm1, vo, vmo, y, cc, dd, mu, d, s, d + s > m, st);
       vk = vo;
       vkm1 = vmo;
-      bytes += mat + (d == 1 ? 2.0 : 4.0) * vec + (d + s > m ? 0.0 : 2.0) * vec;
+      run.bytes += mat + (d == 1 ? 2.0 : 4.0) * vec + (d + s > m ? 0.0 : 2.0) * vec;
+      run.launches++;
     }
-    return bytes;
+    return run;
   }
   T *b[3] = {w, w + n, w + 2 * (size_t)n};
   YPlan yp;
@@ -559,14 +557,15 @@ double cheb_run(const DevCsr &A, const double *mu, int m, double cc, double dd, 
                         k > 2 ? mu[k - 2] : 0.0, mu[k - 1], mu[k], ymode, st);
     vkm1 = vk;
     vk = vkp1;
-    bytes += mat + ((k == 1 ? 2 : 3) + y_passes(ymode)) * vec;
+    run.bytes += mat + ((k == 1 ? 2 : 3) + y_passes(ymode)) * vec;
+    run.launches++;
   }
-  return bytes;
+  return run;
 }
-template double cheb_run<double>(const DevCsr &, const double *, int, double, double,
-                                 const double *, double *, double *, hipStream_t);
-template double cheb_run<float>(const DevCsr &, const double *, int, double, double, const float *,
-                                float *, float *, hipStream_t);
+template ChebRun cheb_run<double>(const DevCsr &, const MultiPlan &, const double *, int, double,
+                                  double, const double *, double *, double *, hipStream_t);
+template ChebRun cheb_run<float>(const DevCsr &, const MultiPlan &, const double *, int, double,
+                                 double, const float *, float *, float *, hipStream_t);
 
 // runs of kThreads (row, piece) items per workgroup: as many as leave about
 // kKpmBlocks workgroups (four per CU).  100^3 FP32, 64 vectors: 512 29.5 ms,

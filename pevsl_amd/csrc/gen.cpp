@@ -54,7 +54,7 @@ void lspol_apply(const LSPolData &L, const double *dx, double *dy, double *wk, h
     scale_vec(n, dy, nullptr, mu[0], s);
     return;
   }
-  cheb_run<double>(B, mu, m, L.cc, L.dd, dx, dy, wk, s);
+  cheb_run<double>(B, dia_multi_plan(B, 8, m), mu, m, L.cc, L.dd, dx, dy, wk, s);
 }
 
 // sum_{j <= m} mu_j T_j(x) by the three-term recurrence (chebxPltd,

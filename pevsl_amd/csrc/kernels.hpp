@@ -84,6 +84,13 @@ struct DevCsr {
 // index bytes per nonzero read by the CSR-stream and row-block kernels
 inline int index_bytes(const DevCsr &A) { return A.jo16 ? 2 : 4; }
 
+// bytes of the matrix that a step reads: its diagonal layout, or the CSR form
+// with `idx` index bytes per nonzero
+inline double matrix_bytes(const DevCsr &A, int elem, int idx, bool dia) {
+  if (dia) return (double)A.n * (dia_mask_bytes(A.dia) + (A.dia.qd >= 0 ? elem : 0));
+  return (double)A.nnz * (elem + idx) + 4.0 * (A.n + 1);
+}
+
 // Rows longer than this are uneven: the CSR-stream kernels sum them by a wave,
 // and the batched filter defaults to the nnz-balanced block kernels.
 constexpr int kUnevenRow = 64;
@@ -176,19 +183,23 @@ template <typename T>
 void dia_clen_blk(const DevCsr &A, int B, const T *b1, const T *b2, const T *v, T *out, double cc,
                   double t, const double *mus, int k, hipStream_t s);
 
-// The degrees 1..m >= 1 of the filter y = sum mu_k T_k((A - cc)/dd) x for one
-// column in the stream form: a launch per degree, or on the diagonal layout of
-// a small or narrow matrix several degrees per launch (k_cheb_multi), with the
-// same bits.  w: 4 n elements (3 n if n > 2^20).  Returns the bytes of the
-// passes over memory.
-template <typename T>
-double cheb_run(const DevCsr &A, const double *mu, int m, double cc, double dd, const T *x, T *y,
-                T *w, hipStream_t s);
 // launches of several degrees: degrees per launch (1: none), rows per
 // workgroup, widest diagonal
 struct MultiPlan {
   int s = 1, R = 0, bw = 0;
 };
+// The degrees 1..m >= 1 of the filter y = sum mu_k T_k((A - cc)/dd) x for one
+// column in the stream form: a launch per degree, or on the diagonal layout of
+// a small or narrow matrix several degrees per launch (k_cheb_multi), with the
+// same bits.  p = dia_multi_plan(A, sizeof(T), m).  w: 4 n elements (3 n if n >
+// 2^20).  Returns the launches and the bytes of their passes over memory.
+struct ChebRun {
+  long long launches = 0;
+  double bytes = 0.0;
+};
+template <typename T>
+ChebRun cheb_run(const DevCsr &A, const MultiPlan &p, const double *mu, int m, double cc, double dd,
+                 const T *x, T *y, T *w, hipStream_t s);
 constexpr int kMultiMax = 32;      // degrees per launch at most
 // rows of a workgroup's window at most: its two FP64 vectors fill 64 KiB of LDS
 constexpr int kMultiRows = 4080;

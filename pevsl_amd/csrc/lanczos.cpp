@@ -70,12 +70,10 @@ struct Slice {
   std::vector<double> vecs;  // accepted Ritz vectors (host, n x nev)
 };
 
-// Clenshaw step: gathered b1 (counted once), b2 (if any), v, out; idx =
-// index bytes per nonzero the kernel reads (2 with 16-bit column offsets)
-size_t clen_launch_bytes(const DevCsr &A, int elem, int ncol, bool has_b2, int idx) {
-  const double vec = (double)A.n * elem;
-  return (size_t)((double)A.nnz * (elem + idx) + 4.0 * (A.n + 1) +
-                  (has_b2 ? 4.0 : 3.0) * vec * ncol);
+// Clenshaw step: gathered b1 (counted once), b2 (if any), v, out; mat = bytes
+// of the matrix (matrix_bytes)
+double clen_launch_bytes(const DevCsr &A, int elem, int ncol, bool has_b2, double mat) {
+  return mat + (has_b2 ? 4.0 : 3.0) * ((double)A.n * elem) * ncol;
 }
 
 // segmented Clenshaw step: the matrix once if any piece forms the product,
@@ -84,7 +82,7 @@ size_t clen_launch_bytes(const DevCsr &A, int elem, int ncol, bool has_b2, int i
 double clen_seg_launch_bytes(const DevCsr &A, int elem, int seg, int d, int nseg,
                              const SegTops &tops) {
   const double piece = (double)A.n * elem * seg;
-  double b = tops.top[0] > d ? (double)A.nnz * (elem + 4) + 4.0 * (A.n + 1) : 0.0;
+  double b = tops.top[0] > d ? matrix_bytes(A, elem, 4, false) : 0.0;
   for (int s = 0; s < nseg; s++)
     b += (d == tops.top[s] ? 2.0 : d == tops.top[s] - 1 ? 3.0 : 4.0) * piece;
   return b;
@@ -92,27 +90,25 @@ double clen_seg_launch_bytes(const DevCsr &A, int elem, int seg, int d, int nseg
 
 // three-term step: passes = vector passes per column (3: vk gathered, vkm1,
 // vkp1; 2 on the first degree; and those of y)
-size_t filter_launch_bytes(const DevCsr &A, int elem, int ncol, int passes, int idx) {
-  const double vec = (double)A.n * elem;
-  return (size_t)((double)A.nnz * (elem + idx) + 4.0 * (A.n + 1) + passes * vec * ncol);
+double filter_launch_bytes(const DevCsr &A, int elem, int ncol, int passes, double mat) {
+  return mat + passes * ((double)A.n * elem) * ncol;
 }
 
-// What a launch on the diagonal layout does not read of the CSR form the byte
-// counts above assume (they feed pevsl_KernelStats, whose figures compare
-// between layouts; the per-kernel timers count what the kernel reads).
-double dia_saved_bytes(const DevCsr &A, int elem, int idx, bool dia) {
-  if (!dia) return 0.0;
-  return (double)A.nnz * (elem + idx) + 4.0 * (A.n + 1) -
-         (double)A.n * (dia_mask_bytes(A.dia) + (A.dia.qd >= 0 ? elem : 0));
-}
-
-// name of a filter step for the per-kernel timers; the stream and row forms
-// keep their names on the diagonal layout
-std::string filter_kernel_name(bool f32, int kind, int B, bool stream, int lanes) {
+// name of a filter step's kernel for the per-kernel timers: one column (B = 0:
+// the stream form, with p.s > 1 several degrees per launch, or k_cheb_vec) or a
+// block of width B
+std::string filter_kernel_name(const DevCsr &A, bool f32, int kind, int B, bool stream = false,
+                               int lanes = 0, const MultiPlan &p = {}) {
+  const bool dia = use_dia(A, f32 ? 4 : 8, std::max(B, 1));
+  const int slots = dia_slots(A.dia.ndiag);
   const char *t = f32 ? "float" : "double";
   char nm[48];
   if (B == 0) {
-    if (stream)
+    if (stream && p.s > 1)
+      snprintf(nm, sizeof nm, "k_cheb_multi<%s,%d>", t, slots);
+    else if (stream && dia)
+      snprintf(nm, sizeof nm, "k_cheb_dia<%s,%d>", t, slots);
+    else if (stream)
       snprintf(nm, sizeof nm, "k_cheb_stream<%s>", t);
     else
       snprintf(nm, sizeof nm, "k_cheb_vec<%s,%d>", t, lanes);
@@ -120,6 +116,9 @@ std::string filter_kernel_name(bool f32, int kind, int B, bool stream, int lanes
     snprintf(nm, sizeof nm, "k_clen_seg<%s,%d>", t, B);
   } else if (kind >= 3) {
     snprintf(nm, sizeof nm, "k_blk_bal<%s,%d,%s>", t, B, kind == 4 ? "EpiClen" : "EpiCheb");
+  } else if ((kind == 1 || kind == 2) && dia) {
+    const char *epi = kind == 2 ? "EpiClen" : "EpiCheb";
+    snprintf(nm, sizeof nm, "k_dia_blk<%s,%d,%d,%s<%s,%d>>", t, B, slots, epi, t, B);
   } else if (kind == 2) {
     snprintf(nm, sizeof nm, "k_clen_blkrow<%s,%d>", t, B);
   } else if (kind == 1) {
@@ -146,34 +145,30 @@ static void cheb_filter_run(Ctx &c, const pevsl_Polparams *pol, const T *x, T *y
   const int lanes = std::max(c.lanes, 1);
   // default (-1): the stream form
   const bool stream = c.use_stream != 0;
+  const MultiPlan p = stream ? dia_multi_plan(A, elem, m) : MultiPlan{};
   const long tok =
-      timed ? c.kt.begin(s, filter_kernel_name(elem == 4, 0, 0, stream, lanes).c_str()) : -1;
-  // statistics count the CSR form, a launch per degree
-  double csr = 0.0;
-  YPlan yp;
-  for (int k = 1; k <= m; k++) {
-    const int ymode = stream ? yp.next(k, m) : (k == 1 ? kYInit | 1 : 1);
-    csr += (double)filter_launch_bytes(A, elem, 1, (k == 1 ? 2 : 3) + y_passes(ymode),
-                                       stream ? index_bytes(A) : 4);
-  }
-  double bytes = csr;
+      timed ? c.kt.begin(s, filter_kernel_name(A, elem == 4, 0, 0, stream, lanes, p).c_str()) : -1;
+  ChebRun run;
   if (stream) {
-    bytes = cheb_run<T>(A, mu, m, cc, dd, x, y, w, s);
+    run = cheb_run<T>(A, p, mu, m, cc, dd, x, y, w, s);
   } else {
     T *b[3] = {w, w + (size_t)n, w + 2 * (size_t)n};
     const T *vk = x, *vkm1 = nullptr;
+    const double mat = matrix_bytes(A, elem, 4, false);
     for (int k = 1; k <= m; k++) {
       T *vkp1 = b[(k - 1) % 3];
       cheb_step_vec<T>(A, vk, vkm1, vkp1, y, cc, k == 1 ? 1.0 / dd : 2.0 / dd, mu[0], mu[k],
                        k == 1, lanes, s);
       vkm1 = vk;
       vk = vkp1;
+      run.bytes += filter_launch_bytes(A, elem, 1, k == 1 ? 3 : 5, mat);
+      run.launches++;
     }
   }
-  if (tok >= 0) c.kt.end(s, tok, m, bytes);
-  c.kstats.filter_bytes += csr;
+  if (tok >= 0) c.kt.end(s, tok, run.launches, run.bytes);
+  c.kstats.filter_bytes += run.bytes;
   c.kstats.filter_steps += m;
-  c.kstats.filter_launches += m;
+  c.kstats.filter_launches += run.launches;
 }
 
 // y = p((A - cc)/dd) v for one FP64 column in HBM (SRC/chebpol.c:509-574).
@@ -294,7 +289,6 @@ struct GroupGraph {
   hipGraphExec_t exec = nullptr;
   char *blocks = nullptr;  // filter-block allocation the graph was captured on
   double bytes = 0.0;      // algorithmic bytes of one replay
-  double kbytes = 0.0;     // bytes its kernels move
   long long steps = 0, launches = 0;
   std::string kname;
   bool used = false;
@@ -399,7 +393,6 @@ class BatchSolver {
   pevsl_Data *p_;
   int ns_;
   bool capture_ = false;  // filter_block enqueues kernels only (graph capture)
-  double kbytes_ = 0.0;   // bytes the last enqueued group's kernels move
   int n_ = 0;
   bool b32_ = false;  // FP32 basis storage
   size_t vb_ = 8;     // basis element bytes
@@ -607,7 +600,9 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
   const bool clen = kind == 2 || kind == 4;
   const bool bal = kind == 3 || kind == 4;
   const bool dia = (kind == 1 || kind == 2) && use_dia(A, (int)elem, B);
-  kbytes_ = 0.0;
+  // only the row kernels read the 16-bit offsets
+  const double mat =
+      matrix_bytes(A, (int)elem, kind == 1 || kind == 2 ? index_bytes(A) : 4, dia);
   auto run = [&](auto *tag) {
     using T = std::remove_pointer_t<decltype(tag)>;
     T *x = (T *)xb[0], *y = (T *)xb[1];
@@ -624,7 +619,7 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
                            c_.stream);
     }
     T *yout = y;
-    const std::string kname = filter_kernel_name(f32, kind, B, false, 0);
+    const std::string kname = filter_kernel_name(A, f32, kind, B);
     if (segk) {
       // pieces of `seg` columns, each active from its own top degree down
       // (columns are sorted by degree, so a piece's first column has its top)
@@ -659,7 +654,6 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
         b1 = out;
         yout = out;
       }
-      kbytes_ += kbytes;
       if (tok >= 0) c_.kt.end(c_.stream, tok, degmax + 1, kbytes);
     } else if (clen && degmax >= 1) {
       // Clenshaw sums from the top degree down: b_d = mu_d x + (2/dd)(A - cc)
@@ -689,8 +683,7 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
         int nact = 0;  // columns whose series has reached degree d + 1
         while (nact < g && degs[(size_t)nact] >= d + 1) nact++;
         if (b1) {
-          const double lb = (double)clen_launch_bytes(A, (int)elem, nact, b2 != nullptr,
-                                                      bal ? 4 : index_bytes(A));
+          const double lb = clen_launch_bytes(A, (int)elem, nact, b2 != nullptr, mat);
           kbytes += lb;
           c_.kstats.filter_bytes += lb;
           c_.kstats.filter_steps += nact;
@@ -700,8 +693,6 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
         b1 = out;
         yout = out;
       }
-      kbytes -= degmax * dia_saved_bytes(A, (int)elem, index_bytes(A), dia);
-      kbytes_ += kbytes;
       if (tok >= 0) c_.kt.end(c_.stream, tok, degmax, kbytes);
     } else {
     // third work buffer: reuse x once it is no longer read (after step 2)
@@ -739,8 +730,7 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
       else
         cheb_step_blk<T>(A, B, vk, vkm1, vkp1, y, cc, d == 1 ? 1.0 / dd : 2.0 / dd,
                          musp, d, nact, c_.stream);
-      const int ib = rowk && !bal ? index_bytes(A) : 4;  // only the row kernel reads jo16
-      const double lb = (double)filter_launch_bytes(A, (int)elem, nact, d == 1 ? 2 : 3, ib) +
+      const double lb = filter_launch_bytes(A, (int)elem, nact, d == 1 ? 2 : 3, mat) +
                         y_passes(ymode) * (double)n_ * (double)elem * ncol;
       kbytes += lb;
       c_.kstats.filter_bytes += lb;
@@ -749,8 +739,6 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
       vkm1 = vk;
       vk = vkp1;
     }
-    kbytes -= degmax * dia_saved_bytes(A, (int)elem, index_bytes(A), dia);
-    kbytes_ += kbytes;
     if (tok >= 0) c_.kt.end(c_.stream, tok, degmax, kbytes);
     }
     if constexpr (std::is_same<T, float>::value) {
@@ -876,7 +864,7 @@ void BatchSolver::filter_group_graph(const std::vector<int> &grp, int k) {
     graphs_.push_back(std::unique_ptr<GroupGraph>(new GroupGraph()));
     gg = graphs_.back().get();
     gg->key = key;
-    gg->kname = filter_kernel_name(c_.filter_prec == PEVSL_PREC_FP32, kind, B, false, 0);
+    gg->kname = filter_kernel_name(*c_.A, c_.filter_prec == PEVSL_PREC_FP32, kind, B);
     stage_mus(grp, B, gg->mus);
   }
   gg->used = true;
@@ -894,14 +882,13 @@ void BatchSolver::filter_group_graph(const std::vector<int> &grp, int k) {
     gg->blocks = base;
     // the capture counted one application that has not run
     gg->bytes = c_.kstats.filter_bytes - ks.filter_bytes;
-    gg->kbytes = kbytes_;
     gg->steps = c_.kstats.filter_steps - ks.filter_steps;
     gg->launches = c_.kstats.filter_launches - ks.filter_launches;
     c_.kstats = ks;
   }
   const long tok = c_.kt.begin(c_.stream, gg->kname.c_str());
   PV_HIP(hipGraphLaunch(gg->exec, c_.stream));
-  c_.kt.end(c_.stream, tok, gg->launches, gg->kbytes);
+  c_.kt.end(c_.stream, tok, gg->launches, gg->bytes);
   c_.kstats.filter_bytes += gg->bytes;
   c_.kstats.filter_steps += gg->steps;
   c_.kstats.filter_launches += gg->launches;

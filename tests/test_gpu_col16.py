@@ -13,7 +13,9 @@ from its row block's first row when the matrix's offsets all fit.
 * batched solves (FP64 three-term row kernel, FP32 Clenshaw row kernel, two
   block widths) with and without the offsets: the same eigenvalues and step
   counts, and the counted filter bytes fall by 2 bytes per nonzero per
-  launch.
+  launch, on a band of varying values; and the same solves of the 16^3
+  Laplacian, which is read through its diagonal layout instead: there the
+  counted bytes are a mask byte per row in place of the CSR matrix.
 """
 import ctypes as C
 
@@ -115,17 +117,35 @@ def test_stream_filter_with_offsets(lib, which):
         M.free()
 
 
+def varying_band():
+    """Symmetric band of random entries, up to 1,100 columns wide: no diagonal
+    layout, rows of at most 7 entries, offsets within 16 bits."""
+    n, rng = 4096, np.random.default_rng(9)
+    pairs = [(np.arange(n - o), np.arange(o, n), rng.uniform(-1, 0, n - o)) for o in (1, 16, 1100)]
+    return sym_csr(n, pairs, rng.uniform(5.0, 6.0, n))
+
+
 @pytest.mark.parametrize("prec,kind,width", [(capi.PEVSL_PREC_FP64, 1, 4),
                                              (capi.PEVSL_PREC_FP32, 2, 4),
                                              (capi.PEVSL_PREC_FP32, 2, 8),
                                              (capi.PEVSL_PREC_FP32, 1, 8)])
-def test_batched_solve_with_and_without_offsets(lib, prec, kind, width):
-    banner("batched 16^3, 5 slices, prec %d kernel %d width %d, 16-bit offsets on/off" % (
-        prec, kind, width))
-    g = 16
-    ia, ja, a = driver.laplacian3d(g, g, g)
+@pytest.mark.parametrize("which", ["band", "laplacian"])
+def test_batched_solve_with_and_without_offsets(lib, which, prec, kind, width):
+    banner("batched %s, 5 slices, prec %d kernel %d width %d, 16-bit offsets on/off" % (
+        which, prec, kind, width))
+    g, lap = 16, which == "laplacian"
+    ia, ja, a = driver.laplacian3d(g, g, g) if lap else varying_band()
+    if lap:
+        edges = np.linspace(0.5, 1.5, 6)
+        ex = [orc.exact_eig_lap3(g, g, g, edges[i], edges[i + 1]) for i in range(5)]
+    else:
+        n = len(ia) - 1
+        dense = np.zeros((n, n))
+        dense[np.repeat(np.arange(n), np.diff(ia)), ja] = a
+        ev = np.linalg.eigvalsh(dense)
+        edges = [0.5 * (ev[j - 1] + ev[j]) for j in (4, 34, 64, 94, 124, 154)]
+        ex = [ev[(ev > edges[i]) & (ev < edges[i + 1])] for i in range(5)]
     M = driver.Matrix(lib, ia, ja, a)
-    edges = np.linspace(0.5, 1.5, 6)
     intvs = [[edges[i], edges[i + 1], 0.0, 12.0] for i in range(5)]
     pols = [driver.find_pol(lib, iv)[0] for iv in intvs]
     vinit = driver.rand_vinit(lib, M.n)
@@ -135,25 +155,50 @@ def test_batched_solve_with_and_without_offsets(lib, prec, kind, width):
             inst = driver.Instance(lib, M, prec=prec, block_rowkernel=kind, block_width=width,
                                    col16=col16)
             try:
-                assert lib.pEVSL_ColumnOffsets16(inst.p) == (1 if col16 else 0)
+                assert lib.pEVSL_ColumnOffsets16(inst.p) == (1 if col16 and not lap else 0)
+                assert lib.pEVSL_DiagonalLayout(inst.p, None) == (7 if col16 and lap else 0)
                 rc, outs = driver.cheblan_batch(inst, intvs, [400] * 5, 1e-8, vinit, pols)
                 assert rc == 0
-                runs.append((outs, inst.kernel_stats()))
+                runs.append((outs, inst.kernel_stats(), inst.kernel_times()))
             finally:
                 inst.close()
     finally:
         for p_ in pols:
             lib.pEVSL_FreePol(C.byref(p_))
         M.free()
-    (o16, k16), (o32, k32) = runs
-    for iv, x, y in zip(intvs, o16, o32):
+    (o16, k16, t16), (o32, k32, t32) = runs
+    for x, y, e in zip(o16, o32, ex):
         assert x["info"]["its"] == y["info"]["its"]
         np.testing.assert_array_equal(x["lam"], y["lam"])
-        ex = orc.exact_eig_lap3(g, g, g, iv[0], iv[1])
-        assert len(x["lam"]) == len(ex) > 0
-        np.testing.assert_allclose(np.sort(x["lam"]), ex, rtol=1e-10)
-    # every counted launch reads the matrix once: 2 index bytes per nonzero
-    # fewer with the offsets
-    assert k16["filter_launches"] == k32["filter_launches"] > 0
-    saved = k32["filter_bytes"] - k16["filter_bytes"]
-    assert saved == 2.0 * int(ia[-1]) * k16["filter_launches"], (saved, k16["filter_launches"])
+        assert len(x["lam"]) == len(e) > 0
+        if lap:
+            np.testing.assert_allclose(np.sort(x["lam"]), e, rtol=1e-10)
+        else:  # an eigenvalue lies within each residual (and eigvalsh's rounding)
+            k = np.argsort(x["lam"])
+            assert np.all(np.abs(x["lam"][k] - e) <= np.asarray(x["res"])[k] + 1e-12)
+    assert k16["filter_steps"] == k32["filter_steps"]
+    name = "k_c%s_blkrow<%s,%d>" % ("heb" if kind == 1 else "len",
+                                    "float" if prec else "double", width)
+    assert name in t32
+    nnz, n, elem = int(ia[-1]), len(ia) - 1, 4 if prec else 8
+    if not lap:
+        # every counted launch reads the matrix once: 2 index bytes per
+        # nonzero fewer with the offsets
+        assert name in t16
+        assert k16["filter_launches"] == k32["filter_launches"] > 0
+        saved = k32["filter_bytes"] - k16["filter_bytes"]
+        assert saved == 2.0 * nnz * k16["filter_launches"], (saved, k16["filter_launches"])
+        return
+    # the counts are of what ran: the timers' launches and bytes add up to the
+    # statistics', and a block launch reads n mask bytes in place of the CSR
+    # matrix (its values, 4-byte indices and row pointers)
+    for ks, kt in ((k16, t16), (k32, t32)):
+        filt = [v for k_, v in kt.items() if k_.startswith("k_")]
+        assert sum(v["launches"] for v in filt) == ks["filter_launches"] > 0
+        assert abs(sum(v["bytes"] for v in filt) - ks["filter_bytes"]) <= 1e-9 * ks["filter_bytes"]
+    t = "float" if prec else "double"
+    dia = "k_dia_blk<%s,%d,7,Epi%s<%s,%d>>" % (t, width, "Cheb" if kind == 1 else "Clen", t, width)
+    assert not any("blkrow" in k_ or "stream" in k_ for k_ in t16), t16.keys()
+    assert t16[dia]["launches"] == t32[name]["launches"]
+    saved = (t32[name]["bytes"] - t16[dia]["bytes"]) / t32[name]["launches"]
+    assert abs(saved - (nnz * (elem + 4) + 4 * (n + 1) - n)) <= 1e-6 * saved

@@ -5,8 +5,9 @@ is compared with the plain CSR form of the same instance
 
 The filter's terms are the same in the same order, each rounded on its own,
 so outputs are equal bit for bit; a product on the CSR side may sum a row in
-several lanes, and is compared to 1e-15 times the row's absolute sum and
-against numpy.
+several lanes, and both forms are compared with numpy to the rounding of a sum.
+Which layout and which kernel a matrix gets is asserted as well
+(pEVSL_DiagonalLayout, the per-kernel timers).
 """
 import ctypes as C
 
@@ -445,3 +446,86 @@ def test_kpm_by_diagonal_count(lib, count, prec):
     assert rc == 0
     # as in test_kpm_on_both_layouts
     assert np.max(np.abs(mu - np.array(ref))) <= (1e-13 if prec == 0 else 2e-5)
+
+
+# kernel of a filter of degree 70 in FP64: several degrees per launch on chains
+# and bands of at most 8 diagonals, one above that or where the window of a
+# workgroup would not fit the band, the CSR-stream kernel without a layout
+STEP = {"chain_wide": "k_cheb_multi<double,3>", "band_31": "k_cheb_multi<double,5>",
+        "lap2d": "k_cheb_multi<double,5>", "block_edge_1": "k_cheb_multi<double,3>",
+        "band_400": "k_cheb_multi<double,7>", "8_diags": "k_cheb_dia<double,8>",
+        "9_diags": "k_cheb_dia<double,9>",
+        "count_10": "k_cheb_dia<double,13>", "32_diags": "k_cheb_dia<double,32>",
+        "33_diags": "k_cheb_stream<double>", "two_vary": "k_cheb_stream<double>",
+        "sparse_diags": "k_cheb_stream<double>"}
+
+
+@pytest.mark.parametrize("name", sorted(STEP))
+def test_filter_runs_the_kernel_meant_for_the_layout(lib, name):
+    """...and its launches and bytes are counted as they ran."""
+    print("\n[gpu case] filter kernel, %s" % name, flush=True)
+    ia, ja, a = CASES[name]()
+    n, deg = len(ia) - 1, 70
+    M = driver.Matrix(lib, ia, ja, a)
+    try:
+        inst = driver.Instance(lib, M)
+        try:
+            mu = np.linspace(1, 2, deg + 1)
+            pol = capi.Polparams()
+            pol.deg, pol.cc, pol.dd = deg, 0.0, 1e3
+            pol.mu = mu.ctypes.data_as(capi.c_double_p)
+            v, y = np.ones(n), np.zeros(n)
+            pv, py = capi.Parvec(), capi.Parvec()
+            for p, x in ((pv, v), (py, y)):
+                lib.pEVSL_ParvecCreateShell(n, n, 0, 0, C.byref(p),
+                                            x.ctypes.data_as(capi.c_double_p))
+            assert lib.pEVSL_ChebAv(inst.p, C.byref(pol), C.byref(pv), C.byref(py), None) == 0
+            kt, ks = inst.kernel_times(), inst.kernel_stats()
+        finally:
+            inst.close()
+    finally:
+        M.free()
+    assert list(kt) == [STEP[name]]
+    t = kt[STEP[name]]
+    assert ks["filter_steps"] == deg
+    assert ks["filter_launches"] == t["launches"] and ks["filter_bytes"] == t["bytes"]
+    if "multi" in STEP[name]:
+        assert t["launches"] * 2 <= deg
+    else:
+        assert t["launches"] == deg
+        # at least the two vectors that every degree reads or writes
+        assert t["bytes"] >= 2.0 * 8 * n * deg
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_product_on_and_off_the_layout(lib, name):
+    """pEVSL_DeviceMatvec through the layout and through plain CSR: each within
+    the rounding of the row's sum, in whichever order."""
+    print("\n[gpu case] product on and off the layout, %s" % name, flush=True)
+    ia, ja, a = CASES[name]()
+    n = len(ia) - 1
+    x = np.random.default_rng(n).uniform(-1, 1, n)
+    rows = np.repeat(np.arange(n), np.diff(ia))
+    ref = np.bincount(rows, a * x[ja], n)
+    mag = np.bincount(rows, np.abs(a * x[ja]), n)
+    M = driver.Matrix(lib, ia, ja, a)
+    hip, d, nb = C.CDLL("libamdhip64.so"), C.c_void_p(), C.c_size_t(8 * n)
+    try:
+        assert hip.hipMalloc(C.byref(d), C.c_size_t(16 * n)) == 0
+        dx, dy = C.c_void_p(d.value), C.c_void_p(d.value + 8 * n)
+        for on in (True, False):
+            y = np.full(n, np.nan)
+            inst = driver.Instance(lib, M, col16=on)
+            try:
+                assert hip.hipMemcpy(dx, x.ctypes.data_as(C.c_void_p), nb, 1) == 0
+                assert hip.hipMemcpy(dy, y.ctypes.data_as(C.c_void_p), nb, 1) == 0
+                assert lib.pEVSL_DeviceMatvec(inst.p, dx, dy) == 0
+                assert hip.hipMemcpy(y.ctypes.data_as(C.c_void_p), dy, nb, 2) == 0
+            finally:
+                inst.close()
+            # two summation orders of at most 33 terms
+            assert np.all(np.abs(y - ref) <= 33 * 2.3e-16 * mag), on
+    finally:
+        if d.value:
+            hip.hipFree(d)
+        M.free()

@@ -456,7 +456,7 @@ def test_segmented_clenshaw_equals_row_kernel(lib, basis):
             lib.pEVSL_FreePol(C.byref(p_))
         M.free()
     assert "k_clen_seg<float,8>" in runs[5][1], runs[5][1].keys()
-    assert "k_clen_blkrow<float,8>" in runs[2][1], runs[2][1].keys()
+    assert "k_dia_blk<float,8,7,EpiClen<float,8>>" in runs[2][1], runs[2][1].keys()
     # both count every column's products once per degree
     assert runs[5][2]["filter_steps"] == runs[2][2]["filter_steps"]
     for iv, o2, o5 in zip(intvs, runs[2][0], runs[5][0]):
