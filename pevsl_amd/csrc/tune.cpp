@@ -15,10 +15,15 @@ using namespace pevsl;
 
 namespace {
 
-// idx: index bytes per nonzero the kernel reads (2 for the row-block kernels
-// on a matrix with 16-bit column offsets)
-double step_bytes(const DevCsr &A, int elem, int ncol, int idx = 4) {
-  return (double)A.nnz * (elem + idx) + 4.0 * (A.n + 1) + 5.0 * (double)A.n * elem * ncol;
+// Bytes of one filter step of block kernel `kind` (see time_blk; 0 is also the
+// one-column vector kernel's): the matrix in the form the kernel reads, and the
+// vector passes: four in Clenshaw form, three and y's two every third degree in
+// the three-term forms, five where y is updated at every degree.
+double step_bytes(const DevCsr &A, int elem, int ncol, int kind) {
+  const bool row = kind == 1 || kind == 2;
+  const double passes = kind == 0 ? 5.0 : kind == 1 || kind == 3 ? 11.0 / 3.0 : 4.0;
+  return matrix_bytes(A, elem, row ? index_bytes(A) : 4, row && use_dia(A, elem, ncol)) +
+         passes * (double)A.n * elem * ncol;
 }
 
 // lanes == 0: the CSR-stream kernel
@@ -123,7 +128,7 @@ int pEVSL_Autotune(pevsl_Data *p, int reps, pevsl_TuneResult *res) {
       bl = L;
     }
   }
-  res->bytes_lanes = step_bytes(*c.A, elem, 1);
+  res->bytes_lanes = step_bytes(*c.A, elem, 1, 0);
   res->t_stream = f32 ? time_vec<float>(c, 0, reps) : time_vec<double>(c, 0, reps);
   DBuf<double> mus;
   mus.ensure(3 * 64);
@@ -139,7 +144,7 @@ int pEVSL_Autotune(pevsl_Data *p, int reps, pevsl_TuneResult *res) {
     const double t = f32 ? time_blk<float>(c, B, reps, mus, 0)
                          : time_blk<double>(c, B, reps, mus, 0);
     res->t_block[i] = t;
-    res->bytes_block[i] = step_bytes(*c.A, elem, B);
+    res->bytes_block[i] = step_bytes(*c.A, elem, B, 0);
     if (t / B < bestc) {
       bestc = t / B;
       bw = B;
@@ -178,8 +183,7 @@ int pEVSL_Autotune(pevsl_Data *p, int reps, pevsl_TuneResult *res) {
       if (f32) {
         const double tc = time_blk<float>(c, B, reps, mus, 2);
         res->t_blockclen[i] = tc;
-        res->bytes_clen[i] =
-            step_bytes(*c.A, elem, B, index_bytes(*c.A)) - (double)c.A->n * B * elem;
+        res->bytes_clen[i] = step_bytes(*c.A, elem, B, 2);
         if (tc / B < bestc) {
           bestc = tc / B;
           bw = B;
@@ -220,11 +224,7 @@ int pEVSL_BenchBlock(pevsl_Data *p, int B, int reps, double *sec, double *bytes)
   std::vector<double> mh(3 * 64, 0.01);
   PV_HIP(hipMemcpy(mus.p, mh.data(), sizeof(double) * mh.size(), hipMemcpyHostToDevice));
   *sec = f32 ? time_blk<float>(c, B, reps, mus, kind) : time_blk<double>(c, B, reps, mus, kind);
-  const int idx = (kind == 1 || kind == 2) ? index_bytes(*c.A) : 4;
-  // four vector passes per degree for all but the lane-per-(row, column)
-  // kernel (Clenshaw; three-term kernels with y every third degree move 3 2/3)
-  *bytes = kind != 0 ? step_bytes(*c.A, elem, B, idx) - (double)c.A->n * B * elem
-                     : step_bytes(*c.A, elem, B, idx);
+  *bytes = step_bytes(*c.A, elem, B, kind);
   return 0;
 }
 

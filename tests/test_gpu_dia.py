@@ -529,3 +529,36 @@ def test_product_on_and_off_the_layout(lib, name):
         if d.value:
             hip.hipFree(d)
         M.free()
+
+
+@pytest.mark.parametrize("which", ["lap3d", "pot", "two_vary"])
+@pytest.mark.parametrize("prec,kind", [(0, 0), (0, 1), (0, 3), (1, 1), (1, 2), (1, 4), (1, 5)])
+def test_benchblock_counts_the_form_it_reads(lib, which, prec, kind):
+    """Bytes of a timed block step: mask bytes (and the varying main diagonal)
+    for the row steps of a matrix read through its diagonals, the CSR matrix
+    for every other kernel; vector passes by kernel."""
+    print("\n[gpu case] block step bytes, %s prec %d kind %d" % (which, prec, kind), flush=True)
+    ia, ja, a = driver.laplacian3d(13, 11, 7) if which == "pot" else CASES[which]()
+    n, nnz, B, elem = len(ia) - 1, int(ia[-1]), 8, 4 if prec else 8
+    if which == "pot":
+        a = np.where(ja == np.repeat(np.arange(n), np.diff(ia)),
+                     a + np.random.default_rng(3).random(nnz), a)
+    M = driver.Matrix(lib, ia, ja, a)
+    sec, got = C.c_double(), C.c_double()
+    try:
+        for on in (True, False):
+            inst = driver.Instance(lib, M, prec=prec, block_rowkernel=kind, col16=on)
+            try:
+                assert lib.pEVSL_BenchBlock(inst.p, B, 2, C.byref(sec), C.byref(got)) == 0
+            finally:
+                inst.close()
+            if on and kind in (1, 2) and which != "two_vary":
+                mat = n * (1 + (elem if which == "pot" else 0))
+            else:
+                idx = 2 if on and kind in (1, 2) else 4
+                mat = nnz * (elem + idx) + 4 * (n + 1)
+            passes = {0: 5.0, 1: 11 / 3.0, 3: 11 / 3.0}.get(kind, 4.0)
+            assert abs(got.value - (mat + passes * n * B * elem)) <= 1e-9 * got.value
+            assert sec.value > 0
+    finally:
+        M.free()
