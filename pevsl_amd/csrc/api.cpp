@@ -253,8 +253,8 @@ struct HostDia {
 };
 
 // Fills D and returns true if the matrix has a diagonal layout: columns
-// ascend strictly within rows, at most kMaxDiags diagonals, each of one finite
-// value (bit for bit), the main diagonal excepted, and at least half of the
+// ascend strictly within rows, at most kMaxDiags diagonals, each of one
+// value (bit for bit, finite in FP32), the main diagonal excepted, and at least half of the
 // diagonals' places taken (a kernel loads x for every diagonal of a row).
 // A matrix without the layout is recognised after its first rows: random
 // sparsity has more than kMaxDiags diagonals within two or three rows, and
@@ -300,7 +300,8 @@ bool find_dia(int n, const int *ia, const int *ja, const double *a, HostDia &D) 
       while (q < nd && off[q] != o) q++;
       if (q == nd) {
         if (nd == kMaxDiags) return false;
-        if (!std::isfinite(a[b + j])) return false;
+        // in FP32 too: the LDS windows multiply it by zero where it is absent
+        if (!std::isfinite((float)a[b + j])) return false;
         off[nd] = o;
         c[nd] = a[b + j];
         varies[nd++] = false;

@@ -80,6 +80,10 @@ CASES = {
     "33_diags": lambda: banded(900, list(range(-16, 17))),
     "two_vary": lambda: banded(900, [-1, 0, 1], vary=[0, 1]),
     "sparse_diags": lambda: banded(900, [-40, -20, 0, 20, 40], drop=0.9),
+    # ...and a value that FP32 does not hold, which zero must not multiply
+    "beyond_fp32": lambda: (lambda ia, ja, a: (ia, ja, np.where(
+        ja - np.repeat(np.arange(900), np.diff(ia)) == 3, 1e39, a)))(
+            *banded(900, [-1, 0, 3], drop=0.2)),
 }
 
 
@@ -353,7 +357,7 @@ def test_kpm_without_symmetry(lib, which, prec):
 LAYOUT = {"1x1": 1, "one_row_block": 3, "block_edge": 3, "block_edge_1": 3, "3_of_4_dropped": 3,
           "4_no_main": 4, "chain_wide": 3, "band_31": 5, "band_400": 7, "lower_only": 3, "lap2d": 5,
           "lap3d": 7, "6_diags": 6, "8_diags": 8, "9_diags": 9, "32_diags": 32, "empty_rows": 2,
-          "33_diags": 0, "two_vary": 0, "sparse_diags": 0,
+          "33_diags": 0, "two_vary": 0, "sparse_diags": 0, "beyond_fp32": 0,
           **{"count_%d" % k: k for k in (10, 13, 14, 19, 20, 27, 28)}}
 
 
