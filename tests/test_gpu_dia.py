@@ -245,8 +245,10 @@ def test_kpm_on_both_layouts(lib, prec, Mdeg, nvec):
             finally:
                 inst.close()
             assert rc == 0
-            # FP64: a few roundings of unit quantities; FP32: the path's 2e-5
-            assert np.max(np.abs(mu - ref)) <= (1e-13 if prec == 0 else 2e-5)
+            # FP64: a few roundings of unit quantities; FP32 as CSR: the path's
+            # 2e-5; on the layout: vectors rounded to FP32 once a step and
+            # everything else in FP64, which numpy puts at up to 1.9e-9 here
+            assert np.max(np.abs(mu - ref)) <= (1e-13 if prec == 0 else 6e-9 if on else 2e-5)
     finally:
         M.free()
 
@@ -281,8 +283,67 @@ def test_kpm_several_runs_of_rows(lib, prec):
         w = (A @ u - 6.0 * u) * ((2.0 if k else 1.0) / 6.0) - (um if k else 0.0)
         um, u = u, w
         ref.append(2.0 / (nvec * np.pi) * float((w * v).sum()))
-    # as in test_kpm_on_both_layouts
-    assert np.max(np.abs(mu - np.array(ref))) <= (1e-13 if prec == 0 else 2e-5)
+    # as in test_kpm_on_both_layouts; numpy: 9.4e-11 (1.4e-8 in FP32 arithmetic)
+    assert np.max(np.abs(mu - np.array(ref))) <= (1e-13 if prec == 0 else 2e-9)
+
+
+@pytest.mark.parametrize("grid,nvec", [((20, 20, 20), 1), ((7, 9, 5), 4)])
+def test_kpm_fp32_rounds_once_a_step(lib, grid, nvec):
+    """Two moments per product keep FP32 vectors' accuracy only with the row
+    sums and the recurrence in FP64.  Bound: four times the error that numpy
+    finds for that form on the same vectors; the same form in FP32 arithmetic
+    throughout is beyond it."""
+    print("\n[gpu case] KPM accuracy in FP32, %dx%dx%d, %d vectors" % (*grid, nvec), flush=True)
+    sp = pytest.importorskip("scipy.sparse")
+    ia, ja, a = driver.laplacian3d(*grid)
+    n, Mdeg, f = len(ia) - 1, 200, np.float32
+    A = sp.csr_matrix((a, ja, ia), shape=(n, n))
+    libc = C.CDLL(None)
+    libc.srand(7)
+    t = 2147483647.0 / 2
+    v = (np.array([libc.rand() for _ in range(n * nvec)], float).reshape(nvec, n).T - t) / t
+    v /= np.linalg.norm(v, axis=0)
+
+    def scaled(dots):
+        return np.array([2.0 / (nvec * np.pi) * float(np.sum(d)) for d in dots])
+
+    u, um, dots = v, 0.0, []
+    for k in range(Mdeg):
+        um, u = u, (A @ u - 6.0 * u) * ((2.0 if k else 1.0) / 6.0) - um
+        dots.append((u * v).sum(0))
+    ref = scaled(dots)
+
+    def two_moments(arith):
+        B, ctr = A.astype(arith), arith(6.0)
+        U, um = [v.astype(f)], np.zeros((n, nvec), f)
+        for k in range(Mdeg // 2):
+            x = U[-1].astype(arith)
+            w = (B @ x - ctr * x) * arith((2.0 if k else 1.0) / 6.0) - um.astype(arith)
+            um = U[-1]
+            U.append(w.astype(f))
+        D = [x.astype(float) for x in U]
+        vv, d1 = (D[0] * D[0]).sum(0), (D[1] * D[0]).sum(0)
+        dots = [d1 / vv]
+        for k in range(2, Mdeg + 1):
+            j = k // 2
+            dots.append(((2 * (D[j] * D[j]).sum(0) - vv) if k % 2 == 0
+                         else (2 * (D[j + 1] * D[j]).sum(0) - d1)) / vv)
+        return np.max(np.abs(scaled(dots) - ref))
+
+    bound = 4 * two_moments(np.float64)
+    assert two_moments(f) > bound
+    M = driver.Matrix(lib, ia, ja, a)
+    try:
+        inst = driver.Instance(lib, M, prec=1)
+        try:
+            lib.pEVSL_RandSeed(7)
+            rc, mu, _ = inst.kpmdos(Mdeg, 0, nvec, [3.0, 5.0, 0.0, 12.0])
+        finally:
+            inst.close()
+    finally:
+        M.free()
+    assert rc == 0
+    assert np.max(np.abs(mu[1:] - ref)) <= bound
 
 
 def not_symmetric(which):
@@ -448,8 +509,8 @@ def test_kpm_by_diagonal_count(lib, count, prec):
     finally:
         M.free()
     assert rc == 0
-    # as in test_kpm_on_both_layouts
-    assert np.max(np.abs(mu - np.array(ref))) <= (1e-13 if prec == 0 else 2e-5)
+    # as in test_kpm_on_both_layouts (numpy: at most 1.6e-9)
+    assert np.max(np.abs(mu - np.array(ref))) <= (1e-13 if prec == 0 else 5e-9)
 
 
 # kernel of a filter of degree 70 in FP64: several degrees per launch on chains
