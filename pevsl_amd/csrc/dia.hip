@@ -85,11 +85,13 @@ k_dia_spmv(int n, DiaArg<double, UC> d, const DiaMask<UC> *__restrict__ mask,
 // vector passes (vk, vkm1, vkp1, and y every third degree) and, below about
 // 1e5 rows, by the launch and one trip of independent loads.  Microseconds per
 // degree of a whole filter call, CSR-stream kernel -> this kernel:
-//   100^3 Laplacian, FP64  19.96 -> 8.36 (30 MB: 3.6 TB/s)   FP32 15.8 -> 5.1
-//   113x97x83 with a potential, FP32  15.3 -> 5.0
-//   60^3, FP64  6.6 -> 3.8      20^3, FP64  5.4 -> 2.7
-// Two and four rows per thread were no faster at 1e6 rows (8.29 and 8.93) and
-// slower below (60^3: 4.1 and 4.6): one row gives the most waves.
+//   100^3 Laplacian, FP64  19.96 -> 7.85 (30 MB: 3.8 TB/s)   FP32 15.8 -> 5.3
+//   113x97x83 with a potential, FP64 7.7   FP32  15.3 -> 5.3
+//   60^3, FP64  6.6 -> 4.5
+// of which a launch of its own (HIP events, back to back) takes FP64 7.8 and
+// FP32 4.7 at 100^3, 3.7 and 2.75 at 60^3, 2.6-3.0 below.  With 8 slots for the
+// 7 diagonals, 100^3 FP64: one, two and four rows per thread 8.36, 8.29 and
+// 8.93, 60^3 3.8, 4.1 and 4.6: one row gives the most waves.
 template <typename T, int UC>
 __global__ void __launch_bounds__(kThreads)
 k_cheb_dia(int n, DiaArg<T, UC> d, const DiaMask<UC> *__restrict__ mask,
@@ -125,15 +127,16 @@ struct MuArg {
 // overlap of two windows are computed by both.
 //
 // For grids and chains whose degree takes less than the launch around it:
-// k_cheb_dia needs 2.7-4 us a degree at any size below 1e5 rows (launch, one
-// trip to memory).  Bound by LDS reads and barriers inside, by the overlap of
-// the windows where the band is wide.  FP64, microseconds per degree, a launch
-// per degree -> best s:
-//   chain 64,000 rows 3.8 -> 0.46 (s = 32)   1e6 rows 6.6 -> 1.3 (s = 32)
-//   12^3 3.7 -> 1.06 (s = 12)   20^3 3.0-4.1 -> 1.89 (s = 5), FP32 1.86
-//   60^2 3.8 -> 0.75 (s = 8)    250^2 3.7 -> 1.65 (s = 7)  400^2 3.8 -> 2.7
-// (with a select per absent diagonal instead of the zeros below: 20^3 2.4,
-// 250^2 2.1)
+// k_cheb_dia needs 2.6-3.0 us a degree at any size below 1e5 rows (launch, one
+// trip to memory), up to 4 where the host launches no faster.  Bound by LDS
+// reads and barriers inside, by the overlap of the windows where the band is
+// wide.  FP64, microseconds per degree, launches of one degree back to back ->
+// this kernel in a whole filter call at the plan's s:
+//   chain 64,000 rows 2.9 -> 0.34 (s = 32)   1e6 rows 5.8 -> 1.15 (s = 32)
+//   12^3 2.8 -> 0.96 (s = 10)   20^3 2.9 -> 1.72 (s = 5), FP32 1.60
+//   60^2 2.9 -> 0.62 (s = 16)   250^2 2.8 -> 1.48 (s = 7)  400^2 2.9 -> 2.55 (4)
+// (with a select per absent diagonal instead of the zeros below, and 8 slots:
+// 20^3 2.4 against 1.95, 250^2 2.1 against 1.8)
 // K rows of the window per thread, blockDim.x apart.
 template <typename T, int UC, int K, bool DV>
 __global__ void __launch_bounds__(1024)
@@ -454,8 +457,11 @@ template void dia_clen_blk<float>(const DevCsr &, int, const float *, const floa
 // k_cheb_multi: a launch costs 4.5 and 0.8e-3 per row of the window it loads; a
 // degree inside it 0.2, and 0.35e-3 (U + 3)/10 per row it steps for U diagonals,
 // for each round of workgroups over the CUs; one launch per degree costs 3.0 +
-// 5.6e-6 n.  The window must fit 64 KiB of LDS, which ends the gain where the
-// band is wide (30^3: 900 rows either side per degree) or the grid large.
+// 5.6e-6 n.  The window must fit kMultiRows, 64 KiB of LDS (of the CU's 160:
+// the kernel packs its neighbours' byte offsets in 16 bits), and as one of
+// contiguous rows it grows by the whole band per degree, which ends the gain
+// where the band is wide (30^3: 900 rows either side per degree) or the grid
+// large.
 MultiPlan dia_multi_plan(const DevCsr &A, int elem, int m) {
   MultiPlan best;
   if (!use_dia(A, elem, 1) || m < 2 || A.n > (1 << 20) || A.dia.ndiag > 8) return best;

@@ -48,7 +48,7 @@ KpmPlan kpm_plan(const DevCsr &A, int elem, int nvec) {
          (!p.dia || p.B < 4 || 4.0 * A.n * p.B * elem <= kResident))
     p.B *= 2;
   const double gbytes = 2.0 * A.n * p.B * elem;
-  p.ng = std::max(1, std::min((nvec + p.B - 1) / p.B, (int)std::min(64.0, kResident / gbytes)));
+  p.ng = std::max(1, std::min((nvec - 1) / p.B + 1, (int)std::min(64.0, kResident / gbytes)));
   return p;
 }
 

@@ -123,8 +123,8 @@ struct KernTimers {
 };
 
 // Highest filter degree a batched FP32 group runs in Clenshaw form; above it
-// the group runs the three-term form (same vector passes with y updated every
-// other degree, smaller rounding error at high degree).
+// the group runs the three-term form (y updated every third degree: 11/3
+// vector passes against four; smaller rounding error at high degree).
 constexpr int kClenMaxDeg = 400;
 
 // Per-instance device context (attached to pevsl_Data.dev).

@@ -8,8 +8,9 @@
 //   * k_cheb_stream : one column, CSR-stream form.  A row block (<= 256 rows,
 //     <= 2048 nonzeros) multiplies its nonzeros with the gathered x values in
 //     coalesced order into LDS, then each thread sums one row sequentially
-//     (the reference's order); a longer row is one block, reduced by all of
-//     its threads.  The default single-slice filter.
+//     (the reference's order), or a wave a row of more than 64 entries; a row
+//     longer than the block is one block, reduced by all of its threads.  The
+//     default single-slice filter.
 //   * (dia.hip) the same steps on matrices with a diagonal layout.
 //   * k_cheb_vec : one column with L lanes per row (tuning alternative).
 //   * k_cheb_blkrow / k_clen_blkrow : B slices as interleaved columns
@@ -22,7 +23,8 @@
 //     steps only, at 4-column granularity).
 //   * k_blk_bal (epilogues EpiCheb / EpiClen) : the same steps
 //     for matrices with uneven rows, parallel over (nonzero, 16-byte piece)
-//     with the products staged in LDS and summed per row in column order.
+//     with the products staged in LDS and summed per row, in column order up
+//     to 64 entries.
 //   * k_cheb_blk : B columns with one lane per (row, column).
 //   * k_kpm_bal : one degree of the KPM recurrence (SRC/kpmdos.c:129-156) for
 //     up to 32 random vectors a group, fused with the per-column dot products
@@ -720,9 +722,11 @@ __global__ void k_blk_colscale(size_t n, int B, const T *__restrict__ v, T *__re
 //            column order and runs the fused epilogue on its piece.
 // Rows beyond kUnevenRow entries are summed by a wave; a row with more nonzeros
 // than a block stages is a block alone and is reduced by the whole workgroup
-// (shuffles, then LDS across waves).  Products are
-// rounded before they are added and staged rows are summed in column order,
-// so those rows round exactly as in the row-per-thread kernels.
+// (shuffles, then LDS across waves).  Products are rounded before they are
+// added.  Rows of up to kUnevenRow entries are summed in column order and round
+// exactly as in the row-per-thread kernels; the order of a longer row's sum
+// depends on the width B (lanes 64/Q entries apart), so a slice of a matrix
+// with such rows may differ in its last bits between blocks of other widths.
 
 // U = NZ / S = 8 products per thread and block: each thread first issues
 // its 8 index and value loads (nontemporal: the matrix streams once per step

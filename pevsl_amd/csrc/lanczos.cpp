@@ -769,6 +769,11 @@ void BatchSolver::enqueue_block(const std::vector<int> &grp, int B, int kind,
 //     a launch then costs much the same at every width (20^3, FP32: 8 0.37, 32
 //     0.09; 48x40x44: 8 0.47, 16 0.34; wider groups run more columns past their
 //     own degree), else 8 (100^3, FP64: 4 4.6, 8 4.1);
+//   A group runs to its highest degree; groups are cut from the slices in order
+//   of degree, and even one slice of degree 400 beside 15 of 40 takes less time
+//   in the wide group than it did in CSR groups of 4 (FP64) and 8 (FP32) (ms,
+//   FP64 / FP32: 2e5-row power law 32.4 -> 27.2 / 28.2 -> 17.4, 20^3 3.1 -> 1.6
+//   / 2.5 -> 1.6, 48x40x44 3.7 -> 2.6 / 2.8 -> 2.2);
 //   row kernels: 8 (FP32) / 4 (FP64), as wider row gathers cost more per column.
 int BatchSolver::group_max() const {
   const int elem = c_.filter_prec == PEVSL_PREC_FP32 ? 4 : 8, kind = block_kind();
